@@ -25,14 +25,15 @@
  * which also lists the work items (expert, chunk of its slots) -> quantize x ->
  * grouped gate+up product with fused SwiGLU over (column tiles x work items) ->
  * quantize h -> grouped down product scaled by the routing weight -> combine.
- * Q4_K experts whose rows fit the LDS run on the matrix cores, 8 to 32 tokens of
- * an expert per work item; the other formats and longer rows use the decode
+ * Q4_K experts run on the matrix cores, up to 64 tokens of an expert per work item from
+ * twelve tokens an expert on (moe_tile_device.h), 8 to 32 below; the other formats and longer rows use the decode
  * GEMV's engine, four tokens per pass over an expert's weights. Both carry the
  * reference's bits for every single-row product. Chunks of 17 to a few dozen tokens
  * over many experts take a form without the sort (gate_up_self_kernel below): four
  * launches, one workgroup row per expert.
  */
 #include "gemv_device.h"
+#include "moe_tile_device.h"
 #include "quantize_device.h"
 
 namespace {
@@ -604,10 +605,30 @@ __global__ void scatter_kernel(const int32_t *__restrict__ idx, int P, int topk,
   tok_slots[rank_in_token(idx, i, topk)] = slot;
 }
 
+/* sigmoid(g) * g with the sigmoid in double on the float-rounded exponential, as the reference:
+ *   en = float(exp(double(-g))), sig = float(1.0 / (1.0 + double(en))).
+ * Both double results are only kept to float, so neither needs the library's last-bit exp and
+ * division (about a hundred double instructions a value; in the products of many tokens they were
+ * half of a workgroup's time outside its loop). exp: 2^k e^r with r = x - k ln 2 in two fused steps,
+ * |r| < 0.35, and the Taylor sum of e^r to r^11 (relative error below 2^-46). Division: the hardware
+ * reciprocal and one cubic step y (1 + e + e^2), e = 1 - d y. Both round to the library forms' float
+ * on all of 150 million inputs compared on the host. Beyond +-200 the exponential is 0 or infinite as a float. */
 __device__ __forceinline__ float silu_ref(float g) {
-  /* sigmoid in double on the float-rounded exponential, as the reference */
-  const float en = (float)exp((double)(-g));
-  const float sig = (float)(1.0 / (1.0 + (double)en));
+  const double x = (double)fminf(fmaxf(-g, -200.f), 200.f);
+  const double kbig = fma(x, 1.4426950408889634, 6755399441055744.0); /* 1.5 * 2^52: k in the low bits */
+  const double k = kbig - 6755399441055744.0;
+  const double r = fma(k, -2.3190468138462996e-17, fma(k, -0.6931471805599453, x));
+  constexpr double C[11] = {1.0 / 3628800, 1.0 / 362880, 1.0 / 40320, 1.0 / 5040, 1.0 / 720, 1.0 / 120,
+                            1.0 / 24,      1.0 / 6,      0.5,         1.0,        1.0};
+  double p = 1.0 / 39916800;
+#pragma unroll
+  for (int i = 0; i < 11; ++i) p = fma(p, r, C[i]);
+  const uint64_t bits = __builtin_bit_cast(uint64_t, p) + (__builtin_bit_cast(uint64_t, kbig) << 52);
+  const float en = (float)__builtin_bit_cast(double, bits);
+  const double d = 1.0 + (double)en;
+  const double y = __builtin_amdgcn_rcp(d);
+  const double e = fma(-d, y, 1.0);
+  const float sig = en == INFINITY ? 0.f : (float)fma(y, fma(e, e, e), y);
   return sig * g;
 }
 
@@ -1351,6 +1372,119 @@ __global__ __launch_bounds__(256, TC <= 8 ? 4 : TC <= 16 ? 2 : 1) void down_mma_
     stage);
 }
 
+/* ---- Many tokens per expert (moe_tile_device.h) -------------------------------------------
+ * An item is up to 64 slots of one expert; 32 or fewer take the one-tile form. The workgroups of an
+ * item follow each other on one XCD (they share the item's rows, and consecutive items of an expert
+ * its weights through the last-level cache). */
+__device__ __forceinline__ bool tile_item(int cols, const int *__restrict__ items, const int *__restrict__ offsets,
+                                          int &col, int &e, int &s0, int &n) {
+  const int id = blockIdx.x, xcd = id & 7, q = id >> 3;
+  const int item = (q / cols) * 8 + xcd;
+  col = q % cols;
+  if (item >= items[0]) return false; /* uniform per workgroup */
+  e = items[2 + 2 * item];
+  s0 = items[3 + 2 * item];
+  n = min(moe_tile::ROWS, offsets[e + 1] - s0);
+  return true;
+}
+
+/* h of 64 columns: wavefronts 0 and 1 form the two gate tiles, 2 and 3 the up tiles; each pair then
+ * exchanges half its sums through LDS, so that all four evaluate the activation. */
+template <int TM>
+__device__ __forceinline__ void gate_up_tile_pass(moe_tile::Lds &l, const QView &xq, int T, int col, int e, int s0, int n,
+                                                  const WView &wg, const WView &wu, int I, float *__restrict__ h,
+                                                  const hipq::MoeEpi &ep) {
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  const int tile = 2 * col + (wave & 1); /* I % 256 == 0 */
+  const bool up = wave >= 2;
+  float v[TM * 16];
+  moe_tile::run<TM>(
+    l, xq, (uint32_t)T, 1,
+    [&](int) { return (up ? wu : wg).qs + (size_t)tile * (size_t)((xq.K >> 8) * hipq::EXPERT_TILE_BYTES); },
+    [&](int, const float(&acc)[TM][16], const float(&accm)[TM][16]) {
+#pragma unroll
+      for (int i = 0; i < TM * 16; ++i) v[i] = acc[i >> 4][i & 15] - accm[i >> 4][i & 15];
+    });
+  constexpr int HALF = TM * 8;
+  float *xch = (float *)l.q[0]; /* [wavefront][HALF][64 lanes] */
+  float *mine = xch + (size_t)wave * HALF * 64 + lane, *theirs = xch + (size_t)(wave ^ 2) * HALF * 64 + lane;
+#pragma unroll
+  for (int i = 0; i < HALF; ++i) mine[i * 64] = up ? v[i] : v[HALF + i];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < HALF; ++i) {
+    const float other = theirs[i * 64];
+    const int k = (up ? HALF : 0) + i, row = moe_tile::out_row(k >> 4, k & 15, lane), c = tile * 32 + (lane & 31);
+    const float own = up ? v[HALF + i] : v[i];
+    if (row < n) h[(size_t)(s0 + row) * I + c] = moe_act(ep, e, I, c, up ? other : own, up ? own : other);
+  }
+}
+__global__ __launch_bounds__(256, 3) void gate_up_tile_kernel(const WView *__restrict__ views, int E_, QView xq, int T,
+                                                              const int *__restrict__ offsets,
+                                                              const int *__restrict__ items,
+                                                              const int *__restrict__ slot_pair, int topk, int I,
+                                                              float *__restrict__ h, hipq::MoeEpi ep) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char xmoe_lds[];
+  moe_tile::Lds &l = *reinterpret_cast<moe_tile::Lds *>(xmoe_lds);
+  int col, e, s0, n;
+  if (!tile_item(I >> 6, items, offsets, col, e, s0, n)) return;
+  const WView wg = views[e], wu = views[E_ + e];
+  if (threadIdx.x < moe_tile::ROWS) l.rows[threadIdx.x] = slot_pair[s0 + min((int)threadIdx.x, n - 1)] / topk;
+  __syncthreads();
+  if (n > 32)
+    gate_up_tile_pass<2>(l, xq, T, col, e, s0, n, wg, wu, I, h, ep);
+  else
+    gate_up_tile_pass<1>(l, xq, T, col, e, s0, n, wg, wu, I, h, ep);
+}
+
+/* contrib of 256 columns, two tiles a wavefront one after the other; the rows of h are quantized (a row of
+ * the activation planes is a slot) */
+template <int TM>
+__device__ __forceinline__ void down_tile_pass(moe_tile::Lds &l, const QView &hq, int P, int col, int e, int s0, int n,
+                                               const WView &wd, const float *wrow, int H, float *__restrict__ contrib,
+                                               const hipq::MoeEpi &ep) {
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  const int tile0 = (col * 4 + wave) * 2; /* H % 256 == 0 */
+  moe_tile::run<TM>(
+    l, hq, (uint32_t)P, 2,
+    [&](int t) { return wd.qs + (size_t)(tile0 + t) * (size_t)((hq.K >> 8) * hipq::EXPERT_TILE_BYTES); },
+    [&](int t, const float(&acc)[TM][16], const float(&accm)[TM][16]) {
+      const int c = (tile0 + t) * 32 + (lane & 31), g4 = 4 * (lane >> 5);
+      const uint32_t off = (uint32_t)(g4 * H + c); /* the rest of an address is uniform */
+#pragma unroll
+      for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int urow = 32 * tm + 8 * (r >> 2) + (r & 3); /* out_row = urow + g4 */
+          float *base = contrib + (size_t)(s0 + urow) * H;
+          if (urow + g4 < n) base[off] = moe_out(ep, e, H, c, acc[tm][r] - accm[tm][r], wrow[urow + g4]);
+        }
+    });
+}
+__global__ __launch_bounds__(256, 3) void down_tile_kernel(const WView *__restrict__ views, int E_, QView hq, int P,
+                                                           const int *__restrict__ offsets,
+                                                           const int *__restrict__ items,
+                                                           const int *__restrict__ slot_pair,
+                                                           const float *__restrict__ wgt, int H,
+                                                           float *__restrict__ contrib, hipq::MoeEpi ep) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char xmoe_lds[];
+  moe_tile::Lds &l = *reinterpret_cast<moe_tile::Lds *>(xmoe_lds);
+  float *wrow = (float *)(xmoe_lds + sizeof(moe_tile::Lds)); /* [ROWS] the routing weights of the item's rows */
+  int col, e, s0, n;
+  if (!tile_item(H >> 8, items, offsets, col, e, s0, n)) return;
+  const WView wd = views[2 * E_ + e];
+  if (threadIdx.x < moe_tile::ROWS) {
+    const int slot = s0 + min((int)threadIdx.x, n - 1);
+    l.rows[threadIdx.x] = slot;
+    wrow[threadIdx.x] = wgt[slot_pair[slot]];
+  }
+  __syncthreads();
+  if (n > 32)
+    down_tile_pass<2>(l, hq, P, col, e, s0, n, wd, wrow, H, contrib, ep);
+  else
+    down_tile_pass<1>(l, hq, P, col, e, s0, n, wd, wrow, H, contrib, ep);
+}
+
 /* ---- The block without a pair sort ------------------------------------------------------
  * For chunks of a few dozen tokens the sort is a launch of its own (4-5 us of a block of 80) and
  * puts three dependent reads (item, offsets, pairs) in front of every workgroup's first weight
@@ -1791,11 +1925,35 @@ int launch_grouped_mma(const hipq::MoeArgs *a, const MoeBufs &b, const WView *vi
   return HIPQ_OK;
 }
 
+int launch_tile_mma(const hipq::MoeArgs *a, const MoeBufs &b, const WView *views, const QAct &xq, const QAct &hq,
+                    hipStream_t s) {
+  const hipq_moe_desc &d = a->desc;
+  const int64_t P = (int64_t)d.tokens * d.topk;
+  const int max_items = (int)((P < d.experts ? P : d.experts) + P / moe_tile::ROWS);
+  const unsigned groups = (unsigned)((max_items + 7) / 8 * 8);
+  hipq::launch_kernel("gate_up_tile_kernel", gate_up_tile_kernel, dim3(groups * (unsigned)(d.intermediate / 64)), dim3(256),
+                      sizeof(moe_tile::Lds), s, views, d.experts, qview(xq), d.tokens, b.offsets, b.items, b.slot_pair,
+                      d.topk, d.intermediate, b.h, a->epi);
+  HIPQ_HIP(hipGetLastError());
+  if (int rc = hipq::launch_quantize_q8_K_rowmma(b.h, P, d.intermediate, d.intermediate, &hq, s)) return rc;
+  hipq::launch_kernel("down_tile_kernel", down_tile_kernel, dim3(groups * (unsigned)(d.hidden / 256)), dim3(256),
+                      sizeof(moe_tile::Lds) + moe_tile::ROWS * sizeof(float), s, views, d.experts, qview(hq), (int)P,
+                      b.offsets, b.items, b.slot_pair, (const float *)b.wgt, d.hidden, b.contrib, a->epi);
+  HIPQ_HIP(hipGetLastError());
+  return HIPQ_OK;
+}
+
 /* Token chunk of the matrix-core expert kernels for P pairs over E experts: the
  * smallest of 8, 16, 32 that holds twice the mean tokens per expert (an expert with
  * more becomes several work items), reduced until the activation rows fit the LDS. */
 int mma_chunk(const hipq_moe_desc &d, int64_t P, int E) {
   const int64_t mean2 = (2 * P + E - 1) / E;
+  /* From twelve tokens an expert on the 64-row tiles are the faster form (us a block, items of 8 to 32 tokens ->
+   * tiles): 2048 / 768 / 128 experts, top 8, with 128 / 200 / 512 / 1000 tokens 92 -> 113 / 140 -> 117 / 243 -> 160 /
+   * 375 -> 221; 1024 / 2048 / 32, top 4, with 64 / 128 / 1000 tokens 59 -> 61 / 89 -> 63 / 250 -> 148. The planes
+   * are addressed with 32 bits. */
+  if (mean2 >= 24 && P * d.intermediate < (int64_t(1) << 32) && (int64_t)d.tokens * d.hidden < (int64_t(1) << 32))
+    return moe_tile::ROWS;
   int tc = mean2 <= 8 ? 8 : mean2 <= 16 ? 16 : 32;
   const int kmax = d.hidden > d.intermediate ? d.hidden : d.intermediate;
   while (tc > 8 && xlds_bytes(tc, kmax) + tc * 256 > XLDS_MAX) tc >>= 1; /* + the paired form's exchange area */
@@ -1957,7 +2115,8 @@ int launch_moe(const MoeArgs *a, void *workspace, size_t workspace_bytes, const 
     rc = launch_self_mma(a, b, views, xq, s);
   } else if (mma) {
     const int tc = chunk;
-    rc = tc == 8    ? launch_grouped_mma<8>(a, b, views, xq, hq, s, one_token)
+    rc = tc == 64   ? launch_tile_mma(a, b, views, xq, hq, s)
+         : tc == 8  ? launch_grouped_mma<8>(a, b, views, xq, hq, s, one_token)
          : tc == 16 ? launch_grouped_mma<16>(a, b, views, xq, hq, s)
                     : launch_grouped_mma<32>(a, b, views, xq, hq, s);
   } else if (dt == HIPQ_Q4_0)

@@ -197,6 +197,36 @@ def test_moe_long_chunk_uses_the_multi_kernel_sort(hipq, cr):
         w.destroy()
 
 
+@pytest.mark.parametrize("h,i", [(256, 768), (1280, 256), (3328, 512)])
+def test_moe_tiles_of_64_rows(hipq, cr, h, i):
+    """Twelve tokens an expert and more: work items of up to 64 rows. Experts with exactly one and two row
+    tiles of 32, one row more than each, a single row and none; one super-block, an odd number, and more than
+    the mins' pass holds at once."""
+    import gpu_util as gu
+    import torch
+    counts = [64, 65, 32, 33, 1, 0, 130]
+    t, e, k = sum(counts), len(counts), 1
+    gate, up, down = _experts(cr, e, i, h, seed=9500)
+    x = synth.normal(9600, (t, h))
+    logits = synth.normal(9601, (t, e))
+    owner = np.repeat(np.arange(e), counts)[np.random.default_rng(3).permutation(t)]
+    logits[np.arange(t), owner] += 20.0
+    ref_y, ref_idx, _ = cr.moe_forward(x, logits, gate, up, down, k)
+    assert np.array_equal(np.bincount(ref_idx.ravel(), minlength=e), counts)
+    wg = [capi.Weight("q4_K", i, h, b) for b in gate]
+    wu = [capi.Weight("q4_K", i, h, b) for b in up]
+    wd = [capi.Weight("q4_K", h, i, b) for b in down]
+    y = torch.full((t, h), float("nan"), device="cuda")
+    for _ in range(2):
+        capi.moe_forward(t, h, i, e, k, wg, wu, wd, gu.dev(x), y, router_logits=gu.dev(logits), stream=gu.stream())
+    torch.cuda.synchronize()
+    got = y.cpu().numpy()
+    assert not np.isnan(got).any()
+    assert gu.rel_err(got, ref_y) <= 2e-6, gu.rel_err(got, ref_y)
+    for w in wg + wu + wd:
+        w.destroy()
+
+
 def test_expert_weights_serve_the_moe_block_only(hipq, cr):
     """Q4_K experts are re-stored for the expert kernels at the first block; a plain
     matmul on such a handle is refused, the block keeps giving the same bits."""
