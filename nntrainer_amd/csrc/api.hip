@@ -14,6 +14,7 @@
  * a gfx950 device hipq_init fails and every other call reports
  * HIPQ_ERR_NOT_INITIALIZED.
  */
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -755,19 +756,60 @@ int matmul_rows(const hipq_weight *w, const float *A, int64_t M, int64_t lda, fl
   return hipq::launch_gemm_rows_q4k(w, &qa, (int)M, (int)mat_rows, C, ldc, s); /* up to two passes of eight rows */
 }
 
+/* Whether a launch of Q4_0 weights of one K takes the six-bit GEMM (gemm_f6.hip; the reference's bits like every
+ * kernel of the format, so the row count only picks the fastest): from 65 rows always; from nine rows of a K that the
+ * few-rows kernel and the int8 GEMM do not take; in between where the few-rows kernel's work, (column tiles) x (passes of
+ * eight rows) x (rounds of 1024 of K, and one), is beyond what measured equal (us a call, few rows / six-bit):
+ * 12288 x 4096 with 16 / 24 / 64 rows 18.6 / 18.6, 25.8 / 18.4, 28.6 / 18.1; 4096 x 4096 with 48 / 64 17.9 / 17.4,
+ * 22.3 / 18.3; 40000 x 2048 with 8 / 12 16.9 / 17.8, 27.0 / 18.6; rows of up to 1024, which cost the six-bit GEMM
+ * little: 3072 x 1024 with 48 / 64 9.5 / 9.2, 9.8 / 9.1, 33000 x 512 with 12 13.4 / 10.2. */
+bool wants_f6(int count, const hipq_weight *const *w, int64_t M) {
+  if (M < 9 || w[0]->dtype != HIPQ_Q4_0) return false;
+  const int64_t K = w[0]->K;
+  if (M > 64 || K % 256) return true;
+  int64_t tiles = 0;
+  for (int i = 0; i < count; ++i) tiles += (w[i]->N + 31) / 32;
+  return tiles * ((M + 7) / 8) * ((K + 1023) / 1024 + 1) > (K <= 1024 ? 1100 : 3900);
+}
+
+/* The six-bit copies of the weights are there, or could be made: a call that may not allocate, a stream that is being
+ * captured into a graph and a full device use the kernels that read the weights as they are stored. */
+bool f6_ready(int count, const hipq_weight *const *w, int64_t M, hipStream_t s, const Scratch &sc) {
+  if (sc.fixed && hipq::qact_f6_bytes(M, w[0]->K) > NOALLOC_SCRATCH_BYTES) return false;
+  for (int i = 0; i < count; ++i) {
+    if (w[i]->gf_base) continue;
+    if (sc.fixed) return false;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cs) != hipSuccess) (void)hipGetLastError();
+    if (cs != hipStreamCaptureStatusNone) return false;
+    if (hipq::ensure_f6(const_cast<hipq_weight *>(w[i]))) return false;
+  }
+  return true;
+}
+
+/* count (1 to 4) weights with their copies, one quantization (unless the last call on the scratch made it) and launch */
+int matmul_f6(int count, const hipq_weight *const *w, const float *A, int64_t M, int64_t lda, float *const *C,
+              const int64_t *ldc, hipStream_t s, const Scratch &sc, bool quantize = true) {
+  void *mem = nullptr;
+  if (int rc = sc.get(hipq::qact_f6_bytes(M, w[0]->K), &mem)) return rc;
+  const QActF6 qa = hipq::qact_f6_carve(mem, M, w[0]->K);
+  if (quantize)
+    if (int rc = hipq::launch_quantize_q8_0_f6(A, M, w[0]->K, lda, &qa, s)) return rc;
+  return hipq::launch_gemm_f6(count, w, &qa, (int)M, C, ldc, s);
+}
+
 /* each_row: every row as a product of its own with M = 1 (the bits of M separate calls): for Q4_0
  * and Q6_K that is what up to 16 rows give anyway; Q4_K drops the 4-row quantizer and the pairwise
  * sums the reference applies to rows it multiplies together. The caller passes at most 16 rows. */
 int matmul_device(hipq_weight_t w, const float *A, int64_t M, int64_t lda, float *C, int64_t ldc,
                   hipStream_t s, const Scratch &sc, bool each_row = false) {
   if (M == 0) return HIPQ_OK;
+  const hipq_weight *one = w;
+  if (wants_f6(1, &one, M) && f6_ready(1, &one, M, s, sc)) return matmul_f6(1, &one, A, M, lda, &C, &ldc, s, sc);
   if (wants_rows(w, M, !sc.fixed)) return matmul_rows(w, A, M, lda, C, ldc, s, 0, sc, each_row);
   if (!each_row && wants_tiled(w, M, !sc.fixed)) return matmul_tiled(w, A, M, lda, C, ldc, s, 0, sc);
   if (M == 1 && hipq::gemv_fuses_quantizer(w, A)) return hipq::launch_gemv_fused(w, A, C, s);
-  {
-    const hipq_weight *one = w;
-    if (hipq::gemm_rows_q40_fuses(1, &one, M, A, lda)) return hipq::launch_gemm_rows_q40_fused(1, &one, A, lda, (int)M, &C, &ldc, s);
-  }
+  if (hipq::gemm_rows_q40_fuses(1, &one, M, A, lda)) return hipq::launch_gemm_rows_q40_fused(1, &one, A, lda, (int)M, &C, &ldc, s);
   const int is_k = w->dtype != HIPQ_Q4_0;
   void *mem = nullptr;
   int rc = sc.get(qact_bytes(is_k, M, w->K), &mem);
@@ -979,6 +1021,7 @@ int hipq_weight_create(int dtype, int layout, int64_t N, int64_t K, const void *
   w->device = g.device;
   w->expert_tiles = 0;
   w->gt_base = nullptr;
+  w->gf_base = nullptr;
   w->gt_qs = w->gt_qh = w->gt_hdr = nullptr;
   w->N = N;
   w->K = K;
@@ -1119,6 +1162,7 @@ int hipq_weight_destroy(hipq_weight_t w) {
     (void)hipDeviceSynchronize();
     (void)hipFree(w->base);
     if (w->gt_base) (void)hipFree(w->gt_base);
+    if (w->gf_base) (void)hipFree(w->gf_base);
     std::lock_guard<std::mutex> lk(g.mu);
     g.live_weights--;
     /* drop the expert tables that name w, and only those: the tables of other layers stay
@@ -1524,7 +1568,8 @@ int hipq_matmul_multi(int count, const hipq_weight_t *w, const float *A, int64_t
         const size_t parts = x->dtype == HIPQ_Q4_K ? hipq::gemm_q4k_split_bytes(x, M) : hipq::gemm_q6k_split_bytes(x, M);
         const size_t tiled = ((qact_tiled_bytes(M, x->K) + 255) & ~(size_t)255) + parts;
         if (tiled > n) n = tiled;
-      }
+      } else if (x->dtype == HIPQ_Q4_0 && M >= 9)
+        n = std::max(n, hipq::qact_f6_bytes(M, x->K));
       if (n > need) need = n;
     }
     void *reserve = nullptr;
@@ -1620,6 +1665,22 @@ int hipq_matmul_multi(int count, const hipq_weight_t *w, const float *A, int64_t
       }
     if (first < 0) continue;
     const int is_k = k != 0;
+    if (k == 0) { /* the six-bit GEMM: one quantization, four weights a launch */
+      const hipq_weight *fw[64];
+      float *fc[64];
+      int64_t fl[64];
+      int nf = 0, members = 0;
+      for (int i = 0; i < count; ++i)
+        if (klass(w[i]) == 0 && ++members <= 64) fw[nf] = w[i], fc[nf] = C[i], fl[nf] = ldc[i], ++nf;
+      const Scratch sc{false, s};
+      if (members <= 64 && wants_f6(std::min(nf, 4), fw, M) && f6_ready(nf, fw, M, s, sc)) {
+        for (int i = 0; i < nf; i += 4) {
+          if ((rc = workspace_unmoved(s, gen))) return rc;
+          if ((rc = matmul_f6(std::min(4, nf - i), fw + i, A, M, lda, fc + i, fl + i, s, sc, i == 0))) return rc;
+        }
+        continue;
+      }
+    }
     if (k == 0) { /* up to four Q4_0 weights and a few rows: one launch that quantizes the rows itself */
       const hipq_weight *fw[4];
       float *fc[4];

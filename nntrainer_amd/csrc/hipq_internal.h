@@ -80,6 +80,12 @@ struct hipq_weight {
    *   gt_hdr [N/32][K/256][64][16 B]: the lane's eight int8 scales, then the fp16 d */
   uint8_t *gt_base;
   const uint8_t *gt_qs, *gt_qh, *gt_hdr;
+  /* Built by the first prefill product of a Q4_0 weight (ensure_f6): the weights as six-bit floats in
+   * the operand order of gemm_f6.hip, per 32 columns and 256 of K (rows padded to that with zeros):
+   *   [6][64][16 B]: lane (column, g) holds sixteen 6-bit codes of each of the eight blocks, values
+   *     16 g .. 16 g + 15, three dwords a block one behind the other, four dwords a piece;
+   *   [32][8] fp16 block scales. */
+  uint8_t *gf_base;
 };
 
 /* Plain-data view of a weight passed to kernels by value. */
@@ -147,7 +153,24 @@ struct QActTiled {
 size_t qact_tiled_bytes(int64_t M, int64_t K);
 QActTiled qact_tiled_carve(void *mem, int64_t M, int64_t K);
 
+/* ------------------------------------------------------------------------- */
+/* Q8_0 activations for the six-bit GEMM (gemm_f6.hip), per 64 rows (padded    */
+/* with zeros) and 256 of K (padded with zeros), one run of bytes:             */
+/*   [row tile 2][block 8]{[64 lanes][16 B], [64 lanes][8 B]}: lane (row, g)   */
+/*       takes 24 bytes, 32 bf6 codes: the first parts of values 16 g ..       */
+/*       16 g + 15 of the block, then their second parts                       */
+/*   [64][8] fp16 block scales                                                 */
+/* ------------------------------------------------------------------------- */
+struct QActF6 {
+  uint8_t *p;
+  int M, K, chunks;
+};
+
 namespace hipq {
+
+constexpr int F6_ROWS = 64;
+constexpr int F6_CHUNK = F6_ROWS * 384 + F6_ROWS * 16; /* bytes of 64 rows and one chunk */
+constexpr int F6_WTILE = 6144 + 512;                   /* bytes of 32 columns and one chunk */
 
 /* error plumbing (api.hip) */
 int fail(int code, const char *fmt, ...);
@@ -206,6 +229,11 @@ int launch_quantize_q8_K_rowmma(const float *A, int64_t M, int64_t K, int64_t ld
 int launch_quantize_q8_K_tiled(const float *A, int64_t M, int64_t K, int64_t lda,
                                int64_t mat_rows, const QActTiled *qa, hipStream_t s);
 
+/* the values of launch_quantize_q8_0 in the form of the six-bit GEMM */
+size_t qact_f6_bytes(int64_t M, int64_t K);
+QActF6 qact_f6_carve(void *mem, int64_t M, int64_t K);
+int launch_quantize_q8_0_f6(const float *A, int64_t M, int64_t K, int64_t lda, const QActF6 *qa, hipStream_t s);
+
 /* gemv.hip ---------------------------------------------------------------- */
 /* C[m][n] for m < M <= 8: one pass over the weights, M activation rows.
  * Rows below pair_rows use the reference GEMM kernel's fp32 order (Q4_K). */
@@ -230,6 +258,10 @@ int launch_gemm(const hipq_weight *w, const QAct *qa, int M, float *C,
 /* up to four Q4_0 weights of one K against the same quantized rows, one launch */
 int launch_gemm_multi(int count, const hipq_weight *const *w, const QAct *qa, int M, float *const *C,
                       const int64_t *ldc, hipStream_t s);
+/* gemm_f6.hip: up to four Q4_0 weights of one K, each with its six-bit copy, one launch */
+int ensure_f6(hipq_weight *w); /* allocates once; synchronous */
+int launch_gemm_f6(int count, const hipq_weight *const *w, const QActF6 *qa, int M, float *const *C, const int64_t *ldc,
+                   hipStream_t s);
 /* gemm_q4k.hip: Q4_K with the sub-block scales folded into two int8 digit planes */
 int launch_gemm_q4k_multi(int count, const hipq_weight *const *w, const QActTiled *qa, int M, float *const *C,
                           const int64_t *ldc, hipStream_t s);

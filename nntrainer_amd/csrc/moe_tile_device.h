@@ -167,7 +167,7 @@ __device__ __forceinline__ void run(Lds &l, const QView &a, uint32_t a_rows, int
 #pragma unroll
     for (int i = 0; i < 4; ++i) W[i] = load_q(0, i);
     hd0 = load_hd(0);
-    asm volatile("s_waitcnt vmcnt(5)\n\ts_barrier" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
     int sb = 0;
     for (; sb + 1 < nsb; sb += 2) {
       super_block(sb, 0, hd0, hd1);

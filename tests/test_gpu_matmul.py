@@ -137,6 +137,29 @@ def test_q4_0_few_rows_on_the_matrix_cores_match_oracle(hipq, cr, m, n, k):
         "%d of %d outputs differ in bits" % ((got.view(np.uint32) != ref.view(np.uint32)).sum(), got.size)
 
 
+@pytest.mark.parametrize("m,n,k", [(65, 33, 32), (96, 128, 256), (97, 130, 544), (129, 1000, 768), (9, 300, 96),
+                                   (31, 260, 1056), (200, 257, 2080), (2100, 1030, 288)])
+def test_q4_0_on_six_bit_operands_matches_oracle(hipq, cr, m, n, k):
+    """Q4_0 through gemm_f6.hip: row counts around the 32-row tile and the quantizer's 64, columns that end inside a
+    tile and inside a workgroup's four, one to nine chunks of 256 of K with the last one whole, one block and three,
+    and a launch of more than 512 workgroups. Activations with every 8-bit value. Same bits as the reference; a second
+    call after another product of the stream's workspace."""
+    import gpu_util as gu
+    blocks = _weights(cr, "q4_0", n, k, seed=1400 + m)
+    a = synth.normal(1401 + k + m, (m, k))
+    ramp = (np.arange(k, dtype=np.float32) % 256 - 127.5) / 127.5
+    a[::7] = ramp * np.abs(a[::7, :1])  # rows whose blocks run through the quantizer's range
+    a[3::11, ::5] = 0.0
+    ref = cr.gemm(cr.oracle(), "q4_0", a, blocks, n)
+    w = capi.Weight("q4_0", n, k, blocks)
+    for rep in range(2):
+        got = gu.gpu_matmul(w, a)
+        assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), \
+            "%d of %d outputs differ in bits" % ((got.view(np.uint32) != ref.view(np.uint32)).sum(), got.size)
+        gu.gpu_matmul(w, synth.normal(rep, (70, k)))
+    w.destroy()
+
+
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("n,k", [(32800, 1024), (33000, 512), (40010, 256), (32768, 768), (50000, 1280)])
 def test_single_row_against_wide_matrices_of_short_rows(hipq, cr, kind, n, k):
