@@ -777,12 +777,13 @@ bool wants_f6(int count, const hipq_weight *const *w, int64_t M) {
 bool f6_ready(int count, const hipq_weight *const *w, int64_t M, hipStream_t s, const Scratch &sc) {
   if (sc.fixed && hipq::qact_f6_bytes(M, w[0]->K) > NOALLOC_SCRATCH_BYTES) return false;
   for (int i = 0; i < count; ++i) {
-    if (w[i]->gf_base) continue;
-    if (sc.fixed) return false;
+    const bool made = __atomic_load_n(&w[i]->gf_base, __ATOMIC_ACQUIRE) != nullptr;
+    if (made && (!w[i]->gf_event || w[i]->gf_stream == s)) continue;
+    if (sc.fixed && !made) return false;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cs) != hipSuccess) (void)hipGetLastError();
     if (cs != hipStreamCaptureStatusNone) return false;
-    if (hipq::ensure_f6(const_cast<hipq_weight *>(w[i]))) return false;
+    if (hipq::ensure_f6(const_cast<hipq_weight *>(w[i]), s)) return false;
   }
   return true;
 }
@@ -1022,6 +1023,8 @@ int hipq_weight_create(int dtype, int layout, int64_t N, int64_t K, const void *
   w->expert_tiles = 0;
   w->gt_base = nullptr;
   w->gf_base = nullptr;
+  w->gf_event = nullptr;
+  w->gf_stream = nullptr;
   w->gt_qs = w->gt_qh = w->gt_hdr = nullptr;
   w->N = N;
   w->K = K;
@@ -1162,6 +1165,7 @@ int hipq_weight_destroy(hipq_weight_t w) {
     (void)hipDeviceSynchronize();
     (void)hipFree(w->base);
     if (w->gt_base) (void)hipFree(w->gt_base);
+    if (w->gf_event) (void)hipEventDestroy(w->gf_event);
     if (w->gf_base) (void)hipFree(w->gf_base);
     std::lock_guard<std::mutex> lk(g.mu);
     g.live_weights--;

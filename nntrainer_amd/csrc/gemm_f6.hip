@@ -263,10 +263,23 @@ __global__ __launch_bounds__(256) void f6_weights_kernel(const uint8_t *__restri
 
 namespace hipq {
 
-int ensure_f6(hipq_weight *w) {
+int ensure_f6(hipq_weight *w, hipStream_t s) {
   static std::mutex mu; /* two threads may run their first prefill product on one weight */
   std::lock_guard<std::mutex> lk(mu);
-  if (w->gf_base) return HIPQ_OK;
+  if (w->gf_base) {
+    if (w->gf_event && s != w->gf_stream) { /* made on another stream a moment ago */
+      const hipError_t q = hipEventQuery(w->gf_event);
+      if (q == hipErrorNotReady) {
+        (void)hipGetLastError();
+        HIPQ_HIP(hipStreamWaitEvent(s, w->gf_event, 0));
+      } else if (q == hipSuccess) {
+        (void)hipEventDestroy(w->gf_event);
+        w->gf_event = nullptr;
+      } else
+        return fail(HIPQ_ERR_RUNTIME, "six-bit copy: %s", hipGetErrorString(q));
+    }
+    return HIPQ_OK;
+  }
   if (w->dtype != HIPQ_Q4_0 || w->expert_tiles)
     return fail(HIPQ_ERR_INVALID_ARGUMENT, "only Q4_0 weights in the plane layout have a six-bit copy");
   const int nb = (int)(w->K / 32), chunks = (nb + 7) / 8;
@@ -275,15 +288,22 @@ int ensure_f6(hipq_weight *w) {
   uint8_t *p = nullptr;
   hipError_t e = hipMalloc((void **)&p, bytes);
   if (e != hipSuccess) return fail(HIPQ_ERR_OUT_OF_MEMORY, "six-bit copy of %zu bytes: %s", bytes, hipGetErrorString(e));
-  launch_kernel("f6_weights_kernel", f6_weights_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, nullptr, w->qs,
-                w->d, (int)w->N, nb, chunks, threads, p);
+  /* on the caller's stream, in front of the product that asked for it: nothing waits. Other streams wait for the
+   * event, until it is seen to have passed. */
+  launch_kernel("f6_weights_kernel", f6_weights_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, w->qs, w->d,
+                (int)w->N, nb, chunks, threads, p);
   e = hipGetLastError();
-  if (e == hipSuccess) e = hipStreamSynchronize(nullptr); /* the caller's stream may be another one */
+  if (e == hipSuccess) e = hipEventCreateWithFlags(&w->gf_event, hipEventDisableTiming);
+  if (e == hipSuccess) e = hipEventRecord(w->gf_event, s);
   if (e != hipSuccess) {
+    (void)hipStreamSynchronize(s);
+    if (w->gf_event) (void)hipEventDestroy(w->gf_event);
+    w->gf_event = nullptr;
     (void)hipFree(p);
     return fail(HIPQ_ERR_RUNTIME, "six-bit copy: %s", hipGetErrorString(e));
   }
-  w->gf_base = p; /* readers test this field */
+  w->gf_stream = s;
+  __atomic_store_n(&w->gf_base, p, __ATOMIC_RELEASE); /* last: readers test this field */
   return HIPQ_OK;
 }
 

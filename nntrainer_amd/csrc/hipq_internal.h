@@ -86,6 +86,8 @@ struct hipq_weight {
    *     16 g .. 16 g + 15, three dwords a block one behind the other, four dwords a piece;
    *   [32][8] fp16 block scales. */
   uint8_t *gf_base;
+  hipEvent_t gf_event;   /* recorded behind the copy on gf_stream, or null once it is known to have passed */
+  hipStream_t gf_stream;
 };
 
 /* Plain-data view of a weight passed to kernels by value. */
@@ -259,7 +261,7 @@ int launch_gemm(const hipq_weight *w, const QAct *qa, int M, float *C,
 int launch_gemm_multi(int count, const hipq_weight *const *w, const QAct *qa, int M, float *const *C,
                       const int64_t *ldc, hipStream_t s);
 /* gemm_f6.hip: up to four Q4_0 weights of one K, each with its six-bit copy, one launch */
-int ensure_f6(hipq_weight *w); /* allocates once; synchronous */
+int ensure_f6(hipq_weight *w, hipStream_t s); /* the copy is there for what is enqueued on s next (allocates once) */
 int launch_gemm_f6(int count, const hipq_weight *const *w, const QActF6 *qa, int M, float *const *C, const int64_t *ldc,
                    hipStream_t s);
 /* gemm_q4k.hip: Q4_K with the sub-block scales folded into two int8 digit planes */
