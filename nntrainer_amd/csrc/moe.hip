@@ -223,6 +223,75 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const float *__restr
   }
 }
 
+/* Many tokens: the same sums on the matrix core. The kernel above reads all of Wr for every four tokens (1000 tokens of
+ * 2048 x 128: 46 us; this one 10.8). Here a workgroup of sixteen
+ * wavefronts takes sixteen tokens and 32 experts, and wavefront p the rows h = 256 j + 16 p + q (q = 0 .. 15) of Wr:
+ * exactly the four chains (one for each q / 4, over j and q % 4) whose sum is partial sum p above. A chain's step over
+ * four rows is one v_mfma_f32_16x16x4_f32, which adds its four products in order, each with one rounding, so every
+ * logit has the bits of the kernel above. Needs H % 256 == 0. */
+constexpr int ROUTER_MANY_T = 16, ROUTER_MANY_E = 32;
+constexpr int ROUTER_XS = 20, ROUTER_WS = 48; /* floats of a staged row of x, of Wr: a step's 64 reads fall into 64 banks */
+constexpr int ROUTER_STAGE = 16 * (ROUTER_XS + ROUTER_WS); /* floats of a wavefront's stage: 16 tokens, 16 rows of Wr */
+__global__ __launch_bounds__(1024) void router_logits_many_kernel(const float *__restrict__ x, const float *__restrict__ wr,
+                                                                  int T, int H, int E, const float *__restrict__ bias,
+                                                                  float *__restrict__ logits) {
+  typedef float v4f __attribute__((ext_vector_type(4)));
+  extern __shared__ __attribute__((aligned(16))) float router_x[]; /* [wavefront 16][ROUTER_STAGE] */
+  const int lane = threadIdx.x & 63, i16 = lane & 15, k = lane >> 4;
+  const int p = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int t0 = blockIdx.y * ROUTER_MANY_T, e0 = blockIdx.x * ROUTER_MANY_E;
+  /* A step's operands are single values out of sixteen rows; they are loaded as whole 64- and 128-byte pieces and turned
+   * through the wavefront's own part of LDS (as loaded dwords they were sixteen lines an instruction: 26 us for 1000
+   * tokens). Columns past the end repeat the last four; they are not stored. */
+  float *sx = router_x + p * ROUTER_STAGE, *sw = sx + 16 * ROUTER_XS;
+  const float *px = x + (size_t)min(t0 + (lane >> 2), T - 1) * H + 16 * p + 4 * (lane & 3);
+  const float *pw = wr + (size_t)(16 * p + (lane >> 3)) * E + min(e0 + 4 * (lane & 7), E - 4);
+  const int nj = H >> 8;
+  v4f acc[4][2] = {}; /* [q / 4][half of the experts] */
+  v4f xv, wv[2];
+  auto load = [&](int j) {
+    xv = *(const v4f *)(px + 256 * j);
+    wv[0] = *(const v4f *)(pw + (size_t)(256 * j) * E);
+    wv[1] = *(const v4f *)(pw + (size_t)(256 * j + 8) * E);
+  };
+  load(0);
+  for (int j = 0; j < nj; ++j) {
+    *(v4f *)(sx + (lane >> 2) * ROUTER_XS + 4 * (lane & 3)) = xv;
+    *(v4f *)(sw + (lane >> 3) * ROUTER_WS + 4 * (lane & 7)) = wv[0];
+    *(v4f *)(sw + (8 + (lane >> 3)) * ROUTER_WS + 4 * (lane & 7)) = wv[1];
+    load(min(j + 1, nj - 1));
+    float a[4], b[4][2];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      a[q] = sx[i16 * ROUTER_XS + 4 * q + k];
+      b[q][0] = sw[(4 * q + k) * ROUTER_WS + i16];
+      b[q][1] = sw[(4 * q + k) * ROUTER_WS + 16 + i16];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int n = 0; n < 2; ++n) acc[q][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q], b[q][n], acc[q][n], 0, 0, 0);
+  }
+  __syncthreads(); /* the stages are free */
+  float *part = router_x; /* [partial sum 16][token][expert] */
+  constexpr int TE = ROUTER_MANY_T * ROUTER_MANY_E;
+#pragma unroll
+  for (int n = 0; n < 2; ++n)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) /* token 4 k + r, expert 16 n + i16 */
+      part[p * TE + (4 * k + r) * ROUTER_MANY_E + 16 * n + i16] = (acc[3][n][r] + acc[2][n][r]) + (acc[1][n][r] + acc[0][n][r]);
+  __syncthreads();
+  if (threadIdx.x < TE) {
+    const int t = t0 + (threadIdx.x >> 5), e = e0 + (threadIdx.x & 31);
+    if (t < T && e < E) {
+      float sum = part[threadIdx.x];
+#pragma unroll
+      for (int q = 1; q < 16; ++q) sum += part[q * TE + threadIdx.x];
+      logits[(size_t)t * E + e] = bias ? sum + bias[e] : sum;
+    }
+  }
+}
+
 /* Routing of token t by one wavefront: softmax, top-k, optional renormalisation, into registers:
  * lane kk < topk ends up with the kk-th choice's expert and weight. */
 template <int MAXV> /* logits per lane: E <= 64 * MAXV */
@@ -408,10 +477,10 @@ __device__ __forceinline__ void route_token(const float *__restrict__ logits, in
 template <int MAXV>
 __global__ __launch_bounds__(256) void route_kernel(const float *__restrict__ logits, int T, int E,
                                                     int topk, int renorm, int32_t *__restrict__ idx,
-                                                    float *__restrict__ wgt) {
+                                                    float *__restrict__ wgt, int *__restrict__ by_expert) {
   const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (t >= T) return; /* uniform per wavefront */
-  route_token<MAXV>(logits, t, E, topk, renorm, idx, wgt);
+  route_token<MAXV>(logits, t, E, topk, renorm, idx, wgt, by_expert);
 }
 
 /* Where the slot of pair i goes in tok_slots: a token's slots in ascending expert
@@ -432,28 +501,17 @@ __device__ __forceinline__ int rank_in_token(const int32_t *idx, int i, int topk
  * Count, scan and scatter of the (token, k) pairs by expert in one workgroup of
  * 1024 threads: the sort of a decode step or a short prefill chunk is a few thousand
  * pairs, and four tiny launches would cost more than the work. E <= 1024. */
-__device__ __forceinline__ void sort_pairs(const int32_t *idx, int P, int E, int topk, int *__restrict__ offsets,
-                                           int *__restrict__ slot_pair, int *__restrict__ tok_slots, int chunk,
-                                           int *__restrict__ items) {
-  __shared__ int cnt[1024];
-  __shared__ int off[1024];
+/* From the experts' pair counts cnt[1024]: the first slot of every expert (off, offsets) and the work items. 1024 threads. */
+__device__ __forceinline__ void pair_offsets(const int *cnt, int *off, int E, int *__restrict__ offsets, int chunk,
+                                             int *__restrict__ items) {
   __shared__ int wsum[16];
   __shared__ int nitems;
   const int t = threadIdx.x;
-  cnt[t] = 0;
   if (t == 0) nitems = 0;
-  __syncthreads();
-  for (int i = t; i < P; i += 1024) atomicAdd(&cnt[idx[i]], 1);
-  __syncthreads();
   /* exclusive scan over the 1024 slots: prefix sums inside each wavefront, then the
    * sixteen wavefront totals */
   const int own = cnt[t];
-  int winc = own;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int v = __shfl_up(winc, d, 64);
-    if ((t & 63) >= d) winc += v;
-  }
+  const int winc = hipq_wave_prefix_sum_i(own);
   if ((t & 63) == 63) wsum[t >> 6] = winc;
   __syncthreads();
   int wbase = 0;
@@ -467,15 +525,10 @@ __device__ __forceinline__ void sort_pairs(const int32_t *idx, int P, int E, int
    * with one atomic (the order of the wavefronts' ranges does not matter). */
   if (chunk > 0) {
     const int nch = t < E ? (own + chunk - 1) / chunk : 0;
-    int incl = nch;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int v = __shfl_up(incl, d, 64);
-      if ((t & 63) >= d) incl += v;
-    }
+    const int incl = hipq_wave_prefix_sum_i(nch);
     int base = 0;
     if ((t & 63) == 63 && incl > 0) base = atomicAdd(&nitems, incl);
-    base = __shfl(base, 63, 64);
+    base = __builtin_amdgcn_readlane(base, 63);
     const int at = base + incl - nch;
     for (int c = 0; c < nch; ++c) {
       items[2 + 2 * (at + c)] = t;
@@ -485,6 +538,19 @@ __device__ __forceinline__ void sort_pairs(const int32_t *idx, int P, int E, int
     if (t == 0) items[0] = nitems;
   }
   off[t] = excl;
+  __syncthreads();
+}
+__device__ __forceinline__ void sort_pairs(const int32_t *idx, int P, int E, int topk, int *__restrict__ offsets,
+                                           int *__restrict__ slot_pair, int *__restrict__ tok_slots, int chunk,
+                                           int *__restrict__ items) {
+  __shared__ int cnt[1024];
+  __shared__ int off[1024];
+  const int t = threadIdx.x;
+  cnt[t] = 0;
+  __syncthreads();
+  for (int i = t; i < P; i += 1024) atomicAdd(&cnt[idx[i]], 1);
+  __syncthreads();
+  pair_offsets(cnt, off, E, offsets, chunk, items);
   cnt[t] = 0;
   __syncthreads();
   for (int i = t; i < P; i += 1024) {
@@ -495,11 +561,46 @@ __device__ __forceinline__ void sort_pairs(const int32_t *idx, int P, int E, int
   }
 }
 
-__global__ __launch_bounds__(1024) void sort_pairs_kernel(const int32_t *__restrict__ idx, int P, int E, int topk,
+/* Up to 16384 pairs behind the routing launch, which has written every token's pairs in ascending expert id to tok_slots.
+ * All of a thread's pairs are loaded before the first is counted, the count hands out the pair's place in its expert, and
+ * the slots of the pairs pass through LDS to the places tok_slots names (in place). 8000 pairs: 15.5 -> 7 us (a second pass
+ * over idx with its own atomics, and topk reads a pair for its rank, one round trip after the other). */
+constexpr int SORT_MANY = 16384;
+__global__ __launch_bounds__(1024) void sort_pairs_kernel(const int32_t *__restrict__ idx, int P, int E,
                                                           int *__restrict__ offsets, int *__restrict__ slot_pair,
-                                                          int *__restrict__ tok_slots, int chunk,
-                                                          int *__restrict__ items) {
-  sort_pairs(idx, P, E, topk, offsets, slot_pair, tok_slots, chunk, items);
+                                                          int *tok_slots, int chunk, int *__restrict__ items) {
+  constexpr int NP = SORT_MANY / 1024;
+  __shared__ int cnt[1024];
+  __shared__ int off[1024];
+  __shared__ uint16_t slot_of[SORT_MANY];
+  const int t = threadIdx.x;
+  int e[NP], place[NP], pair[NP];
+#pragma unroll
+  for (int u = 0; u < NP; ++u)
+    if (1024 * u < P) { /* uniform */
+      e[u] = idx[min(1024 * u + t, P - 1)];
+      pair[u] = tok_slots[min(1024 * u + t, P - 1)];
+    }
+  cnt[t] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < NP; ++u)
+    if (1024 * u < P && 1024 * u + t < P) place[u] = atomicAdd(&cnt[e[u]], 1);
+  __syncthreads();
+  pair_offsets(cnt, off, E, offsets, chunk, items);
+#pragma unroll
+  for (int u = 0; u < NP; ++u) {
+    const int i = 1024 * u + t;
+    if (1024 * u < P && i < P) {
+      const int slot = off[e[u]] + place[u];
+      slot_pair[slot] = i;
+      slot_of[i] = (uint16_t)slot;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < NP; ++u)
+    if (1024 * u < P && 1024 * u + t < P) tok_slots[1024 * u + t] = slot_of[pair[u]];
 }
 
 /* Routing and sort of up to 16 tokens (a decode step) in one launch: a wavefront
@@ -2012,7 +2113,15 @@ int launch_moe(const MoeArgs *a, void *workspace, size_t workspace_bytes, const 
     /* the rows of x of a workgroup's tokens go to LDS: four tokens, or as many as there are or fit 64 KB with the partial sums */
     int tb_n = d.hidden > 0 ? (int)std::min<int64_t>(std::min(ROUTER_TB, T), 15000 / d.hidden) : 0;
     tb_n = tb_n >= 4 ? 4 : tb_n >= 2 ? 2 : tb_n;
-    if ((E & 3) || (d.hidden & 3) || tb_n < 1 || (((uintptr_t)a->router_weight | (uintptr_t)a->x) & 15)) {
+    /* level with the kernel above at 100 to 150 tokens of 32 experts and more (2048 x 128: 100 tokens 77 -> 83 us a block,
+     * 200 106 -> 100, 1000 229 -> 186), at 500 to 1000 of eight */
+    if ((int64_t)T * std::min(E, 32) >= 128 * 32 && d.hidden % 256 == 0 && !(E & 3) && (((uintptr_t)a->router_weight | (uintptr_t)a->x) & 15) == 0) {
+      constexpr size_t lds = 16 * ROUTER_STAGE * sizeof(float);
+      HIPQ_HIP(hipFuncSetAttribute((const void *)router_logits_many_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+      hipq::launch_kernel("router_logits_many_kernel", router_logits_many_kernel,
+                          dim3((E + ROUTER_MANY_E - 1) / ROUTER_MANY_E, (T + ROUTER_MANY_T - 1) / ROUTER_MANY_T), dim3(1024), lds, s,
+                          a->x, a->router_weight, T, d.hidden, E, a->router_bias, b.logits);
+    } else if ((E & 3) || (d.hidden & 3) || tb_n < 1 || (((uintptr_t)a->router_weight | (uintptr_t)a->x) & 15)) {
       hipq::launch_kernel("router_logits_scalar_kernel", router_logits_scalar_kernel, dim3(T), dim3(256), 0, s, a->x,
                           a->router_weight, d.hidden, E, a->router_bias, b.logits);
     } else {
@@ -2036,6 +2145,7 @@ int launch_moe(const MoeArgs *a, void *workspace, size_t workspace_bytes, const 
   b.wgt = wgt;
   b.idx_used = idx;
   const bool self = mma && mma_self(d, chunk); /* no pair sort: the expert kernels find their pairs in idx */
+  const bool one_sort = !self && P <= SORT_MANY && E <= 1024; /* the pairs are sorted by one workgroup */
   /* the router is instantiated for 2, 4 and 16 logits per lane (E <= 128, 256, 1024):
    * a short kernel whose code is mostly fetched cold, so its length is its time.
    * For the matrix-core expert kernels the same launch quantizes x. */
@@ -2084,9 +2194,10 @@ int launch_moe(const MoeArgs *a, void *workspace, size_t workspace_bytes, const 
     auto launch = [&](auto fused, auto plain) {
       if (mma)
         hipq::launch_kernel("fused", fused, dim3(rblocks + qblocks), dim3(256), 0, s, logits, T, E, d.topk, d.renormalize,
-                           idx, wgt, rblocks, xqa, self ? b.tok_slots : (int *)nullptr);
+                           idx, wgt, rblocks, xqa, self || one_sort ? b.tok_slots : (int *)nullptr);
       else
-        hipq::launch_kernel("plain", plain, dim3(rblocks), dim3(256), 0, s, logits, T, E, d.topk, d.renormalize, idx, wgt);
+        hipq::launch_kernel("plain", plain, dim3(rblocks), dim3(256), 0, s, logits, T, E, d.topk, d.renormalize, idx, wgt,
+                            one_sort ? b.tok_slots : (int *)nullptr);
     };
     if (E <= 128) launch(route_quantize_kernel<2>, route_kernel<2>);
     else if (E <= 256) launch(route_quantize_kernel<4>, route_kernel<4>);
@@ -2095,8 +2206,8 @@ int launch_moe(const MoeArgs *a, void *workspace, size_t workspace_bytes, const 
   }
   if ((T <= 16 && E <= 1024) || self || one_token) {
     /* routed and sorted above, or no sort needed */
-  } else if (P <= 16384 && E <= 1024) {
-    hipq::launch_kernel("sort_pairs_kernel", sort_pairs_kernel, dim3(1), dim3(1024), 0, s, idx, P, E, d.topk, b.offsets,
+  } else if (one_sort) {
+    hipq::launch_kernel("sort_pairs_kernel", sort_pairs_kernel, dim3(1), dim3(1024), 0, s, idx, P, E, b.offsets,
                        b.slot_pair, b.tok_slots, chunk, b.items);
   } else {
     hipq::launch_kernel("fill_int_kernel", fill_int_kernel, dim3((E + 255) / 256), dim3(256), 0, s, b.counts, E, 0);

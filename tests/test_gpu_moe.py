@@ -294,6 +294,40 @@ def test_moe_block_replays_from_a_captured_graph(hipq, cr, t):
             w.destroy()
 
 
+@pytest.mark.parametrize("t,h,e", [(130, 256, 36), (145, 768, 128), (700, 512, 8)])
+def test_router_logits_of_many_tokens_are_those_of_few(hipq, t, h, e):
+    """Router weight given, 128 tokens and more: the logits come from another kernel with the same chains. The chosen
+    experts and their weights equal those of calls of eight tokens bit for bit; token and expert counts that end
+    inside a workgroup's sixteen and 32."""
+    import gpu_util as gu
+    import torch
+    k, i = 4, 256
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(11)
+    blocks = torch.empty(capi.weight_nbytes("q4_K", 1, 256) * i * h // 256, dtype=torch.uint8, device="cuda")
+    capi.quantize_weights("q4_K", torch.randn((i, h), generator=gen, device="cuda") * 0.02, i, h, blocks, stream=gu.stream())
+    torch.cuda.synchronize()
+    ws = [[capi.Weight("q4_K", n, kk, blocks, mem=capi.MEM_DEVICE) for _ in range(e)] for n, kk in ((i, h), (i, h), (h, i))]
+    ex = capi.Experts(*ws)
+    x = torch.randn((t, h), generator=gen, device="cuda")
+    wr = torch.randn((h, e), generator=gen, device="cuda") * h ** -0.5
+    out = []
+    for step in (t, 8):
+        y = torch.empty((t, h), device="cuda")
+        idx = torch.zeros((t, k), dtype=torch.int32, device="cuda")
+        wt = torch.empty((t, k), device="cuda")
+        for t0 in range(0, t, step):
+            n = min(step, t - t0)
+            capi.moe_forward(n, h, i, e, k, ex, None, None, x[t0:], y[t0:], router_weight=wr, topk_idx=idx[t0:],
+                             topk_w=wt[t0:], stream=gu.stream())
+        torch.cuda.synchronize()
+        out.append((idx, wt, y))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+    assert torch.equal(out[0][2], out[1][2])
+    for w in sum(ws, []):
+        w.destroy()
+
+
 def test_moe_router_weight_path(hipq, cr):
     """Logits computed on the device from the fp32 router weight."""
     import gpu_util as gu
