@@ -4,6 +4,7 @@ Device buffers are passed as raw addresses (``tensor.data_ptr()``); torch is onl
 the allocator and stream provider of the callers, it is not imported here.
 """
 import ctypes as C
+import importlib.util
 import os
 import subprocess
 
@@ -114,6 +115,7 @@ def lib():
         L.hipq_device_download.argtypes = [vp, vp, C.c_size_t, vp]
         L.hipq_launch_timing_begin.argtypes = [i32]
         L.hipq_launch_timing_end.argtypes = [i32, C.POINTER(i32), C.POINTER(C.c_float), C.POINTER(C.c_char_p)]
+        _bind_native(L)
         _lib = L
     return _lib
 
@@ -220,39 +222,35 @@ def quantize_q8_K(a, m, k, out, variant=Q8K_ROW, lda=None, mem=MEM_DEVICE, strea
     check(lib().hipq_quantize_q8_K(_addr(a), m, k, lda or k, variant, _addr(out), mem, stream))
 
 
-def matmul(w, a, m, c, lda=None, ldc=None, mem=MEM_DEVICE, stream=None):
-    check(lib().hipq_matmul(w.handle, _addr(a), m, lda or w.k, _addr(c), ldc or w.n, mem, stream))
+# The matmul calls are native functions (csrc/native_calls.c): a decode call is a few microseconds, and ctypes would
+# take as long again to marshal its arguments.
+_NATIVE = ("matmul", "matmul_each_row", "matmul_noalloc", "matmul_multi", "mlp_swiglu", "mlp_swiglu_down")
 
 
-def matmul_each_row(w, a, rows, c, lda=None, ldc=None, mem=MEM_DEVICE, stream=None):
-    """`rows` independent one-row products in one call (the bits of `rows` calls of matmul with m = 1)."""
-    check(lib().hipq_matmul_each_row(w.handle, _addr(a), rows, lda or w.k, _addr(c), ldc or w.n, mem, stream))
+def _bind_native(L):
+    """Loads the native functions, hands them the library's entry points and puts them in this module."""
+    path = os.path.join(HERE, "lib", "hipq_native.so")
+    if not os.path.exists(path):
+        raise FileNotFoundError("%s is missing: build it with `make -C %s`" % (path, CSRC))
+    spec = importlib.util.spec_from_file_location("hipq_native", path)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    mod.bind(check, *(C.cast(getattr(L, "hipq_" + n), C.c_void_p).value for n in _NATIVE))
+    for n in _NATIVE:
+        globals()[n] = getattr(mod, n)
 
 
-def matmul_noalloc(w, a, m, c, lda=None, ldc=None, stream=None):
-    """hipq_matmul on device buffers with the quantized activations in the library's
-    fixed scratch array: no device allocation inside the call."""
-    check(lib().hipq_matmul_noalloc(w.handle, _addr(a), m, lda or w.k, _addr(c), ldc or w.n, stream))
+def _before_load(name):
+    def call(*args, **kwargs):
+        lib()
+        return globals()[name](*args, **kwargs)
+    call.__name__ = name
+    return call
 
 
-def matmul_multi(ws, a, m, cs, ldc=None, mem=MEM_DEVICE, stream=None, lda=None):
-    n = len(ws)
-    hs = (C.c_void_p * n)(*[w.handle.value for w in ws])
-    cp = (C.c_void_p * n)(*[_addr(c) for c in cs])
-    ld = (C.c_int64 * n)(*(ldc if ldc is not None else [w.n for w in ws]))
-    check(lib().hipq_matmul_multi(n, hs, _addr(a), m, lda or ws[0].k, cp, ld, mem, stream))
-
-
-def mlp_swiglu(w_act, w_mul, a, m, out, lda=None, ldo=None, mem=MEM_DEVICE, stream=None):
-    """out = swiglu(a . w_act^T, a . w_mul^T): the gated half of a dense MLP in one call."""
-    check(lib().hipq_mlp_swiglu(w_act.handle, w_mul.handle, _addr(a), m, lda or w_act.k, _addr(out),
-                                ldo or w_act.n, mem, stream))
-
-
-def mlp_swiglu_down(w_act, w_mul, w_down, a, m, out, lda=None, ldo=None, mem=MEM_DEVICE, stream=None):
-    """out = swiglu(a . w_act^T, a . w_mul^T) . w_down^T: the gated MLP of a decoder layer in one call."""
-    check(lib().hipq_mlp_swiglu_down(w_act.handle, w_mul.handle, w_down.handle, _addr(a), m, lda or w_act.k,
-                                     _addr(out), ldo or w_down.n, mem, stream))
+for _n in _NATIVE:  # until lib() has loaded the library
+    globals()[_n] = _before_load(_n)
+del _n
 
 
 def quantize_weights(dtype, w, n, k, out, mem=MEM_DEVICE, stream=None):

@@ -94,6 +94,22 @@ def test_no_gpu_means_loud_failure():
     assert e.value.code == -2
 
 
+@pytest.mark.parametrize("name,args,kwargs,error", [
+    ("matmul", (None, 1), {}, TypeError),                              # 'm' and 'c' missing
+    ("matmul", (None, 1, 1, 1), {"rows": 1}, TypeError),               # no such keyword
+    ("matmul", (None, 1, 1, 1), {"m": 1}, TypeError),                  # given twice
+    ("matmul", (None,) + (1,) * 8, {}, TypeError),                     # too many
+    ("matmul", (None, 1, 1, 1), {}, AttributeError),                   # not a weight
+    ("matmul_multi", ([], 1, 1, []), {}, ValueError),                  # no weights
+    ("matmul_multi", (None, 1, 1, None), {}, TypeError),               # not sequences
+    ("mlp_swiglu_down", (None, None, None, 1, 1), {}, TypeError),      # 'out' missing
+])
+def test_native_calls_check_their_arguments(name, args, kwargs, error):
+    capi.lib()
+    with pytest.raises(error):
+        getattr(capi, name)(*args, **kwargs)
+
+
 def test_product_never_imports_the_oracle():
     """The package and the library sources must not reach into oracle/."""
     for base, _, files in os.walk(os.path.join(ROOT, "nntrainer_amd")):
