@@ -86,7 +86,15 @@ __global__ __launch_bounds__(256) void gemv_stream_kernel(WView w, QView qa,
  * into LDS (the arithmetic of the quantizer kernels, so the blocks are the same
  * bits) while its weight loads are in flight, and the engine reads the activations
  * from there. Saves the quantizer's launch, which costs more than the redundant
- * quantization as long as the matrix is small. One chunk only (K <= 4096). */
+ * quantization as long as the matrix is small. One chunk only (K <= 4096).
+ *
+ * Up to some millions of weights a launch is bound by the chain of what waits for what: the arguments, the row,
+ * its quantization, the barrier, the products, the fp32 sums in order. A launch of nothing takes 1.5 us of a
+ * stream's time, these took 4.0 to 4.4. So the row is quantized in one pass, eight or sixteen values a lane (four
+ * values a lane took up to four passes of some hundred dependent instructions), the sums read their records
+ * sixteen blocks ahead (GemvCore::chain_batched), and the arguments are asked for together (args_first). Q4_0
+ * 4096 x 4096 5.95 -> 4.55 us a call; 114 launches of a token through 28 layers of 1024 / 3072 453 -> 384 us of
+ * GPU time; a Q4_K layer of 4096 / 12288 36.3 -> 31.8 us. */
 template <int DT> __host__ __device__ constexpr int fused_act_bytes(int K) {
   /* Q8_0: q [K], meta [K/32] u32; Q8_K: q [K], ql [K/2], qh [K/2], bsum [K/16] i16, d [K/256] f32 */
   return ((DT == HIPQ_Q4_0 ? K + K / 8 : 2 * K + K / 8 + K / 64) + 15) & ~15;
@@ -96,7 +104,6 @@ template <int DT, int T, int G, int NW, int LATE, int FK, int WV = 4, typename S
 __device__ __forceinline__ void gemv_fused_rows(const WView (&wv)[NW], const float *__restrict__ x, int block,
                                                 Store store) {
   static_assert(WV == 4 || (DT != HIPQ_Q4_0 && WV == 12), "wavefronts a workgroup");
-  constexpr int XP = 16 / WV + (16 % WV != 0); /* super-blocks of the row a wavefront quantizes, at most (K <= 4096) */
   typedef GemvCore<DT, T, 1, G, false> E;
   const WView &w = wv[0];
   extern __shared__ __attribute__((aligned(16))) uint32_t gemv_lds[];
@@ -112,17 +119,13 @@ __device__ __forceinline__ void gemv_fused_rows(const WView (&wv)[NW], const flo
 
   /* the row first (it comes from the cache), then the weights: the wait for the row
    * leaves the weight loads in flight. Positions beyond the row re-read its end. */
-  float4 xs[4];
-  if (DT == HIPQ_Q4_0) {
-    const int nb = K >> 5;
+  /* values a lane quantizes; K / V lanes do it (at most 256: K <= 4096) */
+  constexpr int V = DT == HIPQ_Q4_0 && FK && FK <= 2048 ? 8 : 16;
+  float4 xs[V / 4];
+  const int at = min((int)threadIdx.x, K / V - 1); /* the lane's place in the row */
+  const bool mine = (int)threadIdx.x < K / V;
 #pragma unroll
-    for (int p = 0; p < 4; ++p)
-      xs[p] = *(const float4 *)(x + min((int)(threadIdx.x >> 3) + 32 * p, nb - 1) * 32 + (threadIdx.x & 7) * 4);
-  } else {
-    const int nsb = K >> 8;
-#pragma unroll
-    for (int p = 0; p < XP; ++p) xs[p] = *(const float4 *)(x + min(wave + WV * p, nsb - 1) * 256 + lane * 4);
-  }
+  for (int p = 0; p < V / 4; ++p) xs[p] = *(const float4 *)(x + at * V + 4 * p);
   /* LATE 0: the weights are asked for in front of the row's quantization; 1: behind it; 2: the first half of
    * the wavefront's rows in front, the other half behind. A template parameter: chosen at run time, the
    * places' loads end in different registers that are copied where the paths meet, which waits for every
@@ -143,45 +146,35 @@ __device__ __forceinline__ void gemv_fused_rows(const WView (&wv)[NW], const flo
   QView qa;
   qa.K = K;
   qa.q = (const int8_t *)ap;
-  if (DT == HIPQ_Q4_0) {
+  if constexpr (DT == HIPQ_Q4_0) {
     int8_t *q = (int8_t *)ap;
     uint32_t *meta = (uint32_t *)(ap + K);
     qa.meta = meta;
     qa.d = nullptr;
     qa.bsum = nullptr;
     qa.ql = qa.qh = nullptr;
-    const int nb = K >> 5, sub = threadIdx.x & 7;
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      if (32 * p >= nb) break; /* uniform */
-      const int blk = (int)(threadIdx.x >> 3) + 32 * p;
-      uint16_t dh;
-      int qsum;
-      const int packed = hipq_quantize_q8_0_lane(xs[p], dh, qsum);
-      const int bsum = hipq_group_sum_i<8>(qsum);
-      if (blk < nb) {
-        *(int *)(q + blk * 32 + sub * 4) = packed;
-        if (sub == 0) meta[blk] = (uint32_t)dh | ((uint32_t)(bsum & 0xffff) << 16);
-      }
+    uint32_t qv[V / 4];
+    uint16_t dh;
+    int bsum;
+    hipq_quantize_q8_0_values<V>(xs, qv, dh, bsum);
+    if (mine) {
+      if constexpr (V == 8)
+        *(uint2 *)(q + at * V) = make_uint2(qv[0], qv[1]);
+      else
+        *(uint4 *)(q + at * V) = make_uint4(qv[0], qv[1], qv[2], qv[3]);
+      if (at % (32 / V) == 0) meta[at / (32 / V)] = (uint32_t)dh | ((uint32_t)(bsum & 0xffff) << 16);
     }
   } else {
     int8_t *q = (int8_t *)ap;
-    uint16_t *ql = (uint16_t *)(ap + K), *qh = (uint16_t *)(ap + K + (K >> 1));
+    uint8_t *ql = ap + K, *qh = ap + K + (K >> 1);
     int16_t *bsum = (int16_t *)(ap + 2 * K);
     float *d = (float *)(ap + 2 * K + (K >> 3));
     qa.meta = nullptr;
     qa.d = d;
     qa.bsum = bsum;
-    qa.ql = (const uint8_t *)ql;
-    qa.qh = (const uint8_t *)qh;
-    const int nsb = K >> 8;
-#pragma unroll
-    for (int p = 0; p < XP; ++p) {
-      const int sb = wave + WV * p;
-      if (sb >= nsb) break; /* uniform per wavefront */
-      hipq_quantize_q8_K_values < DT == HIPQ_Q4_K ? Q8K_DIGITS : Q8K_BYTES > (xs[p], 0, sb, sb, nsb, 0, q, d, bsum,
-                                                                             nullptr, nullptr, ql, qh);
-    }
+    qa.ql = ql;
+    qa.qh = qh;
+    hipq_quantize_q8_K_values16<DT == HIPQ_Q4_K ? Q8K_DIGITS : Q8K_BYTES>(xs, at, mine, q, d, bsum, ql, qh);
   }
   if constexpr (LATE == 1) {
 #pragma unroll
@@ -208,6 +201,15 @@ __device__ __forceinline__ void gemv_fused_rows(const WView (&wv)[NW], const flo
   if (o[0].valid && row0 + o[0].g < w.N) store(row0 + o[0].g, o);
 }
 
+/* Asks for all of a kernel's arguments at once. One that is loaded where it is first used (the weights' pointers
+ * behind the row's, the output's at the end) adds a round trip of its own to a kernel that is nothing but a chain of
+ * them. */
+template <int DT> __device__ __forceinline__ void args_first(const void *x, const void *C, const WView &w) {
+  const void *scale = DT == HIPQ_Q4_K ? (const void *)w.hdr : w.d;
+  const void *qh = DT == HIPQ_Q6_K ? (const void *)w.qh : x, *sc = DT == HIPQ_Q6_K ? (const void *)w.sc : x;
+  asm volatile("" ::"s"(x), "s"(C), "s"(w.qs), "s"(scale), "s"(qh), "s"(sc), "s"(w.N), "s"(w.K));
+}
+
 template <int DT, int T, int G, int LATE, int FK>
 __device__ __forceinline__ void gemv_fused_body(const WView &w, const float *__restrict__ x,
                                                 float *__restrict__ C, int block) {
@@ -227,6 +229,8 @@ __global__ __launch_bounds__(256) void gemv_fused_swiglu_kernel(WView wact, WVie
                                                                 const float *__restrict__ x,
                                                                 float *__restrict__ out) {
   const WView wv[2] = {wact, wmul};
+  args_first<DT>(x, out, wact);
+  args_first<DT>(x, out, wmul);
   gemv_fused_rows<DT, T, G, 2, LATE, FK>(wv, x, (int)blockIdx.x, [&](int row, const GemvOut(&o)[2]) {
     const float y = o[0].v, z = o[1].v;
     out[row] = (y / (1.f + expf(-y))) * z;
@@ -236,6 +240,7 @@ __global__ __launch_bounds__(256) void gemv_fused_swiglu_kernel(WView wact, WVie
 template <int DT, int T, int G, int LATE, int FK>
 __global__ __launch_bounds__(256) void gemv_fused_kernel(WView w, const float *__restrict__ x,
                                                          float *__restrict__ C) {
+  args_first<DT>(x, C, w);
   gemv_fused_body<DT, T, G, LATE, FK>(w, x, C, (int)blockIdx.x);
 }
 /* The same with WV wavefronts a workgroup: one workgroup a CU quantizes the row once where three of four
@@ -244,6 +249,7 @@ template <int DT, int T, int G, int WV, int LATE, int FK>
 __global__ __launch_bounds__(64 * WV) void gemv_fused_wide_kernel(WView w, const float *__restrict__ x,
                                                                   float *__restrict__ C) {
   const WView wv[1] = {w};
+  args_first<DT>(x, C, w);
   gemv_fused_rows<DT, T, G, 1, LATE, FK, WV>(wv, x, (int)blockIdx.x,
                                          [&](int row, const GemvOut(&o)[1]) { C[row] = o[0].v; });
 }
@@ -259,10 +265,10 @@ struct FusedMulti {
 template <int DT, int T, int G, int LATE, int FK>
 __global__ __launch_bounds__(256) void gemv_fused_multi_kernel(FusedMulti mw, const float *__restrict__ x) {
   const int b = (int)blockIdx.x;
-  int i = 0;
+  int i = 0, first = 0;
 #pragma unroll
-  for (int k = 0; k + 1 < FUSED_MAXW; ++k) i += b >= mw.end[k];
-  const int first = i ? mw.end[i - 1] : 0;
+  for (int k = 0; k + 1 < FUSED_MAXW; ++k)
+    if (b >= mw.end[k]) i = k + 1, first = mw.end[k];
   gemv_fused_body<DT, T, G, LATE, FK>(mw.w[i], x, mw.C[i], b - first);
 }
 

@@ -508,6 +508,35 @@ template <int DT, int T, int R, int G, bool PW, int KC = HIPQ_KCHUNK> struct Gem
     }
     return c;
   }
+  /* s = step(load(b), s) for b = 0 .. n - 1. The records come from LDS in batches of B, the next batch's reads in
+   * flight while this one's steps run: a read takes over a hundred clocks and a step four, and a wavefront that
+   * finishes a decode product has nothing else to do. */
+  template <int B, typename Rec, typename State, typename Load, typename Step>
+  __device__ static __forceinline__ State chain_batched(int n, State s, Load load, Step step) {
+    Rec v[2][B];
+    const int full = n / B;
+    if (full) {
+#pragma unroll
+      for (int j = 0; j < B; ++j) v[0][j] = load(j);
+    }
+    auto batch = [&](int i, Rec(&cur)[B], Rec(&next)[B]) {
+      if (i + 1 < full) {
+#pragma unroll
+        for (int j = 0; j < B; ++j) next[j] = load((i + 1) * B + j);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int j = 0; j < B; ++j) s = step(cur[j], s);
+    };
+    int i = 0;
+    for (; i + 1 < full; i += 2) {
+      batch(i, v[0], v[1]);
+      batch(i + 1, v[1], v[0]);
+    }
+    if (i < full) batch(i, v[0], v[1]);
+    for (int b = full * B; b < n; ++b) s = step(load(b), s);
+    return s;
+  }
   /* phase 2: this lane's fp32 chain over the records of one chunk, reference order */
   __device__ static __forceinline__ void chain(Chain &c, int kc, const uint32_t *lds) {
     const uint32_t *crec = lds + (c.cg * R + c.cr) * PER;
@@ -518,20 +547,13 @@ template <int DT, int T, int R, int G, bool PW, int KC = HIPQ_KCHUNK> struct Gem
     (void)l;
     if (chain) {
       if (DT == HIPQ_Q4_0) {
-        const int nb = kc >> 5;
-#pragma unroll 4
-        for (int b = 0; b < nb; ++b) {
-          const float2 v = *(const float2 *)(crec + 2 * b);
-          acc = fmaf(v.x, v.y, acc);
-        }
+        acc = chain_batched<16, float2>(kc >> 5, acc, [&](int b) { return *(const float2 *)(crec + 2 * b); },
+                                        [](const float2 &v, float s) { return fmaf(v.x, v.y, s); });
       } else if (DT == HIPQ_Q4_K && !PW) {
-        const int nb = kc >> 8;
-#pragma unroll 4
-        for (int b = 0; b < nb; ++b) {
-          const float4 v = *(const float4 *)(crec + 4 * b);
-          acc = fmaf(v.x, v.y, acc);
-          accm = fmaf(v.z, v.w, accm);
-        }
+        const float2 sums = chain_batched<8, float4>(
+          kc >> 8, make_float2(acc, accm), [&](int b) { return *(const float4 *)(crec + 4 * b); },
+          [](const float4 &v, const float2 &s) { return make_float2(fmaf(v.x, v.y, s.x), fmaf(v.z, v.w, s.y)); });
+        acc = sums.x, accm = sums.y;
       } else if (DT == HIPQ_Q4_K) {
         const int nb = kc >> 8;
         for (int b = 0; b < nb; ++b) {
@@ -554,12 +576,10 @@ template <int DT, int T, int R, int G, bool PW, int KC = HIPQ_KCHUNK> struct Gem
           }
         }
       } else {
-        const int nb = kc >> 8;
-#pragma unroll 4
-        for (int b = 0; b < nb; ++b) {
-          const uint32_t *o = crec + b * 9;
-          acc = fmaf(__uint_as_float(o[8]), (float)(int)o[l], acc);
-        }
+        acc = chain_batched<8, float2>(
+          kc >> 8, acc,
+          [&](int b) { return make_float2(__uint_as_float(crec[b * 9 + 8]), __uint_as_float(crec[b * 9 + l])); },
+          [](const float2 &v, float s) { return fmaf(v.x, (float)(int)__float_as_uint(v.y), s); });
       }
     }
     c.acc = acc;

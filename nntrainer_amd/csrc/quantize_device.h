@@ -57,6 +57,34 @@ __device__ __forceinline__ int hipq_quantize_q8_0_lane(const float4 &x, uint16_t
   return pack4(q0, q1, q2, q3);
 }
 
+/* The same with V (8 or 16) consecutive values of the block in the calling lane, the 32 / V lanes of the block
+ * consecutive: the bytes packed in q, the block's scale and sum. For one row quantized by a few wavefronts that wait
+ * for it: what is per block (the reductions, the two divisions) is done by a fourth to an eighth of the lanes, and
+ * no value depends on another's. Rounding by the add of 1.5 * 2^23 leaves the byte in the low bits, which two
+ * permutes a dword gather. */
+template <int V>
+__device__ __forceinline__ void hipq_quantize_q8_0_values(const float4 (&x)[V / 4], uint32_t (&q)[V / 4], uint16_t &dh,
+                                                          int &bsum) {
+  float amax = 0.f;
+#pragma unroll
+  for (int i = 0; i < V / 4; ++i)
+    amax = fmaxf(fmaxf(fmaxf(fabsf(x[i].x), fabsf(x[i].y)), fmaxf(fabsf(x[i].z), fabsf(x[i].w))), amax);
+  amax = hipq_group_max<32 / V>(amax);
+  const float id = amax != 0.0f ? __fdiv_rn(127.f, amax) : 0.0f;
+  auto biased = [&](float v) { return __float_as_uint(__fadd_rn(__fmul_rn(v, id), kRoundMagic)); };
+  int sum = 0;
+#pragma unroll
+  for (int i = 0; i < V / 4; ++i) {
+    q[i] = __builtin_amdgcn_perm(biased(x[i].y), biased(x[i].x), 0x0c0c0400u) |
+           __builtin_amdgcn_perm(biased(x[i].w), biased(x[i].z), 0x04000c0cu);
+    sum = hipq_dot4((int)q[i], 0x01010101, sum);
+  }
+  bsum = hipq_group_sum_i<32 / V>(sum);
+  uint32_t h = hipq_f2h(__fdiv_rn(amax, 127.f));
+  asm volatile("" : "+v"(h)); /* here, beside the rest, and not behind the condition that stores it */
+  dh = (uint16_t)h;
+}
+
 /* output forms of the Q8_K quantizer */
 enum {
   Q8K_PLANES = 0,
@@ -155,6 +183,72 @@ __device__ __forceinline__ void hipq_quantize_q8_K_values(
       qh_out[sb * 64 + lane] = (uint16_t)hi;
     }
   }
+}
+
+/* The row quantizer with sixteen consecutive values of the super-block in the calling lane, the super-block's sixteen
+ * lanes consecutive, for one row quantized by a few wavefronts that wait for it: the reductions stay inside a row of
+ * lanes, the two divisions serve four super-blocks a wavefront, and a 16-value group's sum needs no exchange. MODE
+ * Q8K_DIGITS or Q8K_BYTES; `at` is the lane's place in the row (values 16 at .. 16 at + 15), stored where `store`.
+ *
+ * The scale has the sign of the first value of largest magnitude: that of the largest value or of the smallest,
+ * whichever is larger in magnitude, and only where both are the same has the first to be looked for. No value leaves
+ * -127 .. 127 (|iscale x| <= 127 (1 + 2^-23)), so the low byte of the biased float is the value; where iscale is not
+ * finite that byte is 0, as the plain form's is. */
+template <int MODE>
+__device__ __forceinline__ void hipq_quantize_q8_K_values16(const float4 (&x)[4], int at, bool store,
+                                                            int8_t *__restrict__ q_out, float *__restrict__ d_out,
+                                                            int16_t *__restrict__ bsum_out,
+                                                            uint8_t *__restrict__ ql_out,
+                                                            uint8_t *__restrict__ qh_out) {
+  static_assert(MODE == Q8K_DIGITS || MODE == Q8K_BYTES, "the forms that the GEMV kernels read");
+  const float v[16] = {x[0].x, x[0].y, x[0].z, x[0].w, x[1].x, x[1].y, x[1].z, x[1].w,
+                       x[2].x, x[2].y, x[2].z, x[2].w, x[3].x, x[3].y, x[3].z, x[3].w};
+  float hi = v[0], lo = v[0];
+#pragma unroll
+  for (int i = 1; i < 16; ++i) hi = fmaxf(hi, v[i]), lo = fminf(lo, v[i]);
+  hi = hipq_group_max<16>(hi);
+  lo = -hipq_group_max<16>(-lo);
+  const float amax = fmaxf(fabsf(hi), fabsf(lo));
+  float vmax = fabsf(hi) == amax ? hi : lo;
+  if (__ballot(hi == -lo && amax != 0.f) != 0ull) {
+    int key = 1 << 30; /* place of the first such value, twice, plus its sign */
+#pragma unroll
+    for (int i = 15; i >= 0; --i)
+      if (fabsf(v[i]) == amax) key = (((int)(threadIdx.x & 15) * 16 + i) << 1) | (v[i] < 0.f ? 1 : 0);
+    key = min(key, hipq_dpp_i<HIPQ_DPP_XOR1>(key));
+    key = min(key, hipq_dpp_i<HIPQ_DPP_XOR2>(key));
+    key = min(key, hipq_dpp_i<HIPQ_DPP_HALF_MIRROR>(key));
+    key = min(key, hipq_dpp_i<HIPQ_DPP_MIRROR>(key));
+    vmax = (key & 1) ? -amax : amax;
+  }
+  const float iscale = amax != 0.f ? __fdiv_rn(-127.f, vmax) : 0.f;
+  uint32_t p[4];
+  int sum = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    auto biased = [&](int j) { return __float_as_uint(__fmaf_rn(iscale, v[4 * i + j], kRoundMagic)); };
+    p[i] = __builtin_amdgcn_perm(biased(1), biased(0), 0x0c0c0400u) | __builtin_amdgcn_perm(biased(3), biased(2), 0x04000c0cu);
+    sum = hipq_dot4((int)p[i], 0x01010101, sum);
+  }
+  float d = amax != 0.f ? __fdiv_rn(1.f, iscale) : 0.f;
+  asm volatile("" : "+v"(d)); /* here, beside the rest, and not behind the condition that stores it */
+  if (MODE == Q8K_BYTES) {
+    if (store) *(uint4 *)(q_out + 16 * at) = make_uint4(p[0], p[1], p[2], p[3]);
+  } else {
+    /* 4-bit digits, q = 16 * (qh - 8) + ql, eight values a dword in order */
+    auto gather = [](uint32_t a, uint32_t b) { /* the nibbles of eight bytes 0x0n */
+      return __builtin_amdgcn_perm(b | (b >> 4), a | (a >> 4), 0x06040200u);
+    };
+    uint32_t l[4], h[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) l[i] = p[i] & 0x0f0f0f0fu, h[i] = ((p[i] >> 4) & 0x0f0f0f0fu) ^ 0x08080808u;
+    if (store) {
+      *(uint2 *)(ql_out + 8 * at) = make_uint2(gather(l[0], l[1]), gather(l[2], l[3]));
+      *(uint2 *)(qh_out + 8 * at) = make_uint2(gather(h[0], h[1]), gather(h[2], h[3]));
+      bsum_out[at] = (int16_t)sum;
+    }
+  }
+  if (store && (at & 15) == 0) d_out[at >> 4] = d;
 }
 
 /* The same with the values read from row m of A (rows M and beyond read as zeros). */

@@ -402,6 +402,41 @@ def test_decode_row_quantized_in_the_gemv_equals_the_two_launches(hipq, cr, kind
     assert gu.rel_err(one, ref) <= gu.TOL
 
 
+@pytest.mark.parametrize("kind,k", [("q4_0", 32), ("q4_0", 96), ("q4_0", 1024), ("q4_0", 2048), ("q4_0", 2080),
+                                    ("q4_0", 4096), ("q4_K", 256), ("q4_K", 2304), ("q4_K", 4096), ("q6_K", 256),
+                                    ("q6_K", 4096)])
+def test_decode_row_of_unusual_values_is_quantized_like_the_reference(hipq, cr, kind, k):
+    """The quantization inside the decode GEMV: blocks of zeros, of one value, of tiny and of large values, and
+    largest magnitudes that occur with both signs (the K-formats' scale takes the first one's). Same bits."""
+    import gpu_util as gu
+    n = 200
+    blocks = _weights(cr, kind, n, k, seed=2000 + k)
+    w = capi.Weight(kind, n, k, blocks)
+    blk = 32 if kind == "q4_0" else 256
+    for case in range(6):
+        a = synth.normal(2001 + k + case, (1, k)).reshape(-1, blk)
+        top = np.abs(a).max() * 1.5
+        for i in range(a.shape[0]):
+            lo, hi = (7 * i + 5 * case) % 16, 16 + (11 * i + 3 * case) % (blk - 16)
+            if case == 0:
+                a[i, lo], a[i, hi] = top, -top
+            elif case == 1:
+                a[i, lo], a[i, hi] = -top, top
+            elif case == 2 and i % 2 == 0:
+                a[i] = 0.0
+            elif case == 3:
+                a[i] *= 1e-37 if i % 3 else 1e30
+            elif case == 4:
+                a[i] = a[i, 0]
+            elif case == 5:
+                a[i, lo], a[i, lo ^ 1] = top, -top
+        a = a.reshape(1, k)
+        ref = cr.gemm(cr.oracle(), kind, a, blocks, n)
+        got = gu.gpu_matmul(w, a)
+        assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), (case, got[0, :4], ref[0, :4])
+    w.destroy()
+
+
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("k,ns", [(1024, [2048, 1024, 1024]), (1024, [3072, 3072]), (256, [8, 37, 4, 130]),
                                   (4096, [4096]), (2048, [1000, 6150])])
