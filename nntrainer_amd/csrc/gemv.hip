@@ -119,13 +119,27 @@ __device__ __forceinline__ void gemv_fused_rows(const WView (&wv)[NW], const flo
 
   /* the row first (it comes from the cache), then the weights: the wait for the row
    * leaves the weight loads in flight. Positions beyond the row re-read its end. */
-  /* values a lane quantizes; K / V lanes do it (at most 256: K <= 4096) */
-  constexpr int V = DT == HIPQ_Q4_0 && FK && FK <= 2048 ? 8 : 16;
-  float4 xs[V / 4];
-  const int at = min((int)threadIdx.x, K / V - 1); /* the lane's place in the row */
-  const bool mine = (int)threadIdx.x < K / V;
+  /* V values a lane, K / V lanes. Q8_0: as few values as one pass of the workgroup's lanes allows. Q8_K: sixteen, or
+   * four, a super-block a wavefront, where twelve wavefronts have one each (rows of 1024 with four wavefronts 3.0
+   * against 2.5 us with sixteen values a lane, rows of 2048 with twelve 3.8 against 4.15). */
+  float4 xs[4];
+  int at; /* the lane's place in the row */
+  auto with_v = [&](auto f) {
+    constexpr int lanes = 64 * WV;
+    constexpr bool few = DT == HIPQ_Q4_0 || WV > 4;
+    if (few && K <= 4 * lanes)
+      f(std::integral_constant<int, few ? 4 : 16>{});
+    else if (DT == HIPQ_Q4_0 && K <= 8 * lanes)
+      f(std::integral_constant<int, DT == HIPQ_Q4_0 ? 8 : 16>{});
+    else
+      f(std::integral_constant<int, 16>{});
+  };
+  with_v([&](auto v) {
+    constexpr int V = decltype(v)::value;
+    at = min((int)threadIdx.x, K / V - 1);
 #pragma unroll
-  for (int p = 0; p < V / 4; ++p) xs[p] = *(const float4 *)(x + at * V + 4 * p);
+    for (int p = 0; p < V / 4; ++p) xs[p] = *(const float4 *)(x + at * V + 4 * p);
+  });
   /* LATE 0: the weights are asked for in front of the row's quantization; 1: behind it; 2: the first half of
    * the wavefront's rows in front, the other half behind. A template parameter: chosen at run time, the
    * places' loads end in different registers that are copied where the paths meet, which waits for every
@@ -153,17 +167,25 @@ __device__ __forceinline__ void gemv_fused_rows(const WView (&wv)[NW], const flo
     qa.d = nullptr;
     qa.bsum = nullptr;
     qa.ql = qa.qh = nullptr;
-    uint32_t qv[V / 4];
-    uint16_t dh;
-    int bsum;
-    hipq_quantize_q8_0_values<V>(xs, qv, dh, bsum);
-    if (mine) {
-      if constexpr (V == 8)
-        *(uint2 *)(q + at * V) = make_uint2(qv[0], qv[1]);
-      else
-        *(uint4 *)(q + at * V) = make_uint4(qv[0], qv[1], qv[2], qv[3]);
-      if (at % (32 / V) == 0) meta[at / (32 / V)] = (uint32_t)dh | ((uint32_t)(bsum & 0xffff) << 16);
-    }
+    with_v([&](auto v) {
+      constexpr int V = decltype(v)::value;
+      uint32_t qv[V / 4];
+      float4 xv[V / 4];
+      uint16_t dh;
+      int bsum;
+#pragma unroll
+      for (int p = 0; p < V / 4; ++p) xv[p] = xs[p];
+      hipq_quantize_q8_0_values<V>(xv, qv, dh, bsum);
+      if ((int)threadIdx.x < K / V) {
+        if constexpr (V == 4)
+          *(uint32_t *)(q + at * V) = qv[0];
+        else if constexpr (V == 8)
+          *(uint2 *)(q + at * V) = make_uint2(qv[0], qv[1]);
+        else
+          *(uint4 *)(q + at * V) = make_uint4(qv[0], qv[1], qv[2], qv[3]);
+        if (at % (32 / V) == 0) meta[at / (32 / V)] = (uint32_t)dh | ((uint32_t)(bsum & 0xffff) << 16);
+      }
+    });
   } else {
     int8_t *q = (int8_t *)ap;
     uint8_t *ql = ap + K, *qh = ap + K + (K >> 1);
@@ -174,7 +196,14 @@ __device__ __forceinline__ void gemv_fused_rows(const WView (&wv)[NW], const flo
     qa.bsum = bsum;
     qa.ql = ql;
     qa.qh = qh;
-    hipq_quantize_q8_K_values16<DT == HIPQ_Q4_K ? Q8K_DIGITS : Q8K_BYTES>(xs, at, mine, q, d, bsum, ql, qh);
+    constexpr int FORM = DT == HIPQ_Q4_K ? Q8K_DIGITS : Q8K_BYTES;
+    with_v([&](auto v) {
+      if constexpr (decltype(v)::value == 16)
+        hipq_quantize_q8_K_values16<FORM>(xs, at, (int)threadIdx.x < K / 16, q, d, bsum, ql, qh);
+      else if (wave < (K >> 8)) /* a super-block a wavefront */
+        hipq_quantize_q8_K_values<FORM>(xs[0], 0, wave, wave, K >> 8, 0, q, d, bsum, nullptr, nullptr, (uint16_t *)ql,
+                                        (uint16_t *)qh);
+    });
   }
   if constexpr (LATE == 1) {
 #pragma unroll
@@ -193,7 +222,7 @@ __device__ __forceinline__ void gemv_fused_rows(const WView (&wv)[NW], const flo
     typename E::Chain c = E::begin(arow, 0);
     E::compute(W[i], A, K, lds);
     hipq_wave_lds_sync();
-    E::chain(c, K, lds);
+    E::template chain<FK != 0>(c, K, lds); /* with any length the reads ahead sit behind conditions: slower */
     hipq_wave_lds_sync();
     o[i] = E::finish(c);
   }

@@ -510,16 +510,22 @@ template <int DT, int T, int R, int G, bool PW, int KC = HIPQ_KCHUNK> struct Gem
   }
   /* s = step(load(b), s) for b = 0 .. n - 1. The records come from LDS in batches of B, the next batch's reads in
    * flight while this one's steps run: a read takes over a hundred clocks and a step four, and a wavefront that
-   * finishes a decode product has nothing else to do. */
+   * finishes a small decode product has nothing else to do. With B = 0 a plain loop, which leaves the registers to
+   * more wavefronts: the form where many of them hide each other's reads. */
   template <int B, typename Rec, typename State, typename Load, typename Step>
   __device__ static __forceinline__ State chain_batched(int n, State s, Load load, Step step) {
-    Rec v[2][B];
-    const int full = n / B;
+    if constexpr (B == 0) {
+#pragma unroll 4
+      for (int b = 0; b < n; ++b) s = step(load(b), s);
+      return s;
+    }
+    Rec v[2][B ? B : 1];
+    const int full = n / (B ? B : 1);
     if (full) {
 #pragma unroll
       for (int j = 0; j < B; ++j) v[0][j] = load(j);
     }
-    auto batch = [&](int i, Rec(&cur)[B], Rec(&next)[B]) {
+    auto batch = [&](int i, Rec(&cur)[B ? B : 1], Rec(&next)[B ? B : 1]) {
       if (i + 1 < full) {
 #pragma unroll
         for (int j = 0; j < B; ++j) next[j] = load((i + 1) * B + j);
@@ -537,7 +543,8 @@ template <int DT, int T, int R, int G, bool PW, int KC = HIPQ_KCHUNK> struct Gem
     for (int b = full * B; b < n; ++b) s = step(load(b), s);
     return s;
   }
-  /* phase 2: this lane's fp32 chain over the records of one chunk, reference order */
+  /* phase 2: this lane's fp32 chain over the records of one chunk, reference order. AHEAD: chain_batched's batches */
+  template <bool AHEAD = false>
   __device__ static __forceinline__ void chain(Chain &c, int kc, const uint32_t *lds) {
     const uint32_t *crec = lds + (c.cg * R + c.cr) * PER;
     const bool chain = c.on, pairwise = c.pairwise;
@@ -547,10 +554,10 @@ template <int DT, int T, int R, int G, bool PW, int KC = HIPQ_KCHUNK> struct Gem
     (void)l;
     if (chain) {
       if (DT == HIPQ_Q4_0) {
-        acc = chain_batched<16, float2>(kc >> 5, acc, [&](int b) { return *(const float2 *)(crec + 2 * b); },
+        acc = chain_batched<AHEAD ? 8 : 0, float2>(kc >> 5, acc, [&](int b) { return *(const float2 *)(crec + 2 * b); },
                                         [](const float2 &v, float s) { return fmaf(v.x, v.y, s); });
       } else if (DT == HIPQ_Q4_K && !PW) {
-        const float2 sums = chain_batched<8, float4>(
+        const float2 sums = chain_batched<AHEAD ? 4 : 0, float4>(
           kc >> 8, make_float2(acc, accm), [&](int b) { return *(const float4 *)(crec + 4 * b); },
           [](const float4 &v, const float2 &s) { return make_float2(fmaf(v.x, v.y, s.x), fmaf(v.z, v.w, s.y)); });
         acc = sums.x, accm = sums.y;
@@ -576,7 +583,7 @@ template <int DT, int T, int R, int G, bool PW, int KC = HIPQ_KCHUNK> struct Gem
           }
         }
       } else {
-        acc = chain_batched<8, float2>(
+        acc = chain_batched<AHEAD ? 8 : 0, float2>(
           kc >> 8, acc,
           [&](int b) { return make_float2(__uint_as_float(crec[b * 9 + 8]), __uint_as_float(crec[b * 9 + l])); },
           [](const float2 &v, float s) { return fmaf(v.x, (float)(int)__float_as_uint(v.y), s); });

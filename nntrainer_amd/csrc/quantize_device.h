@@ -57,9 +57,9 @@ __device__ __forceinline__ int hipq_quantize_q8_0_lane(const float4 &x, uint16_t
   return pack4(q0, q1, q2, q3);
 }
 
-/* The same with V (8 or 16) consecutive values of the block in the calling lane, the 32 / V lanes of the block
+/* The same with V (4, 8 or 16) consecutive values of the block in the calling lane, the 32 / V lanes of the block
  * consecutive: the bytes packed in q, the block's scale and sum. For one row quantized by a few wavefronts that wait
- * for it: what is per block (the reductions, the two divisions) is done by a fourth to an eighth of the lanes, and
+ * for it: what is per block (the reductions, the two divisions) is done by fewer lanes, and
  * no value depends on another's. Rounding by the add of 1.5 * 2^23 leaves the byte in the low bits, which two
  * permutes a dword gather. */
 template <int V>
