@@ -799,6 +799,42 @@ int matmul_f6(int count, const hipq_weight *const *w, const float *A, int64_t M,
   return hipq::launch_gemm_f6(count, w, &qa, (int)M, C, ldc, s);
 }
 
+/* Whether launch_gated serves the gated pair of an MLP at M rows: where hipq_matmul_multi sends both products through one
+ * launch of a prefill GEMM, whose epilogue can take the activation as well. */
+bool wants_gated(const hipq_weight *wa, const hipq_weight *wm, int64_t M) {
+  if (wa->dtype != wm->dtype || M < 2) return false;
+  const hipq_weight *ws[2] = {wa, wm};
+  if (wa->dtype == HIPQ_Q4_0) return wants_f6(2, ws, M);
+  return wa->dtype == HIPQ_Q4_K && !hipq::gemm_rows_q4k_fits_multi(2, ws, M) && !wants_rows(wa, M, true) && wants_tiled(wa, M);
+}
+
+/* out = swiglu(A . wa) * (A . wm) for a pair that wants_gated names; *done stays false where the pair's six-bit copies
+ * cannot be had now */
+int launch_gated(const hipq_weight *wa, const hipq_weight *wm, const float *A, int64_t M, int64_t lda, float *out,
+                 int64_t ldo, hipStream_t s, bool *done) {
+  const hipq_weight *ws[2] = {wa, wm};
+  const int64_t K = wa->K;
+  void *mem = nullptr;
+  int rc;
+  *done = false;
+  if (wa->dtype == HIPQ_Q4_0) {
+    const Scratch sc{false, s};
+    if (!f6_ready(2, ws, M, s, sc)) return HIPQ_OK;
+    if ((rc = sc.get(hipq::qact_f6_bytes(M, K), &mem))) return rc;
+    const QActF6 qa = hipq::qact_f6_carve(mem, M, K);
+    if ((rc = hipq::launch_quantize_q8_0_f6(A, M, K, lda, &qa, s))) return rc;
+    *done = true;
+    return hipq::launch_gemm_f6_gated(wa, wm, &qa, (int)M, out, ldo, s);
+  }
+  for (const hipq_weight *x : ws)
+    if (!x->gt_base && (rc = hipq::ensure_gemm_tiles(const_cast<hipq_weight *>(x)))) return rc;
+  if ((rc = workspace(s, qact_tiled_bytes(M, K), &mem))) return rc;
+  const QActTiled qa = qact_tiled_carve(mem, M, K);
+  if ((rc = hipq::launch_quantize_q8_K_tiled(A, M, K, lda, (M / 4) * 4, &qa, s))) return rc;
+  *done = true;
+  return hipq::launch_gemm_q4k_gated(wa, wm, &qa, (int)M, out, ldo, s);
+}
+
 /* each_row: every row as a product of its own with M = 1 (the bits of M separate calls): for Q4_0
  * and Q6_K that is what up to 16 rows give anyway; Q4_K drops the 4-row quantizer and the pairwise
  * sums the reference applies to rows it multiplies together. The caller passes at most 16 rows. */
@@ -1358,6 +1394,10 @@ int hipq_mlp_swiglu(hipq_weight_t w_act, hipq_weight_t w_mul, const float *A, in
   const size_t a_bytes = ((size_t)M * K * 4 + 255) & ~(size_t)255, o_bytes = ((size_t)M * N * 4 + 255) & ~(size_t)255;
   if (mem == HIPQ_MEM_DEVICE && M == 1 && hipq::gemv_fuses_swiglu(w_act, w_mul, A))
     return hipq::launch_gemv_fused_swiglu(w_act, w_mul, A, out, s);
+  if (mem == HIPQ_MEM_DEVICE && wants_gated(w_act, w_mul, M)) {
+    bool done = false;
+    if ((rc = launch_gated(w_act, w_mul, A, M, lda, out, ldo, s, &done)) || done) return rc;
+  }
   /* otherwise: both products from one quantization into the stream's operand buffer, then the
    * activation; host operands cross through the same buffer */
   void *io = nullptr;
@@ -1395,8 +1435,12 @@ int hipq_mlp_swiglu(hipq_weight_t w_act, hipq_weight_t w_mul, const float *A, in
       const int64_t n = steps.rows_at(r0);
       float *const cr[2] = {dY + r0 * N, dZ + r0 * N};
       if (M > 1 && (rc = steps.in(dA, A, lda, K, r0, n))) return rc;
-      if ((rc = hipq_matmul_multi(2, ws, dA + r0 * K, n, K, cr, lds, HIPQ_MEM_DEVICE, stream))) return rc;
-      if ((rc = hipq::launch_swiglu_rows(cr[0], cr[1], n, N, dO + r0 * N, N, s))) return rc;
+      bool done = false;
+      if (wants_gated(w_act, w_mul, n) && (rc = launch_gated(w_act, w_mul, dA + r0 * K, n, K, dO + r0 * N, N, s, &done))) return rc;
+      if (!done) {
+        if ((rc = hipq_matmul_multi(2, ws, dA + r0 * K, n, K, cr, lds, HIPQ_MEM_DEVICE, stream))) return rc;
+        if ((rc = hipq::launch_swiglu_rows(cr[0], cr[1], n, N, dO + r0 * N, N, s))) return rc;
+      }
       if ((rc = steps.out(dO, out, ldo, N, r0, n))) return rc;
       r0 += n;
     }
@@ -1459,9 +1503,14 @@ int hipq_mlp_swiglu_down(hipq_weight_t w_act, hipq_weight_t w_mul, hipq_weight_t
   auto rows = [&](int64_t r0, int64_t n) -> int {
     const float *a = a_dev + r0 * a_ld;
     int rr;
+    bool done = false;
     if (n == 1 && hipq::gemv_fuses_swiglu(w_act, w_mul, a)) {
       if ((rr = hipq::launch_gemv_fused_swiglu(w_act, w_mul, a, dH + r0 * N, s))) return rr;
-    } else {
+      done = true;
+    } else if (wants_gated(w_act, w_mul, n)) {
+      if ((rr = launch_gated(w_act, w_mul, a, n, a_ld, dH + r0 * N, N, s, &done))) return rr;
+    }
+    if (!done) {
       float *const cr[2] = {dY + r0 * N, dZ + r0 * N};
       if ((rr = hipq_matmul_multi(2, ws, a, n, a_ld, cr, lds, HIPQ_MEM_DEVICE, stream))) return rr;
       if ((rr = hipq::launch_swiglu_rows(cr[0], cr[1], n, N, dH + r0 * N, N, s))) return rr;

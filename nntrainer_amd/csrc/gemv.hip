@@ -261,8 +261,7 @@ __global__ __launch_bounds__(256) void gemv_fused_swiglu_kernel(WView wact, WVie
   args_first<DT>(x, out, wact);
   args_first<DT>(x, out, wmul);
   gemv_fused_rows<DT, T, G, 2, LATE, FK>(wv, x, (int)blockIdx.x, [&](int row, const GemvOut(&o)[2]) {
-    const float y = o[0].v, z = o[1].v;
-    out[row] = (y / (1.f + expf(-y))) * z;
+    out[row] = hipq_swiglu(o[0].v, o[1].v);
   });
 }
 
@@ -662,8 +661,7 @@ __global__ __launch_bounds__(256) void swiglu_rows_kernel(const float *__restric
                                                           float *__restrict__ out) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n_total) return;
-  const float yv = y[i], zv = z[i];
-  out[(i / N) * ldo + i % N] = (yv / (1.f + expf(-yv))) * zv;
+  out[(i / N) * ldo + i % N] = hipq_swiglu(y[i], z[i]);
 }
 
 int launch_swiglu_rows(const float *y, const float *z, int64_t M, int64_t N, float *out, int64_t ldo, hipStream_t s) {

@@ -62,6 +62,9 @@ static inline QView qview(const QAct &a) {
   return v;
 }
 
+/* the framework's swiglu in fp32 (fallback_internal.cpp:417-423) */
+__device__ __forceinline__ float hipq_swiglu(float y, float z) { return (y / (1.f + expf(-y))) * z; }
+
 /* Exact dot product of one Q4_K sub-block (32 unsigned 4-bit weights, eight per
  * dword) with 32 int8 activations given as 4-bit digits lo in 0..15 and
  * hi = (q >> 4) + 8 in 0..15:  sum w*q = 16*sum w*hi + sum w*lo - 128*sum w.

@@ -264,6 +264,11 @@ int launch_gemm_multi(int count, const hipq_weight *const *w, const QAct *qa, in
 int ensure_f6(hipq_weight *w, hipStream_t s); /* the copy is there for what is enqueued on s next (allocates once) */
 int launch_gemm_f6(int count, const hipq_weight *const *w, const QActF6 *qa, int M, float *const *C, const int64_t *ldc,
                    hipStream_t s);
+/* out = swiglu(x . wa) * (x . wm) of many rows, one launch (gemm_f6.hip, gemm_q4k.hip) */
+int launch_gemm_f6_gated(const hipq_weight *wa, const hipq_weight *wm, const QActF6 *qa, int M, float *out, int64_t ldo,
+                         hipStream_t s);
+int launch_gemm_q4k_gated(const hipq_weight *wa, const hipq_weight *wm, const QActTiled *qa, int M, float *out, int64_t ldo,
+                          hipStream_t s);
 /* gemm_q4k.hip: Q4_K with the sub-block scales folded into two int8 digit planes */
 int launch_gemm_q4k_multi(int count, const hipq_weight *const *w, const QActTiled *qa, int M, float *const *C,
                           const int64_t *ldc, hipStream_t s);

@@ -174,7 +174,9 @@ def test_gpt_oss_moe_router_bias_and_host_memory(hipq, cr):
 @pytest.mark.parametrize("kind,m,k,n,nd", [("q4_0", 1, 1024, 3072, 1024), ("q4_K", 1, 2048, 768, 2048),
                                            ("q6_K", 3, 512, 256, 512), ("q4_0", 24, 1024, 3072, 1024),
                                            ("q4_K", 5, 1024, 512, 768), ("q4_K", 80, 1024, 1024, 512),
-                                           ("q4_0", 1, 96, 320, 64)])
+                                           ("q4_0", 1, 96, 320, 64),
+                                           # the gated pair in the epilogue of a prefill GEMM
+                                           ("q4_0", 65, 256, 96, 64), ("q4_K", 17, 256, 256, 256)])
 @pytest.mark.parametrize("mem", ["device", "host"])
 def test_mlp_swiglu_down_is_the_two_calls_and_matches_the_oracle(hipq, cr, kind, m, k, n, nd, mem):
     """hipq_mlp_swiglu_down: out = swiglu(a . Wup^T, a . Wgate^T) . Wdown^T, the four layers of
@@ -223,7 +225,11 @@ def test_mlp_swiglu_down_is_the_two_calls_and_matches_the_oracle(hipq, cr, kind,
                                         # one row, the row length a constant of the launch (4096, 3072) or not (2304),
                                         # the weights asked for in front of, behind and around the row's quantization
                                         ("q4_K", 1, 4096, 2200), ("q4_K", 1, 3072, 3000), ("q6_K", 1, 4096, 1100),
-                                        ("q4_0", 1, 4096, 2100), ("q4_K", 1, 2304, 1000), ("q4_K", 1, 2048, 4100)])
+                                        ("q4_0", 1, 4096, 2100), ("q4_K", 1, 2304, 1000), ("q4_K", 1, 2048, 4100),
+                                        # the activation in the epilogue of a prefill GEMM: rows at the edges of its tiles,
+                                        # columns that end inside a workgroup's 64, both tile heights and read-aheads
+                                        ("q4_0", 97, 96, 1056), ("q4_0", 2100, 96, 544), ("q4_K", 65, 512, 100),
+                                        ("q4_K", 2177, 256, 1780)])
 @pytest.mark.parametrize("mem", ["device", "host"])
 def test_mlp_swiglu_matches_oracle(hipq, cr, kind, m, k, n, mem):
     """hipq_mlp_swiglu: out = swiglu(a . Wact^T, a . Wmul^T) (swiglu.cpp:40-62 on the outputs of
