@@ -227,6 +227,19 @@ def quantize_q8_K(a, m, k, out, variant=Q8K_ROW, lda=None, mem=MEM_DEVICE, strea
 _NATIVE = ("matmul", "matmul_each_row", "matmul_noalloc", "matmul_multi", "mlp_swiglu", "mlp_swiglu_down")
 
 
+def _pointer_of(x):
+    """The value ctypes passes for x as a c_void_p argument."""
+    return C.cast(x, C.c_void_p).value or 0
+
+
+def _int_of(x):
+    """The value of a ctypes integer."""
+    x = getattr(x, "_as_parameter_", x)
+    if not isinstance(x, (C.c_int64, C.c_int)):
+        raise TypeError("int expected instead of %s instance" % type(x).__name__)
+    return x.value
+
+
 def _bind_native(L):
     """Loads the native functions, hands them the library's entry points and puts them in this module."""
     path = os.path.join(HERE, "lib", "hipq_native.so")
@@ -235,7 +248,7 @@ def _bind_native(L):
     spec = importlib.util.spec_from_file_location("hipq_native", path)
     mod = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(mod)
-    mod.bind(check, *(C.cast(getattr(L, "hipq_" + n), C.c_void_p).value for n in _NATIVE))
+    mod.bind(check, _pointer_of, _int_of, *(C.cast(getattr(L, "hipq_" + n), C.c_void_p).value for n in _NATIVE))
     for n in _NATIVE:
         globals()[n] = getattr(mod, n)
 

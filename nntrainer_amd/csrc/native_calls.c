@@ -24,9 +24,11 @@ static int (*f_multi)(int, const weight_t *, const float *, int64_t, int64_t, fl
 static int (*f_swiglu)(weight_t, weight_t, const float *, int64_t, int64_t, float *, int64_t, int, void *);
 static int (*f_swiglu_down)(weight_t, weight_t, weight_t, const float *, int64_t, int64_t, float *, int64_t, int, void *);
 static PyObject *raise_status; /* capi.check */
-static PyObject *s_h, *s_value, *s_n, *s_k, *s_data_ptr, *s_ctypes, *s_data;
+static PyObject *pointer_of, *int_of; /* capi._pointer_of, _int_of: the rarer forms of a stream and an integer */
+static PyObject *s_h, *s_handle, *s_value, *s_n, *s_k, *s_data_ptr, *s_ctypes, *s_data;
 
-/* An address as capi._addr takes it: None, an int, a torch tensor, a numpy array. */
+/* The address of a buffer as capi._addr takes it: None, an int, a torch tensor, a numpy array; nothing else has one
+ * (a numpy scalar, bytes and a ctypes object raise AttributeError). */
 static int get_addr(PyObject *x, void **out) {
   if (!x || x == Py_None) {
     *out = NULL;
@@ -40,13 +42,17 @@ static int get_addr(PyObject *x, void **out) {
   if (!p) {
     if (!PyErr_ExceptionMatches(PyExc_AttributeError)) return -1;
     PyErr_Clear();
-    Py_buffer view; /* a C-contiguous array; any other by its .ctypes.data */
-    if (PyObject_CheckBuffer(x) && PyObject_GetBuffer(x, &view, PyBUF_SIMPLE) == 0) {
-      *out = view.buf;
-      PyBuffer_Release(&view);
-      return 0;
+    /* .ctypes.data, as numpy's arrays (and no other buffer) have it; a C-contiguous array's is the start of its buffer,
+     * which is had without the object that .ctypes makes */
+    Py_buffer view;
+    if (PyObject_HasAttr((PyObject *)Py_TYPE(x), s_ctypes) && PyObject_CheckBuffer(x)) {
+      if (PyObject_GetBuffer(x, &view, PyBUF_SIMPLE) == 0) {
+        *out = view.buf;
+        PyBuffer_Release(&view);
+        return 0;
+      }
+      PyErr_Clear();
     }
-    PyErr_Clear();
     PyObject *c = PyObject_GetAttr(x, s_ctypes);
     if (!c) return -1;
     p = PyObject_GetAttr(c, s_data);
@@ -58,8 +64,25 @@ static int get_addr(PyObject *x, void **out) {
   return PyErr_Occurred() ? -1 : 0;
 }
 
+/* A stream: None, an int, or whatever ctypes takes for a c_void_p argument (a c_void_p means its value; an object with
+ * _as_parameter_, torch's streams among them, that parameter). */
+static int get_stream(PyObject *x, void **out) {
+  if (!x || x == Py_None) {
+    *out = NULL;
+    return 0;
+  }
+  PyObject *p = NULL;
+  if (!PyLong_Check(x) && !(x = p = PyObject_CallOneArg(pointer_of, x))) return -1;
+  *out = PyLong_AsVoidPtr(x);
+  Py_XDECREF(p);
+  return PyErr_Occurred() ? -1 : 0;
+}
+
 static int get_int(PyObject *x, int64_t *out) {
+  PyObject *p = NULL;
+  if (!PyIndex_Check(x) && !(x = p = PyObject_CallOneArg(int_of, x))) return -1; /* a ctypes integer */
   *out = PyLong_AsLongLong(x);
+  Py_XDECREF(p);
   return *out == -1 && PyErr_Occurred() ? -1 : 0;
 }
 static int get_attr_int(PyObject *x, PyObject *name, int64_t *out) {
@@ -77,10 +100,17 @@ static int get_stride(PyObject *x, PyObject *w, PyObject *dflt, int64_t *out) {
   }
   return get_attr_int(w, dflt, out);
 }
-/* the handle of a capi.Weight: its _h is a ctypes.c_void_p (null once destroyed) */
+/* the handle of a capi.Weight: its _h is a ctypes.c_void_p (null once destroyed); of another object its `handle` */
 static int get_weight(PyObject *w, weight_t *out) {
   PyObject *h = PyObject_GetAttr(w, s_h);
-  if (!h) return -1;
+  if (!h) {
+    if (!PyErr_ExceptionMatches(PyExc_AttributeError)) return -1;
+    PyErr_Clear();
+    if (!(h = PyObject_GetAttr(w, s_handle))) return -1;
+    const int rc = get_stream(h, out); /* the forms of a pointer argument */
+    Py_DECREF(h);
+    return rc;
+  }
   PyObject *v = PyObject_GetAttr(h, s_value);
   Py_DECREF(h);
   if (!v) return -1;
@@ -146,7 +176,7 @@ static PyObject *one_weight(int each_row, PyObject *const *args, Py_ssize_t narg
   if (ready() || parse(each_row ? "matmul_each_row" : "matmul", each_row ? kw_r : kw_m, 4, args, nargs, names, s, 8) ||
       get_weight(s[0], &w) || get_addr(s[1], &a) || get_int(s[2], &m) || get_addr(s[3], &c) ||
       get_stride(s[4], s[0], s_k, &lda) || get_stride(s[5], s[0], s_n, &ldc) || (s[6] && get_int(s[6], &mem)) ||
-      get_addr(s[7], &stream))
+      get_stream(s[7], &stream))
     return NULL;
   int rc;
   Py_BEGIN_ALLOW_THREADS
@@ -169,7 +199,7 @@ static PyObject *matmul_noalloc(PyObject *self, PyObject *const *args, Py_ssize_
   int64_t m, lda, ldc;
   if (ready() || parse("matmul_noalloc", kw, 4, args, nargs, names, s, 7) || get_weight(s[0], &w) || get_addr(s[1], &a) ||
       get_int(s[2], &m) || get_addr(s[3], &c) || get_stride(s[4], s[0], s_k, &lda) || get_stride(s[5], s[0], s_n, &ldc) ||
-      get_addr(s[6], &stream))
+      get_stream(s[6], &stream))
     return NULL;
   int rc;
   Py_BEGIN_ALLOW_THREADS
@@ -213,7 +243,7 @@ static PyObject *matmul_multi(PyObject *self, PyObject *const *args, Py_ssize_t 
       goto out;
     cp[i] = (float *)p;
   }
-  if (get_addr(s[1], &a) || get_int(s[2], &m) || (s[5] && get_int(s[5], &mem)) || get_addr(s[6], &stream) ||
+  if (get_addr(s[1], &a) || get_int(s[2], &m) || (s[5] && get_int(s[5], &mem)) || get_stream(s[6], &stream) ||
       get_stride(s[7], PySequence_Fast_GET_ITEM(ws, 0), s_k, &lda))
     goto out;
   int rc;
@@ -237,7 +267,7 @@ static PyObject *mlp_swiglu(PyObject *self, PyObject *const *args, Py_ssize_t na
   int64_t m, lda, ldo, mem = MEM_DEVICE;
   if (ready() || parse("mlp_swiglu", kw, 5, args, nargs, names, s, 9) || get_weight(s[0], &wa) || get_weight(s[1], &wm) ||
       get_addr(s[2], &a) || get_int(s[3], &m) || get_addr(s[4], &o) || get_stride(s[5], s[0], s_k, &lda) ||
-      get_stride(s[6], s[0], s_n, &ldo) || (s[7] && get_int(s[7], &mem)) || get_addr(s[8], &stream))
+      get_stride(s[6], s[0], s_n, &ldo) || (s[7] && get_int(s[7], &mem)) || get_stream(s[8], &stream))
     return NULL;
   int rc;
   Py_BEGIN_ALLOW_THREADS
@@ -255,7 +285,7 @@ static PyObject *mlp_swiglu_down(PyObject *self, PyObject *const *args, Py_ssize
   if (ready() || parse("mlp_swiglu_down", kw, 6, args, nargs, names, s, 10) || get_weight(s[0], &wa) ||
       get_weight(s[1], &wm) || get_weight(s[2], &wd) || get_addr(s[3], &a) || get_int(s[4], &m) || get_addr(s[5], &o) ||
       get_stride(s[6], s[0], s_k, &lda) || get_stride(s[7], s[2], s_n, &ldo) || (s[8] && get_int(s[8], &mem)) ||
-      get_addr(s[9], &stream))
+      get_stream(s[9], &stream))
     return NULL;
   int rc;
   Py_BEGIN_ALLOW_THREADS
@@ -264,13 +294,17 @@ static PyObject *mlp_swiglu_down(PyObject *self, PyObject *const *args, Py_ssize
   return finish(rc);
 }
 
-/* bind(check, addresses of the six functions in the order of the pointers above) */
+/* bind(check, pointer_of, int_of, addresses of the six functions in the order of the pointers above) */
 static PyObject *bind(PyObject *self, PyObject *args) {
-  PyObject *check;
+  PyObject *check, *pointer, *integer;
   unsigned long long p[6];
-  if (!PyArg_ParseTuple(args, "OKKKKKK", &check, &p[0], &p[1], &p[2], &p[3], &p[4], &p[5])) return NULL;
+  if (!PyArg_ParseTuple(args, "OOOKKKKKK", &check, &pointer, &integer, &p[0], &p[1], &p[2], &p[3], &p[4], &p[5])) return NULL;
   Py_INCREF(check);
   Py_XSETREF(raise_status, check);
+  Py_INCREF(pointer);
+  Py_XSETREF(pointer_of, pointer);
+  Py_INCREF(integer);
+  Py_XSETREF(int_of, integer);
   *(void **)&f_matmul = (void *)(uintptr_t)p[0];
   *(void **)&f_each_row = (void *)(uintptr_t)p[1];
   *(void **)&f_noalloc = (void *)(uintptr_t)p[2];
@@ -293,18 +327,19 @@ static PyMethodDef methods[] = {
                    "out = swiglu(a . w_act^T, a . w_mul^T): the gated half of a dense MLP in one call."),
   FAST(mlp_swiglu_down, "mlp_swiglu_down(w_act, w_mul, w_down, a, m, out, lda=None, ldo=None, mem=MEM_DEVICE, stream=None)\n\n"
                         "out = swiglu(a . w_act^T, a . w_mul^T) . w_down^T: the gated MLP of a decoder layer in one call."),
-  {"bind", bind, METH_VARARGS, "bind(check, six function addresses)"},
+  {"bind", bind, METH_VARARGS, "bind(check, pointer_of, int_of, six function addresses)"},
   {NULL, NULL, 0, NULL}};
 static struct PyModuleDef module = {PyModuleDef_HEAD_INIT, "hipq_native", "The matmul calls of capi.py.", -1, methods};
 
 PyMODINIT_FUNC PyInit_hipq_native(void) {
   s_h = PyUnicode_InternFromString("_h");
+  s_handle = PyUnicode_InternFromString("handle");
   s_value = PyUnicode_InternFromString("value");
   s_n = PyUnicode_InternFromString("n");
   s_k = PyUnicode_InternFromString("k");
   s_data_ptr = PyUnicode_InternFromString("data_ptr");
   s_ctypes = PyUnicode_InternFromString("ctypes");
   s_data = PyUnicode_InternFromString("data");
-  if (!s_h || !s_value || !s_n || !s_k || !s_data_ptr || !s_ctypes || !s_data) return NULL;
+  if (!s_h || !s_handle || !s_value || !s_n || !s_k || !s_data_ptr || !s_ctypes || !s_data) return NULL;
   return PyModule_Create(&module);
 }

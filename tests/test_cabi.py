@@ -110,6 +110,92 @@ def test_native_calls_check_their_arguments(name, args, kwargs, error):
         getattr(capi, name)(*args, **kwargs)
 
 
+class _Calls:
+    """The native functions bound to a stub that notes what each entry point is given."""
+
+    def __enter__(self):
+        import ctypes as C
+        capi.lib()
+        self.args, self.keep, one = None, [], [C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_int64]
+        kinds = {"matmul": one + [C.c_int, C.c_void_p], "matmul_each_row": one + [C.c_int, C.c_void_p], "matmul_noalloc": one + [C.c_void_p],
+                 "matmul_multi": [C.c_int, C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p, C.c_int, C.c_void_p],
+                 "mlp_swiglu": [C.c_void_p] + one + [C.c_int, C.c_void_p], "mlp_swiglu_down": [C.c_void_p] * 2 + one + [C.c_int, C.c_void_p]}
+
+        def note(*args):
+            self.args = [a or 0 for a in args]
+            return 0
+
+        class Stub:
+            pass
+        for name, types in kinds.items():
+            f = C.CFUNCTYPE(C.c_int, *types)(note)
+            setattr(Stub, "hipq_" + name, f)
+        capi._bind_native(Stub)
+        return self
+
+    def __exit__(self, *exc):
+        capi._bind_native(capi.lib())
+
+
+class _Shape:  # a weight's fields
+    n, k = 8, 32
+
+    def __init__(self, address):
+        import ctypes as C
+        self.handle = C.c_void_p(address)
+
+
+class _Stream:
+    def __init__(self, parameter):
+        self._as_parameter_ = parameter
+
+
+def test_native_calls_take_the_streams_ctypes_takes():
+    import ctypes as C
+    import numpy as np
+    forms = [(None, 0), (0, 0), (0x30, 0x30), (C.c_void_p(0x30), 0x30), (C.c_void_p(None), 0), (_Stream(C.c_void_p(0x40)), 0x40),
+             (_Stream(0x50), 0x50)]
+    w = _Shape(16)
+    with _Calls() as calls:
+        for stream, want in forms:
+            for name, args in (("matmul", (w, 64, 2, 128)), ("matmul_each_row", (w, 64, 2, 128)), ("matmul_noalloc", (w, 64, 2, 128)),
+                               ("matmul_multi", ([w], 64, 2, [128])), ("mlp_swiglu", (w, w, 64, 2, 128)),
+                               ("mlp_swiglu_down", (w, w, w, 64, 2, 128))):
+                getattr(capi, name)(*args, stream=stream)
+                assert calls.args[-1] == want, (name, stream)
+        for stream in (np.int64(0x30), np.zeros(4), object(), 1.5):
+            calls.args = None
+            with pytest.raises((TypeError, C.ArgumentError)):
+                capi.matmul(w, 64, 2, 128, stream=stream)
+            assert calls.args is None
+
+
+def test_native_calls_take_the_buffers_the_binding_takes():
+    import ctypes as C
+    import numpy as np
+    import torch
+    w, a = _Shape(16), np.zeros((4, 64), np.float32)
+    w._h = w.handle  # capi.Weight's own field
+    read_only = np.zeros(64, np.float32)
+    read_only.flags.writeable = False
+    t = torch.zeros(64)
+    forms = [(None, 0), (64, 64), (a, a.ctypes.data), (a[1:, 3:], a.ctypes.data + 4 * 67), (a[:, ::2], a.ctypes.data),
+             (read_only, read_only.ctypes.data), (t[5:], t.data_ptr() + 20), (a.view(np.recarray), a.ctypes.data)]
+    with _Calls() as calls:
+        for x, want in forms:
+            capi.matmul(w, x, 2, x)
+            assert calls.args == [16, want, 2, 32, want, 8, capi.MEM_DEVICE, 0]
+        capi.matmul(w, 64, C.c_int64(2), 128, lda=C.c_int64(48), ldc=np.int64(16), mem=C.c_int(0))
+        assert calls.args == [16, 64, 2, 48, 128, 16, 0, 0]
+        for x in (np.int64(64), np.float32(1), b"0123456789abcdef", bytearray(16), memoryview(b"01234567"), C.c_void_p(64),
+                  (C.c_float * 4)(), object()):
+            for args in ((w, x, 2, 128), (w, 64, 2, x)):
+                calls.args = None
+                with pytest.raises(AttributeError):
+                    capi.matmul(*args)
+                assert calls.args is None, x
+
+
 def test_product_never_imports_the_oracle():
     """The package and the library sources must not reach into oracle/."""
     for base, _, files in os.walk(os.path.join(ROOT, "nntrainer_amd")):
