@@ -4,9 +4,12 @@ Device buffers are passed as raw addresses (``tensor.data_ptr()``); torch is onl
 the allocator and stream provider of the callers, it is not imported here.
 """
 import ctypes as C
+import importlib.machinery
 import importlib.util
 import os
 import subprocess
+import sys
+import warnings
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "lib", "libhipq.so")
@@ -65,7 +68,7 @@ def build(force=False):
     """Compile libhipq.so for gfx950 with hipcc (cross-compiles without a GPU)."""
     if force:
         subprocess.check_call(["make", "-C", CSRC, "clean"], stdout=subprocess.DEVNULL)
-    subprocess.check_call(["make", "-C", CSRC, "-j8"], stdout=subprocess.DEVNULL)
+    subprocess.check_call(["make", "-C", CSRC, "-j8", "PYTHON=" + sys.executable], stdout=subprocess.DEVNULL)
     return LIB_PATH
 
 
@@ -222,9 +225,39 @@ def quantize_q8_K(a, m, k, out, variant=Q8K_ROW, lda=None, mem=MEM_DEVICE, strea
     check(lib().hipq_quantize_q8_K(_addr(a), m, k, lda or k, variant, _addr(out), mem, stream))
 
 
-# The matmul calls are native functions (csrc/native_calls.c): a decode call is a few microseconds, and ctypes would
-# take as long again to marshal its arguments.
-_NATIVE = ("matmul", "matmul_each_row", "matmul_noalloc", "matmul_multi", "mlp_swiglu", "mlp_swiglu_down")
+def matmul(w, a, m, c, lda=None, ldc=None, mem=MEM_DEVICE, stream=None):
+    check(lib().hipq_matmul(w.handle, _addr(a), m, lda or w.k, _addr(c), ldc or w.n, mem, stream))
+
+
+def matmul_each_row(w, a, rows, c, lda=None, ldc=None, mem=MEM_DEVICE, stream=None):
+    """`rows` independent one-row products in one call (the bits of `rows` calls of matmul with m = 1)."""
+    check(lib().hipq_matmul_each_row(w.handle, _addr(a), rows, lda or w.k, _addr(c), ldc or w.n, mem, stream))
+
+
+def matmul_noalloc(w, a, m, c, lda=None, ldc=None, stream=None):
+    """hipq_matmul on device buffers with the quantized activations in the library's
+    fixed scratch array: no device allocation inside the call."""
+    check(lib().hipq_matmul_noalloc(w.handle, _addr(a), m, lda or w.k, _addr(c), ldc or w.n, stream))
+
+
+def matmul_multi(ws, a, m, cs, ldc=None, mem=MEM_DEVICE, stream=None, lda=None):
+    n = len(ws)
+    hs = (C.c_void_p * n)(*[w.handle.value for w in ws])
+    cp = (C.c_void_p * n)(*[_addr(c) for c in cs])
+    ld = (C.c_int64 * n)(*(ldc if ldc is not None else [w.n for w in ws]))
+    check(lib().hipq_matmul_multi(n, hs, _addr(a), m, lda or ws[0].k, cp, ld, mem, stream))
+
+
+def mlp_swiglu(w_act, w_mul, a, m, out, lda=None, ldo=None, mem=MEM_DEVICE, stream=None):
+    """out = swiglu(a . w_act^T, a . w_mul^T): the gated half of a dense MLP in one call."""
+    check(lib().hipq_mlp_swiglu(w_act.handle, w_mul.handle, _addr(a), m, lda or w_act.k, _addr(out),
+                                ldo or w_act.n, mem, stream))
+
+
+def mlp_swiglu_down(w_act, w_mul, w_down, a, m, out, lda=None, ldo=None, mem=MEM_DEVICE, stream=None):
+    """out = swiglu(a . w_act^T, a . w_mul^T) . w_down^T: the gated MLP of a decoder layer in one call."""
+    check(lib().hipq_mlp_swiglu_down(w_act.handle, w_mul.handle, w_down.handle, _addr(a), m, lda or w_act.k,
+                                     _addr(out), ldo or w_down.n, mem, stream))
 
 
 def _pointer_of(x):
@@ -240,30 +273,33 @@ def _int_of(x):
     return x.value
 
 
-def _bind_native(L):
-    """Loads the native functions, hands them the library's entry points and puts them in this module."""
-    path = os.path.join(HERE, "lib", "hipq_native.so")
+# The same calls as native functions (csrc/native_calls.c), where they were built for this interpreter: a decode call is
+# a few microseconds, and ctypes takes as long again to marshal its arguments.
+_FORMS = {f.__name__: f for f in (matmul, matmul_each_row, matmul_noalloc, matmul_multi, mlp_swiglu, mlp_swiglu_down)}
+
+
+def _load_native(path):
     if not os.path.exists(path):
-        raise FileNotFoundError("%s is missing: build it with `make -C %s`" % (path, CSRC))
+        return None
     spec = importlib.util.spec_from_file_location("hipq_native", path)
     mod = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(mod)
-    mod.bind(check, _pointer_of, _int_of, *(C.cast(getattr(L, "hipq_" + n), C.c_void_p).value for n in _NATIVE))
-    for n in _NATIVE:
-        globals()[n] = getattr(mod, n)
+    mod.setup(lib, check, _pointer_of, _int_of)
+    return mod
 
 
-def _before_load(name):
-    def call(*args, **kwargs):
-        lib()
-        return globals()[name](*args, **kwargs)
-    call.__name__ = name
-    return call
+_native = _load_native(os.path.join(HERE, "lib", "hipq_native" + importlib.machinery.EXTENSION_SUFFIXES[0]))
+if _native:
+    globals().update((_n, getattr(_native, _n)) for _n in _FORMS)
 
 
-for _n in _NATIVE:  # until lib() has loaded the library
-    globals()[_n] = _before_load(_n)
-del _n
+def _bind_native(L):
+    """Hands the native functions the library's entry points."""
+    if _native:
+        _native.bind(*(C.cast(getattr(L, "hipq_" + n), C.c_void_p).value for n in _FORMS))
+    else:
+        warnings.warn("the native matmul calls are not built for this interpreter (`make -C %s PYTHON=%s`): each call "
+                      "takes 2 to 5 us longer through ctypes" % (CSRC, sys.executable), RuntimeWarning)
 
 
 def quantize_weights(dtype, w, n, k, out, mem=MEM_DEVICE, stream=None):

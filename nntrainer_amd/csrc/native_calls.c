@@ -7,23 +7,26 @@
  * a call spent 2.0 us (one weight) to 5.4 us (three weights: three arrays of handles, addresses and strides)
  * on marshalling, more than the library's own work for a launch, and the stream ran dry: a token through the
  * 28 layers of a 1024-wide decoder took 450 to 520 us for 415 us of kernels. Here the same calls take 0.3 to
- * 0.6 us. Arguments, defaults and errors are those of the functions' Python form; the global interpreter lock
- * is released during the call, as ctypes does.
+ * 0.6 us. Arguments, defaults and errors are those of the functions' ctypes form in capi.py, which an interpreter
+ * without this module uses; the global interpreter lock is released during the call, as ctypes does.
  */
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #include <stdint.h>
 
-typedef void *weight_t;
-enum { MEM_DEVICE = 1, MAX_STACK = 16 };
+#include "hipq.h"
 
-static int (*f_matmul)(weight_t, const float *, int64_t, int64_t, float *, int64_t, int, void *);
-static int (*f_each_row)(weight_t, const float *, int64_t, int64_t, float *, int64_t, int, void *);
-static int (*f_noalloc)(weight_t, const float *, int64_t, int64_t, float *, int64_t, void *);
-static int (*f_multi)(int, const weight_t *, const float *, int64_t, int64_t, float *const *, const int64_t *, int, void *);
-static int (*f_swiglu)(weight_t, weight_t, const float *, int64_t, int64_t, float *, int64_t, int, void *);
-static int (*f_swiglu_down)(weight_t, weight_t, weight_t, const float *, int64_t, int64_t, float *, int64_t, int, void *);
-static PyObject *raise_status; /* capi.check */
+typedef hipq_weight_t weight_t;
+enum { MEM_DEVICE = HIPQ_MEM_DEVICE, MAX_STACK = 16 };
+
+/* the library's entry points; their types are the header's */
+static __typeof__(&hipq_matmul) f_matmul;
+static __typeof__(&hipq_matmul_each_row) f_each_row;
+static __typeof__(&hipq_matmul_noalloc) f_noalloc;
+static __typeof__(&hipq_matmul_multi) f_multi;
+static __typeof__(&hipq_mlp_swiglu) f_swiglu;
+static __typeof__(&hipq_mlp_swiglu_down) f_swiglu_down;
+static PyObject *load, *raise_status; /* capi.lib, check */
 static PyObject *pointer_of, *int_of; /* capi._pointer_of, _int_of: the rarer forms of a stream and an integer */
 static PyObject *s_h, *s_handle, *s_value, *s_n, *s_k, *s_data_ptr, *s_ctypes, *s_data;
 
@@ -102,21 +105,23 @@ static int get_stride(PyObject *x, PyObject *w, PyObject *dflt, int64_t *out) {
 }
 /* the handle of a capi.Weight: its _h is a ctypes.c_void_p (null once destroyed); of another object its `handle` */
 static int get_weight(PyObject *w, weight_t *out) {
+  void *p = NULL;
+  int rc = 0;
   PyObject *h = PyObject_GetAttr(w, s_h);
-  if (!h) {
+  if (h) {
+    PyObject *v = PyObject_GetAttr(h, s_value);
+    if (!v) rc = -1;
+    if (v && v != Py_None) p = PyLong_AsVoidPtr(v);
+    Py_XDECREF(v);
+  } else {
     if (!PyErr_ExceptionMatches(PyExc_AttributeError)) return -1;
     PyErr_Clear();
     if (!(h = PyObject_GetAttr(w, s_handle))) return -1;
-    const int rc = get_stream(h, out); /* the forms of a pointer argument */
-    Py_DECREF(h);
-    return rc;
+    rc = get_stream(h, &p); /* the forms of a pointer argument */
   }
-  PyObject *v = PyObject_GetAttr(h, s_value);
   Py_DECREF(h);
-  if (!v) return -1;
-  *out = v == Py_None ? NULL : PyLong_AsVoidPtr(v);
-  Py_DECREF(v);
-  return PyErr_Occurred() ? -1 : 0;
+  *out = (weight_t)p;
+  return rc || PyErr_Occurred() ? -1 : 0;
 }
 
 /* Positional and keyword arguments into slots by the names of `kw` (null-terminated, `need` required). */
@@ -160,9 +165,12 @@ static PyObject *finish(int rc) {
   return NULL;
 }
 
-static int ready(void) {
+static int ready(void) { /* the first call loads the library, which binds the entry points */
   if (f_matmul) return 0;
-  PyErr_SetString(PyExc_RuntimeError, "the library is not loaded");
+  PyObject *r = load ? PyObject_CallNoArgs(load) : NULL;
+  Py_XDECREF(r);
+  if (r && f_matmul) return 0;
+  if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, "the library is not loaded");
   return -1;
 }
 
@@ -294,17 +302,21 @@ static PyObject *mlp_swiglu_down(PyObject *self, PyObject *const *args, Py_ssize
   return finish(rc);
 }
 
-/* bind(check, pointer_of, int_of, addresses of the six functions in the order of the pointers above) */
+/* setup(lib, check, pointer_of, int_of): the functions of capi.py that are needed here */
+static PyObject *setup(PyObject *self, PyObject *args) {
+  PyObject *p[4];
+  if (!PyArg_ParseTuple(args, "OOOO", &p[0], &p[1], &p[2], &p[3])) return NULL;
+  for (int i = 0; i < 4; ++i) Py_INCREF(p[i]);
+  Py_XSETREF(load, p[0]);
+  Py_XSETREF(raise_status, p[1]);
+  Py_XSETREF(pointer_of, p[2]);
+  Py_XSETREF(int_of, p[3]);
+  Py_RETURN_NONE;
+}
+/* bind(addresses of the six entry points in the order of the pointers above) */
 static PyObject *bind(PyObject *self, PyObject *args) {
-  PyObject *check, *pointer, *integer;
   unsigned long long p[6];
-  if (!PyArg_ParseTuple(args, "OOOKKKKKK", &check, &pointer, &integer, &p[0], &p[1], &p[2], &p[3], &p[4], &p[5])) return NULL;
-  Py_INCREF(check);
-  Py_XSETREF(raise_status, check);
-  Py_INCREF(pointer);
-  Py_XSETREF(pointer_of, pointer);
-  Py_INCREF(integer);
-  Py_XSETREF(int_of, integer);
+  if (!PyArg_ParseTuple(args, "KKKKKK", &p[0], &p[1], &p[2], &p[3], &p[4], &p[5])) return NULL;
   *(void **)&f_matmul = (void *)(uintptr_t)p[0];
   *(void **)&f_each_row = (void *)(uintptr_t)p[1];
   *(void **)&f_noalloc = (void *)(uintptr_t)p[2];
@@ -327,7 +339,8 @@ static PyMethodDef methods[] = {
                    "out = swiglu(a . w_act^T, a . w_mul^T): the gated half of a dense MLP in one call."),
   FAST(mlp_swiglu_down, "mlp_swiglu_down(w_act, w_mul, w_down, a, m, out, lda=None, ldo=None, mem=MEM_DEVICE, stream=None)\n\n"
                         "out = swiglu(a . w_act^T, a . w_mul^T) . w_down^T: the gated MLP of a decoder layer in one call."),
-  {"bind", bind, METH_VARARGS, "bind(check, pointer_of, int_of, six function addresses)"},
+  {"setup", setup, METH_VARARGS, "setup(lib, check, pointer_of, int_of)"},
+  {"bind", bind, METH_VARARGS, "bind(six entry points' addresses)"},
   {NULL, NULL, 0, NULL}};
 static struct PyModuleDef module = {PyModuleDef_HEAD_INIT, "hipq_native", "The matmul calls of capi.py.", -1, methods};
 

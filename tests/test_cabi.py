@@ -1,7 +1,9 @@
 """CPU: the C-ABI library loads, exports every symbol include/hipq.h declares, and
 fails loudly (no fallback) where there is no GPU."""
+import functools
 import os
 import re
+import sys
 
 import pytest
 
@@ -111,30 +113,35 @@ def test_native_calls_check_their_arguments(name, args, kwargs, error):
 
 
 class _Calls:
-    """The native functions bound to a stub that notes what each entry point is given."""
+    """The matmul calls bound to a stub that notes what each entry point is given."""
 
     def __enter__(self):
         import ctypes as C
-        capi.lib()
-        self.args, self.keep, one = None, [], [C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_int64]
+        self.lib = capi.lib()
+        self.args, one = None, [C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_int64]
         kinds = {"matmul": one + [C.c_int, C.c_void_p], "matmul_each_row": one + [C.c_int, C.c_void_p], "matmul_noalloc": one + [C.c_void_p],
                  "matmul_multi": [C.c_int, C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p, C.c_int, C.c_void_p],
                  "mlp_swiglu": [C.c_void_p] + one + [C.c_int, C.c_void_p], "mlp_swiglu_down": [C.c_void_p] * 2 + one + [C.c_int, C.c_void_p]}
 
-        def note(*args):
+        def note(name, *args):
             self.args = [a or 0 for a in args]
+            if name == "matmul_multi":  # arrays of handles, outputs and strides
+                for i, t in ((1, C.c_void_p), (5, C.c_void_p), (6, C.c_int64)):
+                    self.args[i] = list((t * args[0]).from_address(args[i]))
             return 0
 
         class Stub:
             pass
         for name, types in kinds.items():
-            f = C.CFUNCTYPE(C.c_int, *types)(note)
+            f = C.CFUNCTYPE(C.c_int, *types)(functools.partial(note, name))
             setattr(Stub, "hipq_" + name, f)
+        capi._lib = Stub
         capi._bind_native(Stub)
         return self
 
     def __exit__(self, *exc):
-        capi._bind_native(capi.lib())
+        capi._lib = self.lib
+        capi._bind_native(self.lib)
 
 
 class _Shape:  # a weight's fields
@@ -194,6 +201,59 @@ def test_native_calls_take_the_buffers_the_binding_takes():
                 with pytest.raises(AttributeError):
                     capi.matmul(*args)
                 assert calls.args is None, x
+
+
+def test_ctypes_forms_make_the_same_calls():
+    """An interpreter without the native module uses the ctypes forms: the same entry points, arguments and defaults."""
+    import numpy as np
+    w, x, y = _Shape(16), _Shape(24), np.zeros((2, 32), np.float32)
+    y_at = y.ctypes.data
+    cases = [("matmul", (w, y, 2, 128), {}), ("matmul", (w, y, 2, 128, 40), {"ldc": 0, "mem": 0, "stream": 0x30}),
+             ("matmul_each_row", (w, 64, 2, y), {"lda": None, "ldc": 16}), ("matmul_noalloc", (w, 64), {"m": 1, "c": y, "stream": None}),
+             ("matmul_multi", ([w, x], y, 3, (y, 128)), {"lda": 64}), ("matmul_multi", ((w,), 64, 1, [y], [9], 0, 0x30), {}),
+             ("mlp_swiglu", (w, x, y, 2, 128, 33), {"ldo": 10}), ("mlp_swiglu_down", (w, x, w, y, 2, 128), {"stream": 0x30})]
+    with _Calls() as calls:
+        for name, args, kwargs in cases:
+            seen = []
+            for form in (getattr(capi, name), capi._FORMS[name]):
+                assert form(*args, **kwargs) is None
+                seen.append(calls.args)
+            assert seen[0] == seen[1], (name, seen)
+            assert y_at in seen[0] or y_at in seen[0][5]
+
+
+def test_native_module_is_built_per_interpreter_and_optional(tmp_path):
+    import subprocess
+    import sysconfig
+    lib = os.path.dirname(capi.LIB_PATH)
+    assert os.path.exists(os.path.join(lib, "hipq_native" + sysconfig.get_config_var("EXT_SUFFIX")))
+    # no interpreter, no headers: the library's own targets remain
+    out = subprocess.run(["make", "-B", "-n", "-C", capi.CSRC, "PYTHON=/nonexistent"], capture_output=True, text=True, check=True).stdout
+    assert "libhipq.so" in out and "native_calls" not in out
+    # without the module the binding loads and calls through ctypes
+    code = ("import importlib.machinery as m; m.EXTENSION_SUFFIXES.insert(0, '.other-abi.so')\n"
+            "import warnings; warnings.simplefilter('error')\n"
+            "from nntrainer_amd import capi\n"
+            "try: capi.lib()\n"
+            "except RuntimeWarning: print(capi.matmul.__module__)\n")
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, cwd=ROOT)
+    assert r.stdout.split() == ["nntrainer_amd.capi"], r.stderr
+
+
+def test_native_calls_follow_the_headers_signatures(tmp_path):
+    import subprocess
+    import sysconfig
+    text = open(os.path.join(ROOT, "include", "hipq.h")).read()
+    for n, (old, new) in enumerate([("", ""), (r"hipq_matmul\((hipq_weight_t w), ", r"hipq_matmul(\1, int flags, "),
+                                    ("const int64_t \\*ldc", "const int32_t *ldc")]):
+        changed = re.sub(old, new, text) if old else text
+        assert not old or changed != text, old
+        d = tmp_path / str(n)
+        d.mkdir()
+        (d / "hipq.h").write_text(changed)
+        r = subprocess.run(["gcc", "-std=c11", "-fsyntax-only", "-Werror=incompatible-pointer-types", "-Werror=int-conversion", "-I", str(d),
+                            "-I", sysconfig.get_paths()["include"], os.path.join(capi.CSRC, "native_calls.c")], capture_output=True, text=True)
+        assert (r.returncode == 0) == (not old), (old, r.stderr)
 
 
 def test_product_never_imports_the_oracle():
