@@ -100,6 +100,9 @@ int fail(int code, const char *fmt, ...) {
   va_start(ap, fmt);
   vsnprintf(tl_error, sizeof(tl_error), fmt, ap);
   va_end(ap);
+  /* A refused allocation stays the thread's last error until it is read, across calls that succeed: taken here, so that
+   * whoever goes on without the memory does not find it behind its next launch. */
+  if (code == HIPQ_ERR_OUT_OF_MEMORY) (void)hipGetLastError();
   return code;
 }
 
@@ -774,18 +777,21 @@ bool wants_f6(int count, const hipq_weight *const *w, int64_t M) {
 
 /* The six-bit copies of the weights are there, or could be made: a call that may not allocate, a stream that is being
  * captured into a graph and a full device use the kernels that read the weights as they are stored. */
-bool f6_ready(int count, const hipq_weight *const *w, int64_t M, hipStream_t s, const Scratch &sc) {
-  if (sc.fixed && hipq::qact_f6_bytes(M, w[0]->K) > NOALLOC_SCRATCH_BYTES) return false;
+int f6_ready(int count, const hipq_weight *const *w, int64_t M, hipStream_t s, const Scratch &sc, bool *ready) {
+  *ready = false;
+  if (sc.fixed && hipq::qact_f6_bytes(M, w[0]->K) > NOALLOC_SCRATCH_BYTES) return HIPQ_OK;
   for (int i = 0; i < count; ++i) {
     const bool made = __atomic_load_n(&w[i]->gf_base, __ATOMIC_ACQUIRE) != nullptr;
     if (made && (!w[i]->gf_event || w[i]->gf_stream == s)) continue;
-    if (sc.fixed && !made) return false;
+    if (sc.fixed && !made) return HIPQ_OK;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cs) != hipSuccess) (void)hipGetLastError();
-    if (cs != hipStreamCaptureStatusNone) return false;
-    if (hipq::ensure_f6(const_cast<hipq_weight *>(w[i]), s)) return false;
+    if (cs != hipStreamCaptureStatusNone) return HIPQ_OK;
+    const int rc = hipq::ensure_f6(const_cast<hipq_weight *>(w[i]), s);
+    if (rc) return rc == HIPQ_ERR_OUT_OF_MEMORY ? HIPQ_OK : rc;
   }
-  return true;
+  *ready = true;
+  return HIPQ_OK;
 }
 
 /* count (1 to 4) weights with their copies, one quantization (unless the last call on the scratch made it) and launch */
@@ -819,7 +825,8 @@ int launch_gated(const hipq_weight *wa, const hipq_weight *wm, const float *A, i
   *done = false;
   if (wa->dtype == HIPQ_Q4_0) {
     const Scratch sc{false, s};
-    if (!f6_ready(2, ws, M, s, sc)) return HIPQ_OK;
+    bool ready = false;
+    if ((rc = f6_ready(2, ws, M, s, sc, &ready)) || !ready) return rc;
     if ((rc = sc.get(hipq::qact_f6_bytes(M, K), &mem))) return rc;
     const QActF6 qa = hipq::qact_f6_carve(mem, M, K);
     if ((rc = hipq::launch_quantize_q8_0_f6(A, M, K, lda, &qa, s))) return rc;
@@ -842,7 +849,11 @@ int matmul_device(hipq_weight_t w, const float *A, int64_t M, int64_t lda, float
                   hipStream_t s, const Scratch &sc, bool each_row = false) {
   if (M == 0) return HIPQ_OK;
   const hipq_weight *one = w;
-  if (wants_f6(1, &one, M) && f6_ready(1, &one, M, s, sc)) return matmul_f6(1, &one, A, M, lda, &C, &ldc, s, sc);
+  if (wants_f6(1, &one, M)) {
+    bool ready = false;
+    if (int rc = f6_ready(1, &one, M, s, sc, &ready)) return rc;
+    if (ready) return matmul_f6(1, &one, A, M, lda, &C, &ldc, s, sc);
+  }
   if (wants_rows(w, M, !sc.fixed)) return matmul_rows(w, A, M, lda, C, ldc, s, 0, sc, each_row);
   if (!each_row && wants_tiled(w, M, !sc.fixed)) return matmul_tiled(w, A, M, lda, C, ldc, s, 0, sc);
   if (M == 1 && hipq::gemv_fuses_quantizer(w, A)) return hipq::launch_gemv_fused(w, A, C, s);
@@ -1726,7 +1737,9 @@ int hipq_matmul_multi(int count, const hipq_weight_t *w, const float *A, int64_t
       for (int i = 0; i < count; ++i)
         if (klass(w[i]) == 0 && ++members <= 64) fw[nf] = w[i], fc[nf] = C[i], fl[nf] = ldc[i], ++nf;
       const Scratch sc{false, s};
-      if (members <= 64 && wants_f6(std::min(nf, 4), fw, M) && f6_ready(nf, fw, M, s, sc)) {
+      bool ready = false;
+      if (members <= 64 && wants_f6(std::min(nf, 4), fw, M) && (rc = f6_ready(nf, fw, M, s, sc, &ready))) return rc;
+      if (ready) {
         for (int i = 0; i < nf; i += 4) {
           if ((rc = workspace_unmoved(s, gen))) return rc;
           if ((rc = matmul_f6(std::min(4, nf - i), fw + i, A, M, lda, fc + i, fl + i, s, sc, i == 0))) return rc;
