@@ -44,6 +44,7 @@
  * in its middle. Workgroup ids are mapped so that the row tiles sharing weights run on one XCD.
  */
 #include <mutex>
+#include <new>
 
 #include "gemv_device.h"
 
@@ -317,48 +318,184 @@ __global__ __launch_bounds__(256) void f6_weights_kernel(const uint8_t *__restri
 
 namespace hipq {
 
-int ensure_f6(hipq_weight *w, hipStream_t s) {
-  static std::mutex mu; /* two threads may run their first prefill product on one weight */
-  std::lock_guard<std::mutex> lk(mu);
-  if (w->gf_base) {
-    if (w->gf_event && s != w->gf_stream) { /* made on another stream a moment ago */
-      const hipError_t q = hipEventQuery(w->gf_event);
-      if (q == hipErrorNotReady) {
-        (void)hipGetLastError();
-        HIPQ_HIP(hipStreamWaitEvent(s, w->gf_event, 0));
-      } else if (q == hipSuccess) {
-        (void)hipEventDestroy(w->gf_event);
-        w->gf_event = nullptr;
-      } else
-        return fail(HIPQ_ERR_RUNTIME, "six-bit copy: %s", hipGetErrorString(q));
+/* ---- who may read a copy ----
+ * A copy is made on the stream of the product that asks for it, in front of that product, and nothing waits. Until it
+ * is known to be complete it is PENDING, and only the stream it was made on may read it; a product on another stream
+ * takes the kernels that read the weight as stored (the same bits). Complete is what the page-locked word of its batch
+ * says, which the quantizer behind the copies sets: a plain read, so also a call that is being captured into a graph,
+ * where events may not be queried, finds out. A graph may be launched on any stream, so a captured product reads
+ * complete copies only.
+ * The same stream is known by its handle alone, and one handle can stand for two streams (hipStreamPerThread; a stream
+ * made after another was destroyed): the event of the batch orders those. */
+struct F6Batch {
+  uint32_t *word, *word_dev;
+  hipEvent_t ev;
+  hipStream_t s;
+  int refs; /* PENDING weights that point here */
+  F6Batch *next;
+};
+
+namespace {
+std::mutex f6_mu; /* guards what follows and every weight's gf_ fields */
+struct F6Page { /* batches and the page-locked page of their words; given back by f6_shutdown */
+  static constexpr int COUNT = 1024;
+  F6Batch batch[COUNT];
+  uint32_t *words;
+  F6Page *next;
+};
+F6Page *f6_pages = nullptr;
+F6Batch *f6_idle = nullptr; /* batches no weight points to */
+
+void batch_idle(F6Batch *b) {
+  b->next = f6_idle;
+  f6_idle = b;
+}
+int batch_get(hipStream_t s, F6Batch **out) {
+  if (!f6_idle) {
+    F6Page *pg = new (std::nothrow) F6Page();
+    if (!pg) return fail(HIPQ_ERR_OUT_OF_MEMORY, "host allocation failed");
+    uint32_t *dev = nullptr;
+    hipError_t e = hipHostMalloc((void **)&pg->words, F6Page::COUNT * 4, hipHostMallocDefault);
+    if (e == hipSuccess && (e = hipHostGetDevicePointer((void **)&dev, pg->words, 0)) != hipSuccess) (void)hipHostFree(pg->words);
+    if (e != hipSuccess) {
+      delete pg;
+      return fail(HIPQ_ERR_OUT_OF_MEMORY, "page-locked words: %s", hipGetErrorString(e));
     }
+    pg->next = f6_pages;
+    f6_pages = pg;
+    for (int i = F6Page::COUNT; i-- > 0;) {
+      pg->batch[i] = F6Batch{pg->words + i, dev + i, nullptr, nullptr, 0, nullptr};
+      batch_idle(&pg->batch[i]);
+    }
+  }
+  F6Batch *b = f6_idle;
+  if (!b->ev) HIPQ_HIP(hipEventCreateWithFlags(&b->ev, hipEventDisableTiming));
+  f6_idle = b->next;
+  __atomic_store_n(b->word, 0u, __ATOMIC_RELAXED);
+  b->s = s;
+  *out = b;
+  return HIPQ_OK;
+}
+void batch_drop(hipq_weight *w) {
+  F6Batch *b = w->gf_batch;
+  w->gf_batch = nullptr;
+  if (b && --b->refs == 0) batch_idle(b);
+}
+
+/* Whether the weight's copy is complete; looks up to `spins` times more */
+bool complete(hipq_weight *w, int &spins) {
+  if (w->gf_state == F6_PENDING) {
+    while (!__atomic_load_n(w->gf_batch->word, __ATOMIC_ACQUIRE)) {
+      if (spins <= 0) return false;
+      --spins;
+      __builtin_ia32_pause();
+    }
+    batch_drop(w);
+    __atomic_store_n(&w->gf_state, F6_COMPLETE, __ATOMIC_RELEASE);
+  }
+  return w->gf_state == F6_COMPLETE;
+}
+} // namespace
+
+/* *ready: what is enqueued on s next may read the copies of the weights. Missing ones are made where may_make and the
+ * stream is not being captured; the caller then hands *word to the quantizer it launches behind them. */
+int f6_copies(int count, const hipq_weight *const *cw, hipStream_t s, bool may_make, bool *ready, uint32_t **word) {
+  *ready = false;
+  *word = nullptr;
+  int done = 0;
+  for (int i = 0; i < count; ++i) done += __atomic_load_n(&cw[i]->gf_state, __ATOMIC_ACQUIRE) == F6_COMPLETE;
+  if (done == count) {
+    *ready = true;
     return HIPQ_OK;
   }
-  if (w->dtype != HIPQ_Q4_0 || w->expert_tiles)
-    return fail(HIPQ_ERR_INVALID_ARGUMENT, "only Q4_0 weights in the plane layout have a six-bit copy");
-  const int nb = (int)(w->K / 32), chunks = (nb + 7) / 8;
-  const int64_t tiles = (w->N + 31) / 32, threads = tiles * chunks * 512;
-  const size_t bytes = (size_t)tiles * chunks * F6_WTILE;
-  uint8_t *p = nullptr;
-  hipError_t e = hipMalloc((void **)&p, bytes);
-  if (e != hipSuccess) return fail(HIPQ_ERR_OUT_OF_MEMORY, "six-bit copy of %zu bytes: %s", bytes, hipGetErrorString(e));
-  /* on the caller's stream, in front of the product that asked for it: nothing waits. Other streams wait for the
-   * event, until it is seen to have passed. */
-  launch_kernel("f6_weights_kernel", f6_weights_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, w->qs, w->d,
-                (int)w->N, nb, chunks, threads, p);
-  e = hipGetLastError();
-  if (e == hipSuccess) e = hipEventCreateWithFlags(&w->gf_event, hipEventDisableTiming);
-  if (e == hipSuccess) e = hipEventRecord(w->gf_event, s);
-  if (e != hipSuccess) {
-    (void)hipStreamSynchronize(s);
-    if (w->gf_event) (void)hipEventDestroy(w->gf_event);
-    w->gf_event = nullptr;
-    (void)hipFree(p);
-    return fail(HIPQ_ERR_RUNTIME, "six-bit copy: %s", hipGetErrorString(e));
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cs) != hipSuccess) (void)hipGetLastError();
+  const bool capturing = cs != hipStreamCaptureStatusNone;
+  hipq_weight *const *w = const_cast<hipq_weight *const *>(cw);
+  std::lock_guard<std::mutex> lk(f6_mu);
+  int missing = 0;
+  /* the graph keeps the kernels that are chosen now: a copy that is about to complete is waited for, up to about a
+   * millisecond a call */
+  int spins = capturing ? 20000 : 0;
+  F6Batch *behind = nullptr;
+  for (int i = 0; i < count; ++i) {
+    if (w[i]->gf_state == F6_NONE) {
+      if (w[i]->dtype != HIPQ_Q4_0 || w[i]->expert_tiles)
+        return fail(HIPQ_ERR_INVALID_ARGUMENT, "only Q4_0 weights in the plane layout have a six-bit copy");
+      ++missing;
+    } else if (!complete(w[i], spins)) {
+      F6Batch *b = w[i]->gf_batch;
+      if (capturing || b->s != s) return HIPQ_OK;
+      if (b != behind) HIPQ_HIP(hipStreamWaitEvent(s, b->ev, 0));
+      behind = b;
+    }
   }
-  w->gf_stream = s;
-  __atomic_store_n(&w->gf_base, p, __ATOMIC_RELEASE); /* last: readers test this field */
+  if (missing) {
+    if (!may_make || capturing) return HIPQ_OK;
+    F6Batch *b = nullptr;
+    if (int rc = batch_get(s, &b)) return rc;
+    int made = 0, rc = HIPQ_OK;
+    hipq_weight *fresh[64];
+    for (int i = 0; i < count && !rc && made < 64; ++i) {
+      hipq_weight *x = w[i];
+      if (x->gf_state != F6_NONE || x->gf_base) continue; /* a weight may stand in the list twice */
+      const int nb = (int)(x->K / 32), chunks = (nb + 7) / 8;
+      const int64_t tiles = (x->N + 31) / 32, threads = tiles * chunks * 512;
+      const size_t bytes = (size_t)tiles * chunks * F6_WTILE;
+      uint8_t *p = nullptr;
+      hipError_t e = hipMalloc((void **)&p, bytes);
+      if (e != hipSuccess) {
+        rc = fail(HIPQ_ERR_OUT_OF_MEMORY, "six-bit copy of %zu bytes: %s", bytes, hipGetErrorString(e));
+        break;
+      }
+      x->gf_base = p;
+      fresh[made++] = x;
+      launch_kernel("f6_weights_kernel", f6_weights_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, x->qs, x->d,
+                    (int)x->N, nb, chunks, threads, p);
+      if ((e = hipGetLastError()) != hipSuccess) rc = fail(HIPQ_ERR_RUNTIME, "six-bit copy: %s", hipGetErrorString(e));
+    }
+    if (!rc) {
+      const hipError_t e = hipEventRecord(b->ev, s);
+      if (e != hipSuccess) rc = fail(HIPQ_ERR_RUNTIME, "six-bit copy: %s", hipGetErrorString(e));
+    }
+    if (rc) {
+      if (made) (void)hipStreamSynchronize(s);
+      for (int i = 0; i < made; ++i) {
+        (void)hipFree(fresh[i]->gf_base);
+        fresh[i]->gf_base = nullptr;
+      }
+      batch_idle(b);
+      return rc;
+    }
+    for (int i = 0; i < made; ++i) {
+      fresh[i]->gf_batch = b;
+      __atomic_store_n(&fresh[i]->gf_state, F6_PENDING, __ATOMIC_RELEASE);
+    }
+    b->refs = made;
+    *word = b->word_dev;
+  }
+  *ready = true;
   return HIPQ_OK;
+}
+
+void f6_release(hipq_weight *w) {
+  std::lock_guard<std::mutex> lk(f6_mu);
+  batch_drop(w);
+  if (w->gf_base) (void)hipFree(w->gf_base);
+  w->gf_base = nullptr;
+  w->gf_state = F6_NONE;
+}
+
+void f6_shutdown() {
+  std::lock_guard<std::mutex> lk(f6_mu);
+  while (F6Page *pg = f6_pages) {
+    f6_pages = pg->next;
+    for (F6Batch &b : pg->batch)
+      if (b.ev) (void)hipEventDestroy(b.ev);
+    (void)hipHostFree(pg->words);
+    delete pg;
+  }
+  f6_idle = nullptr;
 }
 
 int launch_gemm_f6(int count, const hipq_weight *const *w, const QActF6 *qa, int M, float *const *C, const int64_t *ldc,

@@ -53,6 +53,10 @@
 /*       hipq_weight.hdr points at the first header, 4096 bytes behind qs)      */
 /* Such a weight serves the expert kernels only.                               */
 /* ------------------------------------------------------------------------- */
+namespace hipq {
+struct F6Batch;
+enum { F6_NONE, F6_PENDING, F6_COMPLETE };
+} // namespace hipq
 struct hipq_weight {
   int dtype;
   int device;
@@ -80,14 +84,14 @@ struct hipq_weight {
    *   gt_hdr [N/32][K/256][64][16 B]: the lane's eight int8 scales, then the fp16 d */
   uint8_t *gt_base;
   const uint8_t *gt_qs, *gt_qh, *gt_hdr;
-  /* Built by the first prefill product of a Q4_0 weight (ensure_f6): the weights as six-bit floats in
+  /* Built by the first prefill product of a Q4_0 weight (f6_copies): the weights as six-bit floats in
    * the operand order of gemm_f6.hip, per 32 columns and 256 of K (rows padded to that with zeros):
    *   [6][64][16 B]: lane (column, g) holds sixteen 6-bit codes of each of the eight blocks, values
    *     16 g .. 16 g + 15, three dwords a block one behind the other, four dwords a piece;
    *   [32][8] fp16 block scales. */
   uint8_t *gf_base;
-  hipEvent_t gf_event;   /* recorded behind the copy on gf_stream, or null once it is known to have passed */
-  hipStream_t gf_stream;
+  int gf_state;             /* hipq::F6_NONE, F6_PENDING, F6_COMPLETE: read with acquire, written under f6_copies' mutex */
+  hipq::F6Batch *gf_batch;  /* PENDING: what the copies enqueued with this one have in common */
 };
 
 /* Plain-data view of a weight passed to kernels by value. */
@@ -234,7 +238,8 @@ int launch_quantize_q8_K_tiled(const float *A, int64_t M, int64_t K, int64_t lda
 /* the values of launch_quantize_q8_0 in the form of the six-bit GEMM */
 size_t qact_f6_bytes(int64_t M, int64_t K);
 QActF6 qact_f6_carve(void *mem, int64_t M, int64_t K);
-int launch_quantize_q8_0_f6(const float *A, int64_t M, int64_t K, int64_t lda, const QActF6 *qa, hipStream_t s);
+/* `word` (may be null): a word of page-locked memory the kernel sets to 1 (f6_copies) */
+int launch_quantize_q8_0_f6(const float *A, int64_t M, int64_t K, int64_t lda, const QActF6 *qa, uint32_t *word, hipStream_t s);
 
 /* gemv.hip ---------------------------------------------------------------- */
 /* C[m][n] for m < M <= 8: one pass over the weights, M activation rows.
@@ -261,7 +266,9 @@ int launch_gemm(const hipq_weight *w, const QAct *qa, int M, float *C,
 int launch_gemm_multi(int count, const hipq_weight *const *w, const QAct *qa, int M, float *const *C,
                       const int64_t *ldc, hipStream_t s);
 /* gemm_f6.hip: up to four Q4_0 weights of one K, each with its six-bit copy, one launch */
-int ensure_f6(hipq_weight *w, hipStream_t s); /* the copy is there for what is enqueued on s next (allocates once) */
+int f6_copies(int count, const hipq_weight *const *w, hipStream_t s, bool may_make, bool *ready, uint32_t **word);
+void f6_release(hipq_weight *w); /* the device no longer reads or writes the weight's copy */
+void f6_shutdown();              /* no weight is left */
 int launch_gemm_f6(int count, const hipq_weight *const *w, const QActF6 *qa, int M, float *const *C, const int64_t *ldc,
                    hipStream_t s);
 /* out = swiglu(x . wa) * (x . wm) of many rows, one launch (gemm_f6.hip, gemm_q4k.hip) */

@@ -74,7 +74,9 @@ __device__ __forceinline__ void bf6_parts(int v, uint32_t &first, uint32_t &seco
  * row (128 bytes of a row in, two whole lines of operands out). Rows M and beyond of the last 64 and blocks of K and
  * beyond are written as zeros. */
 __global__ __launch_bounds__(256) void quantize_q8_0_f6_kernel(const float *__restrict__ A, int64_t M, int64_t n_units, int nbp,
-                                                               int K, int64_t lda, uint8_t *__restrict__ out) {
+                                                               int K, int64_t lda, uint8_t *__restrict__ out, uint32_t *word) {
+  /* what was enqueued in front of this kernel is complete: stream order, no fence is needed for it */
+  if (word && blockIdx.x == 0 && threadIdx.x == 0) __hip_atomic_store(word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   constexpr int PARTS = hipq::F6_ROWS * 384;
   const int64_t unit = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   if (unit >= n_units) return; /* uniform per wavefront */
@@ -273,14 +275,15 @@ QActF6 qact_f6_carve(void *mem, int64_t M, int64_t K) {
   return QActF6{(uint8_t *)mem, (int)M, (int)K, (int)((K + 255) / 256)};
 }
 
-int launch_quantize_q8_0_f6(const float *A, int64_t M, int64_t K, int64_t lda, const QActF6 *qa, hipStream_t s) {
+int launch_quantize_q8_0_f6(const float *A, int64_t M, int64_t K, int64_t lda, const QActF6 *qa, uint32_t *word,
+                            hipStream_t s) {
   if (M <= 0) return HIPQ_OK;
   if (K % 32 || lda < K) return fail(HIPQ_ERR_INVALID_ARGUMENT, "Q8_0: K=%lld must be a multiple of 32 and lda >= K", (long long)K);
   if (((uintptr_t)A & 15) || (lda & 3))
     return fail(HIPQ_ERR_INVALID_ARGUMENT, "activation rows must be 16-byte aligned");
   const int64_t units = (M + F6_ROWS - 1) / F6_ROWS * (F6_ROWS / 8) * (qa->chunks * 8); /* padding included */
   launch_kernel("quantize_q8_0_f6_kernel", quantize_q8_0_f6_kernel, dim3((unsigned)((units + 3) / 4)), dim3(256), 0, s, A, M,
-                units, qa->chunks * 8, (int)K, lda, qa->p);
+                units, qa->chunks * 8, (int)K, lda, qa->p, word);
   HIPQ_HIP(hipGetLastError());
   return HIPQ_OK;
 }
