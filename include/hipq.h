@@ -158,15 +158,23 @@ HIPQ_API int hipq_quantize_q8_K(const float *A, int64_t M, int64_t K, int64_t ld
  *  of 2^24 weights or more, up to 4 from 2^25, up to 2 from 2^28: there the matrix cores are
  *  faster, up to several times); with more rows the K-formats run on the
  *  int8 matrix cores and agree with the reference to 1e-4 of the output's maximum (same
- *  quantized activations, another order of the fp32 sums). The first such product of a
- *  weight adds a copy of it in the kernels' load order (allocates; 0.56 bytes per weight
- *  for Q4_K, 0.875 for Q6_K), kept until hipq_weight_destroy. Q4_K with 5..16 rows and 1024
+ *  quantized activations, another order of the fp32 sums). The first product of many rows of
+ *  a weight adds a copy of it in the kernels' load order, kept until hipq_weight_destroy,
+ *  beside the weight as it is stored: Q4_K 0.56 bytes per weight beside 0.56, Q6_K 0.875
+ *  beside 0.82, Q4_0 0.8125 beside 0.5625 (rows padded to 32, K to 256; from nine to 65 rows
+ *  on, by size). The copies of Q4_0 weights lie in blocks of 64 MiB (larger ones in blocks of
+ *  their own) that are given back with the last copy in them, one empty block excepted, which
+ *  hipq_shutdown frees. Q4_K with 5..16 rows and 1024
  *  columns or more (4 rows from 4096, 3 from 8192 columns) reads the same copy: those row
  *  counts run on the matrix cores as well, with the reference's bits (a batch of decode
  *  rows against a 12288 x 4096 matrix: 11 us for eight, 14 us for sixteen, 8 us for one).
  *  Q4_0 has the same kind of kernel for a few rows (gemm_rows_q40.hip, off the weight as it is
  *  stored: eight rows against 12288 x 4096 in 11 us, against 151936 x 1024 in 26 us); every Q4_0
- *  kernel carries the reference's bits, so there the row count only selects the fastest. */
+ *  kernel carries the reference's bits, so there the row count only selects the fastest, and a
+ *  product of many rows that cannot have the weight's copy takes a slower kernel that reads the
+ *  weight as it is stored: on a full device, in a call that is being captured into a graph before
+ *  the weight has had such a product, and on another stream than that product's until the copy is
+ *  complete. */
 HIPQ_API int hipq_matmul(hipq_weight_t w, const float *A, int64_t M, int64_t lda,
                          float *C, int64_t ldc, int mem, void *stream);
 
@@ -359,7 +367,9 @@ HIPQ_API int hipq_launch_timing_end(int capacity, int *count, float *ms, const c
  *  that calls were made on; waits for the stream. When a call needs more scratch than the stream
  *  has, the library allocates a larger block (hipMalloc: not possible while the stream is being
  *  captured into a graph, so run a call of the largest shape once before capturing) and keeps the
- *  smaller one until a later call on the stream finds the stream drained. No counterpart in the reference, whose OpenCL
+ *  smaller one until a later call on the stream finds the stream drained. The scratch belongs to the stream's
+ *  handle: threads that share the handle hipStreamPerThread have streams of their own but one scratch, so
+ *  they order their calls or use streams they made. No counterpart in the reference, whose OpenCL
  *  back-end has one queue (opencl_command_queue_manager.cpp). */
 HIPQ_API int hipq_stream_release(void *stream);
 

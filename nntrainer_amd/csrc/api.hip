@@ -777,22 +777,23 @@ bool wants_f6(int count, const hipq_weight *const *w, int64_t M) {
 
 /* Whether a call can read the weights' six-bit copies: they are there, or could be made. A call that may not allocate,
  * a stream that is being captured into a graph and a full device use the kernels that read the weights as they are
- * stored. *word: for the call's quantizer (f6_copies). */
-int f6_ready(int count, const hipq_weight *const *w, int64_t M, hipStream_t s, const Scratch &sc, bool *ready, uint32_t **word) {
+ * stored. make: for the call's quantizer (f6_copies). */
+int f6_ready(int count, const hipq_weight *const *w, int64_t M, hipStream_t s, const Scratch &sc, bool *ready,
+             hipq::F6Make *make) {
   *ready = false;
   if (sc.fixed && hipq::qact_f6_bytes(M, w[0]->K) > NOALLOC_SCRATCH_BYTES) return HIPQ_OK;
-  const int rc = hipq::f6_copies(count, w, s, !sc.fixed, ready, word);
+  const int rc = hipq::f6_copies(count, w, s, !sc.fixed, ready, make);
   return rc == HIPQ_ERR_OUT_OF_MEMORY ? HIPQ_OK : rc;
 }
 
 /* count (1 to 4) weights with their copies, one quantization (unless the last call on the scratch made it) and launch */
 int matmul_f6(int count, const hipq_weight *const *w, const float *A, int64_t M, int64_t lda, float *const *C,
-              const int64_t *ldc, hipStream_t s, const Scratch &sc, uint32_t *word, bool quantize = true) {
+              const int64_t *ldc, hipStream_t s, const Scratch &sc, hipq::F6Make *make, bool quantize = true) {
   void *mem = nullptr;
   if (int rc = sc.get(hipq::qact_f6_bytes(M, w[0]->K), &mem)) return rc;
-  const QActF6 qa = hipq::qact_f6_carve(mem, M, w[0]->K);
+  QActF6 qa = hipq::qact_f6_carve(mem, M, w[0]->K);
   if (quantize)
-    if (int rc = hipq::launch_quantize_q8_0_f6(A, M, w[0]->K, lda, &qa, word, s)) return rc;
+    if (int rc = hipq::launch_quantize_q8_0_f6(A, M, w[0]->K, lda, &qa, make, s)) return rc;
   return hipq::launch_gemm_f6(count, w, &qa, (int)M, C, ldc, s);
 }
 
@@ -817,11 +818,11 @@ int launch_gated(const hipq_weight *wa, const hipq_weight *wm, const float *A, i
   if (wa->dtype == HIPQ_Q4_0) {
     const Scratch sc{false, s};
     bool ready = false;
-    uint32_t *word = nullptr;
-    if ((rc = f6_ready(2, ws, M, s, sc, &ready, &word)) || !ready) return rc;
+    hipq::F6Make make;
+    if ((rc = f6_ready(2, ws, M, s, sc, &ready, &make)) || !ready) return rc;
     if ((rc = sc.get(hipq::qact_f6_bytes(M, K), &mem))) return rc;
-    const QActF6 qa = hipq::qact_f6_carve(mem, M, K);
-    if ((rc = hipq::launch_quantize_q8_0_f6(A, M, K, lda, &qa, word, s))) return rc;
+    QActF6 qa = hipq::qact_f6_carve(mem, M, K);
+    if ((rc = hipq::launch_quantize_q8_0_f6(A, M, K, lda, &qa, &make, s))) return rc;
     *done = true;
     return hipq::launch_gemm_f6_gated(wa, wm, &qa, (int)M, out, ldo, s);
   }
@@ -843,9 +844,9 @@ int matmul_device(hipq_weight_t w, const float *A, int64_t M, int64_t lda, float
   const hipq_weight *one = w;
   if (wants_f6(1, &one, M)) {
     bool ready = false;
-    uint32_t *word = nullptr;
-    if (int rc = f6_ready(1, &one, M, s, sc, &ready, &word)) return rc;
-    if (ready) return matmul_f6(1, &one, A, M, lda, &C, &ldc, s, sc, word);
+    hipq::F6Make make;
+    if (int rc = f6_ready(1, &one, M, s, sc, &ready, &make)) return rc;
+    if (ready) return matmul_f6(1, &one, A, M, lda, &C, &ldc, s, sc, &make);
   }
   if (wants_rows(w, M, !sc.fixed)) return matmul_rows(w, A, M, lda, C, ldc, s, 0, sc, each_row);
   if (!each_row && wants_tiled(w, M, !sc.fixed)) return matmul_tiled(w, A, M, lda, C, ldc, s, 0, sc);
@@ -1065,6 +1066,7 @@ int hipq_weight_create(int dtype, int layout, int64_t N, int64_t K, const void *
   w->gt_base = nullptr;
   w->gf_base = nullptr;
   w->gf_state = hipq::F6_NONE;
+  w->gf_copy = nullptr;
   w->gf_batch = nullptr;
   w->gt_qs = w->gt_qh = w->gt_hdr = nullptr;
   w->N = N;
@@ -1731,12 +1733,12 @@ int hipq_matmul_multi(int count, const hipq_weight_t *w, const float *A, int64_t
         if (klass(w[i]) == 0 && ++members <= 64) fw[nf] = w[i], fc[nf] = C[i], fl[nf] = ldc[i], ++nf;
       const Scratch sc{false, s};
       bool ready = false;
-      uint32_t *word = nullptr;
-      if (members <= 64 && wants_f6(std::min(nf, 4), fw, M) && (rc = f6_ready(nf, fw, M, s, sc, &ready, &word))) return rc;
+      hipq::F6Make make;
+      if (members <= 64 && wants_f6(std::min(nf, 4), fw, M) && (rc = f6_ready(nf, fw, M, s, sc, &ready, &make))) return rc;
       if (ready) {
         for (int i = 0; i < nf; i += 4) {
           if ((rc = workspace_unmoved(s, gen))) return rc;
-          if ((rc = matmul_f6(std::min(4, nf - i), fw + i, A, M, lda, fc + i, fl + i, s, sc, word, i == 0))) return rc;
+          if ((rc = matmul_f6(std::min(4, nf - i), fw + i, A, M, lda, fc + i, fl + i, s, sc, &make, i == 0))) return rc;
         }
         continue;
       }

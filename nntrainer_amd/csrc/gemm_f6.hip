@@ -43,10 +43,12 @@
  * issued before the multiply-adds of the step before it, also across the end of a chunk; the one barrier a chunk lies
  * in its middle. Workgroup ids are mapped so that the row tiles sharing weights run on one XCD.
  */
+#include <algorithm>
 #include <mutex>
 #include <new>
 
 #include "gemv_device.h"
+#include "quantize_device.h"
 
 namespace {
 
@@ -77,7 +79,13 @@ struct MultiF6 { /* up to four weights of one K, their column tiles side by side
   int64_t ldc[4];
   int N[4];
   int tile_end[4]; /* running sum of the weights' workgroup columns */
+  uint32_t *word;  /* or null: set_word */
 };
+
+/* The copies made in front of this launch are complete, by stream order: said to the host (no fence is needed for it) */
+__device__ __forceinline__ void set_word(uint32_t *word) {
+  if (word && blockIdx.x == 0 && threadIdx.x == 0) __hip_atomic_store(word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 /* The sums of row tile mt and the wavefront's column tile `tile` (lane (column, g), sum r: row 8 (r / 4) + 4 g + r % 4).
  * LOOK: steps an operand is read ahead of its matrix instruction, 1 or 3 */
@@ -232,6 +240,7 @@ __global__ __launch_bounds__(NT, LOOK == 1 ? 3 : 2) void gemm_f6_kernel(MultiF6 
   const int64_t ldc = wi == 0 ? mw.ldc[0] : wi == 1 ? mw.ldc[1] : wi == 2 ? mw.ldc[2] : mw.ldc[3];
   const int N = wi == 0 ? mw.N[0] : wi == 1 ? mw.N[1] : wi == 2 ? mw.N[2] : mw.N[3];
   f6_tile<LOOK>(w, N, chunks, act, M, mt, nt, C, ldc);
+  set_word(mw.word);
 }
 
 /* The gated pair of an MLP: out = swiglu(act sums) * mul sums. Two wavefronts of a workgroup take 32 columns each of the
@@ -243,6 +252,7 @@ struct GatedF6 {
   float *out;
   int64_t ldo;
   int N, ntiles; /* columns, workgroup columns of 64 */
+  uint32_t *word; /* or null: set_word */
 };
 template <int LOOK>
 __device__ __forceinline__ void f6_gated_tile(const GatedF6 &p, int chunks, const uint8_t *act, int M, int mt, int nt) {
@@ -276,42 +286,165 @@ __global__ __launch_bounds__(NT, LOOK == 1 ? 3 : 2) void gemm_f6_gated_kernel(Ga
   const int xcd = id & 7, qd = id >> 3;
   const int mt = qd % mtiles, nt = (qd / mtiles) * 8 + xcd;
   if (nt < p.ntiles) f6_gated_tile<LOOK>(p, chunks, act, M, mt, nt); /* uniform per workgroup */
+  set_word(p.word);
 }
 
 /* ---- the copy of a weight in operand order ---- */
 
-/* thread = lane (column, g) of one (tile, chunk, block): its sixteen weights as 96 bits, dwords 3 j .. 3 j + 2 of the
- * lane's 24, and the block's scale */
-__global__ __launch_bounds__(256) void f6_weights_kernel(const uint8_t *__restrict__ qs, const uint16_t *__restrict__ d, int N,
-                                                         int nb /* blocks a row */, int chunks, int64_t threads,
-                                                         uint8_t *__restrict__ out) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= threads) return;
-  const int lane = (int)(t & 63), j = (int)((t >> 6) & 7), g = lane >> 5, i32 = lane & 31;
-  const int64_t tc = t >> 9; /* tile * chunks + chunk */
-  const int c = (int)(tc % chunks);
-  const int64_t n = tc / chunks * 32 + i32;
-  uint8_t *dst = out + tc * WTILE;
-  const int b = c * 8 + j;
-  const bool in = n < N && b < nb;
-  uint4 x = make_uint4(0x88888888u, 0x88888888u, 0x88888888u, 0x88888888u); /* weights of zero */
-  if (in) x = *(const uint4 *)(qs + (n * nb + b) * 16);
-  const uint32_t x4[4] = {x.x, x.y, x.z, x.w};
-  uint32_t w[3] = {0, 0, 0};
+struct CopyF6 { /* up to four weights of one K; the workgroups of weight i end at end[i] */
+  const uint8_t *qs[4];
+  const uint16_t *d[4];
+  uint8_t *out[4];
+  int N[4], end[4];
+  int nb, chunks; /* blocks and chunks a row */
+};
+
+/* The fp6 codes of four weights, one nibble a byte, as 24 bits: v - 8 is the number itself from 0 to 7, the sign bit and
+ * its magnitude below */
+__device__ __forceinline__ uint32_t f6_codes(uint32_t v) {
+  const uint32_t t = v ^ 0x08080808u, m = (t >> 3) & 0x01010101u; /* m: below zero, where t = v + 8 */
+  const uint32_t code = (((t ^ ((m << 8) - m)) + m) & 0x0f0f0f0fu) | (m << 5);
+  const uint32_t pairs = (code & 0x003f003fu) | ((code >> 2) & 0x0fc00fc0u);
+  return (pairs & 0xfffu) | ((pairs >> 4) & 0xfff000u);
+}
+
+/* A wavefront takes half a chunk (four blocks) of a tile's 32 rows: 64 bytes a row in, four lanes a row, through LDS to
+ * lane (column, g), which writes twelve of its 24 dwords, three whole kilobytes a wavefront. */
+__device__ __forceinline__ void f6_copy(const uint8_t *__restrict__ qs, const uint16_t *__restrict__ d, int N, int nb, int chunks,
+                                        uint8_t *__restrict__ out, int block) {
+  __shared__ __attribute__((aligned(16))) uint4 rows[4][32][5]; /* a row's four blocks, and a gap against bank conflicts */
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, i32 = lane & 31, g = lane >> 5;
+  const uint32_t unit = (uint32_t)block * 4 + wave; /* (tile, chunk, half) */
+  const uint32_t tc = unit >> 1, tile = tc / (uint32_t)chunks; /* tc: tile * chunks + chunk */
+  const int half = (int)(unit & 1);
+  const int64_t n0 = (int64_t)tile * 32;
+  const int b0 = (int)(tc - tile * (uint32_t)chunks) * 8 + half * 4; /* first block in the row */
+  const bool live = n0 < N;                         /* the last workgroup may have wavefronts to spare */
 #pragma unroll
-  for (int i = 0; i < 16; ++i) { /* byte i of a block = elements i (low nibble) and i + 16 */
-    const int v = (int)((x4[i >> 2] >> (8 * (i & 3) + 4 * g)) & 15u) - 8;
-    const uint32_t code = v < 0 ? 0x20u | (uint32_t)(-v) : (uint32_t)v; /* fp6 codes up to 15 are the number itself */
-    const int bit = 6 * i;
-    w[bit >> 5] |= code << (bit & 31);
-    if ((bit & 31) > 26) w[(bit >> 5) + 1] |= code >> (32 - (bit & 31));
+  for (int i = 0; i < 2; ++i) {
+    const int r = i * 16 + (lane >> 2), b = b0 + (lane & 3);
+    uint4 x = make_uint4(0x88888888u, 0x88888888u, 0x88888888u, 0x88888888u); /* weights of zero */
+    if (n0 + r < N && b < nb) x = *(const uint4 *)(qs + ((n0 + r) * nb + b) * 16);
+    rows[wave][r][lane & 3] = x;
   }
+  uint32_t sc = 0; /* the scales of blocks 2 g and 2 g + 1 of the half */
 #pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    const int k = 3 * j + i;
-    *(uint32_t *)(dst + (k >> 2) * 1024 + lane * 16 + (k & 3) * 4) = w[i];
+  for (int i = 0; i < 2; ++i) {
+    const int b = b0 + 2 * g + i;
+    if (n0 + i32 < N && b < nb) sc |= (uint32_t)d[(n0 + i32) * nb + b] << (16 * i);
   }
-  if (!g) *(uint16_t *)(dst + 6144 + i32 * 16 + j * 2) = in ? d[n * nb + b] : (uint16_t)0;
+  __syncthreads();
+  if (!live) return;
+  uint32_t w[12];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) { /* byte i of a block = elements i (low nibble) and i + 16 */
+    const uint4 x = rows[wave][i32][j];
+    const uint32_t a = f6_codes((x.x >> (4 * g)) & 0x0f0f0f0fu), b = f6_codes((x.y >> (4 * g)) & 0x0f0f0f0fu),
+                   c = f6_codes((x.z >> (4 * g)) & 0x0f0f0f0fu), e = f6_codes((x.w >> (4 * g)) & 0x0f0f0f0fu);
+    w[3 * j] = a | (b << 24);
+    w[3 * j + 1] = (b >> 8) | (c << 16);
+    w[3 * j + 2] = (c >> 16) | (e << 8);
+  }
+  uint8_t *dst = out + (size_t)tc * WTILE;
+#pragma unroll
+  for (int p = 0; p < 3; ++p)
+    *(uint4 *)(dst + (3 * half + p) * 1024 + lane * 16) = make_uint4(w[4 * p], w[4 * p + 1], w[4 * p + 2], w[4 * p + 3]);
+  *(uint32_t *)(dst + 6144 + i32 * 16 + half * 8 + g * 4) = sc;
+}
+
+/* f6_copy of workgroup `block`. A macro, so that the struct's members are picked where it is a kernel's argument: picked
+ * through a reference it went to scratch memory */
+#define F6_COPY(cw, block)                                                                                       \
+  do {                                                                                                           \
+    int wi = 0, begin = 0;                                                                                       \
+    if ((block) >= cw.end[0]) wi = 1, begin = cw.end[0];                                                         \
+    if ((block) >= cw.end[1]) wi = 2, begin = cw.end[1];                                                         \
+    if ((block) >= cw.end[2]) wi = 3, begin = cw.end[2];                                                         \
+    f6_copy(wi == 0 ? cw.qs[0] : wi == 1 ? cw.qs[1] : wi == 2 ? cw.qs[2] : cw.qs[3],                             \
+            wi == 0 ? cw.d[0] : wi == 1 ? cw.d[1] : wi == 2 ? cw.d[2] : cw.d[3],                                 \
+            wi == 0 ? cw.N[0] : wi == 1 ? cw.N[1] : wi == 2 ? cw.N[2] : cw.N[3], cw.nb, cw.chunks,               \
+            wi == 0 ? cw.out[0] : wi == 1 ? cw.out[1] : wi == 2 ? cw.out[2] : cw.out[3], (block)-begin);         \
+  } while (0)
+
+__global__ __launch_bounds__(256) void f6_weights_kernel(CopyF6 cw) { F6_COPY(cw, (int)blockIdx.x); }
+
+/* ---- the activations ---- */
+
+/* A value of magnitude at most 128 as two bf6 (e3m2) codes in units of 1/16: the magnitude rounded to three
+ * significant bits, and the rest (at most 8: codes up to 8 are the number itself). */
+__device__ __forceinline__ void bf6_parts(int v, uint32_t &first, uint32_t &second) {
+  const int mag = v < 0 ? -v : v;
+  const uint32_t t = (__float_as_uint((float)mag) + (1u << 20)) >> 21; /* exponent and two mantissa bits */
+  const bool small = mag < 4;
+  const int rest = small ? 0 : mag - (int)__uint_as_float(t << 21);
+  const uint32_t sign = v < 0 ? 0x20u : 0u;
+  first = sign | (small ? (uint32_t)mag : t - 512u);
+  second = (rest < 0 ? (sign ^ 0x20u) | (uint32_t)(-rest) : sign | (uint32_t)rest);
+}
+
+/* Q8_0 in the form of the six-bit GEMM (QActF6). A wavefront takes one block of eight consecutive rows, eight lanes a
+ * row (128 bytes of a row in, two whole lines of operands out). Rows M and beyond of the last 64 and blocks of K and
+ * beyond are written as zeros. */
+struct RowsF6 {
+  const float *A;
+  int64_t M, lda;
+  uint32_t n_units; /* octets of rows (padding included) x blocks */
+  int nbp, K;
+  uint8_t *out;
+};
+__device__ __forceinline__ void f6_quantize(const RowsF6 &p, int block) {
+  const int64_t M = p.M;
+  const int K = p.K, nbp = p.nbp;
+  constexpr int PARTS = hipq::F6_ROWS * 384;
+  const uint32_t unit = (uint32_t)block * 4 + (threadIdx.x >> 6);
+  if (unit >= p.n_units) return; /* uniform per wavefront */
+  const int lane = threadIdx.x & 63, sub = lane & 7;
+  const uint32_t octet = unit / (uint32_t)nbp; /* a 64-bit quotient was half of the kernel's instructions */
+  const int b = (int)(unit - octet * (uint32_t)nbp);
+  const int64_t m = (int64_t)octet * 8 + (lane >> 3);
+  float4 x = *(const float4 *)(p.A + (m < M ? m : M - 1) * p.lda + min(b * 32 + 4 * sub, K - 4));
+  if (m >= M || b * 32 >= K) x = make_float4(0.f, 0.f, 0.f, 0.f);
+  uint16_t dh;
+  int qsum;
+  const uint32_t q = (uint32_t)hipq_quantize_q8_0_lane(x, dh, qsum);
+  uint32_t part[2] = {0, 0}; /* this lane's four codes of each part, 24 bits */
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    uint32_t first, second;
+    bf6_parts((int)(int8_t)(q >> (8 * k)), first, second);
+    part[0] |= first << (6 * k);
+    part[1] |= second << (6 * k);
+  }
+  uint32_t w[6]; /* the quad's sixteen values: 96 bits of each part */
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int mine = (int)part[h];
+    const uint32_t x0 = (uint32_t)hipq_dpp_i<0x00>(mine), x1 = (uint32_t)hipq_dpp_i<0x55>(mine),
+                   x2 = (uint32_t)hipq_dpp_i<0xAA>(mine), x3 = (uint32_t)hipq_dpp_i<0xFF>(mine);
+    w[3 * h] = x0 | (x1 << 24);
+    w[3 * h + 1] = (x1 >> 8) | (x2 << 16);
+    w[3 * h + 2] = (x2 >> 16) | (x3 << 8);
+  }
+  const int r = (int)(m & (hipq::F6_ROWS - 1)), g = sub >> 2, j = b & 7;
+  uint8_t *dst = p.out + ((m / hipq::F6_ROWS) * (nbp >> 3) + (b >> 3)) * hipq::F6_CHUNK;
+  uint8_t *o = dst + (r >> 5) * (PARTS / 2) + j * 1536;
+  const int at = g * 32 + (r & 31);
+  if ((lane & 3) == 0) *(uint4 *)(o + at * 16) = make_uint4(w[0], w[1], w[2], w[3]);
+  if ((lane & 3) == 1) *(uint2 *)(o + 1024 + at * 8) = make_uint2(w[4], w[5]);
+  if (sub == 0) *(uint16_t *)(dst + PARTS + r * 16 + j * 2) = dh;
+}
+
+__global__ __launch_bounds__(256) void quantize_q8_0_f6_kernel(RowsF6 p) { f6_quantize(p, (int)blockIdx.x); }
+
+/* Both in one launch, for the call that makes the copies: the copies' workgroups in front, their reads of weights that
+ * no cache holds beside the quantization. First pass of four decoder layers of 1024 / 3072 over 512 rows, fresh weights:
+ * 470 us with an allocation, an event and a launch a weight, 380 with the copies of a call in a launch of their own in
+ * front of the quantizer's, 329 this way (272 from the second pass on; 360 with the int8 kernel, which needs no copy). */
+__global__ __launch_bounds__(256) void quantize_copy_f6_kernel(RowsF6 p, CopyF6 cw) {
+  if ((int)blockIdx.x < cw.end[3]) /* uniform */
+    F6_COPY(cw, (int)blockIdx.x);
+  else
+    f6_quantize(p, (int)blockIdx.x - cw.end[3]);
 }
 
 } // namespace
@@ -319,12 +452,12 @@ __global__ __launch_bounds__(256) void f6_weights_kernel(const uint8_t *__restri
 namespace hipq {
 
 /* ---- who may read a copy ----
- * A copy is made on the stream of the product that asks for it, in front of that product, and nothing waits. Until it
- * is known to be complete it is PENDING, and only the stream it was made on may read it; a product on another stream
- * takes the kernels that read the weight as stored (the same bits). Complete is what the page-locked word of its batch
- * says, which the quantizer behind the copies sets: a plain read, so also a call that is being captured into a graph,
- * where events may not be queried, finds out. A graph may be launched on any stream, so a captured product reads
- * complete copies only.
+ * A copy is made by the product that asks for it, in the launch of its quantizer, and nothing waits. Until it is known
+ * to be complete it is PENDING, and only the stream it was made on may read it; a product on another stream takes the
+ * kernels that read the weight as stored (the same bits). Complete is what the page-locked word of its batch says, which
+ * the product behind the quantizer sets: a plain read, so also a call that is being captured into a graph, where events
+ * may not be queried, finds out. A graph may be launched on any stream, so a captured product reads complete copies
+ * only.
  * The same stream is known by its handle alone, and one handle can stand for two streams (hipStreamPerThread; a stream
  * made after another was destroyed): the event of the batch orders those. */
 struct F6Batch {
@@ -333,6 +466,22 @@ struct F6Batch {
   hipStream_t s;
   int refs; /* PENDING weights that point here */
   F6Batch *next;
+};
+
+/* The copies' memory: blocks of 64 MiB (a copy of more than half that has one of its own size), the first gap that is
+ * large enough, given back with the last copy in it; one empty block is kept for the next weights. A hipMalloc for each
+ * copy took 13 to 30 us of the first product. */
+struct F6Block;
+struct F6Copy {
+  F6Block *block;
+  size_t at, bytes; /* multiples of 256 */
+  F6Copy *next;     /* the block's copies in the order of their places */
+};
+struct F6Block {
+  uint8_t *base;
+  size_t size;
+  F6Copy *first;
+  F6Block *next;
 };
 
 namespace {
@@ -350,6 +499,73 @@ void batch_idle(F6Batch *b) {
   b->next = f6_idle;
   f6_idle = b;
 }
+
+constexpr size_t F6_BLOCK = (size_t)64 << 20;
+F6Block *f6_blocks = nullptr;
+
+int mem_get(size_t bytes, F6Copy **out) {
+  F6Copy *c = new (std::nothrow) F6Copy();
+  if (!c) return fail(HIPQ_ERR_OUT_OF_MEMORY, "host allocation failed");
+  c->bytes = bytes;
+  for (F6Block *b = f6_blocks; b && !c->block; b = b->next) {
+    size_t end = 0; /* of the copy in front */
+    F6Copy **at = &b->first;
+    for (; *at && (*at)->at - end < bytes; at = &(*at)->next) end = (*at)->at + (*at)->bytes;
+    if (!*at && b->size - end < bytes) continue;
+    c->block = b, c->at = end, c->next = *at;
+    *at = c;
+  }
+  if (!c->block) {
+    F6Block *b = new (std::nothrow) F6Block();
+    hipError_t e = hipErrorOutOfMemory;
+    if (b) {
+      b->size = bytes > F6_BLOCK / 2 ? bytes : F6_BLOCK;
+      e = hipMalloc((void **)&b->base, b->size);
+      if (e != hipSuccess && b->size > bytes) { /* a full device may still have room for this one */
+        (void)hipGetLastError();
+        b->size = bytes;
+        e = hipMalloc((void **)&b->base, b->size);
+      }
+    }
+    if (e != hipSuccess) {
+      delete b;
+      delete c;
+      return fail(HIPQ_ERR_OUT_OF_MEMORY, "six-bit copy of %zu bytes: %s", bytes, hipGetErrorString(e));
+    }
+    c->block = b, b->first = c;
+    b->next = f6_blocks;
+    f6_blocks = b;
+  }
+  *out = c;
+  return HIPQ_OK;
+}
+/* gives back the empty blocks, one of which may stay for the next weights */
+void mem_trim(bool keep) {
+  for (F6Block **at = &f6_blocks; *at;) {
+    F6Block *b = *at;
+    if (!b->first && keep && b->size == F6_BLOCK) {
+      keep = false;
+    } else if (!b->first) {
+      *at = b->next;
+      (void)hipFree(b->base);
+      delete b;
+      continue;
+    }
+    at = &b->next;
+  }
+}
+void copy_put(hipq_weight *w) {
+  F6Copy *c = w->gf_copy;
+  if (!c) return;
+  F6Copy **at = &c->block->first;
+  while (*at != c) at = &(*at)->next;
+  *at = c->next;
+  if (!c->block->first) mem_trim(true);
+  delete c;
+  w->gf_copy = nullptr;
+  w->gf_base = nullptr;
+}
+
 int batch_get(hipStream_t s, F6Batch **out) {
   if (!f6_idle) {
     F6Page *pg = new (std::nothrow) F6Page();
@@ -382,6 +598,15 @@ void batch_drop(hipq_weight *w) {
   if (b && --b->refs == 0) batch_idle(b);
 }
 
+void make_undo(F6Make &m) {
+  for (int i = 0; i < m.count; ++i) {
+    copy_put(m.w[i]);
+    m.w[i]->gf_state = F6_NONE;
+  }
+  m.count = 0;
+  batch_idle(m.batch);
+}
+
 /* Whether the weight's copy is complete; looks up to `spins` times more */
 bool complete(hipq_weight *w, int &spins) {
   if (w->gf_state == F6_PENDING) {
@@ -397,11 +622,10 @@ bool complete(hipq_weight *w, int &spins) {
 }
 } // namespace
 
-/* *ready: what is enqueued on s next may read the copies of the weights. Missing ones are made where may_make and the
- * stream is not being captured; the caller then hands *word to the quantizer it launches behind them. */
-int f6_copies(int count, const hipq_weight *const *cw, hipStream_t s, bool may_make, bool *ready, uint32_t **word) {
+/* *ready: the products a call enqueues on s next may read the copies of the weights. For those that are missing, where
+ * may_make and the stream is not being captured, `make` has the memory; the call hands it to its quantizer. */
+int f6_copies(int count, const hipq_weight *const *cw, hipStream_t s, bool may_make, bool *ready, F6Make *make) {
   *ready = false;
-  *word = nullptr;
   int done = 0;
   for (int i = 0; i < count; ++i) done += __atomic_load_n(&cw[i]->gf_state, __ATOMIC_ACQUIRE) == F6_COMPLETE;
   if (done == count) {
@@ -419,9 +643,11 @@ int f6_copies(int count, const hipq_weight *const *cw, hipStream_t s, bool may_m
   int spins = capturing ? 20000 : 0;
   F6Batch *behind = nullptr;
   for (int i = 0; i < count; ++i) {
+    if (w[i]->gf_state == F6_MAKING) return HIPQ_OK; /* another thread is about to enqueue it */
     if (w[i]->gf_state == F6_NONE) {
       if (w[i]->dtype != HIPQ_Q4_0 || w[i]->expert_tiles)
         return fail(HIPQ_ERR_INVALID_ARGUMENT, "only Q4_0 weights in the plane layout have a six-bit copy");
+      if (w[i]->K != w[0]->K) return fail(HIPQ_ERR_INVALID_ARGUMENT, "the copies of one call are of one K");
       ++missing;
     } else if (!complete(w[i], spins)) {
       F6Batch *b = w[i]->gf_batch;
@@ -431,58 +657,89 @@ int f6_copies(int count, const hipq_weight *const *cw, hipStream_t s, bool may_m
     }
   }
   if (missing) {
-    if (!may_make || capturing) return HIPQ_OK;
-    F6Batch *b = nullptr;
-    if (int rc = batch_get(s, &b)) return rc;
-    int made = 0, rc = HIPQ_OK;
-    hipq_weight *fresh[64];
-    for (int i = 0; i < count && !rc && made < 64; ++i) {
+    if (!may_make || capturing || missing > F6Make::MOST) return HIPQ_OK;
+    if (int rc = batch_get(s, &make->batch)) return rc;
+    const int64_t chunks = (w[0]->K + 255) / 256;
+    for (int i = 0; i < count; ++i) {
       hipq_weight *x = w[i];
-      if (x->gf_state != F6_NONE || x->gf_base) continue; /* a weight may stand in the list twice */
-      const int nb = (int)(x->K / 32), chunks = (nb + 7) / 8;
-      const int64_t tiles = (x->N + 31) / 32, threads = tiles * chunks * 512;
-      const size_t bytes = (size_t)tiles * chunks * F6_WTILE;
-      uint8_t *p = nullptr;
-      hipError_t e = hipMalloc((void **)&p, bytes);
-      if (e != hipSuccess) {
-        rc = fail(HIPQ_ERR_OUT_OF_MEMORY, "six-bit copy of %zu bytes: %s", bytes, hipGetErrorString(e));
-        break;
+      if (x->gf_state != F6_NONE) continue; /* has one, or stands in the list twice */
+      if (int rc = mem_get((size_t)((x->N + 31) / 32 * chunks) * F6_WTILE, &x->gf_copy)) {
+        make_undo(*make);
+        return rc;
       }
-      x->gf_base = p;
-      fresh[made++] = x;
-      launch_kernel("f6_weights_kernel", f6_weights_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, x->qs, x->d,
-                    (int)x->N, nb, chunks, threads, p);
-      if ((e = hipGetLastError()) != hipSuccess) rc = fail(HIPQ_ERR_RUNTIME, "six-bit copy: %s", hipGetErrorString(e));
+      x->gf_base = x->gf_copy->block->base + x->gf_copy->at;
+      x->gf_state = F6_MAKING;
+      make->w[make->count++] = x;
     }
-    if (!rc) {
-      const hipError_t e = hipEventRecord(b->ev, s);
-      if (e != hipSuccess) rc = fail(HIPQ_ERR_RUNTIME, "six-bit copy: %s", hipGetErrorString(e));
-    }
-    if (rc) {
-      if (made) (void)hipStreamSynchronize(s);
-      for (int i = 0; i < made; ++i) {
-        (void)hipFree(fresh[i]->gf_base);
-        fresh[i]->gf_base = nullptr;
-      }
-      batch_idle(b);
-      return rc;
-    }
-    for (int i = 0; i < made; ++i) {
-      fresh[i]->gf_batch = b;
-      __atomic_store_n(&fresh[i]->gf_state, F6_PENDING, __ATOMIC_RELEASE);
-    }
-    b->refs = made;
-    *word = b->word_dev;
   }
   *ready = true;
+  return HIPQ_OK;
+}
+
+F6Make::~F6Make() { /* a call that failed between f6_copies and its quantizer's launch */
+  if (!count) return;
+  std::lock_guard<std::mutex> lk(f6_mu);
+  make_undo(*this);
+}
+
+size_t qact_f6_bytes(int64_t M, int64_t K) {
+  return (size_t)((M + F6_ROWS - 1) / F6_ROWS) * (size_t)((K + 255) / 256) * F6_CHUNK;
+}
+QActF6 qact_f6_carve(void *mem, int64_t M, int64_t K) {
+  return QActF6{(uint8_t *)mem, (int)M, (int)K, (int)((K + 255) / 256), nullptr};
+}
+
+int launch_quantize_q8_0_f6(const float *A, int64_t M, int64_t K, int64_t lda, QActF6 *qa, F6Make *make, hipStream_t s) {
+  if (M <= 0) return HIPQ_OK;
+  if (K % 32 || lda < K) return fail(HIPQ_ERR_INVALID_ARGUMENT, "Q8_0: K=%lld must be a multiple of 32 and lda >= K", (long long)K);
+  if (((uintptr_t)A & 15) || (lda & 3))
+    return fail(HIPQ_ERR_INVALID_ARGUMENT, "activation rows must be 16-byte aligned");
+  const int64_t units = (M + F6_ROWS - 1) / F6_ROWS * (F6_ROWS / 8) * (qa->chunks * 8); /* padding included */
+  if (units > INT32_MAX) return fail(HIPQ_ERR_NOT_SUPPORTED, "%lld x %lld values in one call", (long long)M, (long long)K);
+  const RowsF6 rows{A, M, lda, (uint32_t)units, qa->chunks * 8, (int)K, qa->p};
+  const unsigned blocks = (unsigned)((units + 3) / 4);
+  if (!make || !make->count) {
+    launch_kernel("quantize_q8_0_f6_kernel", quantize_q8_0_f6_kernel, dim3(blocks), dim3(256), 0, s, rows);
+    HIPQ_HIP(hipGetLastError());
+    return HIPQ_OK;
+  }
+  for (int i = (make->count - 1) / 4 * 4; i >= 0; i -= 4) { /* four copies a launch, the last ones with the rows */
+    CopyF6 cw;
+    cw.nb = (int)(K / 32);
+    cw.chunks = qa->chunks;
+    int end = 0;
+    for (int k = 0; k < 4; ++k) {
+      const hipq_weight *x = make->w[std::min(i + k, make->count - 1)];
+      cw.qs[k] = x->qs, cw.d[k] = x->d, cw.out[k] = x->gf_base, cw.N[k] = (int)x->N;
+      if (i + k < make->count) end += (int)(((x->N + 31) / 32 * cw.chunks + 1) / 2); /* four half chunks a workgroup */
+      cw.end[k] = end;
+    }
+    if (i)
+      launch_kernel("f6_weights_kernel", f6_weights_kernel, dim3((unsigned)end), dim3(256), 0, s, cw);
+    else
+      launch_kernel("quantize_copy_f6_kernel", quantize_copy_f6_kernel, dim3((unsigned)end + blocks), dim3(256), 0, s, rows, cw);
+  }
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess) e = hipEventRecord(make->batch->ev, s);
+  if (e != hipSuccess) {
+    (void)hipStreamSynchronize(s); /* before ~F6Make gives the copies' memory back */
+    return fail(HIPQ_ERR_RUNTIME, "six-bit copies: %s", hipGetErrorString(e));
+  }
+  qa->word = make->batch->word_dev;
+  std::lock_guard<std::mutex> lk(f6_mu);
+  for (int i = 0; i < make->count; ++i) {
+    make->w[i]->gf_batch = make->batch;
+    __atomic_store_n(&make->w[i]->gf_state, F6_PENDING, __ATOMIC_RELEASE);
+  }
+  make->batch->refs = make->count;
+  make->count = 0;
   return HIPQ_OK;
 }
 
 void f6_release(hipq_weight *w) {
   std::lock_guard<std::mutex> lk(f6_mu);
   batch_drop(w);
-  if (w->gf_base) (void)hipFree(w->gf_base);
-  w->gf_base = nullptr;
+  copy_put(w);
   w->gf_state = F6_NONE;
 }
 
@@ -496,6 +753,7 @@ void f6_shutdown() {
     delete pg;
   }
   f6_idle = nullptr;
+  mem_trim(false);
 }
 
 int launch_gemm_f6(int count, const hipq_weight *const *w, const QActF6 *qa, int M, float *const *C, const int64_t *ldc,
@@ -514,6 +772,7 @@ int launch_gemm_f6(int count, const hipq_weight *const *w, const QActF6 *qa, int
     if (i < count) tiles += (int)((w[k]->N + BN - 1) / BN);
     mw.tile_end[i] = tiles; /* unused entries repeat the total: no workgroup lands in them */
   }
+  mw.word = qa->word;
   const int mtiles = (M + BM - 1) / BM;
   const dim3 grid((unsigned)(mtiles * ((tiles + 7) / 8) * 8));
   /* up to two workgroups a CU: the deeper read-ahead (512 rows of 1024 x 3072 13.1 -> 12.0 us, 1024 x 1024 7.5 -> 6.7);
@@ -532,7 +791,7 @@ int launch_gemm_f6_gated(const hipq_weight *wa, const hipq_weight *wm, const QAc
                          hipStream_t s) {
   if (!wa->gf_base || !wm->gf_base || wa->K != wm->K || wa->N != wm->N || wa->K != qa->K || M != qa->M)
     return fail(HIPQ_ERR_INVALID_ARGUMENT, "the gated pair has one shape and its six-bit copies");
-  const GatedF6 p{wa->gf_base, wm->gf_base, out, ldo, (int)wa->N, (int)((wa->N + 63) / 64)};
+  const GatedF6 p{wa->gf_base, wm->gf_base, out, ldo, (int)wa->N, (int)((wa->N + 63) / 64), qa->word};
   const int mtiles = (M + BM - 1) / BM;
   const dim3 grid((unsigned)(mtiles * ((p.ntiles + 7) / 8) * 8));
   /* the bound of launch_gemm_f6 */

@@ -55,7 +55,8 @@
 /* ------------------------------------------------------------------------- */
 namespace hipq {
 struct F6Batch;
-enum { F6_NONE, F6_PENDING, F6_COMPLETE };
+struct F6Copy;
+enum { F6_NONE, F6_MAKING, F6_PENDING, F6_COMPLETE };
 } // namespace hipq
 struct hipq_weight {
   int dtype;
@@ -90,7 +91,8 @@ struct hipq_weight {
    *     16 g .. 16 g + 15, three dwords a block one behind the other, four dwords a piece;
    *   [32][8] fp16 block scales. */
   uint8_t *gf_base;
-  int gf_state;             /* hipq::F6_NONE, F6_PENDING, F6_COMPLETE: read with acquire, written under f6_copies' mutex */
+  int gf_state;             /* hipq::F6_NONE, .. F6_COMPLETE: read with acquire, written under f6_copies' mutex */
+  hipq::F6Copy *gf_copy;    /* the memory gf_base points to */
   hipq::F6Batch *gf_batch;  /* PENDING: what the copies enqueued with this one have in common */
 };
 
@@ -170,6 +172,7 @@ QActTiled qact_tiled_carve(void *mem, int64_t M, int64_t K);
 struct QActF6 {
   uint8_t *p;
   int M, K, chunks;
+  uint32_t *word; /* where the quantizer made copies of weights: for the product behind it to set (f6_copies) */
 };
 
 namespace hipq {
@@ -238,8 +241,8 @@ int launch_quantize_q8_K_tiled(const float *A, int64_t M, int64_t K, int64_t lda
 /* the values of launch_quantize_q8_0 in the form of the six-bit GEMM */
 size_t qact_f6_bytes(int64_t M, int64_t K);
 QActF6 qact_f6_carve(void *mem, int64_t M, int64_t K);
-/* `word` (may be null): a word of page-locked memory the kernel sets to 1 (f6_copies) */
-int launch_quantize_q8_0_f6(const float *A, int64_t M, int64_t K, int64_t lda, const QActF6 *qa, uint32_t *word, hipStream_t s);
+struct F6Make;
+int launch_quantize_q8_0_f6(const float *A, int64_t M, int64_t K, int64_t lda, QActF6 *qa, F6Make *make, hipStream_t s);
 
 /* gemv.hip ---------------------------------------------------------------- */
 /* C[m][n] for m < M <= 8: one pass over the weights, M activation rows.
@@ -266,7 +269,17 @@ int launch_gemm(const hipq_weight *w, const QAct *qa, int M, float *C,
 int launch_gemm_multi(int count, const hipq_weight *const *w, const QAct *qa, int M, float *const *C,
                       const int64_t *ldc, hipStream_t s);
 /* gemm_f6.hip: up to four Q4_0 weights of one K, each with its six-bit copy, one launch */
-int f6_copies(int count, const hipq_weight *const *w, hipStream_t s, bool may_make, bool *ready, uint32_t **word);
+struct F6Make { /* copies that a call makes: memory of f6_copies, launched by launch_quantize_q8_0_f6 */
+  static constexpr int MOST = 64;
+  hipq_weight *w[MOST];
+  int count = 0;
+  F6Batch *batch = nullptr;
+  F6Make() {}
+  ~F6Make();
+  F6Make(const F6Make &) = delete;
+  F6Make &operator=(const F6Make &) = delete;
+};
+int f6_copies(int count, const hipq_weight *const *w, hipStream_t s, bool may_make, bool *ready, F6Make *make);
 void f6_release(hipq_weight *w); /* the device no longer reads or writes the weight's copy */
 void f6_shutdown();              /* no weight is left */
 int launch_gemm_f6(int count, const hipq_weight *const *w, const QActF6 *qa, int M, float *const *C, const int64_t *ldc,

@@ -58,64 +58,6 @@ __global__ __launch_bounds__(256) void quantize_q8_0_kernel(
   }
 }
 
-/* A value of magnitude at most 128 as two bf6 (e3m2) codes in units of 1/16: the magnitude rounded to three
- * significant bits, and the rest (at most 8: codes up to 8 are the number itself). */
-__device__ __forceinline__ void bf6_parts(int v, uint32_t &first, uint32_t &second) {
-  const int mag = v < 0 ? -v : v;
-  const uint32_t t = (__float_as_uint((float)mag) + (1u << 20)) >> 21; /* exponent and two mantissa bits */
-  const bool small = mag < 4;
-  const int rest = small ? 0 : mag - (int)__uint_as_float(t << 21);
-  const uint32_t sign = v < 0 ? 0x20u : 0u;
-  first = sign | (small ? (uint32_t)mag : t - 512u);
-  second = (rest < 0 ? (sign ^ 0x20u) | (uint32_t)(-rest) : sign | (uint32_t)rest);
-}
-
-/* Q8_0 in the form of the six-bit GEMM (QActF6). A wavefront takes one block of eight consecutive rows, eight lanes a
- * row (128 bytes of a row in, two whole lines of operands out). Rows M and beyond of the last 64 and blocks of K and
- * beyond are written as zeros. */
-__global__ __launch_bounds__(256) void quantize_q8_0_f6_kernel(const float *__restrict__ A, int64_t M, int64_t n_units, int nbp,
-                                                               int K, int64_t lda, uint8_t *__restrict__ out, uint32_t *word) {
-  /* what was enqueued in front of this kernel is complete: stream order, no fence is needed for it */
-  if (word && blockIdx.x == 0 && threadIdx.x == 0) __hip_atomic_store(word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-  constexpr int PARTS = hipq::F6_ROWS * 384;
-  const int64_t unit = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (unit >= n_units) return; /* uniform per wavefront */
-  const int lane = threadIdx.x & 63, sub = lane & 7;
-  const int64_t octet = unit / nbp;
-  const int b = (int)(unit - octet * nbp);
-  const int64_t m = octet * 8 + (lane >> 3);
-  float4 x = *(const float4 *)(A + (m < M ? m : M - 1) * lda + min(b * 32 + 4 * sub, K - 4));
-  if (m >= M || b * 32 >= K) x = make_float4(0.f, 0.f, 0.f, 0.f);
-  uint16_t dh;
-  int qsum;
-  const uint32_t q = (uint32_t)hipq_quantize_q8_0_lane(x, dh, qsum);
-  uint32_t part[2] = {0, 0}; /* this lane's four codes of each part, 24 bits */
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    uint32_t first, second;
-    bf6_parts((int)(int8_t)(q >> (8 * k)), first, second);
-    part[0] |= first << (6 * k);
-    part[1] |= second << (6 * k);
-  }
-  uint32_t w[6]; /* the quad's sixteen values: 96 bits of each part */
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int mine = (int)part[h];
-    const uint32_t x0 = (uint32_t)hipq_dpp_i<0x00>(mine), x1 = (uint32_t)hipq_dpp_i<0x55>(mine),
-                   x2 = (uint32_t)hipq_dpp_i<0xAA>(mine), x3 = (uint32_t)hipq_dpp_i<0xFF>(mine);
-    w[3 * h] = x0 | (x1 << 24);
-    w[3 * h + 1] = (x1 >> 8) | (x2 << 16);
-    w[3 * h + 2] = (x2 >> 16) | (x3 << 8);
-  }
-  const int r = (int)(m & (hipq::F6_ROWS - 1)), g = sub >> 2, j = b & 7;
-  uint8_t *dst = out + ((m / hipq::F6_ROWS) * (nbp >> 3) + (b >> 3)) * hipq::F6_CHUNK;
-  uint8_t *o = dst + (r >> 5) * (PARTS / 2) + j * 1536;
-  const int at = g * 32 + (r & 31);
-  if ((lane & 3) == 0) *(uint4 *)(o + at * 16) = make_uint4(w[0], w[1], w[2], w[3]);
-  if ((lane & 3) == 1) *(uint2 *)(o + 1024 + at * 8) = make_uint2(w[4], w[5]);
-  if (sub == 0) *(uint16_t *)(dst + PARTS + r * 16 + j * 2) = dh;
-}
-
 /* ---- Q8_K ---------------------------------------------------------------- */
 
 /* One wavefront per (row, super-block). */
@@ -264,26 +206,6 @@ int launch_quantize_q8_0(const float *A, int64_t M, int64_t K, int64_t lda,
   else
     hipq::launch_kernel("quantize_q8_0_kernel<false>", quantize_q8_0_kernel<false>, dim3(grid), dim3(256), 0, s, A, total, nb, lda,
                        qa->q, qa->meta, nullptr);
-  HIPQ_HIP(hipGetLastError());
-  return HIPQ_OK;
-}
-
-size_t qact_f6_bytes(int64_t M, int64_t K) {
-  return (size_t)((M + F6_ROWS - 1) / F6_ROWS) * (size_t)((K + 255) / 256) * F6_CHUNK;
-}
-QActF6 qact_f6_carve(void *mem, int64_t M, int64_t K) {
-  return QActF6{(uint8_t *)mem, (int)M, (int)K, (int)((K + 255) / 256)};
-}
-
-int launch_quantize_q8_0_f6(const float *A, int64_t M, int64_t K, int64_t lda, const QActF6 *qa, uint32_t *word,
-                            hipStream_t s) {
-  if (M <= 0) return HIPQ_OK;
-  if (K % 32 || lda < K) return fail(HIPQ_ERR_INVALID_ARGUMENT, "Q8_0: K=%lld must be a multiple of 32 and lda >= K", (long long)K);
-  if (((uintptr_t)A & 15) || (lda & 3))
-    return fail(HIPQ_ERR_INVALID_ARGUMENT, "activation rows must be 16-byte aligned");
-  const int64_t units = (M + F6_ROWS - 1) / F6_ROWS * (F6_ROWS / 8) * (qa->chunks * 8); /* padding included */
-  launch_kernel("quantize_q8_0_f6_kernel", quantize_q8_0_f6_kernel, dim3((unsigned)((units + 3) / 4)), dim3(256), 0, s, A, M,
-                units, qa->chunks * 8, (int)K, lda, qa->p, word);
   HIPQ_HIP(hipGetLastError());
   return HIPQ_OK;
 }
