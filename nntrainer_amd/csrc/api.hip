@@ -786,15 +786,16 @@ int f6_ready(int count, const hipq_weight *const *w, int64_t M, hipStream_t s, c
   return rc == HIPQ_ERR_OUT_OF_MEMORY ? HIPQ_OK : rc;
 }
 
-/* count (1 to 4) weights with their copies, one quantization (unless the last call on the scratch made it) and launch */
+/* weights with their copies: one quantization, four weights a launch */
 int matmul_f6(int count, const hipq_weight *const *w, const float *A, int64_t M, int64_t lda, float *const *C,
-              const int64_t *ldc, hipStream_t s, const Scratch &sc, hipq::F6Make *make, bool quantize = true) {
+              const int64_t *ldc, hipStream_t s, const Scratch &sc, hipq::F6Make *make) {
   void *mem = nullptr;
   if (int rc = sc.get(hipq::qact_f6_bytes(M, w[0]->K), &mem)) return rc;
   QActF6 qa = hipq::qact_f6_carve(mem, M, w[0]->K);
-  if (quantize)
-    if (int rc = hipq::launch_quantize_q8_0_f6(A, M, w[0]->K, lda, &qa, make, s)) return rc;
-  return hipq::launch_gemm_f6(count, w, &qa, (int)M, C, ldc, s);
+  if (int rc = hipq::launch_quantize_q8_0_f6(A, M, w[0]->K, lda, &qa, make, s)) return rc;
+  for (int i = 0; i < count; i += 4)
+    if (int rc = hipq::launch_gemm_f6(std::min(4, count - i), w + i, &qa, (int)M, C + i, ldc + i, s)) return rc;
+  return HIPQ_OK;
 }
 
 /* Whether launch_gated serves the gated pair of an MLP at M rows: where hipq_matmul_multi sends both products through one
@@ -1736,10 +1737,7 @@ int hipq_matmul_multi(int count, const hipq_weight_t *w, const float *A, int64_t
       hipq::F6Make make;
       if (members <= 64 && wants_f6(std::min(nf, 4), fw, M) && (rc = f6_ready(nf, fw, M, s, sc, &ready, &make))) return rc;
       if (ready) {
-        for (int i = 0; i < nf; i += 4) {
-          if ((rc = workspace_unmoved(s, gen))) return rc;
-          if ((rc = matmul_f6(std::min(4, nf - i), fw + i, A, M, lda, fc + i, fl + i, s, sc, &make, i == 0))) return rc;
-        }
+        if ((rc = matmul_f6(nf, fw, A, M, lda, fc, fl, s, sc, &make))) return rc;
         continue;
       }
     }

@@ -44,6 +44,7 @@
  * in its middle. Workgroup ids are mapped so that the row tiles sharing weights run on one XCD.
  */
 #include <algorithm>
+#include <atomic>
 #include <mutex>
 #include <new>
 
@@ -87,16 +88,59 @@ __device__ __forceinline__ void set_word(uint32_t *word) {
   if (word && blockIdx.x == 0 && threadIdx.x == 0) __hip_atomic_store(word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+/* What a launch reads its rows from (QActF6). */
+struct ActF6 {
+  const uint8_t *p;
+  const uint32_t *flags;
+  uint32_t token;
+};
+
+/* The sums of f6_sums for a row tile with a scale that is not finite (magnitudes of 8.3e6 and more). There the rank-one
+ * instruction may have nothing but the one block's scales on either side: infinity times the zeros that stand for the
+ * other blocks would be NaN in all of them. Masking the rows' side as well in the loop below cost 8 % of every product;
+ * this plain one runs for such tiles only. */
+__device__ __forceinline__ void f6_sums_plain(const uint8_t *wbase, int N, int chunks, const ActF6 &act, int mt, int tile,
+                                              float (&acc)[16]) {
+  const int lane = threadIdx.x & 63, i32 = lane & 31, g = lane >> 5;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  const uint8_t *w = wbase + (size_t)min(tile, ((N + 31) >> 5) - 1) * chunks * WTILE;
+  const uint8_t *rows = act.p + (size_t)(mt >> 1) * chunks * CHUNK;
+#pragma unroll 1
+  for (int c = 0; c < chunks; ++c, w += WTILE, rows += CHUNK)
+#pragma unroll 1
+    for (int j = 0; j < 8; ++j) {
+      const uint8_t *p = rows + (mt & 1) * PARTS + j * 1536;
+      const v4i a0 = *(const v4i *)(p + lane * 16);
+      const v2i a1 = *(const v2i *)(p + 1024 + lane * 8);
+      v8i b;
+#pragma unroll
+      for (int e = 0; e < 3; ++e) {
+        const int q = 3 * j + e;
+        b[e] = b[3 + e] = *(const int *)(w + (q >> 2) * 1024 + lane * 16 + (q & 3) * 4);
+      }
+      b[6] = b[7] = 0;
+      const v2i da{g ? 0 : (int)*(const uint16_t *)(rows + 2 * PARTS + (mt & 1) * 512 + i32 * 16 + j * 2), 0},
+        dw{g ? 0 : (int)*(const uint16_t *)(w + 6144 + i32 * 16 + j * 2), 0};
+      const v16f D = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(v8i{a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], 0, 0}, b, zero16(),
+                                                                     3, 2, 0, 127 + 4, 0, 127 + 3);
+      const v16f P = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(v4h, da), __builtin_bit_cast(v4h, dw), zero16(), 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[r] = fmaf(D[r], P[r], acc[r]);
+    }
+}
+
 /* The sums of row tile mt and the wavefront's column tile `tile` (lane (column, g), sum r: row 8 (r / 4) + 4 g + r % 4).
  * LOOK: steps an operand is read ahead of its matrix instruction, 1 or 3 */
 template <int LOOK>
-__device__ __forceinline__ void f6_sums(const uint8_t *wbase, int N, int chunks, const uint8_t *act, int mt, int tile,
+__device__ __forceinline__ void f6_sums(const uint8_t *wbase, int N, int chunks, const ActF6 &act, int mt, int tile,
                                         float (&acc)[16]) {
+  const uint32_t flag = act.flags[mt]; /* the same for the whole workgroup */
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int lane = threadIdx.x & 63, i32 = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int half = mt & 1; /* of the quantizer's 64 rows */
-  const rsrc_t ra = make_rsrc(act + (size_t)(mt >> 1) * chunks * CHUNK, (uint32_t)chunks * CHUNK);
+  const rsrc_t ra = make_rsrc(act.p + (size_t)(mt >> 1) * chunks * CHUNK, (uint32_t)chunks * CHUNK);
   /* a tile past the last repeats it; it is not stored */
   const rsrc_t rw = make_rsrc(wbase + (size_t)min(tile, ((N + 31) >> 5) - 1) * chunks * WTILE, (uint32_t)chunks * WTILE);
 
@@ -128,6 +172,10 @@ __device__ __forceinline__ void f6_sums(const uint8_t *wbase, int N, int chunks,
     load_dw(min(k, last), k);
   }
   asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+  if (flag == act.token) { /* looked at only here, behind the other loads */
+    f6_sums_plain(wbase, N, chunks, act, mt, tile, acc);
+    return;
+  }
 
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.f;
@@ -205,7 +253,7 @@ __device__ __forceinline__ void f6_sums(const uint8_t *wbase, int N, int chunks,
 }
 
 template <int LOOK>
-__device__ __forceinline__ void f6_tile(const uint8_t *wbase, int N, int chunks, const uint8_t *act, int M, int mt, int nt,
+__device__ __forceinline__ void f6_tile(const uint8_t *wbase, int N, int chunks, const ActF6 &act, int M, int mt, int nt,
                                         float *__restrict__ C, int64_t ldc) {
   const int lane = threadIdx.x & 63, i32 = lane & 31, g = lane >> 5;
   const int tile = nt * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -223,7 +271,7 @@ __device__ __forceinline__ void f6_tile(const uint8_t *wbase, int N, int chunks,
 
 /* LOOK = 3 takes 182 registers (two workgroups a CU), LOOK = 1 fits three */
 template <int LOOK>
-__global__ __launch_bounds__(NT, LOOK == 1 ? 3 : 2) void gemm_f6_kernel(MultiF6 mw, int chunks, const uint8_t *act, int M,
+__global__ __launch_bounds__(NT, LOOK == 1 ? 3 : 2) void gemm_f6_kernel(MultiF6 mw, int chunks, ActF6 act, int M,
                                                                         int mtiles) {
   const int id = blockIdx.x;
   const int xcd = id & 7, qd = id >> 3;
@@ -255,7 +303,7 @@ struct GatedF6 {
   uint32_t *word; /* or null: set_word */
 };
 template <int LOOK>
-__device__ __forceinline__ void f6_gated_tile(const GatedF6 &p, int chunks, const uint8_t *act, int M, int mt, int nt) {
+__device__ __forceinline__ void f6_gated_tile(const GatedF6 &p, int chunks, const ActF6 &act, int M, int mt, int nt) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int lane = threadIdx.x & 63, i32 = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -280,7 +328,7 @@ __device__ __forceinline__ void f6_gated_tile(const GatedF6 &p, int chunks, cons
   }
 }
 template <int LOOK>
-__global__ __launch_bounds__(NT, LOOK == 1 ? 3 : 2) void gemm_f6_gated_kernel(GatedF6 p, int chunks, const uint8_t *act, int M,
+__global__ __launch_bounds__(NT, LOOK == 1 ? 3 : 2) void gemm_f6_gated_kernel(GatedF6 p, int chunks, ActF6 act, int M,
                                                                               int mtiles) {
   const int id = blockIdx.x;
   const int xcd = id & 7, qd = id >> 3;
@@ -391,6 +439,8 @@ struct RowsF6 {
   uint32_t n_units; /* octets of rows (padding included) x blocks */
   int nbp, K;
   uint8_t *out;
+  uint32_t *flags;
+  uint32_t token;
 };
 __device__ __forceinline__ void f6_quantize(const RowsF6 &p, int block) {
   const int64_t M = p.M;
@@ -431,7 +481,10 @@ __device__ __forceinline__ void f6_quantize(const RowsF6 &p, int block) {
   const int at = g * 32 + (r & 31);
   if ((lane & 3) == 0) *(uint4 *)(o + at * 16) = make_uint4(w[0], w[1], w[2], w[3]);
   if ((lane & 3) == 1) *(uint2 *)(o + 1024 + at * 8) = make_uint2(w[4], w[5]);
-  if (sub == 0) *(uint16_t *)(dst + PARTS + r * 16 + j * 2) = dh;
+  if (sub == 0) {
+    *(uint16_t *)(dst + PARTS + r * 16 + j * 2) = dh;
+    if ((dh & 0x7c00) == 0x7c00) p.flags[m >> 5] = p.token; /* not finite: f6_sums_plain */
+  }
 }
 
 __global__ __launch_bounds__(256) void quantize_q8_0_f6_kernel(RowsF6 p) { f6_quantize(p, (int)blockIdx.x); }
@@ -683,10 +736,13 @@ F6Make::~F6Make() { /* a call that failed between f6_copies and its quantizer's 
 }
 
 size_t qact_f6_bytes(int64_t M, int64_t K) {
-  return (size_t)((M + F6_ROWS - 1) / F6_ROWS) * (size_t)((K + 255) / 256) * F6_CHUNK;
+  const size_t tiles = (size_t)((M + F6_ROWS - 1) / F6_ROWS);
+  return tiles * (size_t)((K + 255) / 256) * F6_CHUNK + ((tiles * 8 + 255) & ~(size_t)255); /* the flags: two a tile of 64 rows */
 }
 QActF6 qact_f6_carve(void *mem, int64_t M, int64_t K) {
-  return QActF6{(uint8_t *)mem, (int)M, (int)K, (int)((K + 255) / 256), nullptr};
+  const int64_t chunks = (K + 255) / 256;
+  return QActF6{(uint8_t *)mem, (uint32_t *)((uint8_t *)mem + (size_t)((M + F6_ROWS - 1) / F6_ROWS) * chunks * F6_CHUNK), 0, (int)M, (int)K,
+                (int)chunks, nullptr};
 }
 
 int launch_quantize_q8_0_f6(const float *A, int64_t M, int64_t K, int64_t lda, QActF6 *qa, F6Make *make, hipStream_t s) {
@@ -696,7 +752,9 @@ int launch_quantize_q8_0_f6(const float *A, int64_t M, int64_t K, int64_t lda, Q
     return fail(HIPQ_ERR_INVALID_ARGUMENT, "activation rows must be 16-byte aligned");
   const int64_t units = (M + F6_ROWS - 1) / F6_ROWS * (F6_ROWS / 8) * (qa->chunks * 8); /* padding included */
   if (units > INT32_MAX) return fail(HIPQ_ERR_NOT_SUPPORTED, "%lld x %lld values in one call", (long long)M, (long long)K);
-  const RowsF6 rows{A, M, lda, (uint32_t)units, qa->chunks * 8, (int)K, qa->p};
+  static std::atomic<uint32_t> calls{0};
+  qa->token = ++calls;
+  const RowsF6 rows{A, M, lda, (uint32_t)units, qa->chunks * 8, (int)K, qa->p, qa->flags, qa->token};
   const unsigned blocks = (unsigned)((units + 3) / 4);
   if (!make || !make->count) {
     launch_kernel("quantize_q8_0_f6_kernel", quantize_q8_0_f6_kernel, dim3(blocks), dim3(256), 0, s, rows);
@@ -778,10 +836,10 @@ int launch_gemm_f6(int count, const hipq_weight *const *w, const QActF6 *qa, int
   /* up to two workgroups a CU: the deeper read-ahead (512 rows of 1024 x 3072 13.1 -> 12.0 us, 1024 x 1024 7.5 -> 6.7);
    * beyond, three workgroups a CU cover the reads (512 of 12288 x 4096 67 -> 62 us) */
   if ((int64_t)mtiles * tiles <= 512)
-    launch_kernel("gemm_f6_kernel<3>", gemm_f6_kernel<3>, grid, dim3(NT), 3 * BUF, s, mw, qa->chunks, (const uint8_t *)qa->p, M,
+    launch_kernel("gemm_f6_kernel<3>", gemm_f6_kernel<3>, grid, dim3(NT), 3 * BUF, s, mw, qa->chunks, ActF6{qa->p, qa->flags, qa->token}, M,
                   mtiles);
   else
-    launch_kernel("gemm_f6_kernel<1>", gemm_f6_kernel<1>, grid, dim3(NT), 3 * BUF, s, mw, qa->chunks, (const uint8_t *)qa->p, M,
+    launch_kernel("gemm_f6_kernel<1>", gemm_f6_kernel<1>, grid, dim3(NT), 3 * BUF, s, mw, qa->chunks, ActF6{qa->p, qa->flags, qa->token}, M,
                   mtiles);
   HIPQ_HIP(hipGetLastError());
   return HIPQ_OK;
@@ -797,10 +855,10 @@ int launch_gemm_f6_gated(const hipq_weight *wa, const hipq_weight *wm, const QAc
   /* the bound of launch_gemm_f6 */
   if ((int64_t)mtiles * p.ntiles <= 512)
     launch_kernel("gemm_f6_gated_kernel<3>", gemm_f6_gated_kernel<3>, grid, dim3(NT), 3 * BUF, s, p, qa->chunks,
-                  (const uint8_t *)qa->p, M, mtiles);
+                  ActF6{qa->p, qa->flags, qa->token}, M, mtiles);
   else
     launch_kernel("gemm_f6_gated_kernel<1>", gemm_f6_gated_kernel<1>, grid, dim3(NT), 3 * BUF, s, p, qa->chunks,
-                  (const uint8_t *)qa->p, M, mtiles);
+                  ActF6{qa->p, qa->flags, qa->token}, M, mtiles);
   HIPQ_HIP(hipGetLastError());
   return HIPQ_OK;
 }

@@ -171,6 +171,10 @@ QActTiled qact_tiled_carve(void *mem, int64_t M, int64_t K);
 /* ------------------------------------------------------------------------- */
 struct QActF6 {
   uint8_t *p;
+  /* per 32 rows: the call's token (a number of its own, so that nothing has to be cleared) where one of their block
+   * scales is not finite; a stray match costs time only */
+  uint32_t *flags;
+  uint32_t token;
   int M, K, chunks;
   uint32_t *word; /* where the quantizer made copies of weights: for the product behind it to set (f6_copies) */
 };

@@ -908,3 +908,83 @@ def test_row_counts_across_the_kernel_choices(hipq, cr):
             assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), case
         done += 1
 
+
+
+def _extreme_rows(m, k):
+    """Rows whose Q8_0 block scales are infinite, subnormal and zero as fp16, in whole rows and in single blocks."""
+    a = synth.normal(77, (m, k))
+    for r in range(m):
+        b = slice(32 * (r % (k // 32)), 32 * (r % (k // 32)) + 32)
+        kind = r % 8
+        if kind == 1:
+            a[r] *= 3e7          # every scale infinite
+        elif kind == 2:
+            a[r, b] *= 1e9       # one infinite scale in the row
+        elif kind == 3:
+            a[r, b] = 0.0
+            a[r, b.start] = -2e7  # one product of the block
+        elif kind == 4:
+            a[r] *= 1e-3         # subnormal scales
+        elif kind == 5:
+            a[r, b] *= 3e-6      # the smallest ones
+        elif kind == 6:
+            a[r] *= 1e-9         # scales of zero
+        elif kind == 7:
+            a[r, b] *= 65504 * 127 / np.abs(a[r, b]).max()  # the largest finite scale
+    return a
+
+
+@pytest.mark.parametrize("m,n,k", [(70, 130, 256), (97, 300, 1056), (2100, 520, 288)])
+@pytest.mark.parametrize("call", ["matmul", "swiglu"])
+def test_q4_0_on_six_bit_operands_with_extreme_scales(hipq, cr, call, m, n, k):
+    """gemm_f6.hip: block scales that are infinite, subnormal and zero as fp16. An infinite scale makes the sums of its own
+    row infinite (or NaN, where the reference's are), and no other block's: the reference's bits. Infinite and NaN
+    activations give what the kernels that read the weight as stored give."""
+    import gpu_util as gu
+    import torch
+    blocks = _weights(cr, "q4_0", n, k, seed=3000 + m)
+    blocks2 = _weights(cr, "q4_0", n, k, seed=3001 + m)
+    w, w2 = capi.Weight("q4_0", n, k, blocks), capi.Weight("q4_0", n, k, blocks2)
+
+    def product(a):
+        da, out = gu.dev(a), torch.full((m, n), 7.0, device="cuda")
+        if call == "matmul":
+            capi.matmul(w, da, m, out, stream=gu.stream())
+        else:
+            capi.mlp_swiglu(w, w2, da, m, out, stream=gu.stream())
+        torch.cuda.synchronize()
+        return out.cpu().numpy()
+
+    def same(got, ref):
+        nan = np.isnan(ref)
+        assert np.array_equal(np.isnan(got), nan)
+        bits = got.view(np.uint32) != ref.view(np.uint32)
+        assert not (bits & ~nan).any(), "%d of %d outputs differ in bits" % ((bits & ~nan).sum(), got.size)
+
+    a = _extreme_rows(m, k)
+    if call == "matmul":
+        ref = cr.gemm(cr.oracle(), "q4_0", a, blocks, n)
+        assert np.isinf(ref).any() and np.isfinite(ref[2]).sum() == 0
+        same(product(a), ref)
+    # the stored weights' kernels, by a call that may not allocate
+    v, v2 = capi.Weight("q4_0", n, k, blocks), capi.Weight("q4_0", n, k, blocks2)
+    for extra in (0.0, np.inf, -np.inf, np.nan):
+        if extra != 0.0:
+            a[::5, 7] = extra
+        da, y, z = gu.dev(a), torch.empty((m, n), device="cuda"), torch.empty((m, n), device="cuda")
+        capi.matmul_noalloc(v, da, m, y, stream=gu.stream())
+        capi.matmul_noalloc(v2, da, m, z, stream=gu.stream())
+        torch.cuda.synchronize()
+        y, z = y.cpu().numpy(), z.cpu().numpy()
+        if call == "matmul":
+            same(product(a), y)
+        else:
+            got = product(a)
+            with np.errstate(all="ignore"):
+                want = y / (1.0 + np.exp(-y.astype(np.float64))) * z
+            assert np.array_equal(np.isnan(got), np.isnan(want))
+            fine = np.isfinite(want)
+            assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)].astype(np.float32))
+            assert np.allclose(got[fine], want[fine], rtol=1e-5, atol=1e-30)
+    for x in (w, w2, v, v2):
+        x.destroy()
