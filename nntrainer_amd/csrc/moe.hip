@@ -35,6 +35,7 @@
 #include "gemv_device.h"
 #include "moe_tile_device.h"
 #include "quantize_device.h"
+#include "silu_ref.h"
 
 namespace {
 
@@ -706,31 +707,8 @@ __global__ void scatter_kernel(const int32_t *__restrict__ idx, int P, int topk,
   tok_slots[rank_in_token(idx, i, topk)] = slot;
 }
 
-/* sigmoid(g) * g with the sigmoid in double on the float-rounded exponential, as the reference:
- *   en = float(exp(double(-g))), sig = float(1.0 / (1.0 + double(en))).
- * Both double results are only kept to float, so neither needs the library's last-bit exp and
- * division (about a hundred double instructions a value; in the products of many tokens they were
- * half of a workgroup's time outside its loop). exp: 2^k e^r with r = x - k ln 2 in two fused steps,
- * |r| < 0.35, and the Taylor sum of e^r to r^11 (relative error below 2^-46). Division: the hardware
- * reciprocal and one cubic step y (1 + e + e^2), e = 1 - d y. Both round to the library forms' float
- * on all of 150 million inputs compared on the host. Beyond +-200 the exponential is 0 or infinite as a float. */
 __device__ __forceinline__ float silu_ref(float g) {
-  const double x = (double)fminf(fmaxf(-g, -200.f), 200.f);
-  const double kbig = fma(x, 1.4426950408889634, 6755399441055744.0); /* 1.5 * 2^52: k in the low bits */
-  const double k = kbig - 6755399441055744.0;
-  const double r = fma(k, -2.3190468138462996e-17, fma(k, -0.6931471805599453, x));
-  constexpr double C[11] = {1.0 / 3628800, 1.0 / 362880, 1.0 / 40320, 1.0 / 5040, 1.0 / 720, 1.0 / 120,
-                            1.0 / 24,      1.0 / 6,      0.5,         1.0,        1.0};
-  double p = 1.0 / 39916800;
-#pragma unroll
-  for (int i = 0; i < 11; ++i) p = fma(p, r, C[i]);
-  const uint64_t bits = __builtin_bit_cast(uint64_t, p) + (__builtin_bit_cast(uint64_t, kbig) << 52);
-  const float en = (float)__builtin_bit_cast(double, bits);
-  const double d = 1.0 + (double)en;
-  const double y = __builtin_amdgcn_rcp(d);
-  const double e = fma(-d, y, 1.0);
-  const float sig = en == INFINITY ? 0.f : (float)fma(y, fma(e, e, e), y);
-  return sig * g;
+  return hipq_silu_ref(g, [](double d) { return __builtin_amdgcn_rcp(d); }); /* the hardware's: 24 bits */
 }
 
 /* The activation between the projections and the bias of the down projection, by expert
