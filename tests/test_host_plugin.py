@@ -59,7 +59,7 @@ ADAPTERS = ["hip_context.cpp", "hip_mem_allocator.cpp", "fc_layer_hip.cpp", "moe
             "qkv_layer_hip.cpp", "tie_word_embedding_hip.cpp", "mlp_swiglu_layer_hip.cpp", "hipq_host.cpp"]
 
 
-@pytest.mark.skipif(not os.path.isdir(REFERENCE), reason="reference checkout not present")
+@pytest.mark.skipif(not os.path.isdir(os.path.join(REFERENCE, "nntrainer")), reason="reference checkout not present")
 @pytest.mark.parametrize("src", ADAPTERS)
 def test_adapters_compile_against_framework_headers(src, tmp_path):
     """The adapter sources compile to object code against the framework's own headers, and what
