@@ -30,11 +30,13 @@ template <typename Rcp> HIPQ_SILU_FN float hipq_silu_ref(float g, Rcp rcp) {
   const double kbig = fma(x, 1.4426950408889634, 6755399441055744.0); /* 1.5 * 2^52: k in the low bits */
   const double k = kbig - 6755399441055744.0;
   const double r = fma(k, -2.3190468138462996e-17, fma(k, -0.6931471805599453, x));
-  constexpr double C[13] = {1.0 / 479001600, 1.0 / 39916800, 1.0 / 3628800, 1.0 / 362880, 1.0 / 40320, 1.0 / 5040, 1.0 / 720,
-                            1.0 / 120,       1.0 / 24,       1.0 / 6,       0.5,          1.0,         1.0};
-  double p = 1.0 / 6227020800;
+  const double r2 = r * r;
+  double even = 1.0 / 479001600, odd = 1.0 / 6227020800; /* two chains of the coefficients of r^2 .. r^13 */
+  constexpr double E[5] = {1.0 / 3628800, 1.0 / 40320, 1.0 / 720, 1.0 / 24, 0.5};
+  constexpr double O[5] = {1.0 / 39916800, 1.0 / 362880, 1.0 / 5040, 1.0 / 120, 1.0 / 6};
 #pragma unroll
-  for (int i = 0; i < 13; ++i) p = fma(p, r, C[i]);
+  for (int i = 0; i < 5; ++i) even = fma(even, r2, E[i]), odd = fma(odd, r2, O[i]);
+  const double p = 1.0 + fma(r2, fma(odd, r, even), r);
   const uint64_t bits = __builtin_bit_cast(uint64_t, p) + (__builtin_bit_cast(uint64_t, kbig) << 52);
   const float en = (float)__builtin_bit_cast(double, bits);
   const double d = 1.0 + (double)en;
