@@ -1,8 +1,9 @@
 // SPDX-License-Identifier: Apache-2.0
 /**
  * @file   gemm.hip
- * @brief  Prefill GEMM (M > 8) for Q4_0 x Q8_0 on gfx950 int8 matrix cores.
- *         (Q4_K x Q8_K has its own kernel, gemm_q4k.hip.)
+ * @brief  Q4_0 x Q8_0 of many rows on the gfx950 int8 matrix cores, off the weight as it is stored.
+ *         (Prefill goes to gemm_f6.hip, about twice as fast; this one takes the calls that cannot have a
+ *         weight's six-bit copy, and 5 to 64 rows where neither that one nor the few-rows kernel applies.)
  *
  * Replaces the M > 1 branch of __ggml_q4_0_8x8_q8_0_GEMM
  * (nntrainer/tensor/cpu_backend/ggml_interface/ggml_interface_omp.cpp:330-389 in

@@ -90,11 +90,13 @@ __global__ __launch_bounds__(256) void gemv_stream_kernel(WView w, QView qa,
  *
  * Up to some millions of weights a launch is bound by the chain of what waits for what: the arguments, the row,
  * its quantization, the barrier, the products, the fp32 sums in order. A launch of nothing takes 1.5 us of a
- * stream's time, these took 4.0 to 4.4. So the row is quantized in one pass, eight or sixteen values a lane (four
- * values a lane took up to four passes of some hundred dependent instructions), the sums read their records
- * sixteen blocks ahead (GemvCore::chain_batched), and the arguments are asked for together (args_first). Q4_0
- * 4096 x 4096 5.95 -> 4.55 us a call; 114 launches of a token through 28 layers of 1024 / 3072 453 -> 384 us of
- * GPU time; a Q4_K layer of 4096 / 12288 36.3 -> 31.8 us. */
+ * stream's time, these took 4.0 to 4.4. So the row is quantized in one pass, four to sixteen values a lane (four
+ * values a lane for every length took up to four passes of some hundred dependent instructions), the arguments are
+ * asked for together (args_first), and where the row length is a constant the sums read their records a batch of
+ * eight blocks ahead, of four super-blocks in Q4_K (GemvCore::chain_batched; with any length the batches sit behind
+ * conditions and are slower). Q4_0 4096 x 4096 5.95 -> 4.6 us a call; a pass of a token through 28 layers of
+ * 1024 / 3072 and its lm_head, 113 launches, 508 -> 380 to 430 by box and host (the native calls of the binding in
+ * it); a Q4_K layer of 4096 / 12288 36.4 -> 33.1 us. */
 template <int DT> __host__ __device__ constexpr int fused_act_bytes(int K) {
   /* Q8_0: q [K], meta [K/32] u32; Q8_K: q [K], ql [K/2], qh [K/2], bsum [K/16] i16, d [K/256] f32 */
   return ((DT == HIPQ_Q4_0 ? K + K / 8 : 2 * K + K / 8 + K / 64) + 15) & ~15;

@@ -564,7 +564,7 @@ __device__ __forceinline__ void sort_pairs(const int32_t *idx, int P, int E, int
 
 /* Up to 16384 pairs behind the routing launch, which has written every token's pairs in ascending expert id to tok_slots.
  * All of a thread's pairs are loaded before the first is counted, the count hands out the pair's place in its expert, and
- * the slots of the pairs pass through LDS to the places tok_slots names (in place). 8000 pairs: 15.5 -> 7 us (a second pass
+ * the slots of the pairs pass through LDS to the places tok_slots names (in place). 8000 pairs: 15.5 -> 8.5 us (a second pass
  * over idx with its own atomics, and topk reads a pair for its rank, one round trip after the other). */
 constexpr int SORT_MANY = 16384;
 __global__ __launch_bounds__(1024) void sort_pairs_kernel(const int32_t *__restrict__ idx, int P, int E,
@@ -2091,8 +2091,9 @@ int launch_moe(const MoeArgs *a, void *workspace, size_t workspace_bytes, const 
     /* the rows of x of a workgroup's tokens go to LDS: four tokens, or as many as there are or fit 64 KB with the partial sums */
     int tb_n = d.hidden > 0 ? (int)std::min<int64_t>(std::min(ROUTER_TB, T), 15000 / d.hidden) : 0;
     tb_n = tb_n >= 4 ? 4 : tb_n >= 2 ? 2 : tb_n;
-    /* level with the kernel above at 100 to 150 tokens of 32 experts and more (2048 x 128: 100 tokens 77 -> 83 us a block,
-     * 200 106 -> 100, 1000 229 -> 186), at 500 to 1000 of eight */
+    /* us a block of 2048 x 768, the few-token kernels / this one: of 128 experts, top 8, with 100 tokens 94.9 / 95.5, 128
+     * 96.8 / 97.5, 150 129.9 / 127.1, 200 128.9 / 123.2, 1000 267.7 / 225.0; of eight, top 4, with 500 78.1 / 78.9, 1000
+     * 115.7 / 116.9 */
     if ((int64_t)T * std::min(E, 32) >= 128 * 32 && d.hidden % 256 == 0 && !(E & 3) && (((uintptr_t)a->router_weight | (uintptr_t)a->x) & 15) == 0) {
       constexpr size_t lds = 16 * ROUTER_STAGE * sizeof(float);
       HIPQ_HIP(hipFuncSetAttribute((const void *)router_logits_many_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
