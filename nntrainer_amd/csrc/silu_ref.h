@@ -21,7 +21,8 @@
  * Both double results are only kept to float, so neither needs the library's last-bit exp and
  * division (about a hundred double instructions a value; in the products of many tokens they were
  * half of a workgroup's time outside its loop). exp: 2^k e^r with r = x - k ln 2 in two fused steps,
- * |r| < 0.35, and the Taylor sum of e^r to r^13 (truncated at 2^-57; to r^11 two of all floats had another
+ * |r| < 0.3466, and e^r = 1 + r + r^2 q(r) with q of degree 9 through the ten Chebyshev nodes of that range, in two
+ * chains (r^2 with a half, a constant of the instruction set; off by 2^-54.6 at most; the Taylor sum to r^11 is off by 2^-47, and two of all floats had another
  * exponential). Division: a reciprocal of 22 bits or better and one cubic step y (1 + e + e^2), e = 1 - d y.
  * Both round to the library forms' float for every float from 2^-30 to 250 in magnitude, with glibc's exp as the
  * library form. Beyond +-200 the exponential is 0 or infinite as a float. */
@@ -31,11 +32,11 @@ template <typename Rcp> HIPQ_SILU_FN float hipq_silu_ref(float g, Rcp rcp) {
   const double k = kbig - 6755399441055744.0;
   const double r = fma(k, -2.3190468138462996e-17, fma(k, -0.6931471805599453, x));
   const double r2 = r * r;
-  double even = 1.0 / 479001600, odd = 1.0 / 6227020800; /* two chains of the coefficients of r^2 .. r^13 */
-  constexpr double E[5] = {1.0 / 3628800, 1.0 / 40320, 1.0 / 720, 1.0 / 24, 0.5};
-  constexpr double O[5] = {1.0 / 39916800, 1.0 / 362880, 1.0 / 5040, 1.0 / 120, 1.0 / 6};
+  double even = 0x1.28917e2c43a66p-22, odd = 0x1.af38a0d2d9620p-26; /* coefficients of r^10, r^11 and down */
+  constexpr double E[4] = {0x1.a019b9133a48ap-16, 0x1.6c16c1788a49bp-10, 0x1.5555555553d67p-5, 0.5};
+  constexpr double O[4] = {0x1.71de0db21e27fp-19, 0x1.a01a01a7c327ap-13, 0x1.11111111109b4p-7, 0x1.5555555555556p-3};
 #pragma unroll
-  for (int i = 0; i < 5; ++i) even = fma(even, r2, E[i]), odd = fma(odd, r2, O[i]);
+  for (int i = 0; i < 4; ++i) even = fma(even, r2, E[i]), odd = fma(odd, r2, O[i]);
   const double p = 1.0 + fma(r2, fma(odd, r, even), r);
   const uint64_t bits = __builtin_bit_cast(uint64_t, p) + (__builtin_bit_cast(uint64_t, kbig) << 52);
   const float en = (float)__builtin_bit_cast(double, bits);

@@ -1,4 +1,4 @@
-"""CPU: the series and the reciprocal step of the expert activation (csrc/silu_ref.h) give the reference's float,
+"""CPU: the polynomial and the reciprocal step of the expert activation (csrc/silu_ref.h) give the reference's float,
 sigmoid(g) * g with exp and the division in double, for every float."""
 import os
 import subprocess
