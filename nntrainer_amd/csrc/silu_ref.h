@@ -21,9 +21,10 @@
  * Both double results are only kept to float, so neither needs the library's last-bit exp and
  * division (about a hundred double instructions a value; in the products of many tokens they were
  * half of a workgroup's time outside its loop). exp: 2^k e^r with r = x - k ln 2 in two fused steps,
- * |r| < 0.3466, and e^r = 1 + r + r^2 q(r) with q of degree 9 through the ten Chebyshev nodes of that range, in two
- * chains (r^2 with a half, a constant of the instruction set; off by 2^-54.6 at most; the Taylor sum to r^11 is off by 2^-47, and two of all floats had another
- * exponential). Division: a reciprocal of 22 bits or better and one cubic step y (1 + e + e^2), e = 1 - d y.
+ * |r| < 0.3466, and e^r = 1 + r + r^2 q(r) with q of degree 9 through the ten Chebyshev nodes of that range (its
+ * first coefficient a half, a constant of the instruction set), in two chains. That is off by 2^-54.6 at most; the
+ * Taylor sum to r^11 is off by 2^-47, and two of all floats had another exponential. Division: a reciprocal of 22 bits
+ * or better and one cubic step y (1 + e + e^2), e = 1 - d y.
  * Both round to the library forms' float for every float from 2^-30 to 250 in magnitude, with glibc's exp as the
  * library form. Beyond +-200 the exponential is 0 or infinite as a float. */
 template <typename Rcp> HIPQ_SILU_FN float hipq_silu_ref(float g, Rcp rcp) {
