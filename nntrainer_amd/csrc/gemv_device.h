@@ -137,7 +137,7 @@ __device__ __forceinline__ uint32_t hipq_late_zero() {
   return z;
 }
 
-template <int T, int R, bool PW, int KC> struct GemvQ40 {
+template <int T, int R, bool PW, int KC, bool FULL> struct GemvQ40 {
   static constexpr int MAXU = GemvUnits<HIPQ_Q4_0, T, KC>::MAXU;
   static constexpr int PER = GemvRec<HIPQ_Q4_0, PW>::PER_CHUNK;
   struct Act {
@@ -155,7 +155,7 @@ template <int T, int R, bool PW, int KC> struct GemvQ40 {
     const int units = qa.K >> 5, u0 = k0 >> 5, un = kc >> 5;
 #pragma unroll
     for (int i = 0; i < MAXU; ++i) {
-      if (i * T >= un) break; /* uniform: this step lies beyond the chunk */
+      if (!FULL && i * T >= un) break; /* uniform: this step lies beyond the chunk */
       const int u = min(tl + i * T, un - 1);
 #pragma unroll
       for (int r = 0; r < R; ++r) {
@@ -173,7 +173,7 @@ template <int T, int R, bool PW, int KC> struct GemvQ40 {
     const uint16_t *dw = w.d + (size_t)row * units + u0;
 #pragma unroll
     for (int i = 0; i < MAXU; ++i) {
-      if (i * T >= un) break;
+      if (!FULL && i * T >= un) break;
       const int u = min(tl + i * T, un - 1);
       W.q[i] = hipq_ld_stream(qs + u);
       W.d[i] = hipq_ld_global(dw + u);
@@ -187,7 +187,7 @@ template <int T, int R, bool PW, int KC> struct GemvQ40 {
     const int un = kc >> 5;
 #pragma unroll
     for (int i = 0; i < MAXU; ++i) {
-      if (i * T >= un) break;
+      if (!FULL && i * T >= un) break;
       const int u = tl + i * T;
       const uint4 q = W.q[i];
       const float d = hipq_h2f((uint16_t)(W.d[i] | late));
@@ -215,7 +215,7 @@ template <int T, int R, bool PW, int KC> struct GemvQ40 {
  * consecutive bytes (lanes 32 bytes apart, each taking a sub-block pair with two
  * loads, stream measurably slower). 8 consecutive lanes hold one super-block; its
  * integer sums meet in three DPP steps. */
-template <int T, int R, bool PW, int KC> struct GemvQ4K {
+template <int T, int R, bool PW, int KC, bool FULL> struct GemvQ4K {
   static_assert(T % 8 == 0, "a super-block's eight sub-blocks sit in eight consecutive lanes");
   static constexpr int MAXU = GemvUnits<HIPQ_Q4_K, T, KC>::MAXU;
   static constexpr int PER = GemvRec<HIPQ_Q4_K, PW>::PER_CHUNK;
@@ -233,7 +233,7 @@ template <int T, int R, bool PW, int KC> struct GemvQ4K {
     const int nsb = qa.K >> 8, un = kc >> 5, b0 = k0 >> 8;
 #pragma unroll
     for (int i = 0; i < MAXU; ++i) {
-      if (i * T >= un) break;
+      if (!FULL && i * T >= un) break;
       const int u = min(tl + i * T, un - 1);
       const int b = u >> 3, j = u & 7;
 #pragma unroll
@@ -254,7 +254,7 @@ template <int T, int R, bool PW, int KC> struct GemvQ4K {
     const uint4 *hdr = (const uint4 *)w.hdr + (size_t)row * nsb + b0;
 #pragma unroll
     for (int i = 0; i < MAXU; ++i) {
-      if (i * T >= un) break;
+      if (!FULL && i * T >= un) break;
       const int u = min(tl + i * T, un - 1);
       W.q[i] = hipq_ld_stream(qs + u);
       W.hd[i] = hipq_ld_global(hdr + (u >> 3));
@@ -265,7 +265,7 @@ template <int T, int R, bool PW, int KC> struct GemvQ4K {
     const int un = kc >> 5;
 #pragma unroll
     for (int i = 0; i < MAXU; ++i) {
-      if (i * T >= un) break;
+      if (!FULL && i * T >= un) break;
       const int u = tl + i * T;
       const bool on = u < un;
       const int uc = on ? u : un - 1;
@@ -317,7 +317,7 @@ template <int T, int R, bool PW, int KC> struct GemvQ4K {
 /* A unit is 64 weights = 16 B of each ql plane + 16 B of qh, unit uu = half*2 + hl of
  * a super-block. Dword t of the unit belongs to partial l = hl*4 + t; lanes uu and
  * uu^2 hold the two 128-element halves. */
-template <int T, int R, bool PW, int KC> struct GemvQ6K {
+template <int T, int R, bool PW, int KC, bool FULL> struct GemvQ6K {
   static constexpr int MAXU = GemvUnits<HIPQ_Q6_K, T, KC>::MAXU;
   static constexpr int PER = GemvRec<HIPQ_Q6_K, PW>::PER_CHUNK;
   struct Act {
@@ -334,7 +334,7 @@ template <int T, int R, bool PW, int KC> struct GemvQ6K {
     const int nsb = qa.K >> 8, un = kc >> 6, b0 = k0 >> 8;
 #pragma unroll
     for (int i = 0; i < MAXU; ++i) {
-      if (i * T >= un) break;
+      if (!FULL && i * T >= un) break;
       const int u = min(tl + i * T, un - 1);
       const int b = u >> 2, uu = u & 3, half = uu >> 1, hl = uu & 1;
 #pragma unroll
@@ -358,7 +358,7 @@ template <int T, int R, bool PW, int KC> struct GemvQ6K {
     const uint16_t *drow = w.d + (size_t)row * nsb + b0;
 #pragma unroll
     for (int i = 0; i < MAXU; ++i) {
-      if (i * T >= un) break;
+      if (!FULL && i * T >= un) break;
       const int u = min(tl + i * T, un - 1);
       const int b = u >> 2;
       /* consecutive lanes take consecutive 16-byte pieces of every plane */
@@ -374,7 +374,7 @@ template <int T, int R, bool PW, int KC> struct GemvQ6K {
     const int un = kc >> 6;
 #pragma unroll
     for (int i = 0; i < MAXU; ++i) {
-      if (i * T >= un) break;
+      if (!FULL && i * T >= un) break;
       const int u = tl + i * T;
       const bool on = u < un;
       const int uc = on ? u : un - 1;
@@ -419,10 +419,10 @@ template <int T, int R, bool PW, int KC> struct GemvQ6K {
   }
 };
 
-template <int DT, int T, int R, bool PW, int KC> struct GemvFmt;
-template <int T, int R, bool PW, int KC> struct GemvFmt<HIPQ_Q4_0, T, R, PW, KC> { typedef GemvQ40<T, R, PW, KC> type; };
-template <int T, int R, bool PW, int KC> struct GemvFmt<HIPQ_Q4_K, T, R, PW, KC> { typedef GemvQ4K<T, R, PW, KC> type; };
-template <int T, int R, bool PW, int KC> struct GemvFmt<HIPQ_Q6_K, T, R, PW, KC> { typedef GemvQ6K<T, R, PW, KC> type; };
+template <int DT, int T, int R, bool PW, int KC, bool FULL> struct GemvFmt;
+template <int T, int R, bool PW, int KC, bool FULL> struct GemvFmt<HIPQ_Q4_0, T, R, PW, KC, FULL> { typedef GemvQ40<T, R, PW, KC, FULL> type; };
+template <int T, int R, bool PW, int KC, bool FULL> struct GemvFmt<HIPQ_Q4_K, T, R, PW, KC, FULL> { typedef GemvQ4K<T, R, PW, KC, FULL> type; };
+template <int T, int R, bool PW, int KC, bool FULL> struct GemvFmt<HIPQ_Q6_K, T, R, PW, KC, FULL> { typedef GemvQ6K<T, R, PW, KC, FULL> type; };
 
 /* ---- engine --------------------------------------------------------------------- */
 
@@ -451,8 +451,8 @@ __device__ __forceinline__ void hipq_wave_lds_sync() {
 /* The pieces of the engine, so that callers with several weight-row groups per
  * wavefront can keep the loads of the next group in flight while this one is
  * computed (see gemv_engine for the plain sequence). */
-template <int DT, int T, int R, int G, bool PW, int KC = HIPQ_KCHUNK> struct GemvCore {
-  typedef typename GemvFmt<DT, T, R, PW, KC>::type F;
+template <int DT, int T, int R, int G, bool PW, int KC = HIPQ_KCHUNK, bool FULL = false> struct GemvCore {
+  typedef typename GemvFmt<DT, T, R, PW, KC, FULL>::type F;
   typedef typename F::Act Act;
   static constexpr int RW = 64 / T; /* weight rows streamed at once */
   static constexpr int NP = G / RW; /* passes per group */
@@ -513,8 +513,9 @@ template <int DT, int T, int R, int G, bool PW, int KC = HIPQ_KCHUNK> struct Gem
   }
   /* s = step(load(b), s) for b = 0 .. n - 1. The records come from LDS in batches of B, the next batch's reads in
    * flight while this one's steps run: a read takes over a hundred clocks and a step four, and a wavefront that
-   * finishes a small decode product has nothing else to do. With B = 0 a plain loop, which leaves the registers to
-   * more wavefronts: the form where many of them hide each other's reads. */
+   * finishes a small decode product has nothing else to do. n is a multiple of B (pad() rounds a row's records up), so
+   * that no read sits behind a condition; past the last batch it is read again. With B = 0 a plain loop, which leaves
+   * the registers to more wavefronts: the form where many of them hide each other's reads. */
   template <int B, typename Rec, typename State, typename Load, typename Step>
   __device__ static __forceinline__ State chain_batched(int n, State s, Load load, Step step) {
     if constexpr (B == 0) {
@@ -523,77 +524,96 @@ template <int DT, int T, int R, int G, bool PW, int KC = HIPQ_KCHUNK> struct Gem
       return s;
     }
     Rec v[2][B ? B : 1];
-    const int full = n / (B ? B : 1);
-    if (full) {
+    const int batches = n / (B ? B : 1), last = batches - 1;
+    auto read = [&](int i, Rec(&to)[B ? B : 1]) {
 #pragma unroll
-      for (int j = 0; j < B; ++j) v[0][j] = load(j);
-    }
-    auto batch = [&](int i, Rec(&cur)[B ? B : 1], Rec(&next)[B ? B : 1]) {
-      if (i + 1 < full) {
-#pragma unroll
-        for (int j = 0; j < B; ++j) next[j] = load((i + 1) * B + j);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-#pragma unroll
-      for (int j = 0; j < B; ++j) s = step(cur[j], s);
+      for (int j = 0; j < B; ++j) to[j] = load(i * B + j);
+      __builtin_amdgcn_sched_barrier(0);
     };
-    int i = 0;
-    for (; i + 1 < full; i += 2) {
-      batch(i, v[0], v[1]);
-      batch(i + 1, v[1], v[0]);
+    auto steps = [&](const Rec(&of)[B ? B : 1]) {
+#pragma unroll
+      for (int j = 0; j < B; ++j) s = step(of[j], s);
+    };
+    read(0, v[0]);
+    for (int i = 0;;) {
+      read(min(i + 1, last), v[1]);
+      steps(v[0]);
+      if (++i == batches) break;
+      read(min(i + 1, last), v[0]);
+      steps(v[1]);
+      if (++i == batches) break;
     }
-    if (i < full) batch(i, v[0], v[1]);
-    for (int b = full * B; b < n; ++b) s = step(load(b), s);
     return s;
   }
-  /* phase 2: this lane's fp32 chain over the records of one chunk, reference order. AHEAD: chain_batched's batches */
+  /* records a batch of a padded row: blocks of Q4_0, super-blocks */
+  static constexpr int PADB = DT == HIPQ_Q4_K ? 4 : 8;
+  static constexpr int BLOCK = DT == HIPQ_Q4_0 ? 32 : 256;                    /* weights a record */
+  static constexpr int RECORD = DT == HIPQ_Q4_0 ? 2 : DT == HIPQ_Q4_K ? 4 : 9; /* dwords (one activation row) */
+  /* Records of zero behind the G rows' last ones, up to whole batches: their steps add nothing (fma(0, 0, s) with s no
+   * negative zero: it starts from +0). One activation row; stride: dwords between rows. */
+  __device__ static __forceinline__ void pad(int k, uint32_t *lds, int stride) {
+    const int n = k / BLOCK, missing = -n & (PADB - 1), lane = threadIdx.x & 63;
+    static_assert(G * (PADB - 1) <= 64, "one lane a record");
+    const int g = lane / (PADB - 1), e = lane % (PADB - 1);
+    if (g < G && e < missing) {
+      uint32_t *o = lds + g * stride + (n + e) * RECORD;
+#pragma unroll
+      for (int i = 0; i < RECORD; ++i) o[i] = 0;
+    }
+  }
+  /* phase 2 of one chain over n records (not the pairwise form), reference order */
+  template <bool AHEAD>
+  __device__ static __forceinline__ void sums(const uint32_t *crec, int k, int l, float &acc, float &accm) {
+    const int n = k / BLOCK, padded = AHEAD ? (n + PADB - 1) & ~(PADB - 1) : n;
+    constexpr int B = AHEAD ? PADB : 0;
+    if constexpr (DT == HIPQ_Q4_0) {
+      acc = chain_batched<B, float2>(padded, acc, [&](int b) { return *(const float2 *)(crec + 2 * b); },
+                                     [](const float2 &v, float s) { return fmaf(v.x, v.y, s); });
+    } else if constexpr (DT == HIPQ_Q4_K) {
+      const float2 r = chain_batched<B, float4>(
+        padded, make_float2(acc, accm), [&](int b) { return *(const float4 *)(crec + 4 * b); },
+        [](const float4 &v, const float2 &s) { return make_float2(fmaf(v.x, v.y, s.x), fmaf(v.z, v.w, s.y)); });
+      acc = r.x, accm = r.y;
+    } else {
+      acc = chain_batched<B, float2>(
+        padded, acc,
+        [&](int b) { return make_float2(__uint_as_float(crec[b * 9 + 8]), __uint_as_float(crec[b * 9 + l])); },
+        [](const float2 &v, float s) { return fmaf(v.x, (float)(int)__float_as_uint(v.y), s); });
+    }
+  }
+  /* phase 2: this lane's fp32 chain over the records of one chunk, reference order. AHEAD: in batches, over rows that
+   * pad() has rounded up */
   template <bool AHEAD = false>
   __device__ static __forceinline__ void chain(Chain &c, int kc, const uint32_t *lds) {
     const uint32_t *crec = lds + (c.cg * R + c.cr) * PER;
-    const bool chain = c.on, pairwise = c.pairwise;
-    const int l = c.l;
-    float acc = c.acc, accm = c.accm;
-    (void)pairwise;
-    (void)l;
-    if (chain) {
-      if (DT == HIPQ_Q4_0) {
-        acc = chain_batched<AHEAD ? 8 : 0, float2>(kc >> 5, acc, [&](int b) { return *(const float2 *)(crec + 2 * b); },
-                                        [](const float2 &v, float s) { return fmaf(v.x, v.y, s); });
-      } else if (DT == HIPQ_Q4_K && !PW) {
-        const float2 sums = chain_batched<AHEAD ? 4 : 0, float4>(
-          kc >> 8, make_float2(acc, accm), [&](int b) { return *(const float4 *)(crec + 4 * b); },
-          [](const float4 &v, const float2 &s) { return make_float2(fmaf(v.x, v.y, s.x), fmaf(v.z, v.w, s.y)); });
-        acc = sums.x, accm = sums.y;
-      } else if (DT == HIPQ_Q4_K) {
-        const int nb = kc >> 8;
-        for (int b = 0; b < nb; ++b) {
-          const uint32_t *o = crec + b * 10;
-          const int I0 = (int)o[0], I1 = (int)o[1], I2 = (int)o[2], I3 = (int)o[3];
-          const int M0 = (int)o[4], M1 = (int)o[5], M2 = (int)o[6], M3 = (int)o[7];
-          const float sd = __uint_as_float(o[8]), sm = __uint_as_float(o[9]);
-          if (pairwise) {
-            acc = fmaf((float)I0, sd, acc);
-            accm = fmaf((float)M0, sm, accm);
-            acc = fmaf((float)I1, sd, acc);
-            accm = fmaf((float)M1, sm, accm);
-            acc = fmaf((float)I2, sd, acc);
-            accm = fmaf((float)M2, sm, accm);
-            acc = fmaf((float)I3, sd, acc);
-            accm = fmaf((float)M3, sm, accm);
-          } else {
-            acc = fmaf((float)(I0 + I1 + I2 + I3), sd, acc);
-            accm = fmaf((float)(M0 + M1 + M2 + M3), sm, accm);
-          }
+    if (!c.on) return;
+    if constexpr (DT == HIPQ_Q4_K && PW) {
+      float acc = c.acc, accm = c.accm;
+      const int nb = kc >> 8;
+      for (int b = 0; b < nb; ++b) {
+        const uint32_t *o = crec + b * 10;
+        const int I0 = (int)o[0], I1 = (int)o[1], I2 = (int)o[2], I3 = (int)o[3];
+        const int M0 = (int)o[4], M1 = (int)o[5], M2 = (int)o[6], M3 = (int)o[7];
+        const float sd = __uint_as_float(o[8]), sm = __uint_as_float(o[9]);
+        if (c.pairwise) {
+          acc = fmaf((float)I0, sd, acc);
+          accm = fmaf((float)M0, sm, accm);
+          acc = fmaf((float)I1, sd, acc);
+          accm = fmaf((float)M1, sm, accm);
+          acc = fmaf((float)I2, sd, acc);
+          accm = fmaf((float)M2, sm, accm);
+          acc = fmaf((float)I3, sd, acc);
+          accm = fmaf((float)M3, sm, accm);
+        } else {
+          acc = fmaf((float)(I0 + I1 + I2 + I3), sd, acc);
+          accm = fmaf((float)(M0 + M1 + M2 + M3), sm, accm);
         }
-      } else {
-        acc = chain_batched<AHEAD ? 8 : 0, float2>(
-          kc >> 8, acc,
-          [&](int b) { return make_float2(__uint_as_float(crec[b * 9 + 8]), __uint_as_float(crec[b * 9 + l])); },
-          [](const float2 &v, float s) { return fmaf(v.x, (float)(int)__float_as_uint(v.y), s); });
       }
+      c.acc = acc;
+      c.accm = accm;
+    } else {
+      sums<AHEAD>(crec, kc, c.l, c.acc, c.accm);
     }
-    c.acc = acc;
-    c.accm = accm;
   }
   __device__ static __forceinline__ GemvOut finish(const Chain &c) {
     const bool chain = c.on;
@@ -625,25 +645,29 @@ template <int DT, int T, int R, int G, bool PW, int KC = HIPQ_KCHUNK> struct Gem
   }
 };
 
-template <int DT, int T, int R, int G, bool PW, int KC = HIPQ_KCHUNK, int FK = 0>
+/* FK: the row length where the launcher has seen one of the usual ones (one chunk); -KC: any length up to KC, the
+ * capacity; 0: any number of chunks */
+template <int DT, int T, int R, int G, bool PW, int KC0 = HIPQ_KCHUNK, int FK = 0>
 __device__ __forceinline__ GemvOut gemv_engine(const WView &w, int row0, const QView &qa,
                                                const int (&arow)[R], int pair_rows,
                                                uint32_t *lds) {
-  typedef GemvCore<DT, T, R, G, PW, KC> E;
+  constexpr int KC = FK < 0 ? -FK : KC0;
+  typedef GemvCore<DT, T, R, G, PW, KC, (FK < 0)> E;
   typename E::Chain c = E::begin(arow, pair_rows);
   if constexpr (FK != 0) {
-    /* FK: the row length, where the launcher has seen one of the usual ones (one chunk). With it a constant no
-     * load sits behind a condition and the waits can count them: the activations' loads first, nothing moved
-     * across, then the weights', and each pass over the weight rows waits for its own loads only. */
+    /* With the row length or its number of steps a constant no load sits behind a condition and the waits can
+     * count them: the activations' loads first, nothing moved across, then the weights', and each pass over the
+     * weight rows waits for its own loads only. */
+    const int K = FK > 0 ? FK : w.K;
     typename E::Act A;
-    E::load_act(A, qa, arow, 0, FK);
+    E::load_act(A, qa, arow, 0, K);
     __builtin_amdgcn_sched_barrier(0);
     typename E::Wts W;
-    E::load_w(W, w, row0, 0, FK);
+    E::load_w(W, w, row0, 0, K);
     __builtin_amdgcn_sched_barrier(0);
-    E::compute(W, A, FK, lds);
+    E::compute(W, A, K, lds);
     hipq_wave_lds_sync();
-    E::chain(c, FK, lds);
+    E::chain(c, K, lds);
     hipq_wave_lds_sync();
     return E::finish(c);
   }

@@ -44,9 +44,8 @@ def test_gemv_matches_oracle(hipq, cr, kind, n, k):
                                  (1000, 1024), (40000, 1024)])
 def test_single_row_against_the_instances_by_row_length(hipq, cr, kind, n, k):
     """One row against shapes chosen by what the library picks for them: the kernels with the row length as
-    a constant (1024, 2048, 3072, 4096) and the ones that take any length (2304, 2560),
-    workgroups of twelve wavefronts whose last one hangs over the matrix's end (6150, 12290), four wavefronts
-    of four rows (8200), the plain and the streamed kernel behind the quantizer's launch (33000 and 40000
+    a constant (1024, 2048, 3072, 4096) and the ones that take any length (2304, 2560), last workgroups that
+    hang over the matrix's end (6150, 8200, 12290), the kernel behind the quantizer's launch (33000 and 40000
     columns). Same bits as the reference's row product."""
     import gpu_util as gu
     blocks = _weights(cr, kind, n, k, seed=900 + n % 97)
@@ -58,6 +57,71 @@ def test_single_row_against_the_instances_by_row_length(hipq, cr, kind, n, k):
     assert not np.isnan(got).any()
     assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), \
         "%d of %d outputs differ in bits" % ((got.view(np.uint32) != ref.view(np.uint32)).sum(), got.size)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("n,k", [
+    # rows within one chunk: at, above and below whole steps of the 16, 32 and 64 lanes a row, and of the sums' batches
+    (100, 512), (6144, 768), (70, 1280), (1024, 1792), (1025, 2304), (2049, 2816), (2051, 3328), (3000, 3840), (4100, 3584),
+    # rows that a workgroup's wavefronts share, quantized in the kernel: one to four rows a wavefront, parts of unequal
+    # length, the longest row
+    (3, 4352), (1024, 4608), (1025, 6400), (1030, 8192), (4096, 16384), (37, 12544), (8192, 4352),
+    # the same behind the quantizer's launch: more rows, rows longer than one pass of a workgroup quantizes
+    (8193, 4352), (9, 16640), (70, 32768),
+    # longer than 32768 (Q6_K: 65536): walked in chunks
+    (5, 33024),
+    # the wide matrices behind the quantizer's launch
+    (32769, 512), (32771, 1792), (32770, 2816), (32773, 3840)])
+def test_single_row_by_length_and_rows(hipq, cr, kind, n, k):
+    """One row against matrices around the lines of the GEMV's dispatch (lanes a row, rows a wavefront, steps of a lane,
+    parts of a long row). Same bits as the reference's row product; the weights are random blocks of few distinct rows."""
+    import gpu_util as gu
+    few = _weights(cr, kind, min(n, 61), k, seed=2000 + n % 97)
+    rows = np.random.RandomState(n).randint(0, min(n, 61), n)
+    blocks = np.ascontiguousarray(few.reshape(min(n, 61), -1)[rows])
+    a = synth.normal(2100 + k % 89, (1, k))
+    ref = cr.gemm(cr.oracle(), kind, a, few, min(n, 61))[:, rows]
+    w = capi.Weight(kind, n, k, blocks)
+    got = gu.gpu_matmul(w, a)
+    w.destroy()
+    assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), \
+        "%d of %d outputs differ in bits" % ((got.view(np.uint32) != ref.view(np.uint32)).sum(), got.size)
+
+
+@pytest.mark.parametrize("k", [32, 800, 2336, 4128, 6112, 16352, 33056])
+def test_single_q4_0_row_of_whole_blocks_only(hipq, cr, k):
+    """Rows of whole blocks of 32 that end inside a batch of the sums' records and inside a part of a long row."""
+    import gpu_util as gu
+    for n in (33, 2100):
+        few = _weights(cr, "q4_0", 33, k, seed=2200 + k % 97)
+        rows = np.random.RandomState(n).randint(0, 33, n)
+        a = synth.normal(2300 + k % 89, (1, k))
+        ref = cr.gemm(cr.oracle(), "q4_0", a, few, 33)[:, rows]
+        w = capi.Weight("q4_0", n, k, np.ascontiguousarray(few.reshape(33, -1)[rows]))
+        got = gu.gpu_matmul(w, a)
+        w.destroy()
+        assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), (n, k)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("n,k", [(770, 1792), (1024, 2304), (2050, 2816), (2048, 3072), (600, 3584), (2500, 3840)])
+def test_gated_pair_of_one_row_by_length_and_rows(hipq, cr, kind, n, k):
+    """mlp_swiglu on one row takes the same forms with two matrices a wavefront: its sums have the bits of the two single
+    products, seen through the activation as numpy forms it from them (a few units in the last place of its exponential)."""
+    import gpu_util as gu
+    a = synth.normal(2400 + k % 89, (1, k))
+    few = [_weights(cr, kind, 41, k, seed=2500 + i) for i in range(2)]
+    rows = [np.random.RandomState(n + i).randint(0, 41, n) for i in range(2)]
+    y, z = (cr.gemm(cr.oracle(), kind, a, few[i], 41)[0, rows[i]] for i in range(2))
+    ws = [capi.Weight(kind, n, k, np.ascontiguousarray(few[i].reshape(41, -1)[rows[i]])) for i in range(2)]
+    da, out = gu.dev(a), gu.dev(np.full((1, n), np.nan, np.float32))
+    capi.mlp_swiglu(ws[0], ws[1], da, 1, out, stream=gu.stream())
+    got = out.cpu().numpy()[0].astype(np.float64)
+    for w in ws:
+        w.destroy()
+    want = y.astype(np.float64) / (1 + np.exp(-y.astype(np.float64))) * z.astype(np.float64)
+    # exp, sum, quotient and product: under eight roundings of 2^-24 relative
+    assert (np.abs(got - want) <= 8 * 2.0 ** -24 * np.abs(want) + 1e-30).all(), np.abs(got / want - 1).max()
 
 
 @pytest.mark.parametrize("kind", KINDS)
