@@ -347,7 +347,8 @@ __global__ __launch_bounds__(NT, TM == 2 ? 3 : 2) void gemm_q4k_kernel(WView w, 
  * workgroups, each walking all of K: 31 us at 12288 x 4096 whatever the row count): blockIdx.y
  * takes a part of K and writes its partial product to part[y]; split_sum_kernel adds the parts
  * in ascending order. */
-__global__ __launch_bounds__(NT, 3) void gemm_q4k_split_kernel(WView w, const int8_t *__restrict__ qt,
+template <int TM>
+__global__ __launch_bounds__(NT, TM == 2 ? 3 : 2) void gemm_q4k_split_kernel(WView w, const int8_t *__restrict__ qt,
                                                                const uint16_t *__restrict__ amin,
                                                                const float *__restrict__ dAt, int M, int mtiles,
                                                                int ntiles, int sb_per_part, float *__restrict__ part,
@@ -358,7 +359,7 @@ __global__ __launch_bounds__(NT, 3) void gemm_q4k_split_kernel(WView w, const in
   if (nt >= ntiles) return; /* uniform per workgroup */
   const int sb0 = blockIdx.y * sb_per_part;
   const int n = min(sb_per_part, (w.K >> 8) - sb0);
-  gemm_q4k_tile<2, true, true>(w, qt, amin, dAt, M, mt, nt, part + (int64_t)blockIdx.y * part_stride, w.N, sb0, n);
+  gemm_q4k_tile<TM, true, true>(w, qt, amin, dAt, M, mt, nt, part + (int64_t)blockIdx.y * part_stride, w.N, sb0, n);
 }
 
 __global__ __launch_bounds__(256) void split_sum_kernel(const float *__restrict__ part, int parts, int64_t part_stride,
@@ -536,38 +537,35 @@ int launch_gemm_q4k_gated(const hipq_weight *wa, const hipq_weight *wm, const QA
   return HIPQ_OK;
 }
 
-/* Parts of K for a product whose 64-row tiles would leave most of the chip idle (0: none), and
- * the bytes of partial products they need. */
-int gemm_q4k_split_parts(const hipq_weight *w, int64_t M) {
-  if (w->dtype != HIPQ_Q4_K || !w->gt_base || (w->N & 3)) return 0;
-  const int64_t tiles = ((M + 63) / 64) * ((w->N + BN - 1) / BN), nsb = w->K / 256;
-  /* measured at 12288 x 4096 (us, whole K a workgroup -> parts): 17..64 rows 31 -> 17-20, 128 rows
-   * 33 -> 28; with more than 192 tiles the parts cost what they gain (256 rows 39.4 -> 40.8) */
-  if (tiles > 192 || nsb < 8) return 0;
-  int parts = (int)(768 / tiles); /* three workgroups a CU */
-  if (parts > 8) parts = 8;
-  if (parts > nsb / 4) parts = (int)(nsb / 4);
-  return parts >= 2 ? parts : 0;
+static constexpr TileCost COST = {{0.f, 1.35f, 1.93f, 2.58f}, {0.f, 2.41f, 3.3f}};
+static TilePlan plan(const hipq_weight *w, int64_t M) {
+  return tile_plan(COST, M, w->N, w->K, w->dtype == HIPQ_Q4_K && w->gt_base && !(w->N & 3));
 }
+/* bytes of the partial products of a product in parts of K (0: whole) */
 size_t gemm_q4k_split_bytes(const hipq_weight *w, int64_t M) {
-  return (size_t)gemm_q4k_split_parts(w, M) * (size_t)M * (size_t)w->N * 4;
+  const TilePlan t = plan(w, M);
+  return t.parts > 1 ? (size_t)t.parts * (size_t)M * (size_t)w->N * 4 : 0;
 }
 
 int launch_gemm_q4k(const hipq_weight *w, const QActTiled *qa, int M, float *C, int64_t ldc, hipStream_t s,
                     void *partials) {
   if ((M + 127) / 128 != qa->mtiles || qa->K != w->K)
     return fail(HIPQ_ERR_INVALID_ARGUMENT, "tiled activations do not match the matmul shape");
-  const int parts = partials ? gemm_q4k_split_parts(w, M) : 0;
-  if (parts && !(ldc & 3) && !((uintptr_t)C & 15)) {
+  const TilePlan tp = plan(w, M);
+  const int parts = tp.parts;
+  if (partials && parts > 1 && !(ldc & 3) && !((uintptr_t)C & 15)) {
+    const int tm = tp.rows / 32;
     const int nsb = (int)(w->K / 256), per = (nsb + parts - 1) / parts;
-    const int mtiles = (M + 63) / 64, ntiles = (int)((w->N + BN - 1) / BN), ngroups = (ntiles + 7) / 8;
+    const int mtiles = (M + 32 * tm - 1) / (32 * tm), ntiles = (int)((w->N + BN - 1) / BN), ngroups = (ntiles + 7) / 8;
     const int64_t stride = (int64_t)M * w->N;
     WView v = wview(w);
     v.qs = w->gt_qs;
     v.hdr = w->gt_hdr;
-    hipq::launch_kernel("gemm_q4k_split_kernel", gemm_q4k_split_kernel, dim3((unsigned)(mtiles * ngroups * 8), (unsigned)((nsb + per - 1) / per)),
-                  dim3(NT), sizeof(Smem<2>), s, v, (const int8_t *)qa->qt, (const uint16_t *)qa->amin,
-                  (const float *)qa->dAt, M, mtiles, ntiles, per, (float *)partials, stride);
+    const dim3 grid((unsigned)(mtiles * ngroups * 8), (unsigned)((nsb + per - 1) / per));
+    if (tm == 2)
+      hipq::launch_kernel("gemm_q4k_split_kernel<2>", gemm_q4k_split_kernel<2>, grid, dim3(NT), sizeof(Smem<2>), s, v, (const int8_t *)qa->qt, (const uint16_t *)qa->amin, (const float *)qa->dAt, M, mtiles, ntiles, per, (float *)partials, stride);
+    else
+      hipq::launch_kernel("gemm_q4k_split_kernel<4>", gemm_q4k_split_kernel<4>, grid, dim3(NT), sizeof(Smem<4>), s, v, (const int8_t *)qa->qt, (const uint16_t *)qa->amin, (const float *)qa->dAt, M, mtiles, ntiles, per, (float *)partials, stride);
     HIPQ_HIP(hipGetLastError());
     const int64_t quads = stride / 4;
     hipq::launch_kernel("split_sum_kernel", split_sum_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s,
@@ -576,12 +574,8 @@ int launch_gemm_q4k(const hipq_weight *w, const QActTiled *qa, int M, float *C, 
     return HIPQ_OK;
   }
   /* 128-row tiles do a fifth more work per CU and time (the weight expansion is
-   * shared by twice the rows) but only two workgroups fit a CU: 512 tiles per round
-   * against 768 of the 64-row kind. Pick by the number of rounds. */
-  const int64_t nt = (w->N + BN - 1) / BN;
-  const int64_t rounds64 = (((int64_t)(M + 63) / 64) * nt + 767) / 768;
-  const int64_t rounds128 = (((int64_t)(M + 127) / 128) * nt + 511) / 512;
-  if (rounds128 * 6 < rounds64 * 5) return launch_tiles<4>(w, qa, M, C, ldc, s);
+   * shared by twice the rows) but only two workgroups fit a CU. */
+  if (tile_plan(COST, M, w->N, w->K, false).rows == 128) return launch_tiles<4>(w, qa, M, C, ldc, s);
   return launch_tiles<2>(w, qa, M, C, ldc, s);
 }
 

@@ -302,12 +302,13 @@ __global__ __launch_bounds__(NT, TM == 2 ? 3 : 2) void gemm_q6k_kernel(WView w, 
 /* Few tiles (up to 128 rows against a matrix of a few thousand columns make under two hundred
  * workgroups, each walking all of K): blockIdx.y takes a part of K and writes its partial product to
  * part[y]; split_sum6_kernel adds the parts in ascending order. */
-__global__ __launch_bounds__(NT, 3) void gemm_q6k_split_kernel(WView w, const int8_t *__restrict__ qt,
+template <int TM>
+__global__ __launch_bounds__(NT, TM == 2 ? 3 : 2) void gemm_q6k_split_kernel(WView w, const int8_t *__restrict__ qt,
                                                                const float *__restrict__ dAt, int M, int mtiles,
                                                                int ntiles, int sb_per_part, float *__restrict__ part,
                                                                int64_t part_stride) {
   const int sb0 = blockIdx.y * sb_per_part;
-  gemm_q6k_tile<2, true>(w, qt, dAt, M, mtiles, ntiles, part + (int64_t)blockIdx.y * part_stride, w.N, sb0,
+  gemm_q6k_tile<TM, true>(w, qt, dAt, M, mtiles, ntiles, part + (int64_t)blockIdx.y * part_stride, w.N, sb0,
                          min(sb_per_part, (w.K >> 8) - sb0));
 }
 
@@ -344,19 +345,14 @@ static int launch_tiles6(const hipq_weight *w, const QActTiled *qa, int M, float
   return HIPQ_OK;
 }
 
-/* Parts of K for a product whose 64-row tiles would leave most of the chip idle (0: none), and the
- * bytes of partial products they need (the rule of the Q4_K product, gemm_q4k.hip). */
-int gemm_q6k_split_parts(const hipq_weight *w, int64_t M) {
-  if (w->dtype != HIPQ_Q6_K || !w->gt_base || (w->N & 3)) return 0;
-  const int64_t tiles = ((M + 63) / 64) * ((w->N + BN - 1) / BN), nsb = w->K / 256;
-  if (tiles > 192 || nsb < 8) return 0;
-  int parts = (int)(768 / tiles); /* three workgroups a CU */
-  if (parts > 8) parts = 8;
-  if (parts > nsb / 4) parts = (int)(nsb / 4);
-  return parts >= 2 ? parts : 0;
+static constexpr TileCost COST = {{0.f, 1.68f, 2.43f, 3.2f}, {0.f, 2.56f, 3.62f}};
+static TilePlan plan(const hipq_weight *w, int64_t M) {
+  return tile_plan(COST, M, w->N, w->K, w->dtype == HIPQ_Q6_K && w->gt_base && !(w->N & 3));
 }
+/* bytes of the partial products of a product in parts of K (0: whole) */
 size_t gemm_q6k_split_bytes(const hipq_weight *w, int64_t M) {
-  return (size_t)gemm_q6k_split_parts(w, M) * (size_t)M * (size_t)w->N * 4;
+  const TilePlan t = plan(w, M);
+  return t.parts > 1 ? (size_t)t.parts * (size_t)M * (size_t)w->N * 4 : 0;
 }
 
 int launch_gemm_q6k(const hipq_weight *w, const QActTiled *qa, int M, float *C, int64_t ldc, hipStream_t s,
@@ -364,18 +360,22 @@ int launch_gemm_q6k(const hipq_weight *w, const QActTiled *qa, int M, float *C, 
   if ((M + 127) / 128 != qa->mtiles || qa->K != w->K)
     return fail(HIPQ_ERR_INVALID_ARGUMENT, "tiled activations do not match the matmul shape");
   if (!w->gt_base) return fail(HIPQ_ERR_INVALID_ARGUMENT, "the Q6_K prefill product needs the weight's tile copy");
-  const int parts = partials ? gemm_q6k_split_parts(w, M) : 0;
-  if (parts && !(ldc & 3) && !((uintptr_t)C & 15)) {
+  const TilePlan tp = plan(w, M);
+  const int parts = tp.parts;
+  if (partials && parts > 1 && !(ldc & 3) && !((uintptr_t)C & 15)) {
+    const int tm = tp.rows / 32;
     const int nsb = (int)(w->K / 256), per = (nsb + parts - 1) / parts;
-    const int mtiles = (M + 63) / 64, ntiles = (int)((w->N + BN - 1) / BN), ngroups = (ntiles + 7) / 8;
+    const int mtiles = (M + 32 * tm - 1) / (32 * tm), ntiles = (int)((w->N + BN - 1) / BN), ngroups = (ntiles + 7) / 8;
     const int64_t stride = (int64_t)M * w->N;
     WView v = wview(w);
     v.qs = w->gt_qs;
     v.qh = w->gt_qh;
     v.hdr = w->gt_hdr;
-    hipq::launch_kernel("gemm_q6k_split_kernel", gemm_q6k_split_kernel, dim3((unsigned)(mtiles * ngroups * 8), (unsigned)((nsb + per - 1) / per)),
-                  dim3(NT), sizeof(Smem6<2>), s, v, (const int8_t *)qa->qt, (const float *)qa->dAt, M, mtiles, ntiles,
-                  per, (float *)partials, stride);
+    const dim3 grid((unsigned)(mtiles * ngroups * 8), (unsigned)((nsb + per - 1) / per));
+    if (tm == 2)
+      hipq::launch_kernel("gemm_q6k_split_kernel<2>", gemm_q6k_split_kernel<2>, grid, dim3(NT), sizeof(Smem6<2>), s, v, (const int8_t *)qa->qt, (const float *)qa->dAt, M, mtiles, ntiles, per, (float *)partials, stride);
+    else
+      hipq::launch_kernel("gemm_q6k_split_kernel<4>", gemm_q6k_split_kernel<4>, grid, dim3(NT), sizeof(Smem6<4>), s, v, (const int8_t *)qa->qt, (const float *)qa->dAt, M, mtiles, ntiles, per, (float *)partials, stride);
     HIPQ_HIP(hipGetLastError());
     hipq::launch_kernel("split_sum6_kernel", split_sum6_kernel, dim3((unsigned)((stride / 4 + 255) / 256)), dim3(256), 0, s,
                        (const float *)partials, (nsb + per - 1) / per, stride, M, (int)w->N, C, ldc);
@@ -383,12 +383,9 @@ int launch_gemm_q6k(const hipq_weight *w, const QActTiled *qa, int M, float *C, 
     return HIPQ_OK;
   }
   /* 128-row tiles halve the expansion per row (the larger part of this kernel's vector work):
-   * 862 against 726 TOP/s at 2048 x 12288 x 4096, 835 against 729 at 512 x 151936 x 4096. Two
-   * of their workgroups fit a CU instead of three, so they never need more rounds than the
-   * 64-row tiles (512 tiles of twice the rows against 768 per round); they lose only where
-   * there are too few of them to give every CU one. */
-  const int64_t tiles128 = ((int64_t)(M + 127) / 128) * ((w->N + BN - 1) / BN);
-  if (M > 64 && tiles128 >= 256) return launch_tiles6<4>(w, qa, M, C, ldc, s);
+   * 862 against 726 TOP/s at 2048 x 12288 x 4096, 835 against 729 at 512 x 151936 x 4096; two
+   * of their workgroups fit a CU instead of three. */
+  if (tile_plan(COST, M, w->N, w->K, false).rows == 128) return launch_tiles6<4>(w, qa, M, C, ldc, s);
   return launch_tiles6<2>(w, qa, M, C, ldc, s);
 }
 

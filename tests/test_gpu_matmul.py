@@ -375,6 +375,29 @@ def test_k_format_gemm_in_parts_of_k(hipq, cr, kind, m, n, k):
         w.destroy()
 
 
+@pytest.mark.parametrize("kind,m,n,k", [("q4_K", 700, 3000, 8192), ("q6_K", 700, 3000, 8192), ("q6_K", 520, 2052, 6144),
+                                        ("q4_K", 400, 4096, 6400), ("q6_K", 200, 1000, 2304)])
+def test_k_format_gemm_in_parts_of_k_by_tile_height(hipq, cr, kind, m, n, k):
+    """Products that the plan of tile height and parts forms in parts of K beyond 128 rows: 128-row tiles in three parts of
+    11, 11 and 10 super-blocks and in six, 64-row tiles in parts of unequal length. Within 1e-4 of every row's own
+    maximum, the same bits from call to call, nothing written between the rows of C."""
+    import gpu_util as gu
+    import torch
+    few = _weights(cr, kind, 61, k, seed=340 + m)
+    cols = np.random.RandomState(m).randint(0, 61, n)
+    a = synth.normal(341 + m, (m, k))
+    ref = cr.gemm(cr.oracle(), kind, a, few, 61)[:, cols]
+    w = capi.Weight(kind, n, k, np.ascontiguousarray(few.reshape(61, -1)[cols]))
+    first = gu.gpu_matmul(w, a)
+    dc = torch.full((m, n + 12), float("nan"), device="cuda")
+    capi.matmul(w, gu.dev(a), m, dc, ldc=n + 12, stream=gu.stream())
+    got = dc[:, :n].cpu().numpy()
+    assert torch.isnan(dc[:, n:]).all(), "the call wrote between the rows of C"
+    w.destroy()
+    assert (np.abs(got - ref).max(axis=1) / np.abs(ref).max(axis=1)).max() <= gu.TOL
+    assert np.array_equal(got, first), "the first call differs from the second"
+
+
 def test_q4_K_gemm_tall_tiles(hipq, cr):
     """A shape for which the Q4_K GEMM picks its 128-row tiles (two rounds of 64-row
     tiles against one of 128-row tiles), with M not a multiple of the tile height."""
