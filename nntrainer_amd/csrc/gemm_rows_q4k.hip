@@ -40,24 +40,34 @@ typedef _Float16 rv8h __attribute__((ext_vector_type(8)));
 typedef __amdgpu_buffer_rsrc_t rrsrc_t;
 
 constexpr int TC = 8;    /* activation rows a workgroup holds */
-constexpr int NREG = 4;  /* result registers of a matrix step that carry them */
 constexpr int SBR = 4;   /* super-blocks a round = wavefronts a workgroup */
 constexpr int NT = 64 * SBR;
-/* a round's partial sums: [wavefront][register][integer sums | min sums][lane][pair 0-3], so that a
- * lane writes, and a chain reads, the four pairs of one kind as one 128-bit access, consecutive
- * lanes consecutive in memory */
-constexpr int REC_DWORDS = SBR * NREG * 2 * 64 * 4;
+constexpr int NREG = 4;  /* result registers of a matrix step that carry them */
+/* PAIRS: some rows of the launch are under the 4-row rule, which adds a super-block's four sub-block pairs one after the
+ * other: a round's records are the pairs' sums. Without such rows (two and three rows, rows that are products of their own)
+ * they are the super-blocks' totals: a quarter of the LDS, so that two rounds' records fit and a round needs one barrier,
+ * a third of the chains' steps and one instruction of the mins instead of four. us a call, pairs' sums -> totals:
+ * 8 rows of 12288 x 4096 14.2 -> 12.3, of 8192 x 12288 23.0 -> 18.8, 12 of 32000 x 4096 36.6 -> 31.7, 3 of 20000 x 2048 12.1 -> 11.0
+ * (the quantizer's launch in them). Eight wavefronts a workgroup, which halve the rounds, do not fit the registers that two
+ * such workgroups a CU leave (48 spilled: 27 us at the first size). */
+template <bool PAIRS> struct Rows {
+  /* a round's partial sums. Pairs: [wavefront][register][integer sums | min sums][lane][pair 0-3], so that a
+   * lane writes, and a chain reads, the four pairs of one kind as one 128-bit access, consecutive
+   * lanes consecutive in memory. Totals: [wavefront][register][lane]{integer sum, min sum}. */
+  static constexpr int REC_DWORDS = SBR * NREG * 64 * (PAIRS ? 8 : 2);
+  static constexpr int RECS = PAIRS ? 1 : 2; /* rounds whose records (and d, dmin) are in LDS */
 
-/* LDS of a workgroup: the quantized rows of the current and of the next round (four
- * super-blocks of every row: int8 values, the sub-block sums as two fp16-exact parts, the
- * scales), the round's partial sums, and d and dmin of its super-blocks per column. */
-constexpr int QROW = SBR * 256 + 16; /* a staged row, padded so that the lanes of a 128-bit read fall into different banks */
-constexpr int ACT_Q = 0, ACT_AMIN = TC * QROW, ACT_DA = ACT_AMIN + TC * SBR * 32;
-constexpr int ACT_BYTES = ACT_DA + SBR * TC * 4;
-constexpr int LDS_REC = (2 * ACT_BYTES + 255) / 256 * 256;
-constexpr int LDS_DW = LDS_REC + REC_DWORDS * 4;
-constexpr int LDS_BYTES = LDS_DW + SBR * 2 * 32 * 4;
-static_assert(ACT_BYTES % 16 == 0 && 3 * LDS_BYTES <= 160 * 1024, "three workgroups a CU");
+  /* LDS of a workgroup: the quantized rows of the current and of the next round (SBR
+   * super-blocks of every row: int8 values, the sub-block sums as two fp16-exact parts, the
+   * scales), the round's partial sums, and d and dmin of its super-blocks per column. */
+  static constexpr int QROW = SBR * 256 + 16; /* a staged row, padded so that the lanes of a 128-bit read fall into different banks */
+  static constexpr int ACT_Q = 0, ACT_AMIN = TC * QROW, ACT_BYTES = ACT_AMIN + TC * SBR * 32;
+  static constexpr int LDS_DA = 2 * ACT_BYTES; /* the rows' scales, four rounds of them */
+  static constexpr int LDS_REC = (LDS_DA + 4 * SBR * TC * 4 + 255) / 256 * 256;
+  static constexpr int LDS_DW = LDS_REC + RECS * REC_DWORDS * 4;
+  static constexpr int LDS_BYTES = LDS_DW + RECS * SBR * 2 * 32 * 4;
+  static_assert(ACT_BYTES % 16 == 0 && 3 * LDS_BYTES <= 160 * 1024, "three workgroups a CU");
+};
 
 struct RowsRegs {
   rv4i q[4];
@@ -75,7 +85,11 @@ struct MultiRowsQ4K {
 
 /* blockIdx.y: the pass, rows 8 y .. 8 y + 7 of the call's M_all (the first pair_all of them under
  * the 4-row rule); the passes of one launch run side by side */
-__global__ __launch_bounds__(NT, 2) void gemm_rows_q4k_kernel(MultiRowsQ4K mw, QView a, int M_all, int pair_all) {
+template <bool PAIRS>
+__global__ __launch_bounds__(NT, PAIRS ? 2 : 3) void gemm_rows_q4k_kernel(MultiRowsQ4K mw, QView a, int M_all, int pair_all) {
+  typedef Rows<PAIRS> R;
+  constexpr int QROW = R::QROW, ACT_Q = R::ACT_Q, ACT_AMIN = R::ACT_AMIN, ACT_BYTES = R::ACT_BYTES, LDS_REC = R::LDS_REC,
+                LDS_DW = R::LDS_DW;
   extern __shared__ __attribute__((aligned(16))) unsigned char rows_lds[];
   /* which weight this workgroup's column tile belongs to (uniform) */
   int tile = blockIdx.x, wi = 0;
@@ -95,8 +109,7 @@ __global__ __launch_bounds__(NT, 2) void gemm_rows_q4k_kernel(MultiRowsQ4K mw, Q
   C += (int64_t)r0 * ldc;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int lane = threadIdx.x & 63, i32 = lane & 31, g = lane >> 5;
-  uint32_t *const lrec = (uint32_t *)(rows_lds + LDS_REC);
-  float *const ldw = (float *)(rows_lds + LDS_DW);
+  float *const lda_ = (float *)(rows_lds + R::LDS_DA);
 
   /* the tile's nibbles and headers as buffer descriptors in scalar registers */
   const rrsrc_t rq = __builtin_amdgcn_make_buffer_rsrc((void *)(w.qs + (size_t)tile * (size_t)(16 * K)), 0, 16 * K, 0x00020000);
@@ -121,29 +134,29 @@ __global__ __launch_bounds__(NT, 2) void gemm_rows_q4k_kernel(MultiRowsQ4K mw, Q
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int c = t + u * NT;
-      const int row = min(c >> 6, M - 1), off = min(rho * (SBR * 256) + (c & 63) * 16, K - 16);
+      const int row = min(c / (16 * SBR), M - 1), off = min(rho * (SBR * 256) + c % (16 * SBR) * 16, K - 16);
       r.q[u] = *(const rv4i *)(a.q + (size_t)row * K + off);
     }
     {
-      const int tt = t & 63, row = min(tt >> 3, M - 1);
-      const int off = min(rho * (SBR * 32) + (tt & 7) * 16, nsb * 32 - 16);
+      const int tt = t & (16 * SBR - 1), row = min(tt / (2 * SBR), M - 1);
+      const int off = min(rho * (SBR * 32) + tt % (2 * SBR) * 16, nsb * 32 - 16);
       r.amin = *(const rv4i *)((const uint8_t *)a.bsum + (size_t)row * nsb * 32 + off);
     }
     {
-      const int tt = t & 31, row = min(tt >> 2, M - 1);
-      r.dA = a.d[(size_t)row * nsb + min(rho * SBR + (tt & 3), nsb - 1)];
+      const int tt = t & (8 * SBR - 1), row = min(tt / SBR, M - 1);
+      r.dA = a.d[(size_t)row * nsb + min(rho * SBR + tt % SBR, nsb - 1)];
     }
   };
-  auto act_store = [&](const ActRegs &r, int which) {
-    unsigned char *base = rows_lds + which * ACT_BYTES;
+  auto act_store = [&](const ActRegs &r, int rho) {
+    unsigned char *base = rows_lds + (rho & 1) * ACT_BYTES;
     const int t = threadIdx.x;
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int c = t + u * NT;
-      *(rv4i *)(base + ACT_Q + (c >> 6) * QROW + (c & 63) * 16) = r.q[u];
+      *(rv4i *)(base + ACT_Q + c / (16 * SBR) * QROW + c % (16 * SBR) * 16) = r.q[u];
     }
-    if (t < 64) *(rv4i *)(base + ACT_AMIN + t * 16) = r.amin; /* [row][super-block of the round][32 bytes] */
-    if (t < 32) ((float *)(base + ACT_DA))[(t & 3) * TC + (t >> 2)] = r.dA; /* [super-block][row] */
+    if (t < 16 * SBR) *(rv4i *)(base + ACT_AMIN + t * 16) = r.amin; /* [row][super-block of the round][32 bytes] */
+    if (t < 8 * SBR) lda_[(rho & 3) * (SBR * TC) + t % SBR * TC + t / SBR] = r.dA; /* [round][super-block][row] */
   };
   ActRegs AR;
   act_load(AR, 0);
@@ -168,6 +181,8 @@ __global__ __launch_bounds__(NT, 2) void gemm_rows_q4k_kernel(MultiRowsQ4K mw, Q
 
   auto round = [&](const RowsRegs &W, int rho) {
     const unsigned char *act = rows_lds + (rho & 1) * ACT_BYTES;
+    uint32_t *const lrec = (uint32_t *)(rows_lds + LDS_REC) + (PAIRS ? 0 : (rho & 1) * R::REC_DWORDS);
+    float *const ldw = (float *)(rows_lds + LDS_DW) + (PAIRS ? 0 : (rho & 1) * (SBR * 2 * 32));
     const int sb = rho * SBR + wave;
     if (sb < nsb) { /* uniform per wavefront */
       const rv16i zero16 = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
@@ -187,9 +202,10 @@ __global__ __launch_bounds__(NT, 2) void gemm_rows_q4k_kernel(MultiRowsQ4K mw, Q
       const uint4 hd = make_uint4((uint32_t)W.hd[0], (uint32_t)W.hd[1], (uint32_t)W.hd[2], (uint32_t)W.hd[3]);
       const uint32_t s03 = hd.y & 0x3f3f3f3fu;
       const uint32_t s47 = hd.z & 0x3f3f3f3fu;
-      int I[4][NREG];
+      constexpr int NP = PAIRS ? 4 : 1; /* sums of a kind an output and super-block */
+      int I[NP][NREG];
 #pragma unroll
-      for (int p = 0; p < 4; ++p)
+      for (int p = 0; p < NP; ++p)
 #pragma unroll
         for (int r = 0; r < NREG; ++r) I[p][r] = 0;
       /* With two wavefronts a SIMD nobody else hides a step's latencies: the eight operands are
@@ -214,49 +230,61 @@ __global__ __launch_bounds__(NT, 2) void gemm_rows_q4k_kernel(MultiRowsQ4K mw, Q
         if (j + 1 < 8) step(j + 1);
         const int scj = (int)(((j < 4 ? s03 : s47) >> (8 * (j & 3))) & 0xff);
 #pragma unroll
-        for (int r = 0; r < NREG; ++r) I[j >> 1][r] = __mul24(D[j & 1][r], scj) + I[j >> 1][r];
+        for (int r = 0; r < NREG; ++r) I[PAIRS ? j >> 1 : 0][r] = __mul24(D[j & 1][r], scj) + I[PAIRS ? j >> 1 : 0][r];
       }
       const uint32_t mlo = (hd.w & 0x0f0f0f0fu) | ((hd.y >> 2) & 0x30303030u);
       const uint32_t mhi = ((hd.w >> 4) & 0x0f0f0f0fu) | ((hd.z >> 2) & 0x30303030u);
-      float Sm[4][NREG];
+      float Sm[NP][NREG];
 #pragma unroll
-      for (int p = 0; p < 4; ++p) {
-        /* the mins of pair p against the sub-block sums (both halves of the K index carry the same
+      for (int p = 0; p < NP; ++p) {
+        /* the mins (of pair p) against the sub-block sums (both halves of the K index carry the same
          * mins: one half meets the sums' low parts, the other the rest) */
-        const uint32_t mw = p < 2 ? mlo : mhi;
         rv8h bmin = {0, 0, 0, 0, 0, 0, 0, 0};
-        bmin[2 * p] = (_Float16)(float)((mw >> (16 * (p & 1))) & 0xff);
-        bmin[2 * p + 1] = (_Float16)(float)((mw >> (16 * (p & 1) + 8)) & 0xff);
+#pragma unroll
+        for (int j = 2 * p; j < (PAIRS ? 2 * p + 2 : 8); ++j) bmin[j] = (_Float16)(float)(((j < 4 ? mlo : mhi) >> (8 * (j & 3))) & 0xff);
         const rv16f S = __builtin_amdgcn_mfma_f32_32x32x16_f16(amin, bmin, zero16f, 0, 0, 0);
 #pragma unroll
         for (int r = 0; r < NREG; ++r) Sm[p][r] = S[r];
       }
-      uint32_t *rec = lrec + wave * (NREG * 2 * 256) + lane * 4;
+      if constexpr (PAIRS) {
+        uint32_t *rec = lrec + wave * (NREG * 2 * 256) + lane * 4;
 #pragma unroll
-      for (int r = 0; r < NREG; ++r) {
-        *(rv4i *)(rec + (r * 2) * 256) = rv4i{I[0][r], I[1][r], I[2][r], I[3][r]};
-        *(rv4i *)(rec + (r * 2 + 1) * 256) =
-          rv4i{(int)__float_as_uint(Sm[0][r]), (int)__float_as_uint(Sm[1][r]), (int)__float_as_uint(Sm[2][r]),
-               (int)__float_as_uint(Sm[3][r])};
+        for (int r = 0; r < NREG; ++r) {
+          *(rv4i *)(rec + (r * 2) * 256) = rv4i{I[0][r], I[1][r], I[2][r], I[3][r]};
+          *(rv4i *)(rec + (r * 2 + 1) * 256) =
+            rv4i{(int)__float_as_uint(Sm[0][r]), (int)__float_as_uint(Sm[1][r]), (int)__float_as_uint(Sm[2][r]),
+                 (int)__float_as_uint(Sm[3][r])};
+        }
+      } else {
+        uint32_t *rec = lrec + wave * (NREG * 128) + lane * 2;
+#pragma unroll
+        for (int r = 0; r < NREG; ++r) *(rv2i *)(rec + r * 128) = rv2i{I[0][r], (int)__float_as_uint(Sm[0][r])};
       }
       if (g == 0) {
         ldw[(wave * 2) * 32 + i32] = hipq_h2f((uint16_t)(hd.x & 0xffff));
         ldw[(wave * 2 + 1) * 32 + i32] = hipq_h2f((uint16_t)(hd.x >> 16));
       }
     }
+    /* the next round's rows: that buffer was last read in front of the last round's barrier, the place of the scales, which
+     * the chains behind it read, four rounds ago */
+    act_store(AR, rho + 1);
     __syncthreads();
-    act_store(AR, (rho + 1) & 1); /* the next round's rows: that buffer was last read a round ago */
     /* the chains of this round's super-blocks, ascending; everything a chain reads is requested
      * before the first step (the records of a wavefront that had no super-block are read as well
      * and not used: a read behind a branch would wait for its own latency) */
-    rv4i ivs[SBR], mvs[SBR];
+    rv4i ivs[PAIRS ? SBR : 1], mvs[PAIRS ? SBR : 1];
+    rv2i tot[PAIRS ? 1 : SBR];
     float dAs[SBR], dws[SBR], dms[SBR];
 #pragma unroll
     for (int ws = 0; ws < SBR; ++ws) {
-      const uint32_t *rec = lrec + ws * (NREG * 2 * 256) + (cr * 2) * 256 + cl * 4;
-      ivs[ws] = *(const rv4i *)rec;
-      mvs[ws] = *(const rv4i *)(rec + 256);
-      dAs[ws] = ((const float *)(act + ACT_DA))[ws * TC + cm];
+      if constexpr (PAIRS) {
+        const uint32_t *rec = lrec + ws * (NREG * 2 * 256) + (cr * 2) * 256 + cl * 4;
+        ivs[ws] = *(const rv4i *)rec;
+        mvs[ws] = *(const rv4i *)(rec + 256);
+      } else {
+        tot[ws] = *(const rv2i *)(lrec + ws * (NREG * 128) + cr * 128 + cl * 2);
+      }
+      dAs[ws] = lda_[(rho & 3) * (SBR * TC) + ws * TC + cm];
       dws[ws] = ldw[(ws * 2) * 32 + cn];
       dms[ws] = ldw[(ws * 2 + 1) * 32 + cn];
     }
@@ -264,29 +292,34 @@ __global__ __launch_bounds__(NT, 2) void gemm_rows_q4k_kernel(MultiRowsQ4K mw, Q
     for (int ws = 0; ws < SBR; ++ws) {
       const int sbw = rho * SBR + ws;
       if (sbw < nsb) { /* uniform */
-        const rv4i iv = ivs[ws], mv = mvs[ws];
-        const int I0 = iv[0], I1 = iv[1], I2 = iv[2], I3 = iv[3];
-        const float M0 = __int_as_float(mv[0]), M1 = __int_as_float(mv[1]), M2 = __int_as_float(mv[2]),
-                    M3 = __int_as_float(mv[3]);
         const float dA = dAs[ws];
         const float sd = dws[ws] * dA, sm = dms[ws] * dA;
-        if (pairwise) {
-          acc = fmaf((float)I0, sd, acc);
-          accm = fmaf(M0, sm, accm);
-          acc = fmaf((float)I1, sd, acc);
-          accm = fmaf(M1, sm, accm);
-          acc = fmaf((float)I2, sd, acc);
-          accm = fmaf(M2, sm, accm);
-          acc = fmaf((float)I3, sd, acc);
-          accm = fmaf(M3, sm, accm);
+        if constexpr (PAIRS) {
+          const rv4i iv = ivs[ws], mv = mvs[ws];
+          const int I0 = iv[0], I1 = iv[1], I2 = iv[2], I3 = iv[3];
+          const float M0 = __int_as_float(mv[0]), M1 = __int_as_float(mv[1]), M2 = __int_as_float(mv[2]),
+                      M3 = __int_as_float(mv[3]);
+          if (pairwise) {
+            acc = fmaf((float)I0, sd, acc);
+            accm = fmaf(M0, sm, accm);
+            acc = fmaf((float)I1, sd, acc);
+            accm = fmaf(M1, sm, accm);
+            acc = fmaf((float)I2, sd, acc);
+            accm = fmaf(M2, sm, accm);
+            acc = fmaf((float)I3, sd, acc);
+            accm = fmaf(M3, sm, accm);
+          } else {
+            /* the partial sums of the mins are integers below 2^24: their fp32 sum is exact */
+            acc = fmaf((float)(I0 + I1 + I2 + I3), sd, acc);
+            accm = fmaf((M0 + M1) + (M2 + M3), sm, accm);
+          }
         } else {
-          /* the partial sums of the mins are integers below 2^24: their fp32 sum is exact */
-          acc = fmaf((float)(I0 + I1 + I2 + I3), sd, acc);
-          accm = fmaf((M0 + M1) + (M2 + M3), sm, accm);
+          acc = fmaf((float)tot[ws][0], sd, acc);
+          accm = fmaf(__int_as_float(tot[ws][1]), sm, accm);
         }
       }
     }
-    __syncthreads(); /* the next round overwrites the records */
+    if constexpr (PAIRS) __syncthreads(); /* the next round overwrites the records */
   };
   /* NB rounds a trip so that each register set has a fixed name; all conditions are uniform */
   for (int rho0 = 0; rho0 < rounds; rho0 += NB) {
@@ -378,8 +411,13 @@ int launch_gemm_rows_q4k_multi(int count, const hipq_weight *const *w, const QAc
     mw.ldc[i] = ldc[j];
     mw.tile_end[i] = tiles; /* unused entries repeat the total: no workgroup lands in them */
   }
-  hipq::launch_kernel("gemm_rows_q4k_kernel", gemm_rows_q4k_kernel, dim3((unsigned)tiles, (unsigned)((M + TC - 1) / TC)), dim3(NT), LDS_BYTES, s, mw,
-                     qview(*qa), M, pair_rows);
+  const dim3 grid((unsigned)tiles, (unsigned)((M + TC - 1) / TC));
+  if (pair_rows)
+    hipq::launch_kernel("gemm_rows_q4k_kernel<true>", gemm_rows_q4k_kernel<true>, grid, dim3(NT), Rows<true>::LDS_BYTES, s, mw,
+                        qview(*qa), M, pair_rows);
+  else
+    hipq::launch_kernel("gemm_rows_q4k_kernel<false>", gemm_rows_q4k_kernel<false>, grid, dim3(NT), Rows<false>::LDS_BYTES, s,
+                        mw, qview(*qa), M, 0);
   HIPQ_HIP(hipGetLastError());
   return HIPQ_OK;
 }

@@ -965,6 +965,24 @@ def test_matmul_each_row_has_the_bits_of_single_row_products(hipq, cr, kind, row
         w.destroy()
 
 
+@pytest.mark.parametrize("rows,n,k", [(5, 1030, 256), (8, 1056, 2304), (13, 1100, 4352), (61, 1027, 1280), (16, 2049, 1024)])
+def test_q4_K_few_rows_of_their_own_by_rounds(hipq, cr, rows, n, k):
+    """Rows that are products of their own take the few-rows kernel whose records are super-block totals: one super-block, whole
+    rounds of four and a rest of one, row counts that leave the last pass partly empty, columns beyond the last tile of 32.
+    The bits of the row products."""
+    import gpu_util as gu
+    few = _weights(cr, "q4_K", 37, k, seed=2600 + k % 97)
+    cols = np.random.RandomState(n).randint(0, 37, n)
+    a = synth.normal(2601 + k % 89, (rows, k))
+    ref = np.concatenate([cr.gemm(cr.oracle(), "q4_K", a[r:r + 1], few, 37) for r in range(rows)])[:, cols]
+    w = capi.Weight("q4_K", n, k, np.ascontiguousarray(few.reshape(37, -1)[cols]))
+    out = gu.dev(np.full((rows, n), np.nan, np.float32))
+    capi.matmul_each_row(w, gu.dev(a), rows, out, stream=gu.stream())
+    got = out.cpu().numpy()
+    w.destroy()
+    assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
+
+
 def test_row_counts_across_the_kernel_choices(hipq, cr):
     """hipq_matmul picks among the GEMV engine, the few-rows matrix-core kernel (one to eight passes),
     the prefill GEMMs (whole K or parts of K) by format, row count and matrix size. Shapes drawn
