@@ -836,6 +836,29 @@ int launch_gated(const hipq_weight *wa, const hipq_weight *wm, const float *A, i
   return hipq::launch_gemm_q4k_gated(wa, wm, &qa, (int)M, out, ldo, s);
 }
 
+/* The whole gated MLP of a prompt on six-bit operands: the rows' quantizer, the gated pair, whose epilogue quantizes the
+ * hidden rows, the down projection. *done stays false where a copy is missing that could not be had now (or would be made by
+ * the down projection's quantizer, which falls away here): the products one by one. */
+int mlp_f6(const hipq_weight *wa, const hipq_weight *wm, const hipq_weight *wd, const float *A, int64_t M, int64_t lda,
+           float *out, int64_t ldo, hipStream_t s, bool *done) {
+  const hipq_weight *ws[2] = {wa, wm};
+  *done = false;
+  const Scratch sc{false, s};
+  bool ready = false;
+  hipq::F6Make none, make;
+  int rc;
+  if ((rc = hipq::f6_copies(1, &wd, s, false, &ready, &none)) || !ready) return rc;
+  if ((rc = f6_ready(2, ws, M, s, sc, &ready, &make)) || !ready) return rc;
+  const size_t x_bytes = (hipq::qact_f6_bytes(M, wa->K) + 255) & ~(size_t)255;
+  void *mem = nullptr;
+  if ((rc = sc.get(x_bytes + hipq::qact_f6_bytes(M, wd->K), &mem))) return rc;
+  QActF6 qa = hipq::qact_f6_carve(mem, M, wa->K), qh = hipq::qact_f6_carve((char *)mem + x_bytes, M, wd->K);
+  if ((rc = hipq::launch_quantize_q8_0_f6(A, M, wa->K, lda, &qa, &make, s))) return rc;
+  *done = true;
+  if ((rc = hipq::launch_gemm_f6_gated(wa, wm, &qa, (int)M, nullptr, 0, s, &qh))) return rc;
+  return hipq::launch_gemm_f6(1, &wd, &qh, (int)M, &out, &ldo, s);
+}
+
 /* each_row: every row as a product of its own with M = 1 (the bits of M separate calls): for Q4_0
  * and Q6_K that is what up to 16 rows give anyway; Q4_K drops the 4-row quantizer and the pairwise
  * sums the reference applies to rows it multiplies together. The caller passes at most 16 rows. */
@@ -1528,6 +1551,10 @@ int hipq_mlp_swiglu_down(hipq_weight_t w_act, hipq_weight_t w_mul, hipq_weight_t
       if ((rr = hipq::launch_gemv_fused_swiglu(w_act, w_mul, a, dH + r0 * N, s))) return rr;
       done = true;
     } else if (wants_gated(w_act, w_mul, n)) {
+      const hipq_weight *wd = w_down;
+      if (w_act->dtype == HIPQ_Q4_0 && wants_f6(1, &wd, n)) {
+        if ((rr = mlp_f6(w_act, w_mul, w_down, a, n, a_ld, o_dev + r0 * o_ld, o_ld, s, &done)) || done) return rr;
+      }
       if ((rr = launch_gated(w_act, w_mul, a, n, a_ld, dH + r0 * N, N, s, &done))) return rr;
     }
     if (!done) {

@@ -291,18 +291,73 @@ __global__ __launch_bounds__(NT, LOOK == 1 ? 3 : 2) void gemm_f6_kernel(MultiF6 
   set_word(mw.word);
 }
 
+/* A value of magnitude at most 128 as two bf6 (e3m2) codes in units of 1/16: the magnitude rounded to three
+ * significant bits, and the rest (at most 8: codes up to 8 are the number itself). */
+__device__ __forceinline__ void bf6_parts(int v, uint32_t &first, uint32_t &second) {
+  const int mag = v < 0 ? -v : v;
+  const uint32_t t = (__float_as_uint((float)mag) + (1u << 20)) >> 21; /* exponent and two mantissa bits */
+  const bool small = mag < 4;
+  const int rest = small ? 0 : mag - (int)__uint_as_float(t << 21);
+  const uint32_t sign = v < 0 ? 0x20u : 0u;
+  first = sign | (small ? (uint32_t)mag : t - 512u);
+  second = (rest < 0 ? (sign ^ 0x20u) | (uint32_t)(-rest) : sign | (uint32_t)rest);
+}
+
+/* Block b (of nbp a row) of row m: the calling lane's four of its values in x, the block's eight lanes consecutive */
+__device__ __forceinline__ void f6_quantize_block(const float4 &x, int64_t m, int b, int nbp, uint8_t *__restrict__ out,
+                                                  uint32_t *__restrict__ flags, uint32_t token) {
+  const int lane = threadIdx.x & 63, sub = lane & 7;
+  constexpr int PARTS = hipq::F6_ROWS * 384;
+  uint16_t dh;
+  int qsum;
+  const uint32_t q = (uint32_t)hipq_quantize_q8_0_lane(x, dh, qsum);
+  uint32_t part[2] = {0, 0}; /* this lane's four codes of each part, 24 bits */
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    uint32_t first, second;
+    bf6_parts((int)(int8_t)(q >> (8 * k)), first, second);
+    part[0] |= first << (6 * k);
+    part[1] |= second << (6 * k);
+  }
+  uint32_t w[6]; /* the quad's sixteen values: 96 bits of each part */
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int mine = (int)part[h];
+    const uint32_t x0 = (uint32_t)hipq_dpp_i<0x00>(mine), x1 = (uint32_t)hipq_dpp_i<0x55>(mine),
+                   x2 = (uint32_t)hipq_dpp_i<0xAA>(mine), x3 = (uint32_t)hipq_dpp_i<0xFF>(mine);
+    w[3 * h] = x0 | (x1 << 24);
+    w[3 * h + 1] = (x1 >> 8) | (x2 << 16);
+    w[3 * h + 2] = (x2 >> 16) | (x3 << 8);
+  }
+  const int r = (int)(m & (hipq::F6_ROWS - 1)), g = sub >> 2, j = b & 7;
+  uint8_t *dst = out + ((m / hipq::F6_ROWS) * (nbp >> 3) + (b >> 3)) * hipq::F6_CHUNK;
+  uint8_t *o = dst + (r >> 5) * (PARTS / 2) + j * 1536;
+  const int at = g * 32 + (r & 31);
+  if ((lane & 3) == 0) *(uint4 *)(o + at * 16) = make_uint4(w[0], w[1], w[2], w[3]);
+  if ((lane & 3) == 1) *(uint2 *)(o + 1024 + at * 8) = make_uint2(w[4], w[5]);
+  if (sub == 0) {
+    *(uint16_t *)(dst + PARTS + r * 16 + j * 2) = dh;
+    if ((dh & 0x7c00) == 0x7c00) flags[m >> 5] = token; /* not finite: f6_sums_plain */
+  }
+}
+
 /* The gated pair of an MLP: out = swiglu(act sums) * mul sums. Two wavefronts of a workgroup take 32 columns each of the
  * one matrix, the other two the same columns of the other; at the end each keeps half of its tile's rows and hands the
  * other half over through LDS. The two products never reach memory: as products and a launch of the activation 512 rows of
- * 3072 columns wrote and read 25 MB more (294 -> 273 us for four decoder layers). */
+ * 3072 columns wrote and read 25 MB more (294 -> 273 us for four decoder layers). QUANT: the result goes out quantized, as the
+ * operand of the down projection behind it: 32 columns of a tile are the blocks of 32 rows, which pass through LDS to the
+ * lanes that the quantizer gives them. As fp32 rows and a quantizer's launch 512 rows of 3072 columns wrote and read 12.6 MB
+ * more (four decoder layers of 1024 and 3072 over 512 rows 271.6 -> 253.7 us). */
 struct GatedF6 {
   const uint8_t *act, *mul;
   float *out;
   int64_t ldo;
-  int N, ntiles; /* columns, workgroup columns of 64 */
+  int N, ntiles; /* columns, workgroup columns of 64 (QUANT: with those that fill the last chunk, written as zeros) */
   uint32_t *word; /* or null: set_word */
+  uint8_t *q;     /* QUANT: where the quantized rows go (QActF6) */
+  uint32_t *flags, token;
 };
-template <int LOOK>
+template <int LOOK, bool QUANT>
 __device__ __forceinline__ void f6_gated_tile(const GatedF6 &p, int chunks, const ActF6 &act, int M, int mt, int nt) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int lane = threadIdx.x & 63, i32 = lane & 31, g = lane >> 5;
@@ -317,6 +372,25 @@ __device__ __forceinline__ void f6_gated_tile(const GatedF6 &p, int chunks, cons
 #pragma unroll
   for (int r = 0; r < 8; ++r) mine[r * 64 + lane] = second ? acc[r] : acc[8 + r];
   __syncthreads();
+  if constexpr (QUANT) {
+    constexpr int LD = 36; /* floats between the rows of a tile: whole 16 bytes, and rows on different banks */
+    float *hs = (float *)smem + 4 * 512, *ht = hs + (wave & 1) * (32 * LD) + i32;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const float o = other[r * 64 + lane];
+      ht[((second ? 16 : 0) + 8 * (r >> 2) + (r & 3) + 4 * g) * LD] = second ? hipq_swiglu(o, acc[8 + r]) : hipq_swiglu(acc[r], o);
+    }
+    __syncthreads();
+    const int row = threadIdx.x >> 3;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int b = nt * 2 + t;
+      float4 x = *(const float4 *)(hs + t * (32 * LD) + row * LD + (threadIdx.x & 7) * 4);
+      if (b * 32 >= p.N) x = make_float4(0.f, 0.f, 0.f, 0.f); /* uniform */
+      f6_quantize_block(x, (int64_t)mt * BM + row, b, p.ntiles * 2, p.q, p.flags, p.token);
+    }
+    return;
+  }
   const int m0 = mt * BM + (second ? 16 : 0), n = tile * 32 + i32;
   const uint32_t off = (uint32_t)(4 * g) * (uint32_t)p.ldo + (uint32_t)n;
 #pragma unroll
@@ -327,13 +401,13 @@ __device__ __forceinline__ void f6_gated_tile(const GatedF6 &p, int chunks, cons
     if (m + 4 * g < M && n < p.N) (p.out + (int64_t)m * p.ldo)[off] = h;
   }
 }
-template <int LOOK>
+template <int LOOK, bool QUANT>
 __global__ __launch_bounds__(NT, LOOK == 1 ? 3 : 2) void gemm_f6_gated_kernel(GatedF6 p, int chunks, ActF6 act, int M,
                                                                               int mtiles) {
   const int id = blockIdx.x;
   const int xcd = id & 7, qd = id >> 3;
   const int mt = qd % mtiles, nt = (qd / mtiles) * 8 + xcd;
-  if (nt < p.ntiles) f6_gated_tile<LOOK>(p, chunks, act, M, mt, nt); /* uniform per workgroup */
+  if (nt < p.ntiles) f6_gated_tile<LOOK, QUANT>(p, chunks, act, M, mt, nt); /* uniform per workgroup */
   set_word(p.word);
 }
 
@@ -418,18 +492,6 @@ __global__ __launch_bounds__(256) void f6_weights_kernel(CopyF6 cw) { F6_COPY(cw
 
 /* ---- the activations ---- */
 
-/* A value of magnitude at most 128 as two bf6 (e3m2) codes in units of 1/16: the magnitude rounded to three
- * significant bits, and the rest (at most 8: codes up to 8 are the number itself). */
-__device__ __forceinline__ void bf6_parts(int v, uint32_t &first, uint32_t &second) {
-  const int mag = v < 0 ? -v : v;
-  const uint32_t t = (__float_as_uint((float)mag) + (1u << 20)) >> 21; /* exponent and two mantissa bits */
-  const bool small = mag < 4;
-  const int rest = small ? 0 : mag - (int)__uint_as_float(t << 21);
-  const uint32_t sign = v < 0 ? 0x20u : 0u;
-  first = sign | (small ? (uint32_t)mag : t - 512u);
-  second = (rest < 0 ? (sign ^ 0x20u) | (uint32_t)(-rest) : sign | (uint32_t)rest);
-}
-
 /* Q8_0 in the form of the six-bit GEMM (QActF6). A wavefront takes one block of eight consecutive rows, eight lanes a
  * row (128 bytes of a row in, two whole lines of operands out). Rows M and beyond of the last 64 and blocks of K and
  * beyond are written as zeros. */
@@ -445,7 +507,6 @@ struct RowsF6 {
 __device__ __forceinline__ void f6_quantize(const RowsF6 &p, int block) {
   const int64_t M = p.M;
   const int K = p.K, nbp = p.nbp;
-  constexpr int PARTS = hipq::F6_ROWS * 384;
   const uint32_t unit = (uint32_t)block * 4 + (threadIdx.x >> 6);
   if (unit >= p.n_units) return; /* uniform per wavefront */
   const int lane = threadIdx.x & 63, sub = lane & 7;
@@ -454,37 +515,7 @@ __device__ __forceinline__ void f6_quantize(const RowsF6 &p, int block) {
   const int64_t m = (int64_t)octet * 8 + (lane >> 3);
   float4 x = *(const float4 *)(p.A + (m < M ? m : M - 1) * p.lda + min(b * 32 + 4 * sub, K - 4));
   if (m >= M || b * 32 >= K) x = make_float4(0.f, 0.f, 0.f, 0.f);
-  uint16_t dh;
-  int qsum;
-  const uint32_t q = (uint32_t)hipq_quantize_q8_0_lane(x, dh, qsum);
-  uint32_t part[2] = {0, 0}; /* this lane's four codes of each part, 24 bits */
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    uint32_t first, second;
-    bf6_parts((int)(int8_t)(q >> (8 * k)), first, second);
-    part[0] |= first << (6 * k);
-    part[1] |= second << (6 * k);
-  }
-  uint32_t w[6]; /* the quad's sixteen values: 96 bits of each part */
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int mine = (int)part[h];
-    const uint32_t x0 = (uint32_t)hipq_dpp_i<0x00>(mine), x1 = (uint32_t)hipq_dpp_i<0x55>(mine),
-                   x2 = (uint32_t)hipq_dpp_i<0xAA>(mine), x3 = (uint32_t)hipq_dpp_i<0xFF>(mine);
-    w[3 * h] = x0 | (x1 << 24);
-    w[3 * h + 1] = (x1 >> 8) | (x2 << 16);
-    w[3 * h + 2] = (x2 >> 16) | (x3 << 8);
-  }
-  const int r = (int)(m & (hipq::F6_ROWS - 1)), g = sub >> 2, j = b & 7;
-  uint8_t *dst = p.out + ((m / hipq::F6_ROWS) * (nbp >> 3) + (b >> 3)) * hipq::F6_CHUNK;
-  uint8_t *o = dst + (r >> 5) * (PARTS / 2) + j * 1536;
-  const int at = g * 32 + (r & 31);
-  if ((lane & 3) == 0) *(uint4 *)(o + at * 16) = make_uint4(w[0], w[1], w[2], w[3]);
-  if ((lane & 3) == 1) *(uint2 *)(o + 1024 + at * 8) = make_uint2(w[4], w[5]);
-  if (sub == 0) {
-    *(uint16_t *)(dst + PARTS + r * 16 + j * 2) = dh;
-    if ((dh & 0x7c00) == 0x7c00) p.flags[m >> 5] = p.token; /* not finite: f6_sums_plain */
-  }
+  f6_quantize_block(x, m, b, nbp, p.out, p.flags, p.token);
 }
 
 __global__ __launch_bounds__(256) void quantize_q8_0_f6_kernel(RowsF6 p) { f6_quantize(p, (int)blockIdx.x); }
@@ -538,6 +569,7 @@ struct F6Block {
 };
 
 namespace {
+std::atomic<uint32_t> f6_calls{0}; /* the calls' tokens */
 std::mutex f6_mu; /* guards what follows and every weight's gf_ fields */
 struct F6Page { /* batches and the page-locked page of their words; given back by f6_shutdown */
   static constexpr int COUNT = 1024;
@@ -752,8 +784,7 @@ int launch_quantize_q8_0_f6(const float *A, int64_t M, int64_t K, int64_t lda, Q
     return fail(HIPQ_ERR_INVALID_ARGUMENT, "activation rows must be 16-byte aligned");
   const int64_t units = (M + F6_ROWS - 1) / F6_ROWS * (F6_ROWS / 8) * (qa->chunks * 8); /* padding included */
   if (units > INT32_MAX) return fail(HIPQ_ERR_NOT_SUPPORTED, "%lld x %lld values in one call", (long long)M, (long long)K);
-  static std::atomic<uint32_t> calls{0};
-  qa->token = ++calls;
+  qa->token = ++f6_calls;
   const RowsF6 rows{A, M, lda, (uint32_t)units, qa->chunks * 8, (int)K, qa->p, qa->flags, qa->token};
   const unsigned blocks = (unsigned)((units + 3) / 4);
   if (!make || !make->count) {
@@ -845,20 +876,36 @@ int launch_gemm_f6(int count, const hipq_weight *const *w, const QActF6 *qa, int
   return HIPQ_OK;
 }
 
+/* out: the products' rows, or null and qh: the operand of a product with K = N (carved; its token is set here) */
 int launch_gemm_f6_gated(const hipq_weight *wa, const hipq_weight *wm, const QActF6 *qa, int M, float *out, int64_t ldo,
-                         hipStream_t s) {
-  if (!wa->gf_base || !wm->gf_base || wa->K != wm->K || wa->N != wm->N || wa->K != qa->K || M != qa->M)
+                         hipStream_t s, QActF6 *qh) {
+  if (!wa->gf_base || !wm->gf_base || wa->K != wm->K || wa->N != wm->N || wa->K != qa->K || M != qa->M ||
+      (qh && (qh->K != wa->N || qh->M != M || wa->N % 32)))
     return fail(HIPQ_ERR_INVALID_ARGUMENT, "the gated pair has one shape and its six-bit copies");
-  const GatedF6 p{wa->gf_base, wm->gf_base, out, ldo, (int)wa->N, (int)((wa->N + 63) / 64), qa->word};
+  GatedF6 p{wa->gf_base, wm->gf_base, out, ldo, (int)wa->N, (int)((wa->N + 63) / 64), qa->word, nullptr, nullptr, 0};
+  if (qh) {
+    qh->token = ++f6_calls;
+    p.ntiles = 4 * qh->chunks;
+    p.q = qh->p, p.flags = qh->flags, p.token = qh->token;
+  }
   const int mtiles = (M + BM - 1) / BM;
   const dim3 grid((unsigned)(mtiles * ((p.ntiles + 7) / 8) * 8));
   /* the bound of launch_gemm_f6 */
-  if ((int64_t)mtiles * p.ntiles <= 512)
-    launch_kernel("gemm_f6_gated_kernel<3>", gemm_f6_gated_kernel<3>, grid, dim3(NT), 3 * BUF, s, p, qa->chunks,
-                  ActF6{qa->p, qa->flags, qa->token}, M, mtiles);
-  else
-    launch_kernel("gemm_f6_gated_kernel<1>", gemm_f6_gated_kernel<1>, grid, dim3(NT), 3 * BUF, s, p, qa->chunks,
-                  ActF6{qa->p, qa->flags, qa->token}, M, mtiles);
+  const bool few = (int64_t)mtiles * p.ntiles <= 512;
+  auto go = [&](const char *name, auto kernel) {
+    launch_kernel(name, kernel, grid, dim3(NT), 3 * BUF, s, p, qa->chunks, ActF6{qa->p, qa->flags, qa->token}, M, mtiles);
+  };
+  if (qh) {
+    if (few)
+      go("gemm_f6_gated_kernel<3, true>", gemm_f6_gated_kernel<3, true>);
+    else
+      go("gemm_f6_gated_kernel<1, true>", gemm_f6_gated_kernel<1, true>);
+  } else {
+    if (few)
+      go("gemm_f6_gated_kernel<3, false>", gemm_f6_gated_kernel<3, false>);
+    else
+      go("gemm_f6_gated_kernel<1, false>", gemm_f6_gated_kernel<1, false>);
+  }
   HIPQ_HIP(hipGetLastError());
   return HIPQ_OK;
 }

@@ -290,7 +290,7 @@ int launch_gemm_f6(int count, const hipq_weight *const *w, const QActF6 *qa, int
                    hipStream_t s);
 /* out = swiglu(x . wa) * (x . wm) of many rows, one launch (gemm_f6.hip, gemm_q4k.hip) */
 int launch_gemm_f6_gated(const hipq_weight *wa, const hipq_weight *wm, const QActF6 *qa, int M, float *out, int64_t ldo,
-                         hipStream_t s);
+                         hipStream_t s, QActF6 *qh = nullptr);
 int launch_gemm_q4k_gated(const hipq_weight *wa, const hipq_weight *wm, const QActTiled *qa, int M, float *out, int64_t ldo,
                           hipStream_t s);
 /* The tile height (64 or 128 rows) of a prefill product of Q4_K or Q6_K and the parts of K its tiles are formed in (1:

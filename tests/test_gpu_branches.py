@@ -219,6 +219,41 @@ def test_mlp_swiglu_down_is_the_two_calls_and_matches_the_oracle(hipq, cr, kind,
             w.destroy()
 
 
+@pytest.mark.parametrize("m,k,n,nd", [(65, 96, 32, 33), (97, 256, 288, 200), (128, 544, 1056, 96), (131, 256, 2080, 64),
+                                      (2100, 64, 544, 64)])
+@pytest.mark.parametrize("huge", [False, True])
+def test_q4_0_mlp_of_a_prompt_quantizes_the_hidden_rows_in_its_epilogue(hipq, cr, m, k, n, nd, huge):
+    """hipq_mlp_swiglu_down on six-bit operands once the three weights have their copies: the gated pair's epilogue writes
+    the hidden rows quantized. Rows that leave the last 32 and 64 partly empty, hidden columns of less than a chunk, of one
+    and a quarter and of whole chunks, both read-aheads; hidden blocks whose scale is not finite (huge). The bits of the two
+    calls, from the first call (which makes the copies) to the third."""
+    import gpu_util as gu
+    import torch
+    ws = [capi.Weight("q4_0", r, c, cr.quantize_weights(cr.oracle(), "q4_0", synth.normal(8900 + i, (r, c), 0.05)))
+          for i, (r, c) in enumerate([(n, k), (n, k), (nd, n)])]
+    a = synth.normal(8903 + m, (m, k))
+    if huge:
+        a[m // 2] *= 1e5  # the pair's product of this row passes 8.3e6, where a block's fp16 scale is infinite
+    da = gu.dev(a)
+    got = []
+    for _ in range(3):
+        out = torch.full((m, nd + 4), float("nan"), device="cuda")
+        capi.mlp_swiglu_down(*ws, da, m, out, ldo=nd + 4, stream=gu.stream())
+        torch.cuda.synchronize()
+        assert torch.isnan(out[:, nd:]).all(), "the call wrote between the rows of the output"
+        got.append(out[:, :nd].cpu().numpy())
+    h, two = torch.empty((m, n), device="cuda"), torch.empty((m, nd), device="cuda")
+    capi.mlp_swiglu(ws[0], ws[1], da, m, h, stream=gu.stream())
+    capi.matmul(ws[2], h, m, two, stream=gu.stream())
+    torch.cuda.synchronize()
+    assert bool((h.abs() > 8.4e6).any()) == huge
+    want = two.cpu().numpy()
+    for w in ws:
+        w.destroy()
+    for g in got:
+        assert np.array_equal(g.view(np.uint32), want.view(np.uint32))
+
+
 @pytest.mark.parametrize("kind,m,k,n", [("q4_0", 1, 1024, 3072), ("q4_K", 1, 2048, 768), ("q6_K", 1, 1024, 512),
                                         ("q4_0", 1, 96, 320),      # K below one chunk unit: not fused
                                         ("q4_0", 24, 1024, 3072), ("q4_K", 5, 1024, 512),
