@@ -379,9 +379,11 @@ __device__ __forceinline__ void route_token_regs(const float *__restrict__ logit
  * apart through both roundings; with v_topk > -75 nothing underflows. A NaN or an infinite maximum among
  * the logits, and equal values on the two sides of the cut, take the full routine as well.
  * The topk-th largest v is the topk-th smallest magnitude |v| (as an integer: the bits of a float order
- * like its magnitude), found one bit at a time from counts over the wavefront: 31 steps of two compares
+ * like its magnitude), found one bit at a time from counts over the wavefront: at most 31 steps of two compares
  * and a few scalar instructions, where a round of selection per expert is two dependent reductions over
- * the wavefront each (2.6 us for eight experts of 128, against 0.7 us). */
+ * the wavefront each (2.6 us for eight experts of 128, against 0.7 us). The search ends at the first threshold with
+ * topk magnitudes below it, mostly after a dozen steps, and tests no expert count inside a step (a branch each: both
+ * together 0.9 us of the launch; two bits a step with three counts were slower). */
 template <int MAXV>
 __device__ __forceinline__ bool topk_set_fast(const float *__restrict__ lg, int E, int topk,
                                               unsigned long long (&mask)[MAXV]) {
@@ -412,20 +414,33 @@ __device__ __forceinline__ bool topk_set_fast(const float *__restrict__ lg, int 
     int n = 0;
 #pragma unroll
     for (int i = 0; i < MAXV; ++i)
-      if (64 * i < E) n += __popcll(__ballot(mag[i] <= t));
+      if (MAXV <= 4 || 64 * i < E) n += __popcll(__ballot(mag[i] <= t));
     return n;
   };
-  int cut = 0; /* the smallest t with topk magnitudes <= t */
-  for (int bit = 30; bit >= 0; --bit)
-    if (count_le(cut | ((1 << bit) - 1)) < topk) cut |= 1 << bit;
-  if (count_le(cut) != topk) return false; /* equal values across the cut: the tie rule decides (uniform) */
-  int beyond = 0x7fffffff;
+  int cut = 0; /* at the end the smallest t with topk magnitudes <= t, or, before, any t with exactly so many */
+  bool found = false;
 #pragma unroll
-  for (int i = 0; i < MAXV; ++i) beyond = min(beyond, mag[i] > cut ? mag[i] : 0x7fffffff);
+  for (int bit = 30; bit >= 0; --bit) {
+    const int t = cut | ((1 << bit) - 1), n = count_le(t);
+    if (n == topk) {
+      cut = t;
+      found = true;
+      break;
+    }
+    if (n < topk) cut |= 1 << bit;
+  }
+  if (!found && count_le(cut) != topk) return false; /* equal values across the cut: the tie rule decides (uniform) */
+  int last = 0, beyond = 0x7fffffff;
+#pragma unroll
+  for (int i = 0; i < MAXV; ++i) {
+    last = max(last, mag[i] > cut ? 0 : mag[i]);
+    beyond = min(beyond, mag[i] > cut ? mag[i] : 0x7fffffff);
+  }
+  last = -hipq_wave_min_i(-last); /* the topk-th magnitude */
   beyond = hipq_wave_min_i(beyond); /* the next magnitude, or 0x7fffffff when every expert is selected */
 #pragma unroll
   for (int i = 0; i < MAXV; ++i) mask[i] = 64 * i < E ? __ballot(mag[i] <= cut) : 0ull;
-  const float v_cut = __uint_as_float((uint32_t)cut);
+  const float v_cut = __uint_as_float((uint32_t)last);
   if (!(v_cut < 75.f)) return false;
   return beyond == 0x7fffffff || __uint_as_float((uint32_t)beyond) - v_cut > 1e-6f;
 }
@@ -1222,24 +1237,98 @@ __global__ __launch_bounds__(256, TC <= 8 ? 4 : TC <= 16 ? 2 : 1) void gate_up_m
   }
 }
 
-/* floats of LDS one of (gate, up) needs for the terms of the second half of K in the one-token kernel */
-__host__ __device__ constexpr int one_token_terms(int K) { return ((K >> 8) / 2 + 1) * 128; }
+/* ---- One token (a decode step) ------------------------------------------------------------
+ * With one row an expert tile's 32 columns are 32 row products, and v_dot8_u32_u4 on the nibbles as they are stored takes
+ * half the vector instructions of the matrix form (which unpacks them and waits for each of its eight dependent steps).
+ * The row is in LDS as 4-bit digits; a lane has half the weights of each sub-block of its column. The launches are chains
+ * of latencies (21 MB of weights at eight experts of 2048 x 768 are 3.4 us of the memory's rate), so everything here
+ * shortens the chain; us a launch of that block, with the matrix form / this one: gate and up 9.6 / 6.7, down with the sum
+ * over the experts 8.7 (two launches) / 5.2; the block of 128 experts 20.7 / 16.3. */
+struct OneRow {
+  uint8_t *ql, *qh; /* [K / 2] each: q = 16 (qh - 8) + ql, eight values a dword */
+  int16_t *bsum;    /* [K / 16] */
+  float *d;         /* [K / 256] */
+};
+__host__ __device__ constexpr int one_row_bytes(int K) { return (K + K / 8 + K / 64 + 15) & ~15; }
+__device__ __forceinline__ OneRow one_row_carve(unsigned char *base, int K) {
+  return OneRow{base, base + (K >> 1), (int16_t *)(base + K), (float *)(base + K + (K >> 3))};
+}
+/* a sum over the lanes that hold the two halves of a column: 32 lanes apart, or 16 */
+template <int APART> __device__ __forceinline__ int sum_halves(int v) {
+  if constexpr (APART == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
+    return (int)(r[0] + r[1]);
+  } else {
+    const auto r = __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);
+    return (int)(r[0] + r[1]);
+  }
+}
+/* One super-block's terms of the lane's column: the integer sum fi with its factor si = d * dA, the mins' sum fm with its
+ * factor sm = dmin * dA (the terms of xr_sb_terms). g: which half of every sub-block the lane has, APART lanes from the
+ * other. */
+template <int APART>
+__device__ __forceinline__ void one_sb_terms(const XRegs &W, const OneRow &l, int sb, int g, float &fi, float &si, float &fm,
+                                             float &sm) {
+  const uint8_t *pl = l.ql + sb * 128 + g * 8, *ph = l.qh + sb * 128 + g * 8;
+  uint2 lo[8], hi[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) lo[j] = *(const uint2 *)(pl + j * 16), hi[j] = *(const uint2 *)(ph + j * 16);
+  const int4 bs = *(const int4 *)(l.bsum + sb * 16 + g * 8); /* sub-blocks 4g .. 4g + 3, two sums each */
+  const float dA = l.d[sb];
+  const uint32_t hx = (uint32_t)W.hd[0], hy = (uint32_t)W.hd[1], hz = (uint32_t)W.hd[2], hw = (uint32_t)W.hd[3];
+  int I = 0;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const uint32_t x0 = (uint32_t)W.q[j >> 1][2 * (j & 1)], x1 = (uint32_t)W.q[j >> 1][2 * (j & 1) + 1];
+    /* sum w q = 16 sum w qh + sum w ql - 128 sum w */
+    uint32_t t = __builtin_amdgcn_udot8(x1, hi[j].y, __builtin_amdgcn_udot8(x0, hi[j].x, 0u, false), false) << 4;
+    t = __builtin_amdgcn_udot8(x1, lo[j].y, __builtin_amdgcn_udot8(x0, lo[j].x, t, false), false);
+    const uint32_t u = __builtin_amdgcn_udot8(x1, 0x11111111u, __builtin_amdgcn_udot8(x0, 0x11111111u, 0u, false), false);
+    I = __mul24((int)(((j < 4 ? hy : hz) >> (8 * (j & 3))) & 0x3fu), (int)t - (int)(u << 7)) + I;
+  }
+  /* the mins of the lane's four sub-blocks against their whole sums */
+  const uint32_t m = g ? ((hw >> 4) & 0x0f0f0f0fu) | ((hz >> 2) & 0x30303030u) : (hw & 0x0f0f0f0fu) | ((hy >> 2) & 0x30303030u);
+  const int bw[4] = {bs.x, bs.y, bs.z, bs.w};
+  int Im = 0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) Im = __mul24((int)((m >> (8 * j)) & 0xffu), (int)(int16_t)bw[j] + (bw[j] >> 16)) + Im;
+  fi = (float)sum_halves<APART>(I);
+  fm = (float)sum_halves<APART>(Im);
+  si = hipq_h2f((uint16_t)(hx & 0xffff)) * dA;
+  sm = hipq_h2f((uint16_t)(hx >> 16)) * dA;
+}
 
-/* One token (a decode step), the routing inside the gate/up launch: every wavefront finds the
+/* what the down product of one token reads of the routing: an entry an expert, in ascending id */
+struct OneExpert {
+  const uint8_t *down; /* the expert's tiles */
+  float w;
+  int e;
+};
+
+constexpr int ONE_PARTS = 4; /* of K, a wavefront each, for gate and up */
+/* floats of LDS one of (gate, up) needs for the terms of the parts behind the first */
+__host__ __device__ constexpr int one_token_terms(int K) { return (K >> 8) * 128; }
+
+/* The routing inside the gate/up launch: every wavefront finds the
  * token's set of experts itself (the same arithmetic on the same logits, so all agree; without the
  * softmax's exponentials where topk_set_fast can promise the same set), the workgroup takes the
  * expert whose rank in ascending id is its blockIdx.y, quantizes the row of x into its LDS while
- * its first weights are on their way, and goes on as the paired form of gate_up_mma_kernel.
+ * its first weights are on their way. One tile of 32 columns a workgroup, a wavefront for each of
+ * (gate, up) x (quarters of K): the launch is a chain of latencies, and few super-blocks a wavefront
+ * shorten it (halves of K and the matrix form: 9.6 us, see above). The chain of fp32 sums keeps the reference's order: the wavefronts behind the first quarter leave their
+ * super-blocks' terms in LDS, and the first quarter's adds them to its own after the barrier, one
+ * super-block after the other.
  * One workgroup more than the columns need routes the token in full and writes the routing's
  * outputs and the few table entries the down product and the combine read. One launch (7-8 us of
  * a block of 25) less than routing, sort and quantization as a launch of their own. */
 template <int MAXV>
-__global__ __launch_bounds__(256, 4) void gate_up_one_token_kernel(
+__global__ __launch_bounds__(64 * 2 * ONE_PARTS) void gate_up_one_token_kernel(
   const float *__restrict__ logits, int E, int topk, int renorm, int32_t *__restrict__ idx, float *__restrict__ wgt,
   int *__restrict__ offsets, int *__restrict__ slot_pair, int *__restrict__ tok_slots, int *__restrict__ items,
-  const float *__restrict__ x, const WView *__restrict__ views, int H, int I, float *__restrict__ h, hipq::MoeEpi ep) {
-  constexpr int TC = 8, NREG = TC / 2;
+  OneExpert *__restrict__ table, const float *__restrict__ x, const WView *__restrict__ views, int H, int I,
+  float *__restrict__ h, hipq::MoeEpi ep) {
   extern __shared__ __attribute__((aligned(16))) unsigned char xmoe_lds[];
+  constexpr int NW = 2 * ONE_PARTS;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   int myi;
   float myw;
@@ -1257,18 +1346,19 @@ __global__ __launch_bounds__(256, 4) void gate_up_one_token_kernel(
         offsets[myi + 1] = rank + 1; /* the end of the expert's slots: all the later kernels read of offsets */
         items[2 + 2 * rank] = myi;
         items[3 + 2 * rank] = rank;
+        table[rank] = OneExpert{views[2 * E + myi].qs, myw, myi};
       }
       if (lane == 0) items[0] = topk;
     }
     return; /* uniform per workgroup */
   }
   /* this wavefront's share of the row of x is asked for first: it has arrived when the routing is done */
-  constexpr int XPRE = 4; /* super-blocks a wavefront holds ahead: rows of up to 4096 values */
+  constexpr int XPRE = 2; /* super-blocks a wavefront holds ahead: rows of up to 4096 values */
   const int nsb_x = H >> 8;
   float4 xpre[XPRE];
 #pragma unroll
   for (int j = 0; j < XPRE; ++j)
-    if (wave + 4 * j < nsb_x) xpre[j] = *(const float4 *)(x + (wave + 4 * j) * 256 + lane * 4);
+    if (wave + NW * j < nsb_x) xpre[j] = *(const float4 *)(x + (wave + NW * j) * 256 + lane * 4);
   /* the other workgroups need the set of experts only, which mostly needs no exponential */
   const int item = blockIdx.y; /* < topk */
   unsigned long long set[MAXV];
@@ -1282,40 +1372,17 @@ __global__ __launch_bounds__(256, 4) void gate_up_one_token_kernel(
     e = __shfl(myi, __ffsll((long long)owner) - 1, 64);
   }
   e = __builtin_amdgcn_readfirstlane(e);
-  const WView wg = views[e], wu = views[E + e];
-  const int K = wg.K;
-  const XLds l = xlds_carve(xmoe_lds, TC, K);
-  /* One tile of 32 columns a workgroup, a wavefront for each of (gate, up) x (first, second half of K):
-   * with one wavefront per SIMD a super-block's eight matrix steps wait for each other, so half the
-   * super-blocks per wavefront halve the stream's time. The chain of fp32 sums keeps the reference's
-   * order: the second half's wavefront leaves its super-blocks' terms in LDS, and the first half's adds
-   * them to its own after the barrier, one super-block after the other. */
+  const int first = wave / ONE_PARTS, part = wave % ONE_PARTS; /* 0: gate, 1: up; which part of K */
+  const uint8_t *qs = views[first ? E + e : e].qs;
+  const int K = H;
+  const OneRow l = one_row_carve(xmoe_lds, K);
   const int col0 = blockIdx.x * 32; /* < I: the grid has as many columns (and the one that routes) */
-  const int first = wave >> 1, half = wave & 1; /* 0: gate, 1: up; which half of K */
   const int i32 = lane & 31, g = lane >> 5;
-  const int nsb = K >> 8, n0 = (nsb + 1) >> 1; /* the first half's super-blocks */
-  const int sb0 = half ? n0 : 0, cnt = half ? nsb - n0 : n0;
-  float *terms = (float *)(xmoe_lds + xlds_bytes(TC, K)); /* [gate, up][super-block of the second half][4 terms][32 columns] */
-  float *xch = terms + 2 * one_token_terms(K);            /* [32 columns] the gate values */
-  auto stage = [&]() {
-    /* rows 1 .. 7 of the matrix operand keep what the LDS held: a row of the product depends on
-     * its own activations only, and those rows are not stored */
-#pragma unroll
-    for (int j = 0; j < XPRE; ++j) {
-      const int b = wave + 4 * j;
-      if (b < nsb) /* uniform per wavefront */
-        hipq_quantize_q8_K_values<Q8K_ROWMMA>(xpre[j], 0, b, b, nsb, 0, l.q, l.dA, nullptr, nullptr,
-                                              (uint16_t *)l.amin, nullptr, nullptr, TC);
-    }
-    for (int b = wave + 4 * XPRE; b < nsb; b += 4) { /* longer rows: the rest as it comes */
-      const float4 xv = *(const float4 *)(x + b * 256 + lane * 4);
-      hipq_quantize_q8_K_values<Q8K_ROWMMA>(xv, 0, b, b, nsb, 0, l.q, l.dA, nullptr, nullptr, (uint16_t *)l.amin,
-                                            nullptr, nullptr, TC);
-    }
-    __syncthreads();
-  };
+  const int nsb = K >> 8, each = nsb / ONE_PARTS, more = nsb % ONE_PARTS; /* the first `more` parts have one more */
+  const int n0 = each + (more > 0), sb0 = part * each + min(part, more), cnt = each + (part < more);
+  float *terms = (float *)(xmoe_lds + one_row_bytes(K)); /* [gate, up][super-block behind the first part][4 terms][32 columns] */
+  float *xch = terms + 2 * one_token_terms(K);           /* [32 columns] the gate values */
   /* the tile (nibbles and headers of its super-blocks) as a buffer descriptor in scalar registers */
-  const uint8_t *qs = first ? wu.qs : wg.qs;
   const xrsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(
     (void *)(qs + (size_t)(col0 >> 5) * (size_t)(nsb * hipq::EXPERT_TILE_BYTES)), 0, nsb * hipq::EXPERT_TILE_BYTES,
     0x00020000);
@@ -1332,31 +1399,46 @@ __global__ __launch_bounds__(256, 4) void gate_up_one_token_kernel(
    * not count them, and every super-block's arithmetic waited for the loads just issued for the next. */
   XRegs buf[2];
   load(buf[0], cnt > 0 ? sb0 : nsb);
-  stage(); /* the row of x is quantized while the first weights are on their way */
+  load(buf[1], cnt > 1 ? sb0 + 1 : nsb);
+  /* the row of x is quantized while the first weights are on their way */
+#pragma unroll
+  for (int j = 0; j < XPRE; ++j) {
+    const int b = wave + NW * j;
+    if (b < nsb) /* uniform per wavefront */
+      hipq_quantize_q8_K_values<Q8K_DIGITS>(xpre[j], 0, b, b, nsb, 0, nullptr, l.d, l.bsum, nullptr, nullptr, (uint16_t *)l.ql,
+                                            (uint16_t *)l.qh);
+  }
+  for (int b = wave + NW * XPRE; b < nsb; b += NW) { /* longer rows: the rest as it comes */
+    const float4 xv = *(const float4 *)(x + b * 256 + lane * 4);
+    hipq_quantize_q8_K_values<Q8K_DIGITS>(xv, 0, b, b, nsb, 0, nullptr, l.d, l.bsum, nullptr, nullptr, (uint16_t *)l.ql,
+                                          (uint16_t *)l.qh);
+  }
+  __syncthreads();
   float acc = 0.f, accm = 0.f;
   for (int u0 = 0; u0 < cnt; u0 += 2) {
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       const int u = u0 + k;
       if (u < cnt) { /* uniform per wavefront */
-        load(buf[(k + 1) & 1], u + 1 < cnt ? sb0 + u + 1 : nsb);
-        float fi[NREG], si[NREG], fm[NREG], sm[NREG];
-        xr_sb_terms<TC, NREG>(buf[k], l, K, sb0 + u, i32, g, fi, si, fm, sm);
-        if (half == 0) {
-          acc = fmaf(fi[0], si[0], acc);
-          accm = fmaf(fm[0], sm[0], accm);
+        float fi, si, fm, sm;
+        one_sb_terms<32>(buf[k], l, sb0 + u, g, fi, si, fm, sm);
+        load(buf[k], u + 2 < cnt ? sb0 + u + 2 : nsb);
+        if (part == 0) {
+          acc = fmaf(fi, si, acc);
+          accm = fmaf(fm, sm, accm);
         } else if (lane < 32) {
-          float *t = terms + (size_t)((first * one_token_terms(K) / 128 + u) * 4) * 32 + lane;
-          t[0] = fi[0], t[32] = si[0], t[64] = fm[0], t[96] = sm[0];
+          float *t = terms + first * one_token_terms(K) + (sb0 + u - n0) * 128 + lane;
+          t[0] = fi, t[32] = si, t[64] = fm, t[96] = sm;
         }
       }
     }
   }
   __syncthreads();
   float out = 0.f;
-  if (half == 0) {
-    for (int u = 0; u < nsb - n0; ++u) {
-      const float *t = terms + (size_t)((first * one_token_terms(K) / 128 + u) * 4) * 32 + i32;
+  if (part == 0) {
+    const float *t = terms + first * one_token_terms(K) + i32;
+#pragma unroll 4
+    for (int u = 0; u < nsb - n0; ++u, t += 128) {
       acc = fmaf(t[0], t[32], acc);
       accm = fmaf(t[64], t[96], accm);
     }
@@ -1364,9 +1446,87 @@ __global__ __launch_bounds__(256, 4) void gate_up_one_token_kernel(
     if (first == 0 && lane < 32) xch[lane] = out;
   }
   __syncthreads();
-  if (first == 1 && half == 0 && lane < 32) {
+  if (first == 1 && part == 0 && lane < 32) {
     const int col = col0 + lane;
     if (col < I) h[(size_t)item * I + col] = moe_act(ep, e, I, col, xch[lane], out);
+  }
+}
+
+/* The down product of one token and the sum over its experts: a workgroup owns sixteen columns, its wavefronts an expert
+ * each, which quantize the expert's row of h themselves. Sixteen columns of a tile leave room for two super-blocks side by
+ * side in a wavefront (lanes 0 - 31 the even ones), and twice the CUs of a whole tile. The experts' results meet in LDS and
+ * are added in ascending id, where the combine's launch had read them from memory. */
+__global__ __launch_bounds__(1024) void down_one_token_kernel(const OneExpert *__restrict__ table, int topk,
+                                                              const float *__restrict__ h, int H, int I,
+                                                              float *__restrict__ y, hipq::MoeEpi ep) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char xmoe_lds[];
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  const int n16 = lane & 15, g = (lane >> 4) & 1, p = lane >> 5;
+  const int K = I, nsb = K >> 8, col = blockIdx.x * 16 + n16; /* H % 256 == 0 */
+  const OneExpert ex = table[wave];
+  const OneRow l = one_row_carve(xmoe_lds + wave * one_row_bytes(K), K);
+  float *outs = (float *)(xmoe_lds + topk * one_row_bytes(K)); /* [topk][16] */
+  /* the expert's row, four super-blocks a pass, sixteen values a lane */
+  const float *row = h + (size_t)wave * K;
+  float4 xs[4];
+  int at = min(lane, K / 16 - 1);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) xs[i] = *(const float4 *)(row + at * 16 + 4 * i);
+  const xrsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(
+    (void *)(ex.down + (size_t)(blockIdx.x >> 1) * (size_t)(nsb * hipq::EXPERT_TILE_BYTES)), 0, nsb * hipq::EXPERT_TILE_BYTES,
+    0x00020000);
+  const int n32 = (blockIdx.x & 1) * 16 + n16; /* the column's place in its tile */
+  auto load = [&](XRegs &r, int u) { /* past the end: zeros, without touching memory */
+    const int sb = 2 * u + p;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      r.q[i] = __builtin_bit_cast(
+        mv4i, __builtin_amdgcn_raw_buffer_load_b128(rq, sb * hipq::EXPERT_TILE_BYTES + (g * 32 + n32) * 16, i * 1024, 2));
+    r.hd = __builtin_bit_cast(
+      mv4i, __builtin_amdgcn_raw_buffer_load_b128(rq, sb * hipq::EXPERT_TILE_BYTES + n32 * 16, 4096, 2));
+  };
+  XRegs buf[2];
+  load(buf[0], 0);
+  load(buf[1], 1);
+  for (int b0 = 0;;) {
+    hipq_quantize_q8_K_values16<Q8K_DIGITS>(xs, at, b0 + lane < K / 16, nullptr, l.d, l.bsum, l.ql, l.qh);
+    if ((b0 += 64) >= K / 16) break; /* uniform */
+    at = min(b0 + lane, K / 16 - 1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) xs[i] = *(const float4 *)(row + at * 16 + 4 * i);
+  }
+  hipq_wave_lds_sync(); /* the row is this wavefront's own */
+  float acc = 0.f, accm = 0.f;
+  const int steps = (nsb + 1) >> 1;
+  for (int u0 = 0; u0 < steps; u0 += 2) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int u = u0 + k;
+      if (u < steps) { /* uniform */
+        float fi, si, fm, sm;
+        one_sb_terms<16>(buf[k], l, min(2 * u + p, nsb - 1), g, fi, si, fm, sm);
+        load(buf[k], u + 2);
+        /* the odd super-block's terms to the lanes of the even one */
+        auto other = [](float v) {
+          const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+          return __uint_as_float(r[1]);
+        };
+        const float fi1 = other(fi), si1 = other(si), fm1 = other(fm), sm1 = other(sm);
+        acc = fmaf(fi, si, acc); /* lanes 0 - 31 */
+        accm = fmaf(fm, sm, accm);
+        if (2 * u + 1 < nsb) {
+          acc = fmaf(fi1, si1, acc);
+          accm = fmaf(fm1, sm1, accm);
+        }
+      }
+    }
+  }
+  if (lane < 16) outs[wave * 16 + lane] = moe_out(ep, ex.e, H, col, acc - accm, ex.w);
+  __syncthreads();
+  if (threadIdx.x < 16) {
+    float sum = 0.f;
+    for (int k = 0; k < topk; ++k) sum = sum + outs[k * 16 + threadIdx.x];
+    y[col] = sum;
   }
 }
 
@@ -1970,7 +2130,7 @@ int launch_grouped_mma(const hipq::MoeArgs *a, const MoeBufs &b, const WView *vi
   if (lds_g > 64 * 1024) /* beyond the default limit of a launch */
     HIPQ_HIP(hipFuncSetAttribute(kg, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_g));
   if (gate_up_done) {
-    /* h is there: the routing launch formed it (gate_up_one_token_kernel) */
+    /* h is there: the routing's launch formed it (gate_up_one_token_kernel) */
   } else if (few)
     hipq::launch_kernel("gate_up_mma_kernel<TC, true>", (gate_up_mma_kernel<TC, true>), dim3((d.intermediate + 63) / 64, max_items), dim3(256), lds_g,
                        s, views, d.experts, qview(xq), b.offsets, b.items, b.slot_pair, d.topk, d.intermediate,
@@ -2136,23 +2296,34 @@ int launch_moe(const MoeArgs *a, void *workspace, size_t workspace_bytes, const 
   /* one token on the matrix-core path: routing, the quantization of x and gate/up as one launch */
   const bool one_token = mma && T == 1 && chunk == 8 && mma_few(d, 8) && E <= 1024 && d.topk <= 64;
   if (one_token) {
-    const size_t lds_g = xlds_bytes(8, d.hidden) + (2 * (size_t)one_token_terms(d.hidden) + 32) * sizeof(float);
+    const size_t lds_g = one_row_bytes(d.hidden) + (2 * (size_t)one_token_terms(d.hidden) + 32) * sizeof(float);
     if (lds_g > 64 * 1024) {
       const void *k = E <= 128   ? (const void *)gate_up_one_token_kernel<2>
                       : E <= 256 ? (const void *)gate_up_one_token_kernel<4>
                                  : (const void *)gate_up_one_token_kernel<16>;
       HIPQ_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_g));
     }
+    OneExpert *table = (OneExpert *)b.hq_mem; /* no kernel of this path keeps quantized rows of h in memory */
     /* one block column more than the columns of h need: the routing's outputs are written there */
     const dim3 grid((unsigned)((d.intermediate + 31) / 32) + 1, (unsigned)d.topk);
     auto launch = [&](auto k, const char *name) {
-      hipq::launch_kernel(name, k, grid, dim3(256), lds_g, s, logits, E, d.topk, d.renormalize, idx, wgt, b.offsets,
-                          b.slot_pair, b.tok_slots, b.items, a->x, views, d.hidden, d.intermediate, b.h, a->epi);
+      hipq::launch_kernel(name, k, grid, dim3(64 * 2 * ONE_PARTS), lds_g, s, logits, E, d.topk, d.renormalize, idx, wgt, b.offsets,
+                          b.slot_pair, b.tok_slots, b.items, table, a->x, views, d.hidden, d.intermediate, b.h, a->epi);
     };
     if (E <= 128) launch(gate_up_one_token_kernel<2>, "gate_up_one_token_kernel<2>");
     else if (E <= 256) launch(gate_up_one_token_kernel<4>, "gate_up_one_token_kernel<4>");
     else launch(gate_up_one_token_kernel<16>, "gate_up_one_token_kernel<16>");
     HIPQ_HIP(hipGetLastError());
+    const size_t lds_d = (size_t)d.topk * (one_row_bytes(d.intermediate) + 16 * sizeof(float));
+    /* a workgroup's wavefronts are the token's experts; more of them, or longer rows of h than a launch's plain LDS
+     * limit holds, go on to the grouped product below */
+    if (d.topk <= 16 && lds_d <= 64 * 1024) {
+      hipq::launch_kernel("down_one_token_kernel", down_one_token_kernel, dim3((unsigned)(d.hidden / 16)),
+                          dim3(64u * d.topk), lds_d, s, (const OneExpert *)table, d.topk, (const float *)b.h, d.hidden,
+                          d.intermediate, a->y, a->epi);
+      HIPQ_HIP(hipGetLastError());
+      return HIPQ_OK;
+    }
   } else if (T <= 16 && E <= 1024) {
     const unsigned qblocks = mma ? (unsigned)((xqa.n_sb + 15) / 16) : 0;
     auto launch = [&](auto fused, auto plain) {

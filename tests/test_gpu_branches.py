@@ -52,6 +52,44 @@ def test_moe_without_renormalization(hipq, cr, t, h, i, e, k):
     _run_moe(cr, "q4_K", t, h, i, e, k, False, seed=7000)
 
 
+# one token: rows of one super-block and of odd counts, one expert, sixteen (the most whose down products share a
+# workgroup), more, and rows of h too long to share one's LDS
+@pytest.mark.parametrize("h,i,e,k", [(256, 256, 8, 1), (1280, 768, 16, 16), (768, 1280, 24, 17), (2304, 512, 300, 5),
+                                     (256, 9216, 8, 8), (4352, 256, 6, 2)])
+def test_moe_of_one_token(hipq, cr, h, i, e, k):
+    _run_moe(cr, "q4_K", 1, h, i, e, k, True, seed=7200)
+
+
+@pytest.mark.parametrize("e,k", [(8, 2), (64, 8), (100, 8), (200, 6), (520, 16)])
+def test_moe_of_one_token_selects_as_the_full_routing(hipq, cr, e, k):
+    """The one-token kernel finds its experts by a search over the logits' magnitudes; two tokens with the same logits
+    take the full routing. Ties across the cut, all logits equal, logits a few spacings apart, an infinity, far apart."""
+    import gpu_util as gu
+    import torch
+    h = i = 256
+    gate, up, down = _experts(cr, "q4_K", 4, i, h, 7300)
+    pick = lambda blobs, n, kk: [capi.Weight("q4_K", n, kk, blobs[x % 4]) for x in range(e)]
+    wg, wu, wd = pick(gate, i, h), pick(up, i, h), pick(down, h, i)
+    x = synth.normal(7301, (1, h))
+    base = synth.normal(7302, (1, e))
+    rows = [base, np.round(base), np.zeros_like(base), 1 + base * 2e-7, base * 60, base.copy(), -np.abs(base) * 1e-20]
+    rows[5][0, e // 2] = -np.inf
+    dx1, dx2 = gu.dev(x), gu.dev(np.repeat(x, 2, 0))
+    for lg in rows:
+        lg = lg.astype(np.float32)
+        out = []
+        for t, dx, l in ((1, dx1, lg), (2, dx2, np.repeat(lg, 2, 0))):
+            y = torch.full((t, h), float("nan"), device="cuda")
+            idx = torch.zeros((t, k), dtype=torch.int32, device="cuda")
+            capi.moe_forward(t, h, i, e, k, wg, wu, wd, dx, y, router_logits=gu.dev(l), topk_idx=idx, stream=gu.stream())
+            torch.cuda.synchronize()
+            out.append((y[0], idx[0]))
+        assert torch.equal(out[0][1], out[1][1])
+        assert torch.equal(out[0][0], out[1][0]) and not bool(torch.isnan(out[0][0]).any())
+    for w in wg + wu + wd:
+        w.destroy()
+
+
 @pytest.mark.parametrize("kind", ["q4_0", "q6_K"])
 @pytest.mark.parametrize("t,h,i,e,k,renorm", [(6, 256, 256, 8, 2, True), (33, 512, 256, 8, 4, True),
                                               (1, 1024, 512, 4, 2, True), (12, 256, 512, 8, 3, False)])
