@@ -39,6 +39,7 @@
 
 namespace {
 
+constexpr int ROUTER_PARTS = 16; /* partial sums of a router logit */
 constexpr int RTOK = 4; /* tokens sharing one pass over an expert's weight rows */
 
 struct MoeBufs {
@@ -66,7 +67,7 @@ size_t carve(const hipq_moe_desc &d, int is_k, uint8_t *base, MoeBufs *b) {
     return base ? base + at : (uint8_t *)nullptr;
   };
   uint8_t *p;
-  p = take(T * E * 4);
+  p = take((T == 1 ? ROUTER_PARTS : T) * E * 4); /* one token: the logits' partial sums */
   if (b) b->logits = (float *)p;
   p = take(P * 4);
   if (b) b->idx = (int32_t *)p;
@@ -222,6 +223,53 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const float *__restr
       logits[(size_t)(t0 + tb) * E + e] = bias ? sum + bias[e] : sum;
     }
   }
+}
+
+/* One token whose block goes on in gate_up_one_token_kernel: partial sums only, which that kernel adds (in the order
+ * above, so a logit has the same bits). A workgroup is one of the wavefronts of the kernel above and reads a quarter of
+ * its rows, so four times as many CUs share the matrix, and nothing passes through LDS: the E / 16 CUs of the
+ * form above were bound by what one of them pulls out of the cache (2048 x 128: 4.6 / 3.2 us, of which 1.5 are any launch's). Rows past the last are
+ * loads beyond the descriptor's end, which touch no memory. */
+__global__ __launch_bounds__(64) void router_parts_kernel(const float *__restrict__ x, const float *__restrict__ wr, int H, int E,
+                                                          float *__restrict__ parts) {
+  constexpr int JU = 8; /* groups of four rows a lane has in flight, as above */
+  const int lane = threadIdx.x, r = lane >> 2, q = lane & 3;
+  const int e4 = blockIdx.x * 4 + q, c = min(e4, (E >> 2) - 1); /* columns past the end repeat the last; not stored */
+  const int off = 64 * blockIdx.y + 4 * r;
+  const auto rw = __builtin_amdgcn_make_buffer_rsrc((void *)wr, 0, H * E * 4, 0x00020000);
+  const auto rx = __builtin_amdgcn_make_buffer_rsrc((void *)x, 0, H * 4, 0x00020000);
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int h0 = 0; h0 < H; h0 += 256 * JU) {
+    float4 w[JU][4], xv[JU];
+#pragma unroll
+    for (int j = 0; j < JU; ++j) {
+      const int h = h0 + 256 * j + off; /* H % 4 == 0: the four rows are in or out together */
+      xv[j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rx, h * 4, 0, 0));
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        w[j][i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rw, ((h + i) * E + 4 * c) * 4, 0, 0));
+    }
+#pragma unroll
+    for (int j = 0; j < JU; ++j) {
+      const float xs[4] = {xv[j].x, xv[j].y, xv[j].z, xv[j].w};
+      if (h0 + 256 * j + off < H) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          acc[0] = fmaf(xs[i], w[j][i].x, acc[0]);
+          acc[1] = fmaf(xs[i], w[j][i].y, acc[1]);
+          acc[2] = fmaf(xs[i], w[j][i].z, acc[2]);
+          acc[3] = fmaf(xs[i], w[j][i].w, acc[3]);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    acc[j] += hipq_dpp_f<0x114>(acc[j]); /* row_shr:4 */
+    acc[j] += hipq_dpp_f<0x118>(acc[j]); /* row_shr:8 */
+  }
+  if ((lane & 12) == 12 && e4 < (E >> 2))
+    *(float4 *)(parts + (size_t)(blockIdx.y * 4 + (lane >> 4)) * E + 4 * e4) = make_float4(acc[0], acc[1], acc[2], acc[3]);
 }
 
 /* Many tokens: the same sums on the matrix core. The kernel above reads all of Wr for every four tokens (1000 tokens of
@@ -1243,7 +1291,8 @@ __global__ __launch_bounds__(256, TC <= 8 ? 4 : TC <= 16 ? 2 : 1) void gate_up_m
  * The row is in LDS as 4-bit digits; a lane has half the weights of each sub-block of its column. The launches are chains
  * of latencies (21 MB of weights at eight experts of 2048 x 768 are 3.4 us of the memory's rate), so everything here
  * shortens the chain; us a launch of that block, with the matrix form / this one: gate and up 9.6 / 6.7, down with the sum
- * over the experts 8.7 (two launches) / 5.2; the block of 128 experts 20.7 / 16.3. */
+ * over the experts 8.7 (two launches) / 5.2; the block of 128 experts 20.7 / 16.3,
+ * with the router's sums finished here 15.4. */
 struct OneRow {
   uint8_t *ql, *qh; /* [K / 2] each: q = 16 (qh - 8) + ql, eight values a dword */
   int16_t *bsum;    /* [K / 16] */
@@ -1321,9 +1370,9 @@ __host__ __device__ constexpr int one_token_terms(int K) { return (K >> 8) * 128
  * One workgroup more than the columns need routes the token in full and writes the routing's
  * outputs and the few table entries the down product and the combine read. One launch (7-8 us of
  * a block of 25) less than routing, sort and quantization as a launch of their own. */
-template <int MAXV>
+template <int MAXV, bool PARTS> /* PARTS: the logits come as the partial sums of router_parts_kernel */
 __global__ __launch_bounds__(64 * 2 * ONE_PARTS) void gate_up_one_token_kernel(
-  const float *__restrict__ logits, int E, int topk, int renorm, int32_t *__restrict__ idx, float *__restrict__ wgt,
+  const float *__restrict__ lg_in, const float *__restrict__ router_bias, int E, int topk, int renorm, int32_t *__restrict__ idx, float *__restrict__ wgt,
   int *__restrict__ offsets, int *__restrict__ slot_pair, int *__restrict__ tok_slots, int *__restrict__ items,
   OneExpert *__restrict__ table, const float *__restrict__ x, const WView *__restrict__ views, int H, int I,
   float *__restrict__ h, hipq::MoeEpi ep) {
@@ -1332,6 +1381,31 @@ __global__ __launch_bounds__(64 * 2 * ONE_PARTS) void gate_up_one_token_kernel(
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   int myi;
   float myw;
+  /* this wavefront's share of the row of x is asked for first: it has arrived when the routing is done */
+  constexpr int XPRE = 2; /* super-blocks a wavefront holds ahead: rows of up to 4096 values */
+  const int nsb_x = H >> 8;
+  float4 xpre[XPRE];
+#pragma unroll
+  for (int j = 0; j < XPRE; ++j)
+    if (wave + NW * j < nsb_x) xpre[j] = *(const float4 *)(x + (wave + NW * j) * 256 + lane * 4);
+  float *terms = (float *)(xmoe_lds + one_row_bytes(H)); /* [gate, up][super-block behind the first part][4 terms][32 columns] */
+  float *xch = terms + 2 * one_token_terms(H);           /* [32 columns] the gate values */
+  const float *logits = lg_in;
+  if (PARTS) {
+    float *sums = xch + 32;
+    for (int e = threadIdx.x; e < E; e += 64 * NW) {
+      float v[ROUTER_PARTS];
+#pragma unroll
+      for (int i = 0; i < ROUTER_PARTS; ++i) v[i] = lg_in[i * E + e];
+      const float bias = router_bias ? router_bias[e] : 0.f;
+      float sum = v[0];
+#pragma unroll
+      for (int i = 1; i < ROUTER_PARTS; ++i) sum += v[i];
+      sums[e] = router_bias ? sum + bias : sum;
+    }
+    __syncthreads();
+    logits = sums;
+  }
   if (blockIdx.x == gridDim.x - 1) {
     /* the extra column of the grid: its first workgroup's first wavefront routes the token in full and
      * writes what the launches behind this one read; it multiplies nothing */
@@ -1352,13 +1426,6 @@ __global__ __launch_bounds__(64 * 2 * ONE_PARTS) void gate_up_one_token_kernel(
     }
     return; /* uniform per workgroup */
   }
-  /* this wavefront's share of the row of x is asked for first: it has arrived when the routing is done */
-  constexpr int XPRE = 2; /* super-blocks a wavefront holds ahead: rows of up to 4096 values */
-  const int nsb_x = H >> 8;
-  float4 xpre[XPRE];
-#pragma unroll
-  for (int j = 0; j < XPRE; ++j)
-    if (wave + NW * j < nsb_x) xpre[j] = *(const float4 *)(x + (wave + NW * j) * 256 + lane * 4);
   /* the other workgroups need the set of experts only, which mostly needs no exponential */
   const int item = blockIdx.y; /* < topk */
   unsigned long long set[MAXV];
@@ -1380,8 +1447,6 @@ __global__ __launch_bounds__(64 * 2 * ONE_PARTS) void gate_up_one_token_kernel(
   const int i32 = lane & 31, g = lane >> 5;
   const int nsb = K >> 8, each = nsb / ONE_PARTS, more = nsb % ONE_PARTS; /* the first `more` parts have one more */
   const int n0 = each + (more > 0), sb0 = part * each + min(part, more), cnt = each + (part < more);
-  float *terms = (float *)(xmoe_lds + one_row_bytes(K)); /* [gate, up][super-block behind the first part][4 terms][32 columns] */
-  float *xch = terms + 2 * one_token_terms(K);           /* [32 columns] the gate values */
   /* the tile (nibbles and headers of its super-blocks) as a buffer descriptor in scalar registers */
   const xrsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(
     (void *)(qs + (size_t)(col0 >> 5) * (size_t)(nsb * hipq::EXPERT_TILE_BYTES)), 0, nsb * hipq::EXPERT_TILE_BYTES,
@@ -2246,7 +2311,12 @@ int launch_moe(const MoeArgs *a, void *workspace, size_t workspace_bytes, const 
   if (need > workspace_bytes) return fail(HIPQ_ERR_RUNTIME, "MoE workspace too small");
   const int T = d.tokens, E = d.experts, P = T * d.topk;
 
+  const bool mma = use_mma(d, dt);
+  const int chunk = mma ? mma_chunk(d, P, E) : 0; /* tokens of an expert per work item of the matrix-core kernels */
+  /* one token on the matrix-core path: routing, the quantization of x and gate/up as one launch */
+  const bool one_token = mma && T == 1 && chunk == 8 && mma_few(d, 8) && E <= 1024 && d.topk <= 64;
   const float *logits = a->router_logits;
+  bool parts = false; /* the logits are partial sums */
   if (!logits) {
     /* the rows of x of a workgroup's tokens go to LDS: four tokens, or as many as there are or fit 64 KB with the partial sums */
     int tb_n = d.hidden > 0 ? (int)std::min<int64_t>(std::min(ROUTER_TB, T), 15000 / d.hidden) : 0;
@@ -2260,6 +2330,11 @@ int launch_moe(const MoeArgs *a, void *workspace, size_t workspace_bytes, const 
       hipq::launch_kernel("router_logits_many_kernel", router_logits_many_kernel,
                           dim3((E + ROUTER_MANY_E - 1) / ROUTER_MANY_E, (T + ROUTER_MANY_T - 1) / ROUTER_MANY_T), dim3(1024), lds, s,
                           a->x, a->router_weight, T, d.hidden, E, a->router_bias, b.logits);
+    } else if (one_token && !(E & 3) && (((uintptr_t)a->router_weight | (uintptr_t)a->x) & 15) == 0 &&
+               (int64_t)d.hidden * E < (1 << 28)) { /* a buffer descriptor's offsets */
+      parts = true;
+      hipq::launch_kernel("router_parts_kernel", router_parts_kernel, dim3((E / 4 + 3) / 4, ROUTER_PARTS / 4), dim3(64), 0, s, a->x,
+                          a->router_weight, d.hidden, E, b.logits);
     } else if ((E & 3) || (d.hidden & 3) || tb_n < 1 || (((uintptr_t)a->router_weight | (uintptr_t)a->x) & 15)) {
       hipq::launch_kernel("router_logits_scalar_kernel", router_logits_scalar_kernel, dim3(T), dim3(256), 0, s, a->x,
                           a->router_weight, d.hidden, E, a->router_bias, b.logits);
@@ -2277,8 +2352,6 @@ int launch_moe(const MoeArgs *a, void *workspace, size_t workspace_bytes, const 
     HIPQ_HIP(hipGetLastError());
     logits = b.logits;
   }
-  const bool mma = use_mma(d, dt);
-  const int chunk = mma ? mma_chunk(d, P, E) : 0; /* tokens of an expert per work item of the matrix-core kernels */
   int32_t *idx = a->topk_idx ? a->topk_idx : b.idx;
   float *wgt = a->topk_w ? a->topk_w : b.wgt;
   b.wgt = wgt;
@@ -2293,26 +2366,25 @@ int launch_moe(const MoeArgs *a, void *workspace, size_t workspace_bytes, const 
   const XQuant xqa = {a->x, (int64_t)T * (d.hidden / 256), d.hidden / 256, xq.q, xq.d, (uint16_t *)xq.bsum};
   if (mma && (((uintptr_t)a->x & 15) != 0))
     return fail(HIPQ_ERR_INVALID_ARGUMENT, "activation rows must be 16-byte aligned");
-  /* one token on the matrix-core path: routing, the quantization of x and gate/up as one launch */
-  const bool one_token = mma && T == 1 && chunk == 8 && mma_few(d, 8) && E <= 1024 && d.topk <= 64;
   if (one_token) {
-    const size_t lds_g = one_row_bytes(d.hidden) + (2 * (size_t)one_token_terms(d.hidden) + 32) * sizeof(float);
-    if (lds_g > 64 * 1024) {
-      const void *k = E <= 128   ? (const void *)gate_up_one_token_kernel<2>
-                      : E <= 256 ? (const void *)gate_up_one_token_kernel<4>
-                                 : (const void *)gate_up_one_token_kernel<16>;
-      HIPQ_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_g));
-    }
+    const size_t lds_g = one_row_bytes(d.hidden) + (2 * (size_t)one_token_terms(d.hidden) + 32 + (parts ? E : 0)) * sizeof(float);
     OneExpert *table = (OneExpert *)b.hq_mem; /* no kernel of this path keeps quantized rows of h in memory */
     /* one block column more than the columns of h need: the routing's outputs are written there */
     const dim3 grid((unsigned)((d.intermediate + 31) / 32) + 1, (unsigned)d.topk);
-    auto launch = [&](auto k, const char *name) {
-      hipq::launch_kernel(name, k, grid, dim3(64 * 2 * ONE_PARTS), lds_g, s, logits, E, d.topk, d.renormalize, idx, wgt, b.offsets,
-                          b.slot_pair, b.tok_slots, b.items, table, a->x, views, d.hidden, d.intermediate, b.h, a->epi);
+    auto launch = [&](auto k, const char *name) -> int {
+      if (lds_g > 64 * 1024) HIPQ_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_g));
+      hipq::launch_kernel(name, k, grid, dim3(64 * 2 * ONE_PARTS), lds_g, s, logits, a->router_bias, E, d.topk, d.renormalize,
+                          idx, wgt, b.offsets, b.slot_pair, b.tok_slots, b.items, table, a->x, views, d.hidden, d.intermediate,
+                          b.h, a->epi);
+      return HIPQ_OK;
     };
-    if (E <= 128) launch(gate_up_one_token_kernel<2>, "gate_up_one_token_kernel<2>");
-    else if (E <= 256) launch(gate_up_one_token_kernel<4>, "gate_up_one_token_kernel<4>");
-    else launch(gate_up_one_token_kernel<16>, "gate_up_one_token_kernel<16>");
+    auto by_experts = [&](auto p) -> int {
+      constexpr bool P = decltype(p)::value;
+      return E <= 128   ? launch(gate_up_one_token_kernel<2, P>, "gate_up_one_token_kernel<2>")
+             : E <= 256 ? launch(gate_up_one_token_kernel<4, P>, "gate_up_one_token_kernel<4>")
+                        : launch(gate_up_one_token_kernel<16, P>, "gate_up_one_token_kernel<16>");
+    };
+    if (const int rc = parts ? by_experts(std::true_type{}) : by_experts(std::false_type{})) return rc;
     HIPQ_HIP(hipGetLastError());
     const size_t lds_d = (size_t)d.topk * (one_row_bytes(d.intermediate) + 16 * sizeof(float));
     /* a workgroup's wavefronts are the token's experts; more of them, or longer rows of h than a launch's plain LDS

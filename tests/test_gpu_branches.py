@@ -90,6 +90,40 @@ def test_moe_of_one_token_selects_as_the_full_routing(hipq, cr, e, k):
         w.destroy()
 
 
+@pytest.mark.parametrize("h,e,k", [(256, 8, 2), (768, 100, 4), (2304, 132, 8), (4352, 20, 3), (256, 1024, 8), (512, 6, 2)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_moe_of_one_token_routes_from_the_partial_sums(hipq, cr, h, e, k, bias):
+    """The logits of one token come as partial sums that the gate/up kernel adds; two tokens take the kernel that adds
+    them itself. Each logit has the same bits, so the experts, their weights and the block's result do."""
+    import gpu_util as gu
+    import torch
+    i = 256
+    gate, up, down = _experts(cr, "q4_K", 2, i, h, 7400)
+    pick = lambda blobs, n, kk: [capi.Weight("q4_K", n, kk, blobs[x % 2]) for x in range(e)]
+    wg, wu, wd = pick(gate, i, h), pick(up, i, h), pick(down, h, i)
+    x, wr = synth.normal(7401, (1, h)), gu.dev(synth.normal(7402, (h, e), 0.1))
+    zero, rb = torch.zeros(e, max(h, i), device="cuda"), gu.dev(synth.normal(7403, (e,), 2.0))
+    out = []
+    for t in (1, 2):
+        dx = gu.dev(np.repeat(x, t, 0))
+        y = torch.full((t, h), float("nan"), device="cuda")
+        idx = torch.zeros((t, k), dtype=torch.int32, device="cuda")
+        wt = torch.zeros((t, k), device="cuda")
+        opt = dict(router_weight=wr, topk_idx=idx, topk_w=wt, stream=gu.stream())
+        if bias:
+            gb, db = zero[:, :i].contiguous(), zero[:, :h].contiguous()
+            capi.moe_forward_gpt_oss(t, h, i, e, k, wg, wu, wd, dx, y, gb, gb, db, router_bias=rb, **opt)
+        else:
+            capi.moe_forward(t, h, i, e, k, wg, wu, wd, dx, y, **opt)
+        torch.cuda.synchronize()
+        out.append((y[0], idx[0], wt[0]))
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+    assert not bool(torch.isnan(out[0][0]).any())
+    for w in wg + wu + wd:
+        w.destroy()
+
+
 @pytest.mark.parametrize("kind", ["q4_0", "q6_K"])
 @pytest.mark.parametrize("t,h,i,e,k,renorm", [(6, 256, 256, 8, 2, True), (33, 512, 256, 8, 4, True),
                                               (1, 1024, 512, 4, 2, True), (12, 256, 512, 8, 3, False)])
