@@ -32,6 +32,7 @@
  * over many experts take a form without the sort (gate_up_self_kernel below): four
  * launches, one workgroup row per expert.
  */
+#include <cmath>
 #include "gemv_device.h"
 #include "moe_tile_device.h"
 #include "quantize_device.h"
@@ -40,6 +41,7 @@
 namespace {
 
 constexpr int ROUTER_PARTS = 16; /* partial sums of a router logit */
+constexpr int MOE_FEW = 64; /* tokens, at most, whose pairs may be products of their own */
 constexpr int RTOK = 4; /* tokens sharing one pass over an expert's weight rows */
 
 struct MoeBufs {
@@ -67,7 +69,7 @@ size_t carve(const hipq_moe_desc &d, int is_k, uint8_t *base, MoeBufs *b) {
     return base ? base + at : (uint8_t *)nullptr;
   };
   uint8_t *p;
-  p = take((T == 1 ? ROUTER_PARTS : T) * E * 4); /* one token: the logits' partial sums */
+  p = take(T * (T <= MOE_FEW ? ROUTER_PARTS : 1) * E * 4); /* few tokens: the logits' partial sums */
   if (b) b->logits = (float *)p;
   p = take(P * 4);
   if (b) b->idx = (int32_t *)p;
@@ -236,6 +238,8 @@ __global__ __launch_bounds__(64) void router_parts_kernel(const float *__restric
   const int lane = threadIdx.x, r = lane >> 2, q = lane & 3;
   const int e4 = blockIdx.x * 4 + q, c = min(e4, (E >> 2) - 1); /* columns past the end repeat the last; not stored */
   const int off = 64 * blockIdx.y + 4 * r;
+  x += (size_t)blockIdx.z * H;
+  parts += (size_t)blockIdx.z * ROUTER_PARTS * E;
   const auto rw = __builtin_amdgcn_make_buffer_rsrc((void *)wr, 0, H * E * 4, 0x00020000);
   const auto rx = __builtin_amdgcn_make_buffer_rsrc((void *)x, 0, H * 4, 0x00020000);
   float acc[4] = {0.f, 0.f, 0.f, 0.f};
@@ -1285,7 +1289,8 @@ __global__ __launch_bounds__(256, TC <= 8 ? 4 : TC <= 16 ? 2 : 1) void gate_up_m
   }
 }
 
-/* ---- One token (a decode step) ------------------------------------------------------------
+/* ---- One token (a decode step), or few pairs ----------------------------------------------
+ * The kernels are written for one token; with more of them each is its own layer of the grid.
  * With one row an expert tile's 32 columns are 32 row products, and v_dot8_u32_u4 on the nibbles as they are stored takes
  * half the vector instructions of the matrix form (which unpacks them and waits for each of its eight dependent steps).
  * The row is in LDS as 4-bit digits; a lane has half the weights of each sub-block of its column. The launches are chains
@@ -1381,6 +1386,9 @@ __global__ __launch_bounds__(64 * 2 * ONE_PARTS) void gate_up_one_token_kernel(
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   int myi;
   float myw;
+  const int tok = blockIdx.z, pair0 = tok * topk;
+  x += (size_t)tok * H;
+  lg_in += (size_t)tok * (PARTS ? ROUTER_PARTS : 1) * E;
   /* this wavefront's share of the row of x is asked for first: it has arrived when the routing is done */
   constexpr int XPRE = 2; /* super-blocks a wavefront holds ahead: rows of up to 4096 values */
   const int nsb_x = H >> 8;
@@ -1413,14 +1421,16 @@ __global__ __launch_bounds__(64 * 2 * ONE_PARTS) void gate_up_one_token_kernel(
       route_token_regs<MAXV>(logits, 0, E, topk, renorm, myi, myw);
       const int rank = rank_by_expert(myi, topk);
       if (lane < topk) {
-        idx[lane] = myi;
-        wgt[lane] = myw;
-        slot_pair[rank] = lane; /* slots in ascending expert id; one token: pair = its k */
-        tok_slots[rank] = rank;
-        offsets[myi + 1] = rank + 1; /* the end of the expert's slots: all the later kernels read of offsets */
-        items[2 + 2 * rank] = myi;
-        items[3 + 2 * rank] = rank;
-        table[rank] = OneExpert{views[2 * E + myi].qs, myw, myi};
+        idx[pair0 + lane] = myi;
+        wgt[pair0 + lane] = myw;
+        table[pair0 + rank] = OneExpert{views[2 * E + myi].qs, myw, myi};
+        if (gridDim.z == 1) { /* what the grouped down product reads, if that follows */
+          slot_pair[rank] = lane; /* slots in ascending expert id; one token: pair = its k */
+          tok_slots[rank] = rank;
+          offsets[myi + 1] = rank + 1; /* the end of the expert's slots: all the later kernels read of offsets */
+          items[2 + 2 * rank] = myi;
+          items[3 + 2 * rank] = rank;
+        }
       }
       if (lane == 0) items[0] = topk;
     }
@@ -1513,12 +1523,12 @@ __global__ __launch_bounds__(64 * 2 * ONE_PARTS) void gate_up_one_token_kernel(
   __syncthreads();
   if (first == 1 && part == 0 && lane < 32) {
     const int col = col0 + lane;
-    if (col < I) h[(size_t)item * I + col] = moe_act(ep, e, I, col, xch[lane], out);
+    if (col < I) h[(size_t)(pair0 + item) * I + col] = moe_act(ep, e, I, col, xch[lane], out);
   }
 }
 
-/* The down product of one token and the sum over its experts: a workgroup owns sixteen columns, its wavefronts an expert
- * each, which quantize the expert's row of h themselves. Sixteen columns of a tile leave room for two super-blocks side by
+/* The down product of one token and the sum over its experts: a workgroup owns sixteen columns of a token, its wavefronts an
+ * expert each, which quantize the expert's row of h themselves. Sixteen columns of a tile leave room for two super-blocks side by
  * side in a wavefront (lanes 0 - 31 the even ones), and twice the CUs of a whole tile. The experts' results meet in LDS and
  * are added in ascending id, where the combine's launch had read them from memory. */
 __global__ __launch_bounds__(1024) void down_one_token_kernel(const OneExpert *__restrict__ table, int topk,
@@ -1528,11 +1538,12 @@ __global__ __launch_bounds__(1024) void down_one_token_kernel(const OneExpert *_
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   const int n16 = lane & 15, g = (lane >> 4) & 1, p = lane >> 5;
   const int K = I, nsb = K >> 8, col = blockIdx.x * 16 + n16; /* H % 256 == 0 */
-  const OneExpert ex = table[wave];
+  const int pair = blockIdx.y * topk + wave; /* blockIdx.y: the token */
+  const OneExpert ex = table[pair];
   const OneRow l = one_row_carve(xmoe_lds + wave * one_row_bytes(K), K);
   float *outs = (float *)(xmoe_lds + topk * one_row_bytes(K)); /* [topk][16] */
   /* the expert's row, four super-blocks a pass, sixteen values a lane */
-  const float *row = h + (size_t)wave * K;
+  const float *row = h + (size_t)pair * K;
   float4 xs[4];
   int at = min(lane, K / 16 - 1);
 #pragma unroll
@@ -1591,7 +1602,7 @@ __global__ __launch_bounds__(1024) void down_one_token_kernel(const OneExpert *_
   if (threadIdx.x < 16) {
     float sum = 0.f;
     for (int k = 0; k < topk; ++k) sum = sum + outs[k * 16 + threadIdx.x];
-    y[col] = sum;
+    y[(size_t)blockIdx.y * H + col] = sum;
   }
 }
 
@@ -2156,6 +2167,22 @@ bool mma_few(const hipq_moe_desc &d, int TC) {
   const int64_t max_items = (P < d.experts ? P : d.experts) + P / TC;
   return max_items * ((d.intermediate + 127) / 128) * 4 <= 2048;
 }
+/* LDS of the down product whose workgroups hold all of a token's experts */
+size_t one_token_down_lds(const hipq_moe_desc &d) { return (size_t)d.topk * (one_row_bytes(d.intermediate) + 16 * sizeof(float)); }
+/* Whether every (token, expert) pair's products are its own, in three launches without a sort, instead of products of the
+ * experts with all of their tokens, in five. An expert's weights are then read once a pair. Fitted to 80 blocks of 1 to 64
+ * tokens over 8 to 128 experts, us: pairs of their own 10 + 0.15 a MB of weights over the pairs + 0.06 a MB over the
+ * experts + 0.06 a pair; grouped 23 + 0.04 + 0.14; the line below is within 3 % of the better one in all but two. Measured,
+ * grouped / own: 2 tokens of 128 experts of 2048 x 768, top 8, 28.4 / 18.8, 8 47.2 / 46.2, 10 49.4 / 55.1; 16 of 128 of
+ * 2816 x 512, top 4, 49.4 / 42.3; 4 of eight of 1536 x 1024, top 2, 26.0 / 15.7, 16 29.4 / 26.6; 2 of eight of 2816 x
+ * 1792, top 8, 34.7 / 36.7. */
+bool pairs_apart(const hipq_moe_desc &d) {
+  if (d.tokens > MOE_FEW || d.topk > 16 || one_token_down_lds(d) > 64 * 1024) return false;
+  const double P = (double)d.tokens * d.topk, E = d.experts;
+  const double used = E * (1. - std::pow(1. - std::min(1., d.topk / E), d.tokens)); /* experts with a pair, expected */
+  const double each = 3. * d.hidden * d.intermediate * (hipq::EXPERT_TILE_BYTES / 8192.); /* bytes of an expert's weights */
+  return (1.3 * P - used) * each < 90e6;
+}
 /* The block without a pair sort: the regime of 8-token chunks (a mean expert has at most four
  * pairs), more tokens than the one-launch routing and sort of a decode step takes, an idx[] that
  * a workgroup scans in one go, and rows short enough that four workgroups of the 16-row form fit
@@ -2313,8 +2340,10 @@ int launch_moe(const MoeArgs *a, void *workspace, size_t workspace_bytes, const 
 
   const bool mma = use_mma(d, dt);
   const int chunk = mma ? mma_chunk(d, P, E) : 0; /* tokens of an expert per work item of the matrix-core kernels */
-  /* one token on the matrix-core path: routing, the quantization of x and gate/up as one launch */
-  const bool one_token = mma && T == 1 && chunk == 8 && mma_few(d, 8) && E <= 1024 && d.topk <= 64;
+  /* one token, or few pairs, on the matrix-core path: every pair's products are its own */
+  const bool own = mma && E <= 1024 && pairs_apart(d);
+  /* ... of one token with more experts than a workgroup has wavefronts, the gate/up product only */
+  const bool one_token = own || (mma && T == 1 && chunk == 8 && mma_few(d, 8) && E <= 1024 && d.topk <= 64);
   const float *logits = a->router_logits;
   bool parts = false; /* the logits are partial sums */
   if (!logits) {
@@ -2333,7 +2362,7 @@ int launch_moe(const MoeArgs *a, void *workspace, size_t workspace_bytes, const 
     } else if (one_token && !(E & 3) && (((uintptr_t)a->router_weight | (uintptr_t)a->x) & 15) == 0 &&
                (int64_t)d.hidden * E < (1 << 28)) { /* a buffer descriptor's offsets */
       parts = true;
-      hipq::launch_kernel("router_parts_kernel", router_parts_kernel, dim3((E / 4 + 3) / 4, ROUTER_PARTS / 4), dim3(64), 0, s, a->x,
+      hipq::launch_kernel("router_parts_kernel", router_parts_kernel, dim3((E / 4 + 3) / 4, ROUTER_PARTS / 4, T), dim3(64), 0, s, a->x,
                           a->router_weight, d.hidden, E, b.logits);
     } else if ((E & 3) || (d.hidden & 3) || tb_n < 1 || (((uintptr_t)a->router_weight | (uintptr_t)a->x) & 15)) {
       hipq::launch_kernel("router_logits_scalar_kernel", router_logits_scalar_kernel, dim3(T), dim3(256), 0, s, a->x,
@@ -2370,7 +2399,7 @@ int launch_moe(const MoeArgs *a, void *workspace, size_t workspace_bytes, const 
     const size_t lds_g = one_row_bytes(d.hidden) + (2 * (size_t)one_token_terms(d.hidden) + 32 + (parts ? E : 0)) * sizeof(float);
     OneExpert *table = (OneExpert *)b.hq_mem; /* no kernel of this path keeps quantized rows of h in memory */
     /* one block column more than the columns of h need: the routing's outputs are written there */
-    const dim3 grid((unsigned)((d.intermediate + 31) / 32) + 1, (unsigned)d.topk);
+    const dim3 grid((unsigned)((d.intermediate + 31) / 32) + 1, (unsigned)d.topk, (unsigned)T);
     auto launch = [&](auto k, const char *name) -> int {
       if (lds_g > 64 * 1024) HIPQ_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_g));
       hipq::launch_kernel(name, k, grid, dim3(64 * 2 * ONE_PARTS), lds_g, s, logits, a->router_bias, E, d.topk, d.renormalize,
@@ -2386,11 +2415,9 @@ int launch_moe(const MoeArgs *a, void *workspace, size_t workspace_bytes, const 
     };
     if (const int rc = parts ? by_experts(std::true_type{}) : by_experts(std::false_type{})) return rc;
     HIPQ_HIP(hipGetLastError());
-    const size_t lds_d = (size_t)d.topk * (one_row_bytes(d.intermediate) + 16 * sizeof(float));
-    /* a workgroup's wavefronts are the token's experts; more of them, or longer rows of h than a launch's plain LDS
-     * limit holds, go on to the grouped product below */
-    if (d.topk <= 16 && lds_d <= 64 * 1024) {
-      hipq::launch_kernel("down_one_token_kernel", down_one_token_kernel, dim3((unsigned)(d.hidden / 16)),
+    if (own) { /* otherwise the grouped product below goes on */
+      const size_t lds_d = one_token_down_lds(d);
+      hipq::launch_kernel("down_one_token_kernel", down_one_token_kernel, dim3((unsigned)(d.hidden / 16), (unsigned)T),
                           dim3(64u * d.topk), lds_d, s, (const OneExpert *)table, d.topk, (const float *)b.h, d.hidden,
                           d.intermediate, a->y, a->epi);
       HIPQ_HIP(hipGetLastError());

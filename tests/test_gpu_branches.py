@@ -60,10 +60,20 @@ def test_moe_of_one_token(hipq, cr, h, i, e, k):
     _run_moe(cr, "q4_K", 1, h, i, e, k, True, seed=7200)
 
 
+# pairs whose products are their own, to the most tokens; the last four shapes are beyond the rule (work items of 8, 16 and
+# 32 tokens, and one token more)
+@pytest.mark.parametrize("t,h,i,e,k", [(2, 256, 256, 8, 2), (3, 1280, 768, 16, 16), (7, 768, 512, 300, 5),
+                                       (16, 1536, 512, 8, 2), (33, 512, 256, 64, 3), (64, 256, 256, 8, 1),
+                                       (12, 1024, 1024, 16, 8), (24, 1024, 1024, 8, 4), (48, 1024, 1280, 4, 4),
+                                       (65, 256, 256, 8, 1)])
+def test_moe_of_few_tokens(hipq, cr, t, h, i, e, k):
+    _run_moe(cr, "q4_K", t, h, i, e, k, True, seed=7250)
+
+
 @pytest.mark.parametrize("e,k", [(8, 2), (64, 8), (100, 8), (200, 6), (520, 16)])
 def test_moe_of_one_token_selects_as_the_full_routing(hipq, cr, e, k):
-    """The one-token kernel finds its experts by a search over the logits' magnitudes; two tokens with the same logits
-    take the full routing. Ties across the cut, all logits equal, logits a few spacings apart, an infinity, far apart."""
+    """The one-token kernel finds its experts by a search over the logits' magnitudes; 65 tokens with the same
+    logits take the full routing. Ties across the cut, all logits equal, logits a few spacings apart, an infinity, far apart."""
     import gpu_util as gu
     import torch
     h = i = 256
@@ -74,11 +84,11 @@ def test_moe_of_one_token_selects_as_the_full_routing(hipq, cr, e, k):
     base = synth.normal(7302, (1, e))
     rows = [base, np.round(base), np.zeros_like(base), 1 + base * 2e-7, base * 60, base.copy(), -np.abs(base) * 1e-20]
     rows[5][0, e // 2] = -np.inf
-    dx1, dx2 = gu.dev(x), gu.dev(np.repeat(x, 2, 0))
+    dx1, dx2 = gu.dev(x), gu.dev(np.repeat(x, 65, 0))
     for lg in rows:
         lg = lg.astype(np.float32)
         out = []
-        for t, dx, l in ((1, dx1, lg), (2, dx2, np.repeat(lg, 2, 0))):
+        for t, dx, l in ((1, dx1, lg), (65, dx2, np.repeat(lg, 65, 0))):
             y = torch.full((t, h), float("nan"), device="cuda")
             idx = torch.zeros((t, k), dtype=torch.int32, device="cuda")
             capi.moe_forward(t, h, i, e, k, wg, wu, wd, dx, y, router_logits=gu.dev(l), topk_idx=idx, stream=gu.stream())
@@ -93,7 +103,7 @@ def test_moe_of_one_token_selects_as_the_full_routing(hipq, cr, e, k):
 @pytest.mark.parametrize("h,e,k", [(256, 8, 2), (768, 100, 4), (2304, 132, 8), (4352, 20, 3), (256, 1024, 8), (512, 6, 2)])
 @pytest.mark.parametrize("bias", [False, True])
 def test_moe_of_one_token_routes_from_the_partial_sums(hipq, cr, h, e, k, bias):
-    """The logits of one token come as partial sums that the gate/up kernel adds; two tokens take the kernel that adds
+    """The logits of one token come as partial sums that the gate/up kernel adds; 65 tokens take the kernel that adds
     them itself. Each logit has the same bits, so the experts, their weights and the block's result do."""
     import gpu_util as gu
     import torch
@@ -104,7 +114,7 @@ def test_moe_of_one_token_routes_from_the_partial_sums(hipq, cr, h, e, k, bias):
     x, wr = synth.normal(7401, (1, h)), gu.dev(synth.normal(7402, (h, e), 0.1))
     zero, rb = torch.zeros(e, max(h, i), device="cuda"), gu.dev(synth.normal(7403, (e,), 2.0))
     out = []
-    for t in (1, 2):
+    for t in (1, 3, 65):
         dx = gu.dev(np.repeat(x, t, 0))
         y = torch.full((t, h), float("nan"), device="cuda")
         idx = torch.zeros((t, k), dtype=torch.int32, device="cuda")
@@ -116,9 +126,9 @@ def test_moe_of_one_token_routes_from_the_partial_sums(hipq, cr, h, e, k, bias):
         else:
             capi.moe_forward(t, h, i, e, k, wg, wu, wd, dx, y, **opt)
         torch.cuda.synchronize()
-        out.append((y[0], idx[0], wt[0]))
-    for a, b in zip(*out):
-        assert torch.equal(a, b)
+        out.append((y[t - 1], idx[t - 1], wt[t - 1]))
+    for a, b, c in zip(*out):
+        assert torch.equal(a, c) and torch.equal(b, c)
     assert not bool(torch.isnan(out[0][0]).any())
     for w in wg + wu + wd:
         w.destroy()
