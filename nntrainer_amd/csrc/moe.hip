@@ -1688,10 +1688,10 @@ __global__ __launch_bounds__(256, TC <= 8 ? 4 : TC <= 16 ? 2 : 1) void down_mma_
 }
 
 /* ---- Many tokens per expert (moe_tile_device.h) -------------------------------------------
- * An item is up to 64 slots of one expert; 32 or fewer take the one-tile form. The workgroups of an
+ * An item is up to 64 (`rows`) slots of one expert; 32 or fewer take the one-tile form. The workgroups of an
  * item follow each other on one XCD (they share the item's rows, and consecutive items of an expert
  * its weights through the last-level cache). */
-__device__ __forceinline__ bool tile_item(int cols, const int *__restrict__ items, const int *__restrict__ offsets,
+__device__ __forceinline__ bool tile_item(int cols, int rows, const int *__restrict__ items, const int *__restrict__ offsets,
                                           int &col, int &e, int &s0, int &n) {
   const int id = blockIdx.x, xcd = id & 7, q = id >> 3;
   const int item = (q / cols) * 8 + xcd;
@@ -1699,7 +1699,7 @@ __device__ __forceinline__ bool tile_item(int cols, const int *__restrict__ item
   if (item >= items[0]) return false; /* uniform per workgroup */
   e = items[2 + 2 * item];
   s0 = items[3 + 2 * item];
-  n = min(moe_tile::ROWS, offsets[e + 1] - s0);
+  n = min(rows, offsets[e + 1] - s0);
   return true;
 }
 
@@ -1714,9 +1714,8 @@ __device__ __forceinline__ void gate_up_tile_pass(moe_tile::Lds &l, const QView 
   const bool up = wave >= 2;
   float v[TM * 16];
   moe_tile::run<TM>(
-    l, xq, (uint32_t)T, 1,
-    [&](int) { return (up ? wu : wg).qs + (size_t)tile * (size_t)((xq.K >> 8) * hipq::EXPERT_TILE_BYTES); },
-    [&](int, const float(&acc)[TM][16], const float(&accm)[TM][16]) {
+    l, xq, (uint32_t)T, (up ? wu : wg).qs + (size_t)tile * (size_t)((xq.K >> 8) * hipq::EXPERT_TILE_BYTES),
+    [&](const float(&acc)[TM][16], const float(&accm)[TM][16]) {
 #pragma unroll
       for (int i = 0; i < TM * 16; ++i) v[i] = acc[i >> 4][i & 15] - accm[i >> 4][i & 15];
     });
@@ -1737,12 +1736,12 @@ __device__ __forceinline__ void gate_up_tile_pass(moe_tile::Lds &l, const QView 
 __global__ __launch_bounds__(256, 3) void gate_up_tile_kernel(const WView *__restrict__ views, int E_, QView xq, int T,
                                                               const int *__restrict__ offsets,
                                                               const int *__restrict__ items,
-                                                              const int *__restrict__ slot_pair, int topk, int I,
-                                                              float *__restrict__ h, hipq::MoeEpi ep) {
+                                                              const int *__restrict__ slot_pair, int rows, int topk,
+                                                              int I, float *__restrict__ h, hipq::MoeEpi ep) {
   extern __shared__ __attribute__((aligned(16))) unsigned char xmoe_lds[];
   moe_tile::Lds &l = *reinterpret_cast<moe_tile::Lds *>(xmoe_lds);
   int col, e, s0, n;
-  if (!tile_item(I >> 6, items, offsets, col, e, s0, n)) return;
+  if (!tile_item(I >> 6, rows, items, offsets, col, e, s0, n)) return;
   const WView wg = views[e], wu = views[E_ + e];
   if (threadIdx.x < moe_tile::ROWS) l.rows[threadIdx.x] = slot_pair[s0 + min((int)threadIdx.x, n - 1)] / topk;
   __syncthreads();
@@ -1752,19 +1751,20 @@ __global__ __launch_bounds__(256, 3) void gate_up_tile_kernel(const WView *__res
     gate_up_tile_pass<1>(l, xq, T, col, e, s0, n, wg, wu, I, h, ep);
 }
 
-/* contrib of 256 columns, two tiles a wavefront one after the other; the rows of h are quantized (a row of
- * the activation planes is a slot) */
+/* contrib of 128 columns, a tile a wavefront; the rows of h are quantized (a row of the activation planes is a slot). With
+ * two tiles a wavefront, one after the other, a block of few experts left most of the chip idle and one of many ended
+ * less evenly: us a block, 100 tokens of eight experts of 1536 x 1024, top 2, 43.9 -> 36.3, 250 52 / 44, of 32 of 2560 x 1280,
+ * top 4, 93.2 -> 85.0, 1000 of 128 of 2048 x 768, top 8, 199.9 -> 195.7 (without the router). */
 template <int TM>
 __device__ __forceinline__ void down_tile_pass(moe_tile::Lds &l, const QView &hq, int P, int col, int e, int s0, int n,
                                                const WView &wd, const float *wrow, int H, float *__restrict__ contrib,
                                                const hipq::MoeEpi &ep) {
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
-  const int tile0 = (col * 4 + wave) * 2; /* H % 256 == 0 */
+  const int tile = col * 4 + wave; /* H % 256 == 0 */
   moe_tile::run<TM>(
-    l, hq, (uint32_t)P, 2,
-    [&](int t) { return wd.qs + (size_t)(tile0 + t) * (size_t)((hq.K >> 8) * hipq::EXPERT_TILE_BYTES); },
-    [&](int t, const float(&acc)[TM][16], const float(&accm)[TM][16]) {
-      const int c = (tile0 + t) * 32 + (lane & 31), g4 = 4 * (lane >> 5);
+    l, hq, (uint32_t)P, wd.qs + (size_t)tile * (size_t)((hq.K >> 8) * hipq::EXPERT_TILE_BYTES),
+    [&](const float(&acc)[TM][16], const float(&accm)[TM][16]) {
+      const int c = tile * 32 + (lane & 31), g4 = 4 * (lane >> 5);
       const uint32_t off = (uint32_t)(g4 * H + c); /* the rest of an address is uniform */
 #pragma unroll
       for (int tm = 0; tm < TM; ++tm)
@@ -1780,13 +1780,13 @@ __global__ __launch_bounds__(256, 3) void down_tile_kernel(const WView *__restri
                                                            const int *__restrict__ offsets,
                                                            const int *__restrict__ items,
                                                            const int *__restrict__ slot_pair,
-                                                           const float *__restrict__ wgt, int H,
+                                                           const float *__restrict__ wgt, int rows, int H,
                                                            float *__restrict__ contrib, hipq::MoeEpi ep) {
   extern __shared__ __attribute__((aligned(16))) unsigned char xmoe_lds[];
   moe_tile::Lds &l = *reinterpret_cast<moe_tile::Lds *>(xmoe_lds);
   float *wrow = (float *)(xmoe_lds + sizeof(moe_tile::Lds)); /* [ROWS] the routing weights of the item's rows */
   int col, e, s0, n;
-  if (!tile_item(H >> 8, items, offsets, col, e, s0, n)) return;
+  if (!tile_item(H >> 7, rows, items, offsets, col, e, s0, n)) return;
   const WView wd = views[2 * E_ + e];
   if (threadIdx.x < moe_tile::ROWS) {
     const int slot = s0 + min((int)threadIdx.x, n - 1);
@@ -2257,34 +2257,42 @@ int launch_grouped_mma(const hipq::MoeArgs *a, const MoeBufs &b, const WView *vi
 }
 
 int launch_tile_mma(const hipq::MoeArgs *a, const MoeBufs &b, const WView *views, const QAct &xq, const QAct &hq,
-                    hipStream_t s) {
+                    int rows, hipStream_t s) {
   const hipq_moe_desc &d = a->desc;
   const int64_t P = (int64_t)d.tokens * d.topk;
-  const int max_items = (int)((P < d.experts ? P : d.experts) + P / moe_tile::ROWS);
+  const int max_items = (int)((P < d.experts ? P : d.experts) + P / rows);
   const unsigned groups = (unsigned)((max_items + 7) / 8 * 8);
   hipq::launch_kernel("gate_up_tile_kernel", gate_up_tile_kernel, dim3(groups * (unsigned)(d.intermediate / 64)), dim3(256),
-                      sizeof(moe_tile::Lds), s, views, d.experts, qview(xq), d.tokens, b.offsets, b.items, b.slot_pair,
+                      sizeof(moe_tile::Lds), s, views, d.experts, qview(xq), d.tokens, b.offsets, b.items, b.slot_pair, rows,
                       d.topk, d.intermediate, b.h, a->epi);
   HIPQ_HIP(hipGetLastError());
   if (int rc = hipq::launch_quantize_q8_K_rowmma(b.h, P, d.intermediate, d.intermediate, &hq, s)) return rc;
-  hipq::launch_kernel("down_tile_kernel", down_tile_kernel, dim3(groups * (unsigned)(d.hidden / 256)), dim3(256),
+  hipq::launch_kernel("down_tile_kernel", down_tile_kernel, dim3(groups * (unsigned)(d.hidden / 128)), dim3(256),
                       sizeof(moe_tile::Lds) + moe_tile::ROWS * sizeof(float), s, views, d.experts, qview(hq), (int)P,
-                      b.offsets, b.items, b.slot_pair, (const float *)b.wgt, d.hidden, b.contrib, a->epi);
+                      b.offsets, b.items, b.slot_pair, (const float *)b.wgt, rows, d.hidden, b.contrib, a->epi);
   HIPQ_HIP(hipGetLastError());
   return HIPQ_OK;
 }
 
-/* Token chunk of the matrix-core expert kernels for P pairs over E experts: the
+/* Rows of a work item of the matrix-core expert kernels for P pairs over E experts: of the tiles (tiles is set), or the
  * smallest of 8, 16, 32 that holds twice the mean tokens per expert (an expert with
  * more becomes several work items), reduced until the activation rows fit the LDS. */
-int mma_chunk(const hipq_moe_desc &d, int64_t P, int E) {
+int mma_chunk(const hipq_moe_desc &d, int64_t P, int E, bool *tiles) {
+  *tiles = false;
   const int64_t mean2 = (2 * P + E - 1) / E;
-  /* From twelve tokens an expert on the 64-row tiles are the faster form (us a block, items of 8 to 32 tokens ->
-   * tiles): 2048 / 768 / 128 experts, top 8, with 128 / 200 / 512 / 1000 tokens 92 -> 113 / 140 -> 117 / 243 -> 160 /
-   * 375 -> 221; 1024 / 2048 / 32, top 4, with 64 / 128 / 1000 tokens 59 -> 61 / 89 -> 63 / 250 -> 148. The planes
-   * are addressed with 32 bits. */
-  if (mean2 >= 24 && P * d.intermediate < (int64_t(1) << 32) && (int64_t)d.tokens * d.hidden < (int64_t(1) << 32))
-    return moe_tile::ROWS;
+  /* From eight tokens an expert on the tiles are the faster form (us a block, items of 8 to 32 tokens -> tiles): eight
+   * experts of 1536 x 1024, top 2, with 24 / 40 tokens 29.4 -> 32.3 / 39.1 -> 33.2; 32 of 2560 x 1280, top 4, with 40 / 70
+   * 55.4 -> 63.2 / 96.1 -> 65.3; 64 of 1792 x 768, top 4, with 100 / 160 51.4 -> 60.1 / 73.3 -> 60.5; 128 of 2048 x 768,
+   * top 8, with 100 / 160 83.8 -> 104 / 116 -> 107. The planes are addressed with 32 bits. */
+  if (mean2 > 16 && P * d.intermediate < (int64_t(1) << 32) && (int64_t)d.tokens * d.hidden < (int64_t(1) << 32)) {
+    *tiles = true;
+    /* Items of 32 rows where those of 64 leave the chip unfilled: their number is about P / 64 and half an item an expert,
+     * and the two products have I / 64 and H / 128 workgroups an item. us a block at 64 / 32 rows: eight experts of 1536 x
+     * 1024, top 2, 100 tokens 36.3 / 34.2, 250 44.0 / 39.9, 600 (637 workgroups) 54.1 / 51.2, 1000 (987) 66.1 / 71.8; of 2048 x
+     * 512, top 8, 160 (576) 48.8 / 46.2, 250 (846) 53.1 / 54.7; 32 of 2560 x 1280, top 4, 250 (1280) 85.0 / 97.2. */
+    const int64_t items = std::max<int64_t>(std::min<int64_t>(P, E), P / moe_tile::ROWS + E / 2);
+    return items * (d.intermediate / 64 + d.hidden / 128) <= 700 ? moe_tile::ROWS / 2 : moe_tile::ROWS;
+  }
   int tc = mean2 <= 8 ? 8 : mean2 <= 16 ? 16 : 32;
   const int kmax = d.hidden > d.intermediate ? d.hidden : d.intermediate;
   while (tc > 8 && xlds_bytes(tc, kmax) + tc * 256 > XLDS_MAX) tc >>= 1; /* + the paired form's exchange area */
@@ -2339,7 +2347,8 @@ int launch_moe(const MoeArgs *a, void *workspace, size_t workspace_bytes, const 
   const int T = d.tokens, E = d.experts, P = T * d.topk;
 
   const bool mma = use_mma(d, dt);
-  const int chunk = mma ? mma_chunk(d, P, E) : 0; /* tokens of an expert per work item of the matrix-core kernels */
+  bool tiles = false;
+  const int chunk = mma ? mma_chunk(d, P, E, &tiles) : 0; /* tokens of an expert per work item of the matrix-core kernels */
   /* one token, or few pairs, on the matrix-core path: every pair's products are its own */
   const bool own = mma && E <= 1024 && pairs_apart(d);
   /* ... of one token with more experts than a workgroup has wavefronts, the gate/up product only */
@@ -2475,7 +2484,7 @@ int launch_moe(const MoeArgs *a, void *workspace, size_t workspace_bytes, const 
     rc = launch_self_mma(a, b, views, xq, s);
   } else if (mma) {
     const int tc = chunk;
-    rc = tc == 64   ? launch_tile_mma(a, b, views, xq, hq, s)
+    rc = tiles      ? launch_tile_mma(a, b, views, xq, hq, chunk, s)
          : tc == 8  ? launch_grouped_mma<8>(a, b, views, xq, hq, s, one_token)
          : tc == 16 ? launch_grouped_mma<16>(a, b, views, xq, hq, s)
                     : launch_grouped_mma<32>(a, b, views, xq, hq, s);

@@ -21,7 +21,7 @@
  * beforehand. A row's sixteen 16-byte pieces are stored rotated by an exclusive-or with its number
  * (the lane asks for piece slot ^ row), which spreads the 128-bit reads of eight neighbouring rows
  * over all banks. Weights stream through registers from the expert tiles (hipq_internal.h), a
- * super-block ahead; tile switches do not drain the pipeline.
+ * super-block ahead.
  */
 #ifndef HIPQ_MOE_TILE_DEVICE_H
 #define HIPQ_MOE_TILE_DEVICE_H
@@ -56,12 +56,11 @@ __device__ __forceinline__ uint32_t scale2(uint32_t x, uint32_t digit2) {
 }
 __device__ __forceinline__ int out_row(int tm, int r, int lane) { return 32 * tm + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
 
-/* The wavefront's ntile column tiles over the whole of K for the item's 32 * TM rows (l.rows, all of
- * them valid plane rows). tile_of(t) names the first byte of tile t's expert tile, done(t, acc, accm)
- * receives its sums: acc[tm][r] - accm[tm][r] is row out_row(tm, r, lane), column lane & 31. Every wavefront of
- * the workgroup calls it with the same ntile (the barriers). */
-template <int TM, typename TileOf, typename Done>
-__device__ __forceinline__ void run(Lds &l, const QView &a, uint32_t a_rows, int ntile, TileOf tile_of, Done done) {
+/* The wavefront's column tile (its first byte is tile[0]) over the whole of K for the item's 32 * TM rows (l.rows, all of
+ * them valid plane rows). done(acc, accm) receives the sums: acc[tm][r] - accm[tm][r] is row out_row(tm, r, lane), column
+ * lane & 31. */
+template <int TM, typename Done>
+__device__ __forceinline__ void run(Lds &l, const QView &a, uint32_t a_rows, const uint8_t *tile, Done done) {
   const int K = a.K, nsb = K >> 8;
   const int lane = threadIdx.x & 63, i32 = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -92,139 +91,137 @@ __device__ __forceinline__ void run(Lds &l, const QView &a, uint32_t a_rows, int
   /* LDS byte of this lane's operand of step j: row i32, piece 2 j + g */
   const uint32_t abase = (uint32_t)(i32 * 256 + ((g ^ (i32 & 15)) << 4));
 
-  for (int t = 0; t < ntile; ++t) {
-    const rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)tile_of(t), 0, (int)tile_bytes, 0x00020000);
-    auto load_q = [&](int sb, int i) {
-      return __builtin_bit_cast(
-        v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, lane * 16, sb * hipq::EXPERT_TILE_BYTES + i * 1024, 0));
-    };
-    auto load_hd = [&](int sb) {
-      return __builtin_bit_cast(
-        v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, 4096 + i32 * 16, sb * hipq::EXPERT_TILE_BYTES, 0));
-    };
-    float acc[TM][16];
+  const rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)tile, 0, (int)tile_bytes, 0x00020000);
+  auto load_q = [&](int sb, int i) {
+    return __builtin_bit_cast(
+      v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, lane * 16, sb * hipq::EXPERT_TILE_BYTES + i * 1024, 0));
+  };
+  auto load_hd = [&](int sb) {
+    return __builtin_bit_cast(
+      v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, 4096 + i32 * 16, sb * hipq::EXPERT_TILE_BYTES, 0));
+  };
+  float acc[TM][16];
 #pragma unroll
-    for (int tm = 0; tm < TM; ++tm)
+  for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[tm][r] = 0.f;
-    v4i W[4], hd0, hd1;
+    for (int r = 0; r < 16; ++r) acc[tm][r] = 0.f;
+  v4i W[4], hd0, hd1;
 
-    /* One super-block: the rows of the next are asked for first; a quarter of the nibbles is asked for
-     * again (for the next super-block) as soon as its two steps have taken it, so one set of registers holds
-     * the stream and most of a super-block's time covers every load. */
-    auto super_block = [&](int sb, int buf, const v4i &hd, v4i &hdn) {
-      const int sbn = min(sb + 1, nsb - 1); /* past the end the last one again: a fixed number of loads in flight */
-      copy_rows(sbn, buf ^ 1);
-      const int8_t *pq = l.q[buf];
-      const uint32_t hx = (uint32_t)hd[0], hy = (uint32_t)hd[1], hz = (uint32_t)hd[2];
-      v16i Dlo[TM], Dhi[TM];
+  /* One super-block: the rows of the next are asked for first; a quarter of the nibbles is asked for
+   * again (for the next super-block) as soon as its two steps have taken it, so one set of registers holds
+   * the stream and most of a super-block's time covers every load. */
+  auto super_block = [&](int sb, int buf, const v4i &hd, v4i &hdn) {
+    const int sbn = min(sb + 1, nsb - 1); /* past the end the last one again: a fixed number of loads in flight */
+    copy_rows(sbn, buf ^ 1);
+    const int8_t *pq = l.q[buf];
+    const uint32_t hx = (uint32_t)hd[0], hy = (uint32_t)hd[1], hz = (uint32_t)hd[2];
+    v16i Dlo[TM], Dhi[TM];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        v4i av[TM];
-        uint32_t at = abase;
-        asm("" : "+v"(at)); /* one instruction a step instead of eight registers */
+    for (int j = 0; j < 8; ++j) {
+      v4i av[TM];
+      uint32_t at = abase;
+      asm("" : "+v"(at)); /* one instruction a step instead of eight registers */
 #pragma unroll
-        for (int tm = 0; tm < TM; ++tm) av[tm] = *(const v4i *)(pq + (at ^ (j * 32)) + tm * 8192);
-        const uint32_t sel = 0x0c000c00u | (uint32_t)(j & 3) | ((uint32_t)(j & 3) << 16);
-        const uint32_t sc = j < 4 ? hy : hz;
-        const uint32_t slo = sc & 0x07070707u, shi = (sc >> 3) & 0x07070707u;
-        const uint32_t dl = __builtin_amdgcn_perm(slo, slo, sel), dh = __builtin_amdgcn_perm(shi, shi, sel);
-        const uint32_t x0 = (uint32_t)W[j >> 1][2 * (j & 1)], x1 = (uint32_t)W[j >> 1][2 * (j & 1) + 1];
-        const uint32_t e0 = x0 & HIPQ_M4, e1 = x1 & HIPQ_M4, o0 = (x0 >> 4) & HIPQ_M4, o1 = (x1 >> 4) & HIPQ_M4;
-        const v4i bl = {(int)scale2(e0, dl), (int)scale2(e1, dl), (int)scale2(o0, dl), (int)scale2(o1, dl)};
-        const v4i bh = {(int)scale2(e0, dh), (int)scale2(e1, dh), (int)scale2(o0, dh), (int)scale2(o1, dh)};
-#pragma unroll
-        for (int tm = 0; tm < TM; ++tm) {
-          Dlo[tm] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[tm], bl, j == 0 ? zero16 : Dlo[tm], 0, 0, 0);
-          Dhi[tm] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[tm], bh, j == 0 ? zero16 : Dhi[tm], 0, 0, 0);
-        }
-        if (j & 1) W[j >> 1] = load_q(sbn, j >> 1);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      hdn = load_hd(sbn);
-      const float dw = hipq_h2f((uint16_t)(hx & 0xffff));
+      for (int tm = 0; tm < TM; ++tm) av[tm] = *(const v4i *)(pq + (at ^ (j * 32)) + tm * 8192);
+      const uint32_t sel = 0x0c000c00u | (uint32_t)(j & 3) | ((uint32_t)(j & 3) << 16);
+      const uint32_t sc = j < 4 ? hy : hz;
+      const uint32_t slo = sc & 0x07070707u, shi = (sc >> 3) & 0x07070707u;
+      const uint32_t dl = __builtin_amdgcn_perm(slo, slo, sel), dh = __builtin_amdgcn_perm(shi, shi, sel);
+      const uint32_t x0 = (uint32_t)W[j >> 1][2 * (j & 1)], x1 = (uint32_t)W[j >> 1][2 * (j & 1) + 1];
+      const uint32_t e0 = x0 & HIPQ_M4, e1 = x1 & HIPQ_M4, o0 = (x0 >> 4) & HIPQ_M4, o1 = (x1 >> 4) & HIPQ_M4;
+      const v4i bl = {(int)scale2(e0, dl), (int)scale2(e1, dl), (int)scale2(o0, dl), (int)scale2(o1, dl)};
+      const v4i bh = {(int)scale2(e0, dh), (int)scale2(e1, dh), (int)scale2(o0, dh), (int)scale2(o1, dh)};
 #pragma unroll
       for (int tm = 0; tm < TM; ++tm) {
+        Dlo[tm] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[tm], bl, j == 0 ? zero16 : Dlo[tm], 0, 0, 0);
+        Dhi[tm] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[tm], bh, j == 0 ? zero16 : Dhi[tm], 0, 0, 0);
+      }
+      if (j & 1) W[j >> 1] = load_q(sbn, j >> 1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    hdn = load_hd(sbn);
+    const float dw = hipq_h2f((uint16_t)(hx & 0xffff));
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm) {
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        const v4i dv = *(const v4i *)((const int8_t *)l.dA[buf] + (32 * tm + 8 * q4 + 4 * g) * 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int r = 4 * q4 + e;
+          acc[tm][r] = fmaf((float)((Dhi[tm][r] << 3) + Dlo[tm][r]), dw * __int_as_float(dv[e]), acc[tm][r]);
+        }
+      }
+      /* keeps the arithmetic of a row tile here: sunk past the barrier its operands would all stay live */
+#pragma unroll
+      for (int r = 0; r < 16; ++r) asm volatile("" : "+v"(acc[tm][r]));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    /* the rows copied above have arrived (they were issued before the five weight loads, which stay in flight) */
+    asm volatile("s_waitcnt vmcnt(5) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  };
+
+  copy_rows(0, 0);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) W[i] = load_q(0, i);
+  hd0 = load_hd(0);
+  asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+  int sb = 0;
+  for (; sb + 1 < nsb; sb += 2) {
+    super_block(sb, 0, hd0, hd1);
+    super_block(sb + 1, 1, hd1, hd0);
+  }
+  if (sb < nsb) super_block(sb, 0, hd0, hd1);
+
+  /* the mins: accm = fma(Im, dmin * dA, accm) over the super-blocks, in a pass of its own so that its
+   * chains do not occupy registers during the products */
+  float accm[TM][16];
+#pragma unroll
+  for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) accm[tm][r] = 0.f;
+  MinsLds &ml = *reinterpret_cast<MinsLds *>(&l.q[0][0]);
+  const uint32_t vm = (uint32_t)l.rows[(32 * (wave & 1) + (lane >> 1)) & (32 * TM - 1)] * (uint32_t)(nsb * 32) + (lane & 1) * 16;
+  for (int m0 = 0; m0 < nsb; m0 += MINS_SB) {
+    const int mn = min(MINS_SB, nsb - m0);
+    /* copies of the last super-block of the products may still be under way into the row buffers */
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    for (int k = wave; k < TM * mn; k += 4) { /* 32 rows of a super-block; k % TM is wave % TM, as in vm */
+      const int b = k / TM, part = k % TM;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rm, lds_ptr(ml.amin[b] + part * 1024), 16, (int)vm, (m0 + b) * 32, 0, 0);
+    }
+    for (int b = wave; b < mn; b += 4)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rd, lds_ptr(ml.dA[b]), 4, (int)vd, (m0 + b) * 4, 0, 0);
+    v4i hd = load_hd(m0);
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    for (int b = 0; b < mn; ++b) {
+      const uint32_t hx = (uint32_t)hd[0], hy = (uint32_t)hd[1], hz = (uint32_t)hd[2], hw = (uint32_t)hd[3];
+      hd = load_hd(m0 + min(b + 1, mn - 1));
+      const float dmin = hipq_h2f((uint16_t)(hx >> 16));
+      const uint32_t mlo = (hw & 0x0f0f0f0fu) | ((hy >> 2) & 0x30303030u);
+      const uint32_t mhi = ((hw >> 4) & 0x0f0f0f0fu) | ((hz >> 2) & 0x30303030u);
+      v8h bmin;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        bmin[j] = (_Float16)(float)((mlo >> (8 * j)) & 0xff);
+        bmin[4 + j] = (_Float16)(float)((mhi >> (8 * j)) & 0xff);
+      }
+#pragma unroll
+      for (int tm = 0; tm < TM; ++tm) {
+        const v8h amin = __builtin_bit_cast(v8h, *(const v4i *)(ml.amin[b] + (32 * tm + i32) * 32 + g * 16));
+        const v16f Sm = __builtin_amdgcn_mfma_f32_32x32x16_f16(amin, bmin, zero16f, 0, 0, 0);
 #pragma unroll
         for (int q4 = 0; q4 < 4; ++q4) {
-          const v4i dv = *(const v4i *)((const int8_t *)l.dA[buf] + (32 * tm + 8 * q4 + 4 * g) * 4);
+          const v4i dv = *(const v4i *)((const int8_t *)ml.dA[b] + (32 * tm + 8 * q4 + 4 * g) * 4);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int r = 4 * q4 + e;
-            acc[tm][r] = fmaf((float)((Dhi[tm][r] << 3) + Dlo[tm][r]), dw * __int_as_float(dv[e]), acc[tm][r]);
-          }
-        }
-        /* keeps the arithmetic of a row tile here: sunk past the barrier its operands would all stay live */
-#pragma unroll
-        for (int r = 0; r < 16; ++r) asm volatile("" : "+v"(acc[tm][r]));
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      /* the rows copied above have arrived (they were issued before the five weight loads, which stay in flight) */
-      asm volatile("s_waitcnt vmcnt(5) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    };
-
-    copy_rows(0, 0);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) W[i] = load_q(0, i);
-    hd0 = load_hd(0);
-    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-    int sb = 0;
-    for (; sb + 1 < nsb; sb += 2) {
-      super_block(sb, 0, hd0, hd1);
-      super_block(sb + 1, 1, hd1, hd0);
-    }
-    if (sb < nsb) super_block(sb, 0, hd0, hd1);
-
-    /* the mins: accm = fma(Im, dmin * dA, accm) over the super-blocks, in a pass of its own so that its
-     * chains do not occupy registers during the products */
-    float accm[TM][16];
-#pragma unroll
-    for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) accm[tm][r] = 0.f;
-    MinsLds &ml = *reinterpret_cast<MinsLds *>(&l.q[0][0]);
-    const uint32_t vm = (uint32_t)l.rows[(32 * (wave & 1) + (lane >> 1)) & (32 * TM - 1)] * (uint32_t)(nsb * 32) + (lane & 1) * 16;
-    for (int m0 = 0; m0 < nsb; m0 += MINS_SB) {
-      const int mn = min(MINS_SB, nsb - m0);
-      /* copies of the last super-block of the products may still be under way into the row buffers */
-      asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-      for (int k = wave; k < TM * mn; k += 4) { /* 32 rows of a super-block; k % TM is wave % TM, as in vm */
-        const int b = k / TM, part = k % TM;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rm, lds_ptr(ml.amin[b] + part * 1024), 16, (int)vm, (m0 + b) * 32, 0, 0);
-      }
-      for (int b = wave; b < mn; b += 4)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rd, lds_ptr(ml.dA[b]), 4, (int)vd, (m0 + b) * 4, 0, 0);
-      v4i hd = load_hd(m0);
-      asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-      for (int b = 0; b < mn; ++b) {
-        const uint32_t hx = (uint32_t)hd[0], hy = (uint32_t)hd[1], hz = (uint32_t)hd[2], hw = (uint32_t)hd[3];
-        hd = load_hd(m0 + min(b + 1, mn - 1));
-        const float dmin = hipq_h2f((uint16_t)(hx >> 16));
-        const uint32_t mlo = (hw & 0x0f0f0f0fu) | ((hy >> 2) & 0x30303030u);
-        const uint32_t mhi = ((hw >> 4) & 0x0f0f0f0fu) | ((hz >> 2) & 0x30303030u);
-        v8h bmin;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          bmin[j] = (_Float16)(float)((mlo >> (8 * j)) & 0xff);
-          bmin[4 + j] = (_Float16)(float)((mhi >> (8 * j)) & 0xff);
-        }
-#pragma unroll
-        for (int tm = 0; tm < TM; ++tm) {
-          const v8h amin = __builtin_bit_cast(v8h, *(const v4i *)(ml.amin[b] + (32 * tm + i32) * 32 + g * 16));
-          const v16f Sm = __builtin_amdgcn_mfma_f32_32x32x16_f16(amin, bmin, zero16f, 0, 0, 0);
-#pragma unroll
-          for (int q4 = 0; q4 < 4; ++q4) {
-            const v4i dv = *(const v4i *)((const int8_t *)ml.dA[b] + (32 * tm + 8 * q4 + 4 * g) * 4);
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              accm[tm][4 * q4 + e] = fmaf(Sm[4 * q4 + e], dmin * __int_as_float(dv[e]), accm[tm][4 * q4 + e]);
-          }
+          for (int e = 0; e < 4; ++e)
+            accm[tm][4 * q4 + e] = fmaf(Sm[4 * q4 + e], dmin * __int_as_float(dv[e]), accm[tm][4 * q4 + e]);
         }
       }
     }
-    done(t, acc, accm);
-    __syncthreads(); /* the row buffers are free again */
   }
+  done(acc, accm);
+  __syncthreads(); /* the row buffers are free again */
 }
 
 } // namespace moe_tile

@@ -227,6 +227,34 @@ def test_moe_tiles_of_64_rows(hipq, cr, h, i):
         w.destroy()
 
 
+@pytest.mark.parametrize("h,i", [(1280, 768), (256, 1536), (3328, 256)])
+def test_moe_tiles_of_64_rows_of_many_experts(hipq, cr, h, i):
+    """The counts above among 32 experts: enough work items for 64 rows each; with few they have 32."""
+    import gpu_util as gu
+    import torch
+    counts = [64, 65, 32, 33, 1, 0, 130] + [8] * 25
+    t, e, k = sum(counts), len(counts), 1
+    gate, up, down = ([m[x % 3] for x in range(e)] for m in _experts(cr, 3, i, h, seed=9500))
+    x = synth.normal(9600, (t, h))
+    logits = synth.normal(9601, (t, e))
+    owner = np.repeat(np.arange(e), counts)[np.random.default_rng(3).permutation(t)]
+    logits[np.arange(t), owner] += 20.0
+    ref_y, ref_idx, _ = cr.moe_forward(x, logits, gate, up, down, k)
+    assert np.array_equal(np.bincount(ref_idx.ravel(), minlength=e), counts)
+    wg = [capi.Weight("q4_K", i, h, b) for b in gate]
+    wu = [capi.Weight("q4_K", i, h, b) for b in up]
+    wd = [capi.Weight("q4_K", h, i, b) for b in down]
+    y = torch.full((t, h), float("nan"), device="cuda")
+    for _ in range(2):
+        capi.moe_forward(t, h, i, e, k, wg, wu, wd, gu.dev(x), y, router_logits=gu.dev(logits), stream=gu.stream())
+    torch.cuda.synchronize()
+    got = y.cpu().numpy()
+    assert not np.isnan(got).any()
+    assert gu.rel_err(got, ref_y) <= 2e-6, gu.rel_err(got, ref_y)
+    for w in wg + wu + wd:
+        w.destroy()
+
+
 def test_expert_weights_serve_the_moe_block_only(hipq, cr):
     """Q4_K experts are re-stored for the expert kernels at the first block; a plain
     matmul on such a handle is refused, the block keeps giving the same bits."""
