@@ -359,20 +359,31 @@ __global__ __launch_bounds__(NT, TM == 2 ? 3 : 2) void gemm_q4k_split_kernel(WVi
   if (nt >= ntiles) return; /* uniform per workgroup */
   const int sb0 = blockIdx.y * sb_per_part;
   const int n = min(sb_per_part, (w.K >> 8) - sb0);
-  gemm_q4k_tile<TM, true, true>(w, qt, amin, dAt, M, mt, nt, part + (int64_t)blockIdx.y * part_stride, w.N, sb0, n);
+  gemm_q4k_tile<TM, true, true>(w, qt, amin, dAt, M, mt, nt, part + (int64_t)blockIdx.y * part_stride,
+                                (int)((w.N + 3) & ~3), sb0, n);
 }
 
+/* The partial products' rows are padded to whole quads (stride Np), so rows of any length are read 16 bytes a lane; C is
+ * written so where its rows allow it. */
 __global__ __launch_bounds__(256) void split_sum_kernel(const float *__restrict__ part, int parts, int64_t part_stride,
-                                                        int M, int N, float *__restrict__ C, int64_t ldc) {
-  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4; /* N % 4 == 0 */
-  if (i >= (int64_t)M * N) return;
-  const int m = (int)(i / N), n = (int)(i - (int64_t)m * N);
+                                                        int M, int N, int Np, float *__restrict__ C, int64_t ldc, bool whole) {
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= (int64_t)M * Np) return;
+  const int m = (int)(i / Np), n = (int)(i - (int64_t)m * Np);
   float4 v = *(const float4 *)(part + i);
   for (int p = 1; p < parts; ++p) {
     const float4 u = *(const float4 *)(part + p * part_stride + i);
     v.x += u.x, v.y += u.y, v.z += u.z, v.w += u.w;
   }
-  *(float4 *)(C + (int64_t)m * ldc + n) = v;
+  float *c = C + (int64_t)m * ldc + n;
+  if (whole) {
+    *(float4 *)c = v;
+    return;
+  }
+  c[0] = v.x;
+  if (n + 1 < N) c[1] = v.y;
+  if (n + 2 < N) c[2] = v.z;
+  if (n + 3 < N) c[3] = v.w;
 }
 
 /* Up to four weights of one K (each with its tile copy) against the same activations as ONE
@@ -537,14 +548,23 @@ int launch_gemm_q4k_gated(const hipq_weight *wa, const hipq_weight *wm, const QA
   return HIPQ_OK;
 }
 
+int launch_split_sum(const float *partials, int parts, int M, int64_t N, float *C, int64_t ldc, hipStream_t s) {
+  const int64_t stride = split_stride(M, N);
+  const bool whole = !(N & 3) && !(ldc & 3) && !((uintptr_t)C & 15);
+  launch_kernel("split_sum_kernel", split_sum_kernel, dim3((unsigned)((stride / 4 + 255) / 256)), dim3(256), 0, s, partials, parts,
+                stride, M, (int)N, (int)(stride / M), C, ldc, whole);
+  HIPQ_HIP(hipGetLastError());
+  return HIPQ_OK;
+}
+
 static constexpr TileCost COST = {{0.f, 1.35f, 1.93f, 2.58f}, {0.f, 2.41f, 3.3f}};
 static TilePlan plan(const hipq_weight *w, int64_t M) {
-  return tile_plan(COST, M, w->N, w->K, w->dtype == HIPQ_Q4_K && w->gt_base && !(w->N & 3));
+  return tile_plan(COST, M, w->N, w->K, w->dtype == HIPQ_Q4_K && w->gt_base);
 }
 /* bytes of the partial products of a product in parts of K (0: whole) */
 size_t gemm_q4k_split_bytes(const hipq_weight *w, int64_t M) {
   const TilePlan t = plan(w, M);
-  return t.parts > 1 ? (size_t)t.parts * (size_t)M * (size_t)w->N * 4 : 0;
+  return t.parts > 1 ? (size_t)t.parts * (size_t)split_stride(M, w->N) * 4 : 0;
 }
 
 int launch_gemm_q4k(const hipq_weight *w, const QActTiled *qa, int M, float *C, int64_t ldc, hipStream_t s,
@@ -553,11 +573,11 @@ int launch_gemm_q4k(const hipq_weight *w, const QActTiled *qa, int M, float *C, 
     return fail(HIPQ_ERR_INVALID_ARGUMENT, "tiled activations do not match the matmul shape");
   const TilePlan tp = plan(w, M);
   const int parts = tp.parts;
-  if (partials && parts > 1 && !(ldc & 3) && !((uintptr_t)C & 15)) {
+  if (partials && parts > 1) {
     const int tm = tp.rows / 32;
     const int nsb = (int)(w->K / 256), per = (nsb + parts - 1) / parts;
     const int mtiles = (M + 32 * tm - 1) / (32 * tm), ntiles = (int)((w->N + BN - 1) / BN), ngroups = (ntiles + 7) / 8;
-    const int64_t stride = (int64_t)M * w->N;
+    const int64_t stride = split_stride(M, w->N);
     WView v = wview(w);
     v.qs = w->gt_qs;
     v.hdr = w->gt_hdr;
@@ -567,11 +587,7 @@ int launch_gemm_q4k(const hipq_weight *w, const QActTiled *qa, int M, float *C, 
     else
       hipq::launch_kernel("gemm_q4k_split_kernel<4>", gemm_q4k_split_kernel<4>, grid, dim3(NT), sizeof(Smem<4>), s, v, (const int8_t *)qa->qt, (const uint16_t *)qa->amin, (const float *)qa->dAt, M, mtiles, ntiles, per, (float *)partials, stride);
     HIPQ_HIP(hipGetLastError());
-    const int64_t quads = stride / 4;
-    hipq::launch_kernel("split_sum_kernel", split_sum_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s,
-                       (const float *)partials, (nsb + per - 1) / per, stride, M, (int)w->N, C, ldc);
-    HIPQ_HIP(hipGetLastError());
-    return HIPQ_OK;
+    return launch_split_sum((const float *)partials, (nsb + per - 1) / per, M, w->N, C, ldc, s);
   }
   /* 128-row tiles do a fifth more work per CU and time (the weight expansion is
    * shared by twice the rows) but only two workgroups fit a CU. */

@@ -301,28 +301,15 @@ __global__ __launch_bounds__(NT, TM == 2 ? 3 : 2) void gemm_q6k_kernel(WView w, 
 
 /* Few tiles (up to 128 rows against a matrix of a few thousand columns make under two hundred
  * workgroups, each walking all of K): blockIdx.y takes a part of K and writes its partial product to
- * part[y]; split_sum6_kernel adds the parts in ascending order. */
+ * part[y]; split_sum_kernel (launch_split_sum) adds the parts in ascending order. */
 template <int TM>
 __global__ __launch_bounds__(NT, TM == 2 ? 3 : 2) void gemm_q6k_split_kernel(WView w, const int8_t *__restrict__ qt,
                                                                const float *__restrict__ dAt, int M, int mtiles,
                                                                int ntiles, int sb_per_part, float *__restrict__ part,
                                                                int64_t part_stride) {
   const int sb0 = blockIdx.y * sb_per_part;
-  gemm_q6k_tile<TM, true>(w, qt, dAt, M, mtiles, ntiles, part + (int64_t)blockIdx.y * part_stride, w.N, sb0,
+  gemm_q6k_tile<TM, true>(w, qt, dAt, M, mtiles, ntiles, part + (int64_t)blockIdx.y * part_stride, (w.N + 3) & ~3, sb0,
                          min(sb_per_part, (w.K >> 8) - sb0));
-}
-
-__global__ __launch_bounds__(256) void split_sum6_kernel(const float *__restrict__ part, int parts, int64_t part_stride,
-                                                         int M, int N, float *__restrict__ C, int64_t ldc) {
-  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4; /* N % 4 == 0 */
-  if (i >= (int64_t)M * N) return;
-  const int m = (int)(i / N), n = (int)(i - (int64_t)m * N);
-  float4 v = *(const float4 *)(part + i);
-  for (int p = 1; p < parts; ++p) {
-    const float4 u = *(const float4 *)(part + p * part_stride + i);
-    v.x += u.x, v.y += u.y, v.z += u.z, v.w += u.w;
-  }
-  *(float4 *)(C + (int64_t)m * ldc + n) = v;
 }
 
 } // namespace
@@ -347,12 +334,12 @@ static int launch_tiles6(const hipq_weight *w, const QActTiled *qa, int M, float
 
 static constexpr TileCost COST = {{0.f, 1.68f, 2.43f, 3.2f}, {0.f, 2.56f, 3.62f}};
 static TilePlan plan(const hipq_weight *w, int64_t M) {
-  return tile_plan(COST, M, w->N, w->K, w->dtype == HIPQ_Q6_K && w->gt_base && !(w->N & 3));
+  return tile_plan(COST, M, w->N, w->K, w->dtype == HIPQ_Q6_K && w->gt_base);
 }
 /* bytes of the partial products of a product in parts of K (0: whole) */
 size_t gemm_q6k_split_bytes(const hipq_weight *w, int64_t M) {
   const TilePlan t = plan(w, M);
-  return t.parts > 1 ? (size_t)t.parts * (size_t)M * (size_t)w->N * 4 : 0;
+  return t.parts > 1 ? (size_t)t.parts * (size_t)split_stride(M, w->N) * 4 : 0;
 }
 
 int launch_gemm_q6k(const hipq_weight *w, const QActTiled *qa, int M, float *C, int64_t ldc, hipStream_t s,
@@ -362,11 +349,11 @@ int launch_gemm_q6k(const hipq_weight *w, const QActTiled *qa, int M, float *C, 
   if (!w->gt_base) return fail(HIPQ_ERR_INVALID_ARGUMENT, "the Q6_K prefill product needs the weight's tile copy");
   const TilePlan tp = plan(w, M);
   const int parts = tp.parts;
-  if (partials && parts > 1 && !(ldc & 3) && !((uintptr_t)C & 15)) {
+  if (partials && parts > 1) {
     const int tm = tp.rows / 32;
     const int nsb = (int)(w->K / 256), per = (nsb + parts - 1) / parts;
     const int mtiles = (M + 32 * tm - 1) / (32 * tm), ntiles = (int)((w->N + BN - 1) / BN), ngroups = (ntiles + 7) / 8;
-    const int64_t stride = (int64_t)M * w->N;
+    const int64_t stride = split_stride(M, w->N);
     WView v = wview(w);
     v.qs = w->gt_qs;
     v.qh = w->gt_qh;
@@ -377,10 +364,7 @@ int launch_gemm_q6k(const hipq_weight *w, const QActTiled *qa, int M, float *C, 
     else
       hipq::launch_kernel("gemm_q6k_split_kernel<4>", gemm_q6k_split_kernel<4>, grid, dim3(NT), sizeof(Smem6<4>), s, v, (const int8_t *)qa->qt, (const float *)qa->dAt, M, mtiles, ntiles, per, (float *)partials, stride);
     HIPQ_HIP(hipGetLastError());
-    hipq::launch_kernel("split_sum6_kernel", split_sum6_kernel, dim3((unsigned)((stride / 4 + 255) / 256)), dim3(256), 0, s,
-                       (const float *)partials, (nsb + per - 1) / per, stride, M, (int)w->N, C, ldc);
-    HIPQ_HIP(hipGetLastError());
-    return HIPQ_OK;
+    return launch_split_sum((const float *)partials, (nsb + per - 1) / per, M, w->N, C, ldc, s);
   }
   /* 128-row tiles halve the expansion per row (the larger part of this kernel's vector work):
    * 862 against 726 TOP/s at 2048 x 12288 x 4096, 835 against 729 at 512 x 151936 x 4096; two

@@ -346,7 +346,7 @@ def test_k_format_gemm_in_parts_of_k(hipq, cr, kind, m, n, k):
     the Q4_K and Q6_K prefill products are formed in parts of K that run side by side and are added in
     ascending order (nine super-blocks split 5 + 4, sixteen into four and eight parts). The first
     call, which makes the copy, and the following ones have the same bits, within 1e-4 of the
-    reference; a strided output keeps its padding; N not a multiple of four takes no parts."""
+    reference; a strided output keeps its padding; N not a multiple of four likewise."""
     import gpu_util as gu
     import torch
     blocks = _weights(cr, kind, n, k, seed=330 + m)
@@ -396,6 +396,33 @@ def test_k_format_gemm_in_parts_of_k_by_tile_height(hipq, cr, kind, m, n, k):
     w.destroy()
     assert (np.abs(got - ref).max(axis=1) / np.abs(ref).max(axis=1)).max() <= gu.TOL
     assert np.array_equal(got, first), "the first call differs from the second"
+
+
+@pytest.mark.parametrize("kind", ["q4_K", "q6_K"])
+@pytest.mark.parametrize("m,n,k,off", [(33, 1001, 4096, 0), (96, 2502, 2304, 0), (130, 1503, 6400, 0), (40, 1000, 4096, 1)])
+def test_k_format_gemm_in_parts_of_k_at_any_alignment(hipq, cr, kind, m, n, k, off):
+    """Rows of one to three values behind the last quad, and an output that does not start on sixteen bytes: the product
+    in parts has the bits of the one whose rows are padded to whole quads, and nothing is written beside its rows."""
+    import gpu_util as gu
+    import torch
+    few = _weights(cr, kind, 61, k, seed=350 + m)
+    pad = (n + 3) // 4 * 4
+    cols = np.random.RandomState(n).randint(0, 61, pad)
+    a = synth.normal(351 + m, (m, k))
+    ref = cr.gemm(cr.oracle(), kind, a, few, 61)[:, cols[:n]]
+    blocks = np.ascontiguousarray(few.reshape(61, -1)[cols])
+    even, w = capi.Weight(kind, pad, k, blocks), capi.Weight(kind, n, k, np.ascontiguousarray(blocks[:n]))
+    want = gu.gpu_matmul(even, a)[:, :n]
+    buf = torch.full((m * n + off + 5,), float("nan"), device="cuda")
+    capi.matmul(w, gu.dev(a), m, buf[off:off + m * n], stream=gu.stream())
+    torch.cuda.synchronize()
+    got = buf.cpu().numpy()
+    assert np.isnan(got[:off]).all() and np.isnan(got[off + m * n:]).all(), "the call wrote beside C"
+    got = got[off:off + m * n].reshape(m, n)
+    for x in (even, w):
+        x.destroy()
+    assert np.array_equal(got, want)
+    assert (np.abs(got - ref).max(axis=1) / np.abs(ref).max(axis=1)).max() <= gu.TOL
 
 
 def test_q4_K_gemm_tall_tiles(hipq, cr):
