@@ -68,10 +68,10 @@ template <int TM> struct Smem {
   static constexpr int ASTAGE = BM * 128; /* bytes of one 128-deep activation stage of the tile */
   int8_t a[3][ASTAGE];       /* ring of stages, each [row/32][step 4][lane 64][16] */
   _Float16 amin[2][BM * 16]; /* per super-block: per row 8 low parts, 8 high parts of bsum32_j */
-  float dA[2][BM];
+  float dA[2][TM == 1 ? 64 : BM]; /* a copy moves 64 scales */
 };
-static_assert(sizeof(Smem<2>) * 3 <= 160 * 1024 && sizeof(Smem<4>) * 2 <= 160 * 1024,
-              "three workgroups of 64 rows or two of 128 rows per CU must fit the 160 KB LDS");
+static_assert(sizeof(Smem<1>) * 4 <= 160 * 1024 && sizeof(Smem<2>) * 3 <= 160 * 1024 && sizeof(Smem<4>) * 2 <= 160 * 1024,
+              "four workgroups of 32 rows, three of 64 or two of 128 per CU must fit the 160 KB LDS");
 
 __device__ __forceinline__ uint32_t pk_scale(uint32_t x, uint32_t digit2) {
   const v2us r = __builtin_bit_cast(v2us, x) * __builtin_bit_cast(v2us, digit2);
@@ -134,14 +134,14 @@ template <int TM>
 __device__ __forceinline__ void dma_rows(const Src &sr, Smem<TM> &sm, int sb, int buf) {
   if (sr.wave < TM) /* uniform per wavefront */
     dma16(sr.amin, sr.lane * 16, (uint32_t)sb * (128 * 32) + sr.wave * 1024, (char *)sm.amin[buf] + sr.wave * 1024);
-  if (TM == 2 ? sr.wave == 2 : sr.wave < 2)
-    dma4(sr.dAt, sr.lane * 4, (uint32_t)sb * (128 * 4) + (TM == 2 ? 0 : sr.wave * 256),
-         sm.dA[buf] + (TM == 2 ? 0 : sr.wave * 64));
+  if (TM < 4 ? sr.wave == 2 : sr.wave < 2)
+    dma4(sr.dAt, (TM == 1 ? sr.lane & 31 : sr.lane) * 4, (uint32_t)sb * (128 * 4) + (TM < 4 ? 0 : sr.wave * 256),
+         sm.dA[buf] + (TM < 4 ? 0 : sr.wave * 64));
 }
 /* Loads a wavefront issues at least per stage (some wavefronts copy no per-row
  * data): what may stay in flight at the stage's barrier. First / second half. */
 template <int TM> struct InFlight {
-  static constexpr int FIRST = TM + (TM == 2 ? 0 : 1) + 2; /* copies of the ring, row data, two nibble loads */
+  static constexpr int FIRST = TM + (TM < 4 ? 0 : 1) + 2; /* copies of the ring, row data, two nibble loads */
   static constexpr int SECOND = TM + 3;                    /* copies of the ring, two nibble loads, the header */
 };
 
@@ -234,11 +234,11 @@ __device__ __forceinline__ void gemm_q4k_sums(const WView &w, const int8_t *__re
   const int i32 = lane & 31, g = lane >> 5;
 
   Src sr;
-  /* the quantizer tiles by 128 rows: a 64-row tile is half mt & 1 of quantizer tile mt / 2 */
-  const int qt128 = TM == 2 ? mt >> 1 : mt, hrow = TM == 2 ? mt & 1 : 0;
-  sr.qt = make_rsrc(qt + ((size_t)qt128 * (2 * nsb_all) + 2 * first) * QSTAGE + hrow * 8192, (uint32_t)(2 * nsb) * QSTAGE);
-  sr.amin = make_rsrc(amin + (((size_t)qt128 * nsb_all + first) * 128 + hrow * 64) * 16, (uint32_t)nsb * 128 * 32);
-  sr.dAt = make_rsrc(dAt + ((size_t)qt128 * nsb_all + first) * 128 + hrow * 64, (uint32_t)nsb * 128 * 4);
+  /* the quantizer tiles by 128 rows: a tile of 32 TM rows is part mt % (4 / TM) of quantizer tile mt / (4 / TM) */
+  const int qt128 = mt / (4 / TM), row0 = mt % (4 / TM) * Smem<TM>::BM;
+  sr.qt = make_rsrc(qt + ((size_t)qt128 * (2 * nsb_all) + 2 * first) * QSTAGE + row0 * 128, (uint32_t)(2 * nsb) * QSTAGE);
+  sr.amin = make_rsrc(amin + (((size_t)qt128 * nsb_all + first) * 128 + row0) * 16, (uint32_t)nsb * 128 * 32);
+  sr.dAt = make_rsrc(dAt + ((size_t)qt128 * nsb_all + first) * 128 + row0, (uint32_t)nsb * 128 * 4);
   const int n = min(ncol0 + i32, (int)w.N - 1);
   constexpr int HSTRIDE = TILES ? 32 : 1; /* uint4 between a column's consecutive super-block headers */
   if (TILES) {
@@ -332,7 +332,7 @@ __device__ __forceinline__ void gemm_q4k_tile(const WView &w, const int8_t *__re
 }
 
 template <int TM, bool TILES>
-__global__ __launch_bounds__(NT, TM == 2 ? 3 : 2) void gemm_q4k_kernel(WView w, const int8_t *__restrict__ qt,
+__global__ __launch_bounds__(NT, TM == 1 ? 4 : TM == 2 ? 3 : 2) void gemm_q4k_kernel(WView w, const int8_t *__restrict__ qt,
                                                          const uint16_t *__restrict__ amin,
                                                          const float *__restrict__ dAt, int M, int mtiles,
                                                          int ntiles, float *__restrict__ C, int64_t ldc) {
@@ -348,7 +348,7 @@ __global__ __launch_bounds__(NT, TM == 2 ? 3 : 2) void gemm_q4k_kernel(WView w, 
  * takes a part of K and writes its partial product to part[y]; split_sum_kernel adds the parts
  * in ascending order. */
 template <int TM>
-__global__ __launch_bounds__(NT, TM == 2 ? 3 : 2) void gemm_q4k_split_kernel(WView w, const int8_t *__restrict__ qt,
+__global__ __launch_bounds__(NT, TM == 1 ? 4 : TM == 2 ? 3 : 2) void gemm_q4k_split_kernel(WView w, const int8_t *__restrict__ qt,
                                                                const uint16_t *__restrict__ amin,
                                                                const float *__restrict__ dAt, int M, int mtiles,
                                                                int ntiles, int sb_per_part, float *__restrict__ part,
@@ -396,7 +396,7 @@ struct MultiQ4K {
   int tile_end[4]; /* running sum of the weights' column tiles */
 };
 template <int TM>
-__global__ __launch_bounds__(NT, TM == 2 ? 3 : 2) void gemm_q4k_multi_kernel(MultiQ4K mw, const int8_t *__restrict__ qt,
+__global__ __launch_bounds__(NT, TM == 1 ? 4 : TM == 2 ? 3 : 2) void gemm_q4k_multi_kernel(MultiQ4K mw, const int8_t *__restrict__ qt,
                                                                const uint16_t *__restrict__ amin,
                                                                const float *__restrict__ dAt, int M, int mtiles) {
   const int id = blockIdx.x;
@@ -416,7 +416,7 @@ __global__ __launch_bounds__(NT, TM == 2 ? 3 : 2) void gemm_q4k_multi_kernel(Mul
 }
 
 /* The gated pair of an MLP: out = swiglu(act sums) * mul sums. Two wavefronts of a workgroup take 32 columns each of the
- * one matrix, the other two the same columns of the other; at the end each keeps half of its row tiles and hands the other
+ * one matrix, the other two the same columns of the other; at the end each keeps half of its sums and hands the other
  * half over through LDS. The two products never reach memory: as products and a launch of the activation 1777 rows of
  * 12288 columns wrote and read 350 MB more (870 -> 827 us for a decoder layer of 4096 and 12288). */
 struct GatedQ4K {
@@ -426,7 +426,7 @@ struct GatedQ4K {
   int ntiles; /* workgroup columns of 64 */
 };
 template <int TM>
-__global__ __launch_bounds__(NT, TM == 2 ? 3 : 2) void gemm_q4k_gated_kernel(GatedQ4K p, const int8_t *__restrict__ qt,
+__global__ __launch_bounds__(NT, TM == 1 ? 4 : TM == 2 ? 3 : 2) void gemm_q4k_gated_kernel(GatedQ4K p, const int8_t *__restrict__ qt,
                                                                const uint16_t *__restrict__ amin,
                                                                const float *__restrict__ dAt, int M, int mtiles) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
@@ -442,30 +442,29 @@ __global__ __launch_bounds__(NT, TM == 2 ? 3 : 2) void gemm_q4k_gated_kernel(Gat
   float acc[TM][16];
   gemm_q4k_sums<TM, true>(w, qt, amin, dAt, mt, ncol0, acc);
 
-  constexpr int H = TM / 2; /* row tiles a wavefront hands over */
-  static_assert(4 * H * 4096 <= sizeof(Smem<TM>), "the halves fit the workgroup's LDS");
+  constexpr int H = TM * 8; /* sums of its TM * 16 that a lane hands over */
+  static_assert(4 * H * 256 <= sizeof(Smem<TM>), "the halves fit the workgroup's LDS");
   __syncthreads(); /* no wavefront reads or fills the ring any more */
-  float *mine = (float *)smem_raw + wave * (H * 1024), *other = (float *)smem_raw + (wave ^ 2) * (H * 1024);
+  float *mine = (float *)smem_raw + wave * (H * 64) + lane, *other = (float *)smem_raw + (wave ^ 2) * (H * 64) + lane;
+  auto sum = [&](int i) { return acc[i >> 4][i & 15]; };
 #pragma unroll
-  for (int t = 0; t < H; ++t)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) mine[t * 1024 + r * 64 + lane] = second ? acc[t][r] : acc[H + t][r];
+  for (int i = 0; i < H; ++i) mine[i * 64] = second ? sum(i) : sum(H + i);
   __syncthreads();
-  const int m0 = mt * 32 * TM + (second ? 32 * H : 0);
 #pragma unroll
-  for (int t = 0; t < H; ++t)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const float o = other[t * 1024 + r * 64 + lane];
-      const float h = second ? hipq_swiglu(o, acc[H + t][r]) : hipq_swiglu(acc[t][r], o);
-      const int m = m0 + t * 32 + acc_row(r, lane);
-      if (m < M && ncol < p.act.N) p.out[(int64_t)m * p.ldo + ncol] = h;
-    }
+  for (int i = 0; i < H; ++i) {
+    const float o = other[i * 64];
+    const float h = second ? hipq_swiglu(o, sum(H + i)) : hipq_swiglu(sum(i), o);
+    const int row = second ? (H + i) / 16 * 32 + acc_row((H + i) & 15, lane) : i / 16 * 32 + acc_row(i & 15, lane);
+    const int m = mt * 32 * TM + row;
+    if (m < M && ncol < p.act.N) p.out[(int64_t)m * p.ldo + ncol] = h;
+  }
 }
 
 } // namespace
 
 namespace hipq {
+
+static constexpr TileCost COST = {{0.f, 0.92f, 1.32f, 1.78f, 2.04f}, {0.f, 1.35f, 1.93f, 2.58f}, {0.f, 2.41f, 3.3f}};
 
 template <int TM>
 int launch_tiles(const hipq_weight *w, const QActTiled *qa, int M, float *C, int64_t ldc, hipStream_t s) {
@@ -477,7 +476,7 @@ int launch_tiles(const hipq_weight *w, const QActTiled *qa, int M, float *C, int
   if (w->gt_base) { /* the tile copy, where the weight has one */
     v.qs = w->gt_qs;
     v.hdr = w->gt_hdr;
-    hipq::launch_kernel(TM == 2 ? "gemm_q4k_kernel<2, true>" : "gemm_q4k_kernel<4, true>", gemm_q4k_kernel<TM, true>, dim3(grid), dim3(NT), sizeof(Smem<TM>), s, v, (const int8_t *)qa->qt,
+    hipq::launch_kernel(TM == 1 ? "gemm_q4k_kernel<1, true>" : TM == 2 ? "gemm_q4k_kernel<2, true>" : "gemm_q4k_kernel<4, true>", gemm_q4k_kernel<TM, true>, dim3(grid), dim3(NT), sizeof(Smem<TM>), s, v, (const int8_t *)qa->qt,
                   (const uint16_t *)qa->amin, (const float *)qa->dAt, M, mtiles, ntiles, C, ldc);
   } else
     hipq::launch_kernel(TM == 2 ? "gemm_q4k_kernel<2, false>" : "gemm_q4k_kernel<4, false>", gemm_q4k_kernel<TM, false>, dim3(grid), dim3(NT), sizeof(Smem<TM>), s, v, (const int8_t *)qa->qt,
@@ -510,7 +509,11 @@ int launch_gemm_q4k_multi(int count, const hipq_weight *const *w, const QActTile
   const int64_t rounds64 = (((int64_t)(M + 63) / 64) * tiles + 767) / 768;
   const int64_t rounds128 = (((int64_t)(M + 127) / 128) * tiles + 511) / 512;
   const int ngroups = (tiles + 7) / 8;
-  if (rounds128 * 6 < rounds64 * 5) {
+  if (tile_plan(COST, M, (int64_t)tiles * BN, qa->K, true, false).rows == 32) {
+    const int mtiles = (M + 31) / 32;
+    hipq::launch_kernel("gemm_q4k_multi_kernel<1>", gemm_q4k_multi_kernel<1>, dim3((unsigned)(mtiles * ngroups * 8)), dim3(NT), sizeof(Smem<1>), s, mw,
+                       (const int8_t *)qa->qt, (const uint16_t *)qa->amin, (const float *)qa->dAt, M, mtiles);
+  } else if (rounds128 * 6 < rounds64 * 5) {
     const int mtiles = (M + 127) / 128;
     hipq::launch_kernel("gemm_q4k_multi_kernel<4>", gemm_q4k_multi_kernel<4>, dim3((unsigned)(mtiles * ngroups * 8)), dim3(NT), sizeof(Smem<4>), s, mw,
                        (const int8_t *)qa->qt, (const uint16_t *)qa->amin, (const float *)qa->dAt, M, mtiles);
@@ -535,7 +538,11 @@ int launch_gemm_q4k_gated(const hipq_weight *wa, const hipq_weight *wm, const QA
   const int64_t rounds64 = (((int64_t)(M + 63) / 64) * p.ntiles + 767) / 768;
   const int64_t rounds128 = (((int64_t)(M + 127) / 128) * p.ntiles + 511) / 512;
   const int ngroups = (p.ntiles + 7) / 8;
-  if (rounds128 * 6 < rounds64 * 5) {
+  if (tile_plan(COST, M, (int64_t)p.ntiles * BN, wa->K, true, false).rows == 32) {
+    const int mtiles = (M + 31) / 32;
+    launch_kernel("gemm_q4k_gated_kernel<1>", gemm_q4k_gated_kernel<1>, dim3((unsigned)(mtiles * ngroups * 8)), dim3(NT),
+                  sizeof(Smem<1>), s, p, (const int8_t *)qa->qt, (const uint16_t *)qa->amin, (const float *)qa->dAt, M, mtiles);
+  } else if (rounds128 * 6 < rounds64 * 5) {
     const int mtiles = (M + 127) / 128;
     launch_kernel("gemm_q4k_gated_kernel<4>", gemm_q4k_gated_kernel<4>, dim3((unsigned)(mtiles * ngroups * 8)), dim3(NT),
                   sizeof(Smem<4>), s, p, (const int8_t *)qa->qt, (const uint16_t *)qa->amin, (const float *)qa->dAt, M, mtiles);
@@ -557,9 +564,8 @@ int launch_split_sum(const float *partials, int parts, int M, int64_t N, float *
   return HIPQ_OK;
 }
 
-static constexpr TileCost COST = {{0.f, 1.35f, 1.93f, 2.58f}, {0.f, 2.41f, 3.3f}};
 static TilePlan plan(const hipq_weight *w, int64_t M) {
-  return tile_plan(COST, M, w->N, w->K, w->dtype == HIPQ_Q4_K && w->gt_base);
+  return tile_plan(COST, M, w->N, w->K, w->gt_base, w->dtype == HIPQ_Q4_K && w->gt_base);
 }
 /* bytes of the partial products of a product in parts of K (0: whole) */
 size_t gemm_q4k_split_bytes(const hipq_weight *w, int64_t M) {
@@ -582,7 +588,9 @@ int launch_gemm_q4k(const hipq_weight *w, const QActTiled *qa, int M, float *C, 
     v.qs = w->gt_qs;
     v.hdr = w->gt_hdr;
     const dim3 grid((unsigned)(mtiles * ngroups * 8), (unsigned)((nsb + per - 1) / per));
-    if (tm == 2)
+    if (tm == 1)
+      hipq::launch_kernel("gemm_q4k_split_kernel<1>", gemm_q4k_split_kernel<1>, grid, dim3(NT), sizeof(Smem<1>), s, v, (const int8_t *)qa->qt, (const uint16_t *)qa->amin, (const float *)qa->dAt, M, mtiles, ntiles, per, (float *)partials, stride);
+    else if (tm == 2)
       hipq::launch_kernel("gemm_q4k_split_kernel<2>", gemm_q4k_split_kernel<2>, grid, dim3(NT), sizeof(Smem<2>), s, v, (const int8_t *)qa->qt, (const uint16_t *)qa->amin, (const float *)qa->dAt, M, mtiles, ntiles, per, (float *)partials, stride);
     else
       hipq::launch_kernel("gemm_q4k_split_kernel<4>", gemm_q4k_split_kernel<4>, grid, dim3(NT), sizeof(Smem<4>), s, v, (const int8_t *)qa->qt, (const uint16_t *)qa->amin, (const float *)qa->dAt, M, mtiles, ntiles, per, (float *)partials, stride);
@@ -591,8 +599,10 @@ int launch_gemm_q4k(const hipq_weight *w, const QActTiled *qa, int M, float *C, 
   }
   /* 128-row tiles do a fifth more work per CU and time (the weight expansion is
    * shared by twice the rows) but only two workgroups fit a CU. */
-  if (tile_plan(COST, M, w->N, w->K, false).rows == 128) return launch_tiles<4>(w, qa, M, C, ldc, s);
-  return launch_tiles<2>(w, qa, M, C, ldc, s);
+  const int rows = parts == 1 ? tp.rows : tile_plan(COST, M, w->N, w->K, w->gt_base, false).rows;
+  return rows == 32   ? launch_tiles<1>(w, qa, M, C, ldc, s)
+         : rows == 64 ? launch_tiles<2>(w, qa, M, C, ldc, s)
+                      : launch_tiles<4>(w, qa, M, C, ldc, s);
 }
 
 } // namespace hipq

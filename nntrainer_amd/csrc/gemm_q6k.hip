@@ -46,10 +46,10 @@ template <int TM> struct Smem6 {
   static constexpr int BM = 32 * TM;
   static constexpr int ASTAGE = BM * 128;
   int8_t a[3][ASTAGE]; /* ring of stages, each [row/32][step 4][lane 64][16] */
-  float dA[2][BM];
+  float dA[2][TM == 1 ? 64 : BM]; /* a copy moves 64 scales */
 };
-static_assert(sizeof(Smem6<2>) * 3 <= 160 * 1024 && sizeof(Smem6<4>) * 2 <= 160 * 1024,
-              "three workgroups of 64 rows or two of 128 rows per CU must fit the 160 KB LDS");
+static_assert(sizeof(Smem6<1>) * 4 <= 160 * 1024 && sizeof(Smem6<2>) * 3 <= 160 * 1024 && sizeof(Smem6<4>) * 2 <= 160 * 1024,
+              "four workgroups of 32 rows, three of 64 or two of 128 per CU must fit the 160 KB LDS");
 
 __device__ __forceinline__ rsrc_t make_rsrc(const void *p, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, (int)bytes, 0x00020000);
@@ -97,8 +97,8 @@ __device__ __forceinline__ void dma_a(const Src6 &sr, Smem6<TM> &sm, int stage, 
 /* the rows' scales of a super-block: wavefront 0 (and 1 for 128 rows) copies 64 of them */
 template <int TM>
 __device__ __forceinline__ void dma_rows(const Src6 &sr, Smem6<TM> &sm, int sb, int buf) {
-  if (sr.wave < TM / 2) /* uniform per wavefront */
-    dma4(sr.dAt, sr.lane * 4, (uint32_t)sb * (128 * 4) + sr.wave * 256, sm.dA[buf] + sr.wave * 64);
+  if (sr.wave < (TM + 1) / 2) /* uniform per wavefront */
+    dma4(sr.dAt, (TM == 1 ? sr.lane & 31 : sr.lane) * 4, (uint32_t)sb * (128 * 4) + sr.wave * 256, sm.dA[buf] + sr.wave * 64);
 }
 /* Loads a wavefront issues at least per stage (wavefronts 2 and 3 copy no scales): what
  * may stay in flight at the stage's barrier. */
@@ -216,10 +216,10 @@ __device__ __forceinline__ void gemm_q6k_tile(const WView &w, const int8_t *__re
   const int i32 = lane & 31;
 
   Src6 sr;
-  /* the quantizer tiles by 128 rows: a 64-row tile is half mt & 1 of quantizer tile mt / 2 */
-  const int qt128 = TM == 2 ? mt >> 1 : mt, hrow = TM == 2 ? mt & 1 : 0;
-  sr.qt = make_rsrc(qt + ((size_t)qt128 * (2 * nsb_all) + 2 * first) * QSTAGE + hrow * 8192, (uint32_t)(2 * nsb) * QSTAGE);
-  sr.dAt = make_rsrc(dAt + ((size_t)qt128 * nsb_all + first) * 128 + hrow * 64, (uint32_t)nsb * 128 * 4);
+  /* the quantizer tiles by 128 rows: a tile of 32 TM rows is part mt % (4 / TM) of quantizer tile mt / (4 / TM) */
+  const int qt128 = mt / (4 / TM), row0 = mt % (4 / TM) * BM;
+  sr.qt = make_rsrc(qt + ((size_t)qt128 * (2 * nsb_all) + 2 * first) * QSTAGE + row0 * 128, (uint32_t)(2 * nsb) * QSTAGE);
+  sr.dAt = make_rsrc(dAt + ((size_t)qt128 * nsb_all + first) * 128 + row0, (uint32_t)nsb * 128 * 4);
   /* the copy pads N to 32 rows: a wavefront whose columns start below N has its tile */
   const size_t wt = (size_t)(min(n0 + wave * 32, (int)w.N - 1) >> 5);
   sr.wq = make_rsrc(w.qs + (wt * nsb_all + first) * 4096, (uint32_t)nsb * 4096);
@@ -293,7 +293,7 @@ __device__ __forceinline__ void gemm_q6k_tile(const WView &w, const int8_t *__re
 }
 
 template <int TM>
-__global__ __launch_bounds__(NT, TM == 2 ? 3 : 2) void gemm_q6k_kernel(WView w, const int8_t *__restrict__ qt,
+__global__ __launch_bounds__(NT, TM == 1 ? 4 : TM == 2 ? 3 : 2) void gemm_q6k_kernel(WView w, const int8_t *__restrict__ qt,
                                                                        const float *__restrict__ dAt, int M, int mtiles,
                                                                        int ntiles, float *__restrict__ C, int64_t ldc) {
   gemm_q6k_tile<TM, false>(w, qt, dAt, M, mtiles, ntiles, C, ldc, 0, 0);
@@ -303,7 +303,7 @@ __global__ __launch_bounds__(NT, TM == 2 ? 3 : 2) void gemm_q6k_kernel(WView w, 
  * workgroups, each walking all of K): blockIdx.y takes a part of K and writes its partial product to
  * part[y]; split_sum_kernel (launch_split_sum) adds the parts in ascending order. */
 template <int TM>
-__global__ __launch_bounds__(NT, TM == 2 ? 3 : 2) void gemm_q6k_split_kernel(WView w, const int8_t *__restrict__ qt,
+__global__ __launch_bounds__(NT, TM == 1 ? 4 : TM == 2 ? 3 : 2) void gemm_q6k_split_kernel(WView w, const int8_t *__restrict__ qt,
                                                                const float *__restrict__ dAt, int M, int mtiles,
                                                                int ntiles, int sb_per_part, float *__restrict__ part,
                                                                int64_t part_stride) {
@@ -326,15 +326,15 @@ static int launch_tiles6(const hipq_weight *w, const QActTiled *qa, int M, float
   v.qs = w->gt_qs;
   v.qh = w->gt_qh;
   v.hdr = w->gt_hdr;
-  hipq::launch_kernel(TM == 2 ? "gemm_q6k_kernel<2>" : "gemm_q6k_kernel<4>", gemm_q6k_kernel<TM>, dim3(grid), dim3(NT), sizeof(Smem6<TM>), s, v, (const int8_t *)qa->qt,
+  hipq::launch_kernel(TM == 1 ? "gemm_q6k_kernel<1>" : TM == 2 ? "gemm_q6k_kernel<2>" : "gemm_q6k_kernel<4>", gemm_q6k_kernel<TM>, dim3(grid), dim3(NT), sizeof(Smem6<TM>), s, v, (const int8_t *)qa->qt,
                 (const float *)qa->dAt, M, mtiles, ntiles, C, ldc);
   HIPQ_HIP(hipGetLastError());
   return HIPQ_OK;
 }
 
-static constexpr TileCost COST = {{0.f, 1.68f, 2.43f, 3.2f}, {0.f, 2.56f, 3.62f}};
+static constexpr TileCost COST = {{0.f, 1.32f, 2.01f, 2.72f, 3.2f}, {0.f, 1.68f, 2.43f, 3.2f}, {0.f, 2.56f, 3.62f}};
 static TilePlan plan(const hipq_weight *w, int64_t M) {
-  return tile_plan(COST, M, w->N, w->K, w->dtype == HIPQ_Q6_K && w->gt_base);
+  return tile_plan(COST, M, w->N, w->K, w->gt_base, w->dtype == HIPQ_Q6_K && w->gt_base);
 }
 /* bytes of the partial products of a product in parts of K (0: whole) */
 size_t gemm_q6k_split_bytes(const hipq_weight *w, int64_t M) {
@@ -359,7 +359,9 @@ int launch_gemm_q6k(const hipq_weight *w, const QActTiled *qa, int M, float *C, 
     v.qh = w->gt_qh;
     v.hdr = w->gt_hdr;
     const dim3 grid((unsigned)(mtiles * ngroups * 8), (unsigned)((nsb + per - 1) / per));
-    if (tm == 2)
+    if (tm == 1)
+      hipq::launch_kernel("gemm_q6k_split_kernel<1>", gemm_q6k_split_kernel<1>, grid, dim3(NT), sizeof(Smem6<1>), s, v, (const int8_t *)qa->qt, (const float *)qa->dAt, M, mtiles, ntiles, per, (float *)partials, stride);
+    else if (tm == 2)
       hipq::launch_kernel("gemm_q6k_split_kernel<2>", gemm_q6k_split_kernel<2>, grid, dim3(NT), sizeof(Smem6<2>), s, v, (const int8_t *)qa->qt, (const float *)qa->dAt, M, mtiles, ntiles, per, (float *)partials, stride);
     else
       hipq::launch_kernel("gemm_q6k_split_kernel<4>", gemm_q6k_split_kernel<4>, grid, dim3(NT), sizeof(Smem6<4>), s, v, (const int8_t *)qa->qt, (const float *)qa->dAt, M, mtiles, ntiles, per, (float *)partials, stride);
@@ -369,8 +371,10 @@ int launch_gemm_q6k(const hipq_weight *w, const QActTiled *qa, int M, float *C, 
   /* 128-row tiles halve the expansion per row (the larger part of this kernel's vector work):
    * 862 against 726 TOP/s at 2048 x 12288 x 4096, 835 against 729 at 512 x 151936 x 4096; two
    * of their workgroups fit a CU instead of three. */
-  if (tile_plan(COST, M, w->N, w->K, false).rows == 128) return launch_tiles6<4>(w, qa, M, C, ldc, s);
-  return launch_tiles6<2>(w, qa, M, C, ldc, s);
+  const int rows = parts == 1 ? tp.rows : tile_plan(COST, M, w->N, w->K, true, false).rows;
+  return rows == 32   ? launch_tiles6<1>(w, qa, M, C, ldc, s)
+         : rows == 64 ? launch_tiles6<2>(w, qa, M, C, ldc, s)
+                      : launch_tiles6<4>(w, qa, M, C, ldc, s);
 }
 
 } // namespace hipq

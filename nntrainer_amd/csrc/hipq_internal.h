@@ -293,34 +293,38 @@ int launch_gemm_f6_gated(const hipq_weight *wa, const hipq_weight *wm, const QAc
                          hipStream_t s, QActF6 *qh = nullptr);
 int launch_gemm_q4k_gated(const hipq_weight *wa, const hipq_weight *wm, const QActTiled *qa, int M, float *out, int64_t ldo,
                           hipStream_t s);
-/* The tile height (64 or 128 rows) of a prefill product of Q4_K or Q6_K and the parts of K its tiles are formed in (1:
+/* The tile height (32, 64 or 128 rows) of a prefill product of Q4_K or Q6_K and the parts of K its tiles are formed in (1:
  * whole), by what each choice should take. Per super-block a CU's tiles of 64 rows x 128 columns take c64[n] us with n of
- * them on it (three fit), those of 128 rows c128[n] (two fit); a CU has the launch's tiles in rounds of as many as fit;
+ * them on it (three fit), those of 32 rows c32[n] (four fit), those of 128 c128[n] (two fit); a CU has the launch's tiles in rounds of as many as fit;
  * parts write and read their sums (0.26 us a megabyte, and a launch of 1 us). The figures are fitted (rms 5 %) to 99 sizes
  * a format, 65 to 1000 rows of 1024 x 4096 to 4096 x 12288, each with both heights and 1 to 8 parts: by them the products
  * take 1.7 % (Q4_K) and 2.9 % (Q6_K) less than by the rule before (parts up to 192 tiles of 64 rows), 1 % (Q4_K) and 2 % more
  * than the fastest choice; where that rule had left the chip unevenly filled, 400 rows of 4096 x 12288, 84 -> 69 and 100 ->
- * 72 us. Parts change the order of a sum, so they have to gain 1.5 us. `split`: parts are possible. */
+ * 72 us. Parts change the order of a sum, so they have to gain 1.5 us. Tiles of 32 rows walk a super-block in 0.92 / 1.32 us
+ * where those of 64 take 1.35 / 1.68, and are the faster ones up to about 200 rows wherever the chip is not full otherwise:
+ * over 89 + 63 sizes of 17 to 320 rows (700 x 1536 to 40000 x 2048) 10 % less a call, 30 % at the smallest (us, Q6_K, 64 rows
+ * -> 32: 32 rows of 1000 x 4096 16.9 -> 14.9, of 16822 x 3328 26.6 -> 22.5, 96 of 6000 x 1024 14.7 -> 12.3; Q4_K 160 of 12288 x
+ * 4096 39.2 -> 32.7). `copy`: the weight has its tile copy, which they read; `split`: parts are possible. */
 struct TileCost {
-  float c64[4], c128[3];
+  float c32[5], c64[4], c128[3];
 };
 struct TilePlan {
   int rows, parts;
 };
-inline TilePlan tile_plan(const TileCost &c, int64_t M, int64_t N, int64_t K, bool split) {
+inline TilePlan tile_plan(const TileCost &c, int64_t M, int64_t N, int64_t K, bool copy, bool split) {
   const int64_t nsb = K / 256, nt = (N + 127) / 128;
   TilePlan best{64, 1};
   double least = 1e30;
-  for (int tall = 0; tall < (M > 64 ? 2 : 1); ++tall) {
-    const int64_t mt = (M + (tall ? 127 : 63)) / (tall ? 128 : 64);
-    const int fit = tall ? 2 : 3;
-    const float *t = tall ? c.c128 : c.c64;
+  for (int h = copy ? 32 : 64; h <= (M > 64 ? 128 : 64); h *= 2) {
+    const int64_t mt = (M + h - 1) / h;
+    const int fit = h == 32 ? 4 : h == 64 ? 3 : 2;
+    const float *t = h == 32 ? c.c32 : h == 64 ? c.c64 : c.c128;
     for (int p = 1; p <= (split ? 8 : 1); ++p) {
-      if (p > 1 && (nsb < 4 * p || p * M * N * 4 > ((int64_t)64 << 20))) break;
+      if (p > 1 && (nsb < 3 * p || p * M * N * 4 > ((int64_t)64 << 20))) break;
       const int64_t per = (nsb + p - 1) / p, parts = (nsb + per - 1) / per, a_cu = (mt * nt * parts + 255) / 256;
       double us = (double)per * ((double)(a_cu / fit) * t[fit] + t[a_cu % fit]);
       if (parts > 1) us += 1.5 + 1.0 + 0.26e-6 * 4 * (double)((parts + 1) * M * N);
-      if (us < least) least = us, best = TilePlan{tall ? 128 : 64, (int)parts};
+      if (us < least) least = us, best = TilePlan{h, (int)parts};
     }
   }
   return best;

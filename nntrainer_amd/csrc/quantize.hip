@@ -254,7 +254,10 @@ int launch_quantize_q8_K_tiled(const float *A, int64_t M, int64_t K, int64_t lda
   if (((uintptr_t)A & 15) || (lda & 3))
     return fail(HIPQ_ERR_INVALID_ARGUMENT, "activation rows must be 16-byte aligned");
   const int nsb = (int)(K / 256);
-  const int64_t units = (int64_t)qa->mtiles * 32 * nsb; /* (row quad, super-block) pairs, padding rows included */
+  /* (row quad, super-block) pairs, padding rows included: as many as the tiles can read, which for a product of up to 32 or
+   * 64 rows are not taller than that */
+  const int64_t rows = M <= 32 ? 32 : M <= 64 ? 64 : (int64_t)qa->mtiles * 128;
+  const int64_t units = rows / 4 * nsb;
   const unsigned grid = (unsigned)((units + 3) / 4);
   hipq::launch_kernel("quantize_q8_K_tiled_kernel", quantize_q8_K_tiled_kernel, dim3(grid), dim3(256), 0, s, A, M, units, (int)nsb, lda, mat_rows, qa->qt,
                 qa->dAt, qa->amin);

@@ -425,6 +425,34 @@ def test_k_format_gemm_in_parts_of_k_at_any_alignment(hipq, cr, kind, m, n, k, o
     assert (np.abs(got - ref).max(axis=1) / np.abs(ref).max(axis=1)).max() <= gu.TOL
 
 
+@pytest.mark.parametrize("kind", ["q4_K", "q6_K"])
+@pytest.mark.parametrize("m", [17, 32, 33, 97, 130])
+def test_k_format_gemm_of_32_row_tiles(hipq, cr, kind, m):
+    """Tiles of 32 rows: every quarter of the quantizer's 128-row tiles, an odd number of super-blocks, columns past the last
+    tile; one product, three weights in a launch and the gated pair."""
+    import gpu_util as gu
+    import torch
+    k, ns = 768, (1100, 70, 33)
+    blocks = [_weights(cr, kind, n, k, seed=360 + n) for n in ns]
+    a = synth.normal(361 + m, (m, k))
+    refs = [cr.gemm(cr.oracle(), kind, a, b, n) for b, n in zip(blocks, ns)]
+    ws = [capi.Weight(kind, n, k, b) for b, n in zip(blocks, ns)]
+    mul = capi.Weight(kind, ns[0], k, np.ascontiguousarray(blocks[0].reshape(ns[0], -1)[::-1]))
+    try:
+        outs = [torch.full((m, n), float("nan"), device="cuda") for n in ns]
+        capi.matmul_multi(ws, gu.dev(a), m, outs, stream=gu.stream())
+        h = torch.full((m, ns[0]), float("nan"), device="cuda")
+        capi.mlp_swiglu(ws[0], mul, gu.dev(a), m, h, stream=gu.stream())
+        torch.cuda.synchronize()
+        for got, ref in [(gu.gpu_matmul(ws[0], a), refs[0])] + [(o.cpu().numpy(), r) for o, r in zip(outs, refs)]:
+            assert not np.isnan(got).any()
+            assert (np.abs(got - ref).max(axis=1) / np.abs(ref).max(axis=1)).max() <= gu.TOL
+        assert gu.rel_err(h.cpu().numpy(), cr.swiglu(refs[0], refs[0][:, ::-1])) <= gu.TOL
+    finally:
+        for w in ws + [mul]:
+            w.destroy()
+
+
 def test_q4_K_gemm_tall_tiles(hipq, cr):
     """A shape for which the Q4_K GEMM picks its 128-row tiles (two rounds of 64-row
     tiles against one of 128-row tiles), with M not a multiple of the tile height."""
