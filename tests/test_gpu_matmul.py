@@ -453,6 +453,31 @@ def test_k_format_gemm_of_32_row_tiles(hipq, cr, kind, m):
             w.destroy()
 
 
+@pytest.mark.parametrize("m,n,k", [(40, 8192, 512), (18, 12100, 1024), (24, 1100, 8192)])
+def test_q4_K_few_rows_or_tiles(hipq, cr, m, n, k):
+    """Beyond sixteen rows the faster of the few-rows kernel and the prefill GEMM, here the GEMM: one product and the first of
+    two weights within 1e-4 of every row's own maximum. Rows that are products of their own keep the reference's bits."""
+    import gpu_util as gu
+    import torch
+    few = _weights(cr, "q4_K", 61, k, seed=370 + m)
+    cols = np.random.RandomState(n).randint(0, 61, n)
+    a = synth.normal(371 + m, (m, k))
+    ref = cr.gemm(cr.oracle(), "q4_K", a, few, 61)[:, cols]
+    alone = np.concatenate([cr.gemm(cr.oracle(), "q4_K", a[i:i + 1], few, 61) for i in range(m)])[:, cols]
+    w = capi.Weight("q4_K", n, k, np.ascontiguousarray(few.reshape(61, -1)[cols]))
+    v = capi.Weight("q4_K", 61, k, few)
+    outs = [torch.full((m, x), float("nan"), device="cuda") for x in (n, 61, n)]
+    capi.matmul_multi([w, v], gu.dev(a), m, outs[:2], stream=gu.stream())
+    capi.matmul_each_row(w, gu.dev(a), m, outs[2], stream=gu.stream())
+    torch.cuda.synchronize()
+    got = [o.cpu().numpy() for o in outs] + [gu.gpu_matmul(w, a)]
+    w.destroy(), v.destroy()
+    for x in (got[0], got[3]):
+        assert (np.abs(x - ref).max(axis=1) / np.abs(ref).max(axis=1)).max() <= gu.TOL
+    assert gu.rel_err(got[1], cr.gemm(cr.oracle(), "q4_K", a, few, 61)) <= gu.TOL
+    assert np.array_equal(got[2].view(np.uint32), alone.astype(np.float32).view(np.uint32))
+
+
 def test_q4_K_gemm_tall_tiles(hipq, cr):
     """A shape for which the Q4_K GEMM picks its 128-row tiles (two rounds of 64-row
     tiles against one of 128-row tiles), with M not a multiple of the tile height."""
