@@ -60,6 +60,8 @@ struct MoeBufs {
 
 size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
 
+bool pairs_apart(const hipq_moe_desc &d);
+
 size_t carve(const hipq_moe_desc &d, int is_k, uint8_t *base, MoeBufs *b) {
   const size_t T = d.tokens, H = d.hidden, I = d.intermediate, E = d.experts, P = T * d.topk;
   size_t o = 0;
@@ -69,7 +71,7 @@ size_t carve(const hipq_moe_desc &d, int is_k, uint8_t *base, MoeBufs *b) {
     return base ? base + at : (uint8_t *)nullptr;
   };
   uint8_t *p;
-  p = take(T * (T <= MOE_FEW ? ROUTER_PARTS : 1) * E * 4); /* few tokens: the logits' partial sums */
+  p = take(T * (T == 1 || pairs_apart(d) ? ROUTER_PARTS : 1) * E * 4); /* there the logits' partial sums */
   if (b) b->logits = (float *)p;
   p = take(P * 4);
   if (b) b->idx = (int32_t *)p;
