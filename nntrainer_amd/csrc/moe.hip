@@ -631,6 +631,24 @@ __device__ __forceinline__ void sort_pairs(const int32_t *idx, int P, int E, int
   }
 }
 
+/* The rows of x quantized for the matrix-core expert kernels, in the same launch as the
+ * sort or the routing (neither needs the other): the first workgroups sort or route (or
+ * both, with 1024 threads), the others quantize one super-block per wavefront. */
+struct XQuant {
+  const float *x;
+  int64_t n_sb; /* T * H / 256 */
+  int nsb;
+  int8_t *q;
+  float *d;
+  uint16_t *amin;
+};
+__device__ __forceinline__ void quantize_x(const XQuant &xq, int T, int block) {
+  const int64_t sb = (int64_t)block * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  if (sb >= xq.n_sb) return; /* uniform per wavefront */
+  hipq_quantize_q8_K_wave<Q8K_ROWMMA>(xq.x, T, sb, xq.nsb, (int64_t)xq.nsb * 256, 0, xq.q, xq.d, nullptr, nullptr,
+                                      xq.amin, nullptr, nullptr);
+}
+
 /* Up to 16384 pairs behind the routing launch, which has written every token's pairs in ascending expert id to tok_slots.
  * All of a thread's pairs are loaded before the first is counted, the count hands out the pair's place in its expert, and
  * the slots of the pairs pass through LDS to the places tok_slots names (in place). 8000 pairs: 15.5 -> 8.5 us (a second pass
@@ -638,7 +656,12 @@ __device__ __forceinline__ void sort_pairs(const int32_t *idx, int P, int E, int
 constexpr int SORT_MANY = 16384;
 __global__ __launch_bounds__(1024) void sort_pairs_kernel(const int32_t *__restrict__ idx, int P, int E,
                                                           int *__restrict__ offsets, int *__restrict__ slot_pair,
-                                                          int *tok_slots, int chunk, int *__restrict__ items) {
+                                                          int *tok_slots, int chunk, int *__restrict__ items, XQuant xq,
+                                                          int T) {
+  if (blockIdx.x > 0) {
+    quantize_x(xq, T, blockIdx.x - 1);
+    return;
+  }
   constexpr int NP = SORT_MANY / 1024;
   __shared__ int cnt[1024];
   __shared__ int off[1024];
@@ -685,25 +708,6 @@ __global__ __launch_bounds__(1024) void route_sort_kernel(const float *__restric
   if (t < T) route_token<MAXV>(logits, t, E, topk, renorm, idx, wgt);
   __syncthreads(); /* orders the routing's stores before the sort's loads */
   sort_pairs(idx, T * topk, E, topk, offsets, slot_pair, tok_slots, chunk, items);
-}
-
-/* The rows of x quantized for the matrix-core expert kernels, in the same launch as
- * the routing (neither needs the other): workgroups 0 .. route_blocks - 1 route (or
- * route and sort, with 1024 threads), the others quantize one super-block per
- * wavefront. */
-struct XQuant {
-  const float *x;
-  int64_t n_sb; /* T * H / 256 */
-  int nsb;
-  int8_t *q;
-  float *d;
-  uint16_t *amin;
-};
-__device__ __forceinline__ void quantize_x(const XQuant &xq, int T, int block) {
-  const int64_t sb = (int64_t)block * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (sb >= xq.n_sb) return; /* uniform per wavefront */
-  hipq_quantize_q8_K_wave<Q8K_ROWMMA>(xq.x, T, sb, xq.nsb, (int64_t)xq.nsb * 256, 0, xq.q, xq.d, nullptr, nullptr,
-                                      xq.amin, nullptr, nullptr);
 }
 
 template <int MAXV>
@@ -2452,9 +2456,9 @@ int launch_moe(const MoeArgs *a, void *workspace, size_t workspace_bytes, const 
     const int rblocks = (T + 3) / 4;
     const unsigned qblocks = mma ? (unsigned)((xqa.n_sb + 3) / 4) : 0;
     auto launch = [&](auto fused, auto plain) {
-      if (mma)
+      if (mma && !one_sort)
         hipq::launch_kernel("fused", fused, dim3(rblocks + qblocks), dim3(256), 0, s, logits, T, E, d.topk, d.renormalize,
-                           idx, wgt, rblocks, xqa, self || one_sort ? b.tok_slots : (int *)nullptr);
+                           idx, wgt, rblocks, xqa, self ? b.tok_slots : (int *)nullptr);
       else
         hipq::launch_kernel("plain", plain, dim3(rblocks), dim3(256), 0, s, logits, T, E, d.topk, d.renormalize, idx, wgt,
                             one_sort ? b.tok_slots : (int *)nullptr);
@@ -2467,8 +2471,10 @@ int launch_moe(const MoeArgs *a, void *workspace, size_t workspace_bytes, const 
   if ((T <= 16 && E <= 1024) || self || one_token) {
     /* routed and sorted above, or no sort needed */
   } else if (one_sort) {
-    hipq::launch_kernel("sort_pairs_kernel", sort_pairs_kernel, dim3(1), dim3(1024), 0, s, idx, P, E, b.offsets,
-                       b.slot_pair, b.tok_slots, chunk, b.items);
+    /* the other CUs quantize x beside the one that sorts */
+    const unsigned qblocks = mma ? (unsigned)((xqa.n_sb + 15) / 16) : 0;
+    hipq::launch_kernel("sort_pairs_kernel", sort_pairs_kernel, dim3(1 + qblocks), dim3(1024), 0, s, idx, P, E, b.offsets,
+                       b.slot_pair, b.tok_slots, chunk, b.items, xqa, T);
   } else {
     hipq::launch_kernel("fill_int_kernel", fill_int_kernel, dim3((E + 255) / 256), dim3(256), 0, s, b.counts, E, 0);
     hipq::launch_kernel("count_kernel", count_kernel, dim3((P + 255) / 256), dim3(256), 0, s, idx, P, b.counts);
