@@ -73,6 +73,21 @@ __global__ __launch_bounds__(256) void quantize_q8_K_kernel(
                                 ql_out, qh_out);
 }
 
+/* The row form of the matrix-core kernels where every row follows the row quantizer: sixteen values a lane, four super-blocks
+ * a wavefront, so that the two divisions and the reductions serve four of them (8000 rows of 768: 10.2 -> 6.8 us). */
+__global__ __launch_bounds__(256) void quantize_q8_K_rowmma16_kernel(const float *__restrict__ A, uint32_t groups, uint32_t row_groups,
+                                                                     int64_t lda, int8_t *__restrict__ q_out,
+                                                                     float *__restrict__ d_out, int16_t *__restrict__ amin_out) {
+  const uint32_t t = blockIdx.x * 256 + threadIdx.x;
+  const uint32_t at = t < groups ? t : groups - 16 + (t & 15); /* past the end: the last super-block again, not stored */
+  const uint32_t m = at / row_groups;
+  const float *src = A + (int64_t)m * lda + (int64_t)(at - m * row_groups) * 16;
+  float4 x[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) x[i] = *(const float4 *)(src + 4 * i);
+  hipq_quantize_q8_K_values16<Q8K_ROWMMA>(x, (int)at, t < groups, q_out, d_out, amin_out, nullptr, nullptr);
+}
+
 /* The tiled form for the Q4_K prefill GEMM. A wavefront takes super-block b of four
  * consecutive rows (a 4-aligned quad, so that all four follow the same quantizer's
  * semantics): sixteen lanes per row, sixteen values per lane in four 16-byte loads, lane
@@ -240,6 +255,12 @@ int launch_quantize_q8_K_rowmma(const float *A, int64_t M, int64_t K, int64_t ld
     return fail(HIPQ_ERR_INVALID_ARGUMENT, "activation rows must be 16-byte aligned");
   const int nsb = (int)(K / 256);
   const int64_t total = M * nsb;
+  if (mat_rows == 0 && total < (int64_t(1) << 26)) { /* 32-bit places */
+    hipq::launch_kernel("quantize_q8_K_rowmma16_kernel", quantize_q8_K_rowmma16_kernel, dim3((unsigned)((total + 15) / 16)), dim3(256),
+                        0, s, A, (uint32_t)(total * 16), (uint32_t)(nsb * 16), lda, qa->q, qa->d, (int16_t *)qa->bsum);
+    HIPQ_HIP(hipGetLastError());
+    return HIPQ_OK;
+  }
   const unsigned grid = (unsigned)((total + 3) / 4);
   hipq::launch_kernel("quantize_q8_K_kernel<Q8K_ROWMMA>", quantize_q8_K_kernel<Q8K_ROWMMA>, dim3(grid), dim3(256), 0, s, A, M, total, nsb, lda,
                      mat_rows, qa->q, qa->d, nullptr, nullptr, (uint16_t *)qa->bsum, nullptr, nullptr);

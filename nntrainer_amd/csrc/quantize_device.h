@@ -188,7 +188,7 @@ __device__ __forceinline__ void hipq_quantize_q8_K_values(
 /* The row quantizer with sixteen consecutive values of the super-block in the calling lane, the super-block's sixteen
  * lanes consecutive, for one row quantized by a few wavefronts that wait for it: the reductions stay inside a row of
  * lanes, the two divisions serve four super-blocks a wavefront, and a 16-value group's sum needs no exchange. MODE
- * Q8K_DIGITS or Q8K_BYTES; `at` is the lane's place in the row (values 16 at .. 16 at + 15), stored where `store`.
+ * Q8K_DIGITS, Q8K_BYTES or Q8K_ROWMMA (the sums' fp16 parts then go to bsum_out); `at` is the lane's place in the row (values 16 at .. 16 at + 15), stored where `store`.
  *
  * The scale has the sign of the first value of largest magnitude: that of the largest value or of the smallest,
  * whichever is larger in magnitude, and only where both are the same has the first to be looked for. No value leaves
@@ -200,7 +200,7 @@ __device__ __forceinline__ void hipq_quantize_q8_K_values16(const float4 (&x)[4]
                                                             int16_t *__restrict__ bsum_out,
                                                             uint8_t *__restrict__ ql_out,
                                                             uint8_t *__restrict__ qh_out) {
-  static_assert(MODE == Q8K_DIGITS || MODE == Q8K_BYTES, "the forms that the GEMV kernels read");
+  static_assert(MODE == Q8K_DIGITS || MODE == Q8K_BYTES || MODE == Q8K_ROWMMA, "the forms of one row's quantizer");
   const float v[16] = {x[0].x, x[0].y, x[0].z, x[0].w, x[1].x, x[1].y, x[1].z, x[1].w,
                        x[2].x, x[2].y, x[2].z, x[2].w, x[3].x, x[3].y, x[3].z, x[3].w};
   float hi = v[0], lo = v[0];
@@ -234,6 +234,20 @@ __device__ __forceinline__ void hipq_quantize_q8_K_values16(const float4 (&x)[4]
   asm volatile("" : "+v"(d)); /* here, beside the rest, and not behind the condition that stores it */
   if (MODE == Q8K_BYTES) {
     if (store) *(uint4 *)(q_out + 16 * at) = make_uint4(p[0], p[1], p[2], p[3]);
+  } else if (MODE == Q8K_ROWMMA) {
+    /* the group's 8 even values, then its 8 odd ones; two lanes are a sub-block */
+    const int bs = sum + hipq_dpp_i<HIPQ_DPP_XOR1>(sum);
+    if (store) {
+      *(uint4 *)(q_out + (int64_t)16 * at) =
+        make_uint4(__builtin_amdgcn_perm(p[1], p[0], 0x06040200u), __builtin_amdgcn_perm(p[3], p[2], 0x06040200u),
+                   __builtin_amdgcn_perm(p[1], p[0], 0x07050301u), __builtin_amdgcn_perm(p[3], p[2], 0x07050301u));
+      if ((at & 1) == 0) {
+        const int l6 = bs & 63;
+        uint16_t *amin = (uint16_t *)bsum_out + (at & ~15) + ((at & 15) >> 1);
+        amin[0] = __half_as_ushort(__float2half_rn((float)l6));
+        amin[8] = __half_as_ushort(__float2half_rn((float)(bs - l6)));
+      }
+    }
   } else {
     /* 4-bit digits, q = 16 * (qh - 8) + ql, eight values a dword in order */
     auto gather = [](uint32_t a, uint32_t b) { /* the nibbles of eight bytes 0x0n */

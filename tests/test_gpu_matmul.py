@@ -453,6 +453,32 @@ def test_k_format_gemm_of_32_row_tiles(hipq, cr, kind, m):
             w.destroy()
 
 
+@pytest.mark.parametrize("m,k", [(2, 256), (7, 1280), (17, 1024)])
+def test_q4_K_rows_of_their_own_with_hard_super_blocks(hipq, cr, m, k):
+    """The row form of the quantizer, sixteen values a lane: rounding adversaries, a row of zeros, a largest magnitude with both
+    signs (the first decides), strided rows; a last wavefront that is not full. The reference's bits of every row alone."""
+    import os
+    import gpu_util as gu
+    import torch
+    adv = np.load(os.path.join(os.path.dirname(__file__), "golden", "q8k_rounding_adversaries.npy")).reshape(-1, 256)
+    n = 1030
+    blocks = _weights(cr, "q4_K", n, k, seed=380 + m)
+    a = synth.normal(381 + m, (m, k))
+    for r in range(m):
+        a[r, (r % (k // 256)) * 256:][:256] = adv[r % len(adv)]
+    a[1] = 0.0
+    a[m - 1, 7], a[m - 1, 200], a[m - 1, 90] = 9.25, -9.25, -9.25
+    ref = np.concatenate([cr.gemm(cr.oracle(), "q4_K", a[r:r + 1], blocks, n) for r in range(m)])
+    w = capi.Weight("q4_K", n, k, blocks)
+    wide = torch.full((m, k + 8), float("nan"), device="cuda")
+    wide[:, :k] = gu.dev(a)
+    out = torch.full((m, n), float("nan"), device="cuda")
+    capi.matmul_each_row(w, wide, m, out, lda=k + 8, stream=gu.stream())
+    torch.cuda.synchronize()
+    w.destroy()
+    assert np.array_equal(out.cpu().numpy().view(np.uint32), ref.astype(np.float32).view(np.uint32))
+
+
 @pytest.mark.parametrize("m,n,k", [(40, 8192, 512), (18, 12100, 1024), (24, 1100, 8192)])
 def test_q4_K_few_rows_or_tiles(hipq, cr, m, n, k):
     """Beyond sixteen rows the faster of the few-rows kernel and the prefill GEMM, here the GEMM: one product and the first of
