@@ -629,6 +629,7 @@ struct Scratch {
   bool fixed;
   hipStream_t s;
   void *slot = nullptr; /* fixed: this stream's part of the static array */
+  bool whole = false;   /* products walk K whole */
   int get(size_t bytes, void **out) const {
     if (!fixed) return workspace(s, bytes, out);
     if (bytes > NOALLOC_SCRATCH_BYTES)
@@ -727,7 +728,7 @@ int matmul_tiled(const hipq_weight *w, const float *A, int64_t M, int64_t lda, f
    * scratch of the allocation-free entry point may be too small for them: then none) */
   const size_t act_bytes = (qact_tiled_bytes(M, w->K) + 255) & ~(size_t)255;
   size_t part_bytes = w->dtype == HIPQ_Q4_K ? hipq::gemm_q4k_split_bytes(w, M) : hipq::gemm_q6k_split_bytes(w, M);
-  if (sc.fixed && act_bytes + part_bytes > NOALLOC_SCRATCH_BYTES) part_bytes = 0;
+  if (sc.whole || (sc.fixed && act_bytes + part_bytes > NOALLOC_SCRATCH_BYTES)) part_bytes = 0;
   int rc = sc.get(act_bytes + part_bytes, &mem);
   if (rc) return rc;
   QActTiled qa = qact_tiled_carve(mem, M, w->K);
@@ -910,8 +911,9 @@ bool reads_rows_once(const hipq_weight *w, int64_t M, const float *A, int64_t ld
  * multiplied in steps of RowSteps::STEP (the last one up to twice that). Q4_0: every kernel has the
  * reference's bits, always. Q4_K and Q6_K: where the whole call and every step take the prefill GEMM
  * on whole K (a row's sums there depend on neither the other rows nor the tile height; a product in
- * parts of K adds in another order). The weights' tile copies are made here, as the products would. */
-int steps_keep_bits(int count, const hipq_weight_t *w, int64_t M, bool *keep) {
+ * parts of K adds in another order; whole_steps: the steps' products walk K whole whatever their rows). The weights' tile
+ * copies are made here, as the products would. */
+int steps_keep_bits(int count, const hipq_weight_t *w, int64_t M, bool *keep, bool whole_steps = false) {
   *keep = false;
   if (M < 2 * RowSteps::STEP) return HIPQ_OK;
   const int64_t sizes[3] = {M, RowSteps::STEP, RowSteps::STEP + M % RowSteps::STEP};
@@ -922,7 +924,8 @@ int steps_keep_bits(int count, const hipq_weight_t *w, int64_t M, bool *keep) {
     if (!w[i]->gt_base)
       if (int rc = hipq::ensure_gemm_tiles(const_cast<hipq_weight *>(w[i]))) return rc;
     for (int64_t m : sizes)
-      if (w[i]->dtype == HIPQ_Q4_K ? hipq::gemm_q4k_split_bytes(w[i], m) : hipq::gemm_q6k_split_bytes(w[i], m))
+      if ((m == M || !whole_steps) &&
+          (w[i]->dtype == HIPQ_Q4_K ? hipq::gemm_q4k_split_bytes(w[i], m) : hipq::gemm_q6k_split_bytes(w[i], m)))
         return HIPQ_OK;
   }
   *keep = true;
@@ -1347,13 +1350,14 @@ int hipq_matmul(hipq_weight_t w, const float *A, int64_t M, int64_t lda, float *
     if (rc) return rc;
   }
   bool keep = false;
-  if ((rc = steps_keep_bits(1, &w, M, &keep))) return rc;
+  if ((rc = steps_keep_bits(1, &w, M, &keep, true))) return rc;
   RowSteps steps;
   if ((rc = steps.plan(s, M, keep, A, w->K, 1, &C, w->N))) return rc;
+  const Scratch step_sc{false, s, nullptr, steps.step != 0};
   for (int64_t r0 = 0; r0 < M;) {
     const int64_t n = steps.rows_at(r0);
     if ((rc = steps.in(dA, A, lda, w->K, r0, n))) return rc;
-    if ((rc = matmul_device(w, dA + r0 * w->K, n, w->K, dC + r0 * w->N, w->N, s, sc))) return rc;
+    if ((rc = matmul_device(w, dA + r0 * w->K, n, w->K, dC + r0 * w->N, w->N, s, step_sc))) return rc;
     if ((rc = steps.out(dC, C, ldc, w->N, r0, n))) return rc;
     r0 += n;
   }

@@ -200,6 +200,7 @@ def test_grouped_calls_on_a_few_page_locked_rows(hipq, cr, kind, m):
     ("q4_K", 700, 2048, 12288, 0),      # every step takes the prefill GEMM on whole K: two steps
     ("q4_K", 1100, 2048, 4096, 0),      # a step would run in parts of K (other bits): one piece
     ("q6_K", 1100, 1024, 4096, 4),
+    ("q6_K", 520, 3072, 8448, 0),       # the whole call walks K whole, a step alone would not: two steps on whole K
     ("q4_0", 512, 1024, 3072, 0),       # outputs of 6 MB: one piece
 ])
 def test_prefill_rows_in_steps_give_the_device_bits(hipq, cr, kind, m, k, n, pad):
