@@ -826,7 +826,7 @@ def main():
                                                              "rows_8": round(q4k_qkv_ms[8], 5),
                                                              "rows_16": round(q4k_qkv_ms[16], 5)},
             "note": "16 rows: two passes of the same kernel, still the reference's bits; 64 rows: the prefill GEMM "
-                    "in parts of K (one 64-row tile per 128 columns), within 1e-4; qkv: three Q4_K weights of a layer "
+                    "in parts of K (tiles of 32 or 64 rows), within 1e-4; qkv: three Q4_K weights of a layer "
                     "through hipq_matmul_multi, one quantization and one launch of the few-rows kernel for all three"},
         "decode_gemv_size_sweep": {
             "workload": "Q4_K GEMV M=1 K=4096 over N = 4096 .. 151936, weight copies of more than twice the last-level "

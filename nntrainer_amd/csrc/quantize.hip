@@ -94,7 +94,8 @@ __global__ __launch_bounds__(256) void quantize_q8_K_rowmma16_kernel(const float
  * l of a row holding values 64 i + 4 l .. + 3 of the super-block from load i. That is the
  * arithmetic of hipq_quantize_q8_K_values value by value; the reductions stay inside a
  * 16-lane row (four DPP steps) and the scale's two divisions serve sixteen values per
- * lane instead of four. Rows M and beyond of the last 128-row tile are written as zeros. */
+ * lane instead of four. Rows M and beyond are written as zeros as far
+ * as a tile reads them. */
 __global__ __launch_bounds__(256) void quantize_q8_K_tiled_kernel(
   const float *__restrict__ A, int64_t M, int64_t n_units, int nsb, int64_t lda, int64_t mat_rows,
   int8_t *__restrict__ q_out, float *__restrict__ d_out, uint16_t *__restrict__ amin_out) {
