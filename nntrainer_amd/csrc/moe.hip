@@ -1694,15 +1694,16 @@ __global__ __launch_bounds__(256, TC <= 8 ? 4 : TC <= 16 ? 2 : 1) void down_mma_
 }
 
 /* ---- Many tokens per expert (moe_tile_device.h) -------------------------------------------
- * An item is up to 64 (`rows`) slots of one expert; 32 or fewer take the one-tile form. The workgroups of an
- * item follow each other on one XCD (they share the item's rows, and consecutive items of an expert
- * its weights through the last-level cache). */
+ * An item is up to 64 (`rows`) slots of one expert; 32 or fewer take the one-tile form. An XCD has an eighth of the list,
+ * consecutive items: the workgroups of an item follow each other there (they share its rows) and so do the items of an
+ * expert, whose weights then come from that XCD's L2 the second time. With the items dealt out one by one an expert's second
+ * item fetched its weights again: us a block, 1400 tokens of 64 experts of 1792 x 768, top 8, 5 % less, 600 of eight of 2048 x 1024, top 4, 89.3 -> 86.2, 1000 of 128 of 2048 x 768, top 8, 2 % less. */
 __device__ __forceinline__ bool tile_item(int cols, int rows, const int *__restrict__ items, const int *__restrict__ offsets,
                                           int &col, int &e, int &s0, int &n) {
   const int id = blockIdx.x, xcd = id & 7, q = id >> 3;
-  const int item = (q / cols) * 8 + xcd;
+  const int n_items = items[0], per = (n_items + 7) >> 3, at = q / cols, item = xcd * per + at;
   col = q % cols;
-  if (item >= items[0]) return false; /* uniform per workgroup */
+  if (at >= per || item >= n_items) return false; /* uniform per workgroup */
   e = items[2 + 2 * item];
   s0 = items[3 + 2 * item];
   n = min(rows, offsets[e + 1] - s0);
