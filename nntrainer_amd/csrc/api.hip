@@ -676,6 +676,19 @@ int quantize_for(const hipq_weight *w, const float *A, int64_t M, int64_t lda, c
   return hipq::launch_quantize_q8_K(A, M, w->K, lda, mat_rows, &qa, nullptr, s);
 }
 
+/* The tile copy for the few-rows Q6_K kernel, made at a weight's first product that takes it. A stream that is being
+ * captured and a full device go on with the engine, which has the same bits. */
+int rows_q6k_copy(const hipq_weight *w, int64_t M, hipStream_t s) {
+  if (w->gt_base || !hipq::gemm_rows_q6k_fits(w, M)) return HIPQ_OK;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cs) != hipSuccess) (void)hipGetLastError();
+  if (cs != hipStreamCaptureStatusNone) return HIPQ_OK;
+  const int rc = hipq::ensure_gemm_tiles(const_cast<hipq_weight *>(w));
+  if (rc != HIPQ_ERR_OUT_OF_MEMORY) return rc;
+  (void)hipGetLastError();
+  return HIPQ_OK;
+}
+
 /* Block-dot stage on already quantized activations. */
 int multiply(const hipq_weight *w, const QAct &qa, int64_t M, float *C, int64_t ldc,
              hipStream_t s, bool each_row = false) {
@@ -688,6 +701,7 @@ int multiply(const hipq_weight *w, const QAct &qa, int64_t M, float *C, int64_t 
    * 2^25 weights up, where the GEMV engine's eight-row pass is the slower of the two */
   const bool q40_gemm = w->dtype == HIPQ_Q4_0 && w->K % 256 == 0;
   if (hipq::gemm_rows_q40_fits(w, M)) return hipq::launch_gemm_rows_q40(w, &qa, (int)M, C, ldc, s);
+  if (w->gt_base && hipq::gemm_rows_q6k_fits(w, M)) return hipq::launch_gemm_rows_q6k(w, &qa, (int)M, C, ldc, s);
   if (M <= 8 && !(q40_gemm && M >= 5 && w->N * w->K >= (int64_t(1) << 25)))
     return hipq::launch_gemv(w, &qa, (int)M, pair_rows, C, ldc, s);
   if (q40_gemm) return hipq::launch_gemm(w, &qa, (int)M, C, ldc, s);
@@ -883,7 +897,10 @@ int matmul_device(hipq_weight_t w, const float *A, int64_t M, int64_t lda, float
   if (hipq::gemm_rows_q40_fuses(1, &one, M, A, lda)) return hipq::launch_gemm_rows_q40_fused(1, &one, A, lda, (int)M, &C, &ldc, s);
   const int is_k = w->dtype != HIPQ_Q4_0;
   void *mem = nullptr;
-  int rc = sc.get(qact_bytes(is_k, M, w->K), &mem);
+  int rc;
+  /* the entry point that may not allocate takes the few-rows Q6_K kernel once the copy exists */
+  if (!sc.fixed && (rc = rows_q6k_copy(w, M, s))) return rc;
+  rc = sc.get(qact_bytes(is_k, M, w->K), &mem);
   if (rc) return rc;
   QAct qa = qact_carve(is_k, mem, M, w->K);
   rc = quantize_for(w, A, M, lda, qa, s, each_row);
@@ -1671,6 +1688,7 @@ int hipq_matmul_multi(int count, const hipq_weight_t *w, const float *A, int64_t
     for (int i = 0; i < count; ++i) {
       const hipq_weight *x = w[i];
       size_t n = qact_bytes(x->dtype != HIPQ_Q4_0, M, x->K);
+      if ((rc = rows_q6k_copy(x, M, s))) return rc;
       if (x->dtype != HIPQ_Q4_0 && (wants_tiled(x, M) || (M > 16 && tiles_q4k(x, M)))) {
         if (!x->gt_base && (rc = hipq::ensure_gemm_tiles(const_cast<hipq_weight *>(x)))) return rc;
         const size_t parts = x->dtype == HIPQ_Q4_K ? hipq::gemm_q4k_split_bytes(x, M) : hipq::gemm_q6k_split_bytes(x, M);

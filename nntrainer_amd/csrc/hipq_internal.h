@@ -359,6 +359,12 @@ bool gemm_rows_q4k_fits_multi(int count, const hipq_weight *const *w, int64_t M,
 int launch_gemm_rows_q4k_multi(int count, const hipq_weight *const *w, const QAct *qa, int M, int pair_rows,
                                float *const *C, const int64_t *ldc, hipStream_t s);
 
+/* gemm_rows_q6k.hip: Q6_K for a few rows on the matrix cores with the reference's bits (rows are independent in this
+ * format); fits: the row counts and shapes that should take it; qa in the form of launch_quantize_q8_K; the weight with its
+ * tile copy (ensure_gemm_tiles) */
+bool gemm_rows_q6k_fits(const hipq_weight *w, int64_t M);
+int launch_gemm_rows_q6k(const hipq_weight *w, const QAct *qa, int M, float *C, int64_t ldc, hipStream_t s);
+
 /* gemm_rows_q40.hip: Q4_0 for a few rows on the matrix cores with the reference's bits (rows are
  * independent in this format); fits: the row counts and shapes that should take it; qa in the form
  * of launch_quantize_q8_0; the weight's planes as they are */

@@ -479,6 +479,71 @@ def test_q4_K_rows_of_their_own_with_hard_super_blocks(hipq, cr, m, k):
     assert np.array_equal(out.cpu().numpy().view(np.uint32), ref.astype(np.float32).view(np.uint32))
 
 
+@pytest.mark.parametrize("m,n,k", [(2, 20001, 256), (3, 12310, 512), (5, 9001, 1280), (8, 4100, 1024), (9, 1030, 2304), (16, 610, 256),
+                                   (13, 4100, 4352)])
+def test_q6_K_few_rows_on_the_matrix_cores(hipq, cr, m, n, k):
+    """One pass and two of eight rows, a last pass of one row and more, one round of super-blocks, whole rounds and a part of
+    one, columns behind the last tile of 32, strided rows: every row has the bits of its own product, as one call and as rows of
+    their own, before and after the weight's tile copy exists."""
+    import gpu_util as gu
+    import torch
+    few = _weights(cr, "q6_K", 61, k, seed=390 + m)
+    cols = np.random.RandomState(n).randint(0, 61, n)
+    a = synth.normal(391 + m, (m, k))
+    a[m // 2] = 0.0
+    ref = np.concatenate([cr.gemm(cr.oracle(), "q6_K", a[r:r + 1], few, 61) for r in range(m)])[:, cols].astype(np.float32)
+    w = capi.Weight("q6_K", n, k, np.ascontiguousarray(few.reshape(61, -1)[cols]))
+    wide = torch.full((m, k + 4), float("nan"), device="cuda")
+    wide[:, :k] = gu.dev(a)
+    try:
+        for _ in range(2):
+            out = torch.full((m, n + 5), float("nan"), device="cuda")
+            capi.matmul_each_row(w, wide, m, out, lda=k + 4, ldc=n + 5, stream=gu.stream())
+            torch.cuda.synchronize()
+            got = out.cpu().numpy()
+            assert np.isnan(got[:, n:]).all(), "the call wrote between the rows of C"
+            assert np.array_equal(got[:, :n].copy().view(np.uint32), ref.view(np.uint32))
+        one = gu.gpu_matmul(w, a)
+    finally:
+        w.destroy()
+    if m <= (4 if n * k >= 2 ** 25 else 8 if n * k >= 2 ** 24 else 16):
+        assert np.array_equal(one.view(np.uint32), ref.view(np.uint32))
+    else:
+        assert gu.rel_err(one, ref) <= gu.TOL
+
+
+def test_q6_K_few_rows_captured_before_the_copy_exists(hipq, cr):
+    """The few-rows Q6_K kernel reads a copy of the weight that its first product makes; a call that is being captured, and the
+    one that may not allocate, use the weight as it is stored: the same bits, replayed three times with the copy made between."""
+    import gpu_util as gu
+    import torch
+    m, n, k = 8, 5000, 512
+    blocks = _weights(cr, "q6_K", n, k, seed=395)
+    fresh, warm = capi.Weight("q6_K", n, k, blocks), capi.Weight("q6_K", n, k, blocks)
+    a = gu.dev(synth.normal(396, (m, k)))
+    want, out, na = (torch.full((m, n), float("nan"), device="cuda") for _ in range(3))
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        capi.matmul(warm, a, m, want, stream=side.cuda_stream)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=side):
+        capi.matmul(fresh, a, m, out, stream=torch.cuda.current_stream().cuda_stream)
+    capi.matmul_noalloc(fresh, a, m, na, stream=gu.stream())
+    torch.cuda.synchronize()
+    assert torch.equal(na, want)
+    for _ in range(3):
+        out.fill_(-1.0)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        eager = torch.full((m, n), float("nan"), device="cuda")
+        capi.matmul(fresh, a, m, eager, stream=gu.stream())
+        torch.cuda.synchronize()
+        assert torch.equal(eager, want)
+    fresh.destroy(), warm.destroy()
+
+
 @pytest.mark.parametrize("m,n,k", [(40, 8192, 512), (18, 12100, 1024), (24, 1100, 8192)])
 def test_q4_K_few_rows_or_tiles(hipq, cr, m, n, k):
     """Beyond sixteen rows the faster of the few-rows kernel and the prefill GEMM, here the GEMM: one product and the first of
