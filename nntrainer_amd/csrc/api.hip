@@ -597,9 +597,6 @@ QAct qact_rows(const QAct &a, int is_k, int64_t r0, int64_t rows) {
   return v;
 }
 
-bool tiles_q4k(const hipq_weight *w, int64_t M) {
-  return w->dtype == HIPQ_Q4_K && M > 8 && w->N * (w->K / 2) < (int64_t(1) << 32);
-}
 /* The prefill GEMMs of the K-formats take their activations in the tiled form. The Q4_K one
  * addresses the weight planes with 32-bit byte offsets where it has no tile copy; the Q6_K
  * one reads the tile copy only, which the entry point that may not allocate cannot build
@@ -620,7 +617,7 @@ bool wants_tiled(const hipq_weight *w, int64_t M, bool may_allocate = true) {
   }
   /* up to 16 rows of a Q4_K matrix of 1024 columns or more take the few-rows kernel (wants_rows) */
   if (hipq::gemm_rows_q4k_fits(w, M) && (w->gt_base || may_allocate)) return false;
-  return tiles_q4k(w, M);
+  return w->dtype == HIPQ_Q4_K && M > 8 && w->N * (w->K / 2) < (int64_t(1) << 32);
 }
 
 /* Where a call's quantized activations go: the per-stream workspace (grown on
@@ -760,8 +757,8 @@ int matmul_tiled(const hipq_weight *w, const float *A, int64_t M, int64_t lda, f
  * reference's bits as the GEMV engine's) off the weight's tile copy; the entry point that may not
  * allocate takes that path only once the copy exists.
  * phase: 0 quantizer + product, 1 product only, 2 quantizer only */
-bool wants_rows(const hipq_weight *w, int64_t M, bool may_allocate, bool exact = false) {
-  return hipq::gemm_rows_q4k_fits(w, M, exact) && (w->gt_base || may_allocate);
+bool wants_rows(const hipq_weight *w, int64_t M, bool may_allocate) {
+  return hipq::gemm_rows_q4k_fits(w, M) && (w->gt_base || may_allocate);
 }
 
 int matmul_rows(const hipq_weight *w, const float *A, int64_t M, int64_t lda, float *C, int64_t ldc,
@@ -822,8 +819,7 @@ bool wants_gated(const hipq_weight *wa, const hipq_weight *wm, int64_t M) {
   if (wa->dtype != wm->dtype || M < 2) return false;
   const hipq_weight *ws[2] = {wa, wm};
   if (wa->dtype == HIPQ_Q4_0) return wants_f6(2, ws, M);
-  /* its launch of the activation and the products' way through memory fall away: 3 us */
-  return tiles_q4k(wa, M) && !hipq::gemm_rows_q4k_fits_multi(2, ws, M, 3.) && (M > 16 || !wants_rows(wa, M, true));
+  return wa->dtype == HIPQ_Q4_K && !hipq::gemm_rows_q4k_fits_multi(2, ws, M) && !wants_rows(wa, M, true) && wants_tiled(wa, M);
 }
 
 /* out = swiglu(A . wa) * (A . wm) for a pair that wants_gated names; *done stays false where the pair's six-bit copies
@@ -891,7 +887,7 @@ int matmul_device(hipq_weight_t w, const float *A, int64_t M, int64_t lda, float
     if (int rc = f6_ready(1, &one, M, s, sc, &ready, &make)) return rc;
     if (ready) return matmul_f6(1, &one, A, M, lda, &C, &ldc, s, sc, &make);
   }
-  if (wants_rows(w, M, !sc.fixed, each_row)) return matmul_rows(w, A, M, lda, C, ldc, s, 0, sc, each_row);
+  if (wants_rows(w, M, !sc.fixed)) return matmul_rows(w, A, M, lda, C, ldc, s, 0, sc, each_row);
   if (!each_row && wants_tiled(w, M, !sc.fixed)) return matmul_tiled(w, A, M, lda, C, ldc, s, 0, sc);
   if (M == 1 && hipq::gemv_fuses_quantizer(w, A)) return hipq::launch_gemv_fused(w, A, C, s);
   if (hipq::gemm_rows_q40_fuses(1, &one, M, A, lda)) return hipq::launch_gemm_rows_q40_fused(1, &one, A, lda, (int)M, &C, &ldc, s);
@@ -1417,7 +1413,7 @@ int hipq_matmul_each_row(hipq_weight_t w, const float *A, int64_t rows, int64_t 
     if (w->dtype == HIPQ_Q4_K) /* up to 64 where the few-rows kernel takes that many in one launch */
       for (int64_t c = 64; c > 16; c -= 8) {
         const int64_t t = (rows - r0) < c ? (rows - r0) : c;
-        if (t > 16 && wants_rows(w, t, true, true)) {
+        if (t > 16 && wants_rows(w, t, true)) {
           n = t;
           break;
         }
@@ -1689,7 +1685,7 @@ int hipq_matmul_multi(int count, const hipq_weight_t *w, const float *A, int64_t
       const hipq_weight *x = w[i];
       size_t n = qact_bytes(x->dtype != HIPQ_Q4_0, M, x->K);
       if ((rc = rows_q6k_copy(x, M, s))) return rc;
-      if (x->dtype != HIPQ_Q4_0 && (wants_tiled(x, M) || (M > 16 && tiles_q4k(x, M)))) {
+      if (x->dtype != HIPQ_Q4_0 && wants_tiled(x, M)) {
         if (!x->gt_base && (rc = hipq::ensure_gemm_tiles(const_cast<hipq_weight *>(x)))) return rc;
         const size_t parts = x->dtype == HIPQ_Q4_K ? hipq::gemm_q4k_split_bytes(x, M) : hipq::gemm_q6k_split_bytes(x, M);
         const size_t tiled = ((qact_tiled_bytes(M, x->K) + 255) & ~(size_t)255) + parts;
@@ -1713,7 +1709,6 @@ int hipq_matmul_multi(int count, const hipq_weight_t *w, const float *A, int64_t
   auto klass = [&](const hipq_weight *x) {
     if (x->dtype == HIPQ_Q4_0) return 0;
     if (x->dtype == HIPQ_Q4_K && q4k_rows_group) return 5;
-    if (n_q4k >= 2 && n_q4k < 64 && M > 16 && tiles_q4k(x, M)) return 3; /* all of them in the launches of the prefill GEMM */
     if (wants_rows(x, M, true)) return 5; /* a few rows of Q4_K on the matrix cores: the row form of the MoE kernels */
     if (wants_tiled(x, M)) return x->dtype == HIPQ_Q4_K ? 3 : 4; /* the two tiled forms differ in their rows' quantizer */
     return (x->dtype == HIPQ_Q4_K && M > 1) ? 1 : 2;

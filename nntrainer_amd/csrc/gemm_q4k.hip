@@ -567,7 +567,6 @@ int launch_split_sum(const float *partials, int parts, int M, int64_t N, float *
 static TilePlan plan(const hipq_weight *w, int64_t M) {
   return tile_plan(COST, M, w->N, w->K, w->gt_base, w->dtype == HIPQ_Q4_K && w->gt_base);
 }
-double gemm_q4k_us(int64_t M, int64_t N, int64_t K, bool parts) { return tile_plan(COST, M, N, K, true, parts).us; }
 /* bytes of the partial products of a product in parts of K (0: whole) */
 size_t gemm_q4k_split_bytes(const hipq_weight *w, int64_t M) {
   const TilePlan t = plan(w, M);

@@ -341,17 +341,6 @@ __global__ __launch_bounds__(NT, PAIRS ? 2 : 3) void gemm_rows_q4k_kernel(MultiR
 
 namespace hipq {
 
-/* More than 16 rows: passes of eight side by side in one launch against the prefill GEMM (which rounds less, but not as the
- * reference does). A call takes 4.9 us and 0.35 a super-block for the chain of rounds, and 4.2 + 0.22 K / 256 ns a
- * workgroup (a column tile of a pass); the GEMM its estimate and 7.8. Measured on 170 sizes, us, this kernel / the GEMM: 64
- * rows of 1100 x 1024 8.8 / 10.3, of 2048 x 2048 10.0 / 14.4, of 6000 x 1024 13.4 / 11.3, 32 of 4096 x 4096 13.9 / 15.4, of
- * 8192 x 512 10.2 / 9.2, 24 of 1100 x 8192 17.5 / 15.2, of 20000 x 1024 16.8 / 12.0; by this line 7.5 % less than with all of
- * them here, 0.1 % more than the faster one each time. */
-static bool passes_beat_tiles(int64_t tiles, int64_t M, int64_t K, bool parts, double saved) {
-  const double nsb = (double)(K / 256), workgroups = (double)(tiles * ((M + TC - 1) / TC));
-  return 4.9 + 0.35 * nsb + 1e-3 * workgroups * (4.2 + 0.22 * nsb) <= 7.8 - saved + gemm_q4k_us(M, tiles * 32, K, parts);
-}
-
 /* Where it beats the GEMV engine (measured, kernel us old -> new): five to eight rows from 1024
  * columns up (2048 x 1024: 5.5 -> 4.0; 4096 x 4096: 16.4 -> 8.3; 12288 x 4096: 39.0 -> 11.2;
  * 151936 x 4096: 421 -> 75); with fewer rows where the last lines of the rule below say (at first four
@@ -360,16 +349,19 @@ static bool passes_beat_tiles(int64_t tiles, int64_t M, int64_t K, bool parts, d
  * of a workgroup takes 1.7 us, most of it the issue of its vector instructions (about 290 a
  * wavefront and super-block: nibble expansion, scale multiplies, the chains), so the kernel
  * streams its weights at 2.5-4.6 TB/s. */
-bool gemm_rows_q4k_fits(const hipq_weight *w, int64_t M, bool exact) {
+bool gemm_rows_q4k_fits(const hipq_weight *w, int64_t M) {
   if (w->dtype != HIPQ_Q4_K || w->expert_tiles || w->K % 256 || 16 * w->K > 0x7fffffff) return false;
   /* More than eight rows: passes of eight side by side in one launch (blockIdx.y). Two passes
    * always (12288 x 4096 with 16 rows: 14.7 us against 17.2 for the prefill GEMM in parts of K; 4096 x
    * 4096: 8.5 against 12.5: a launch of one pass leaves half the chip idle there); up to eight where
-   * the launch stays small and, unless the rows have to keep the reference's bits, takes less than that GEMM. */
+   * the launch stays small. Up to that line hipq.h promises the reference's bits, which the GEMM's sums do not have, so it
+   * does not move with what the GEMM takes: us, this kernel / the GEMM, 64 rows of 2048 x 2048 10.0 / 14.4, of 1100 x 1024
+   * 8.8 / 10.3, 32 of 4096 x 4096 13.9 / 15.4, but 64 of 6000 x 1024 13.4 / 11.3, 24 of 20000 x 1024 16.8 / 12.0, of
+   * 1100 x 8192 17.5 / 15.2 (the faster one each time would be 8 % less over 170 sizes up to the line). */
   if (M >= 5 && M <= 2 * TC) return w->N >= 1024;
   if (M > 2 * TC && M <= 8 * TC && w->N >= 1024) {
     const int64_t tiles = (w->N + 31) / 32, passes = (M + TC - 1) / TC;
-    return tiles * passes * (w->K / 256) <= 8192 && (exact || passes_beat_tiles(tiles, M, w->K, true, 0.));
+    return tiles * passes * (w->K / 256) <= 8192;
   }
   /* Two to four rows against the engine with its row lengths compiled in (calls in a row on one
    * stream, us, engine / this kernel). Four rows: 4096 x 4096 10.4 / 11.2, 6144 x 4096 11.7 / 11.4,
@@ -385,7 +377,7 @@ bool gemm_rows_q4k_fits(const hipq_weight *w, int64_t M, bool exact) {
 
 /* Several weights of one K in one launch (hipq_matmul_multi): what counts is the launch's width, the
  * columns of all of them, and the launches it replaces. */
-bool gemm_rows_q4k_fits_multi(int count, const hipq_weight *const *w, int64_t M, double saved) {
+bool gemm_rows_q4k_fits_multi(int count, const hipq_weight *const *w, int64_t M) {
   if (count < 2 || M < 2 || M > 8 * TC) return false;
   int64_t tiles = 0;
   for (int i = 0; i < count; ++i) {
@@ -396,7 +388,7 @@ bool gemm_rows_q4k_fits_multi(int count, const hipq_weight *const *w, int64_t M,
   }
   if (tiles < 32) return false;
   if (M <= 2 * TC) return true;
-  return tiles * ((M + TC - 1) / TC) * (w[0]->K / 256) <= 8192 && passes_beat_tiles(tiles, M, w[0]->K, false, saved);
+  return tiles * ((M + TC - 1) / TC) * (w[0]->K / 256) <= 8192;
 }
 
 int launch_gemm_rows_q4k_multi(int count, const hipq_weight *const *w, const QAct *qa, int M, int pair_rows,

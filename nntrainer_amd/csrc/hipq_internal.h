@@ -310,11 +310,11 @@ struct TileCost {
 };
 struct TilePlan {
   int rows, parts;
-  double us; /* by the estimate, without what every call takes */
 };
 inline TilePlan tile_plan(const TileCost &c, int64_t M, int64_t N, int64_t K, bool copy, bool split) {
   const int64_t nsb = K / 256, nt = (N + 127) / 128;
-  TilePlan best{64, 1, 1e30};
+  TilePlan best{64, 1};
+  double least = 1e30;
   for (int h = copy ? 32 : 64; h <= (M > 64 ? 128 : 64); h *= 2) {
     const int64_t mt = (M + h - 1) / h;
     const int fit = h == 32 ? 4 : h == 64 ? 3 : 2;
@@ -324,7 +324,7 @@ inline TilePlan tile_plan(const TileCost &c, int64_t M, int64_t N, int64_t K, bo
       const int64_t per = (nsb + p - 1) / p, parts = (nsb + per - 1) / per, a_cu = (mt * nt * parts + 255) / 256;
       double us = (double)per * ((double)(a_cu / fit) * t[fit] + t[a_cu % fit]);
       if (parts > 1) us += 1.5 + 1.0 + 0.26e-6 * 4 * (double)((parts + 1) * M * N);
-      if (us < best.us) best = TilePlan{h, (int)parts, us};
+      if (us < least) least = us, best = TilePlan{h, (int)parts};
     }
   }
   return best;
@@ -345,17 +345,15 @@ size_t gemm_q6k_split_bytes(const hipq_weight *w, int64_t M);
 int launch_gemm_q4k(const hipq_weight *w, const QActTiled *qa, int M, float *C,
                     int64_t ldc, hipStream_t s, void *partials = nullptr);
 size_t gemm_q4k_split_bytes(const hipq_weight *w, int64_t M);
-/* what a launch against N columns with tile copies should take, without the quantizer and what every call takes */
-double gemm_q4k_us(int64_t M, int64_t N, int64_t K, bool parts);
 /* gemm_rows_q4k.hip: Q4_K for a few rows on the matrix cores with the reference's bits; fits: the row
  * counts and shapes that should take it (up to 16 rows, in passes of up to 8 for the launcher); qa in
  * the form of launch_quantize_q8_K_rowmma, the first pair_rows rows under the 4-row quantizer's rule;
  * the weight with its tile copy (ensure_gemm_tiles) */
-bool gemm_rows_q4k_fits(const hipq_weight *w, int64_t M, bool exact = false /* the reference's bits are needed */);
+bool gemm_rows_q4k_fits(const hipq_weight *w, int64_t M);
 int launch_gemm_rows_q4k(const hipq_weight *w, const QAct *qa, int M, int pair_rows, float *C, int64_t ldc,
                          hipStream_t s);
 /* up to four weights of one K against the same rows in one launch (the column tiles side by side in the grid) */
-bool gemm_rows_q4k_fits_multi(int count, const hipq_weight *const *w, int64_t M, double saved = 0. /* us, by the GEMM's form */);
+bool gemm_rows_q4k_fits_multi(int count, const hipq_weight *const *w, int64_t M);
 int launch_gemm_rows_q4k_multi(int count, const hipq_weight *const *w, const QAct *qa, int M, int pair_rows,
                                float *const *C, const int64_t *ldc, hipStream_t s);
 
