@@ -504,6 +504,7 @@ int stage_copy(bool to_device, void *dev, void *host, size_t hpitch, size_t widt
   return HIPQ_OK;
 }
 
+struct Scratch;
 /* Rows of a host-memory call in steps. With page-locked operands the copies are asynchronous, and
  * the link carries both directions at once: while the kernels work on one step's rows, the copy
  * engines take the step before out (on a second stream) and, behind the kernels, bring the next
@@ -542,6 +543,7 @@ struct RowSteps {
     step = STEP;
     return HIPQ_OK;
   }
+  Scratch scratch() const; /* of a piece's products */
   /* the rows of the piece that starts at r0 */
   int64_t rows_at(int64_t r0) const { return (!step || M - r0 < 2 * step) ? M - r0 : step; }
   int in(float *dev, const float *host, int64_t lda, int64_t K, int64_t r0, int64_t n) const {
@@ -626,7 +628,7 @@ struct Scratch {
   bool fixed;
   hipStream_t s;
   void *slot = nullptr; /* fixed: this stream's part of the static array */
-  bool whole = false;   /* products walk K whole */
+  int64_t rows = 0;     /* the products are steps of a call of so many rows and take its parts of K (0: no steps) */
   int get(size_t bytes, void **out) const {
     if (!fixed) return workspace(s, bytes, out);
     if (bytes > NOALLOC_SCRATCH_BYTES)
@@ -638,6 +640,8 @@ struct Scratch {
     return HIPQ_OK;
   }
 };
+
+Scratch RowSteps::scratch() const { return Scratch{false, s, nullptr, step ? M : 0}; }
 
 /* The slot of the static array that belongs to stream s (the first four streams that use the
  * allocation-free entry point get one each, until hipq_stream_release gives it back). */
@@ -738,8 +742,8 @@ int matmul_tiled(const hipq_weight *w, const float *A, int64_t M, int64_t lda, f
   /* room for the partial products of a product with few tiles behind the activations (the fixed
    * scratch of the allocation-free entry point may be too small for them: then none) */
   const size_t act_bytes = (qact_tiled_bytes(M, w->K) + 255) & ~(size_t)255;
-  size_t part_bytes = w->dtype == HIPQ_Q4_K ? hipq::gemm_q4k_split_bytes(w, M) : hipq::gemm_q6k_split_bytes(w, M);
-  if (sc.whole || (sc.fixed && act_bytes + part_bytes > NOALLOC_SCRATCH_BYTES)) part_bytes = 0;
+  size_t part_bytes = w->dtype == HIPQ_Q4_K ? hipq::gemm_q4k_split_bytes(w, M, sc.rows) : hipq::gemm_q6k_split_bytes(w, M, sc.rows);
+  if (sc.fixed && act_bytes + part_bytes > NOALLOC_SCRATCH_BYTES) part_bytes = 0;
   int rc = sc.get(act_bytes + part_bytes, &mem);
   if (rc) return rc;
   QActTiled qa = qact_tiled_carve(mem, M, w->K);
@@ -749,8 +753,8 @@ int matmul_tiled(const hipq_weight *w, const float *A, int64_t M, int64_t lda, f
   const int64_t mat_rows = w->dtype == HIPQ_Q4_K ? (M / 4) * 4 : 0;
   if (phase != 1) rc = hipq::launch_quantize_q8_K_tiled(A, M, w->K, lda, mat_rows, &qa, s);
   if (rc || phase == 2) return rc;
-  if (w->dtype == HIPQ_Q6_K) return hipq::launch_gemm_q6k(w, &qa, (int)M, C, ldc, s, partials);
-  return hipq::launch_gemm_q4k(w, &qa, (int)M, C, ldc, s, partials);
+  if (w->dtype == HIPQ_Q6_K) return hipq::launch_gemm_q6k(w, &qa, (int)M, C, ldc, s, partials, sc.rows);
+  return hipq::launch_gemm_q4k(w, &qa, (int)M, C, ldc, s, partials, sc.rows);
 }
 
 /* Three to eight rows of a large Q4_K matrix run on the matrix cores (gemm_rows_q4k.hip, the
@@ -922,24 +926,19 @@ bool reads_rows_once(const hipq_weight *w, int64_t M, const float *A, int64_t ld
 
 /* Whether the products of a call of M rows against these weights have the same bits when the rows are
  * multiplied in steps of RowSteps::STEP (the last one up to twice that). Q4_0: every kernel has the
- * reference's bits, always. Q4_K and Q6_K: where the whole call and every step take the prefill GEMM
- * on whole K (a row's sums there depend on neither the other rows nor the tile height; a product in
- * parts of K adds in another order; whole_steps: the steps' products walk K whole whatever their rows). The weights' tile
- * copies are made here, as the products would. */
-int steps_keep_bits(int count, const hipq_weight_t *w, int64_t M, bool *keep, bool whole_steps = false) {
+ * reference's bits, always. Q4_K and Q6_K: where the whole call and every step take the prefill GEMM,
+ * the steps' products in the whole call's parts of K (Scratch::rows): a row's sums there depend on
+ * neither the other rows nor the tile height, but on the parts. The weights' tile copies are made
+ * here, as the products would. */
+int steps_keep_bits(int count, const hipq_weight_t *w, int64_t M, bool *keep) {
   *keep = false;
   if (M < 2 * RowSteps::STEP) return HIPQ_OK;
-  const int64_t sizes[3] = {M, RowSteps::STEP, RowSteps::STEP + M % RowSteps::STEP};
   for (int i = 0; i < count; ++i) {
     if (w[i]->dtype == HIPQ_Q4_0) continue;
-    for (int64_t m : sizes)
+    for (int64_t m : {M, RowSteps::STEP, RowSteps::STEP + M % RowSteps::STEP})
       if (!wants_tiled(w[i], m)) return HIPQ_OK;
     if (!w[i]->gt_base)
       if (int rc = hipq::ensure_gemm_tiles(const_cast<hipq_weight *>(w[i]))) return rc;
-    for (int64_t m : sizes)
-      if ((m == M || !whole_steps) &&
-          (w[i]->dtype == HIPQ_Q4_K ? hipq::gemm_q4k_split_bytes(w[i], m) : hipq::gemm_q6k_split_bytes(w[i], m)))
-        return HIPQ_OK;
   }
   *keep = true;
   return HIPQ_OK;
@@ -1363,14 +1362,13 @@ int hipq_matmul(hipq_weight_t w, const float *A, int64_t M, int64_t lda, float *
     if (rc) return rc;
   }
   bool keep = false;
-  if ((rc = steps_keep_bits(1, &w, M, &keep, true))) return rc;
+  if ((rc = steps_keep_bits(1, &w, M, &keep))) return rc;
   RowSteps steps;
   if ((rc = steps.plan(s, M, keep, A, w->K, 1, &C, w->N))) return rc;
-  const Scratch step_sc{false, s, nullptr, steps.step != 0};
   for (int64_t r0 = 0; r0 < M;) {
     const int64_t n = steps.rows_at(r0);
     if ((rc = steps.in(dA, A, lda, w->K, r0, n))) return rc;
-    if ((rc = matmul_device(w, dA + r0 * w->K, n, w->K, dC + r0 * w->N, w->N, s, step_sc))) return rc;
+    if ((rc = matmul_device(w, dA + r0 * w->K, n, w->K, dC + r0 * w->N, w->N, s, steps.scratch()))) return rc;
     if ((rc = steps.out(dC, C, ldc, w->N, r0, n))) return rc;
     r0 += n;
   }
@@ -1440,6 +1438,9 @@ int hipq_matmul_noalloc(hipq_weight_t w, const float *A, int64_t M, int64_t lda,
   return matmul_device(w, A, M, lda, C, ldc, s, Scratch{true, s, slot});
 }
 
+static int multi_device(int count, const hipq_weight_t *w, const float *A, int64_t M, int64_t lda, float *const *C,
+                        const int64_t *ldc, hipStream_t s, const Scratch &sc);
+
 int hipq_mlp_swiglu(hipq_weight_t w_act, hipq_weight_t w_mul, const float *A, int64_t M, int64_t lda,
                     float *out, int64_t ldo, int mem, void *stream) {
   int rc = require_ready();
@@ -1502,7 +1503,7 @@ int hipq_mlp_swiglu(hipq_weight_t w_act, hipq_weight_t w_mul, const float *A, in
       bool done = false;
       if (wants_gated(w_act, w_mul, n) && (rc = launch_gated(w_act, w_mul, dA + r0 * K, n, K, dO + r0 * N, N, s, &done))) return rc;
       if (!done) {
-        if ((rc = hipq_matmul_multi(2, ws, dA + r0 * K, n, K, cr, lds, HIPQ_MEM_DEVICE, stream))) return rc;
+        if ((rc = multi_device(2, ws, dA + r0 * K, n, K, cr, lds, s, steps.scratch()))) return rc;
         if ((rc = hipq::launch_swiglu_rows(cr[0], cr[1], n, N, dO + r0 * N, N, s))) return rc;
       }
       if ((rc = steps.out(dO, out, ldo, N, r0, n))) return rc;
@@ -1510,7 +1511,7 @@ int hipq_mlp_swiglu(hipq_weight_t w_act, hipq_weight_t w_mul, const float *A, in
     }
     return steps.finish();
   }
-  if ((rc = hipq_matmul_multi(2, ws, a_dev, M, a_ld, cs, lds, HIPQ_MEM_DEVICE, stream))) return rc;
+  if ((rc = multi_device(2, ws, a_dev, M, a_ld, cs, lds, s, Scratch{false, s}))) return rc;
   if (mem == HIPQ_MEM_DEVICE) return hipq::launch_swiglu_rows(dY, dZ, M, N, out, ldo, s);
   if ((rc = hipq::launch_swiglu_rows(dY, dZ, M, N, h_out, h_ld, s))) return rc;
   return dio.finish();
@@ -1564,7 +1565,7 @@ int hipq_mlp_swiglu_down(hipq_weight_t w_act, hipq_weight_t w_mul, hipq_weight_t
   const hipq_weight_t ws[2] = {w_act, w_mul};
   const int64_t lds[2] = {N, N};
   /* rows [r0, r0 + n): the gated half into dH, the down projection into the output */
-  auto rows = [&](int64_t r0, int64_t n) -> int {
+  auto rows = [&](int64_t r0, int64_t n, const Scratch &sc) -> int {
     const float *a = a_dev + r0 * a_ld;
     int rr;
     bool done = false;
@@ -1580,13 +1581,13 @@ int hipq_mlp_swiglu_down(hipq_weight_t w_act, hipq_weight_t w_mul, hipq_weight_t
     }
     if (!done) {
       float *const cr[2] = {dY + r0 * N, dZ + r0 * N};
-      if ((rr = hipq_matmul_multi(2, ws, a, n, a_ld, cr, lds, HIPQ_MEM_DEVICE, stream))) return rr;
+      if ((rr = multi_device(2, ws, a, n, a_ld, cr, lds, s, sc))) return rr;
       if ((rr = hipq::launch_swiglu_rows(cr[0], cr[1], n, N, dH + r0 * N, N, s))) return rr;
     }
-    return hipq_matmul(w_down, dH + r0 * N, n, N, o_dev + r0 * o_ld, o_ld, HIPQ_MEM_DEVICE, stream);
+    return matmul_device(w_down, dH + r0 * N, n, N, o_dev + r0 * o_ld, o_ld, s, sc);
   };
   if (mem == HIPQ_MEM_DEVICE || direct) {
-    if ((rc = rows(0, M))) return rc;
+    if ((rc = rows(0, M, Scratch{false, s}))) return rc;
     return direct ? dio.finish() : HIPQ_OK;
   }
   /* host rows through the copy engines, in steps where that keeps the bits */
@@ -1598,7 +1599,7 @@ int hipq_mlp_swiglu_down(hipq_weight_t w_act, hipq_weight_t w_mul, hipq_weight_t
   for (int64_t r0 = 0; r0 < M;) {
     const int64_t n = steps.rows_at(r0);
     if ((rc = steps.in(dA, A, lda, K, r0, n))) return rc;
-    if ((rc = rows(r0, n))) return rc;
+    if ((rc = rows(r0, n, steps.scratch()))) return rc;
     if ((rc = steps.out(dO, out, ldo, Nd, r0, n))) return rc;
     r0 += n;
   }
@@ -1640,8 +1641,7 @@ int hipq_matmul_multi(int count, const hipq_weight_t *w, const float *A, int64_t
     if (dio.begin(s, A, M, lda, Kh, count, C, ldc, ns.data(), &rc)) {
       for (int i = 0; i < count; ++i) dC[i] = dio.outs[i].dev, dld[i] = dio.outs[i].dld;
       if ((rc = dio.fetch((float *)io, Kh))) return rc;
-      if ((rc = hipq_matmul_multi(count, w, (const float *)io, M, Kh, dC.data(), dld.data(), HIPQ_MEM_DEVICE, stream)))
-        return rc;
+      if ((rc = multi_device(count, w, (const float *)io, M, Kh, dC.data(), dld.data(), s, Scratch{false, s}))) return rc;
       return dio.finish();
     }
     if (rc) return rc;
@@ -1661,15 +1661,20 @@ int hipq_matmul_multi(int count, const hipq_weight_t *w, const float *A, int64_t
       const int64_t n = steps.rows_at(r0);
       if ((rc = steps.in((float *)io, A, lda, Kh, r0, n))) return rc;
       for (int i = 0; i < count; ++i) dCr[i] = dC[i] + r0 * dld[i];
-      if ((rc = hipq_matmul_multi(count, w, (const float *)io + r0 * Kh, n, Kh, dCr.data(), dld.data(), HIPQ_MEM_DEVICE,
-                                  stream)))
-        return rc;
+      if ((rc = multi_device(count, w, (const float *)io + r0 * Kh, n, Kh, dCr.data(), dld.data(), s, steps.scratch()))) return rc;
       for (int i = 0; i < count; ++i)
         if ((rc = steps.out(dC[i], C[i], ldc[i], w[i]->N, r0, n, i == 0))) return rc;
       r0 += n;
     }
     return steps.finish();
   }
+  return multi_device(count, w, A, M, lda, C, ldc, s, Scratch{false, s});
+}
+
+/* Several weights of one K against rows in device memory; M > 0 */
+static int multi_device(int count, const hipq_weight_t *w, const float *A, int64_t M, int64_t lda, float *const *C,
+                        const int64_t *ldc, hipStream_t s, const Scratch &sc) {
+  int rc;
   if (M == 1 && hipq::gemv_fuses_quantizer_multi(count, w, A))
     return hipq::launch_gemv_fused_multi(count, w, A, C, s);
   /* ONE reservation for the whole call, before anything is quantized: the largest scratch any
@@ -1687,7 +1692,8 @@ int hipq_matmul_multi(int count, const hipq_weight_t *w, const float *A, int64_t
       if ((rc = rows_q6k_copy(x, M, s))) return rc;
       if (x->dtype != HIPQ_Q4_0 && wants_tiled(x, M)) {
         if (!x->gt_base && (rc = hipq::ensure_gemm_tiles(const_cast<hipq_weight *>(x)))) return rc;
-        const size_t parts = x->dtype == HIPQ_Q4_K ? hipq::gemm_q4k_split_bytes(x, M) : hipq::gemm_q6k_split_bytes(x, M);
+        const size_t parts =
+          x->dtype == HIPQ_Q4_K ? hipq::gemm_q4k_split_bytes(x, M, sc.rows) : hipq::gemm_q6k_split_bytes(x, M, sc.rows);
         const size_t tiled = ((qact_tiled_bytes(M, x->K) + 255) & ~(size_t)255) + parts;
         if (tiled > n) n = tiled;
       } else if (x->dtype == HIPQ_Q4_0 && M >= 9)
@@ -1724,7 +1730,7 @@ int hipq_matmul_multi(int count, const hipq_weight_t *w, const float *A, int64_t
       if (i < count && klass(w[i]) != 5) continue;
       if (i < count) {
         if (first) { /* the one quantization, in the row form of the matrix-core kernels */
-          if ((rc = matmul_rows(w[i], A, M, lda, C[i], ldc[i], s, 2, Scratch{false, s}))) return rc;
+          if ((rc = matmul_rows(w[i], A, M, lda, C[i], ldc[i], s, 2, sc))) return rc;
           void *mem = nullptr;
           if ((rc = workspace(s, qact_bytes(1, M, w[i]->K), &mem))) return rc;
           qa = qact_carve(1, mem, M, w[i]->K);
@@ -1774,7 +1780,7 @@ int hipq_matmul_multi(int count, const hipq_weight_t *w, const float *A, int64_t
       if (klass(w[i]) == k) {
         /* the products after the first read the rows the first one quantized */
         if (!first && (rc = workspace_unmoved(s, gen))) return rc;
-        if ((rc = matmul_tiled(w[i], A, M, lda, C[i], ldc[i], s, first ? 0 : 1, Scratch{false, s}))) return rc;
+        if ((rc = matmul_tiled(w[i], A, M, lda, C[i], ldc[i], s, first ? 0 : 1, sc))) return rc;
         first = false;
       }
   }
@@ -1794,7 +1800,6 @@ int hipq_matmul_multi(int count, const hipq_weight_t *w, const float *A, int64_t
       int nf = 0, members = 0;
       for (int i = 0; i < count; ++i)
         if (klass(w[i]) == 0 && ++members <= 64) fw[nf] = w[i], fc[nf] = C[i], fl[nf] = ldc[i], ++nf;
-      const Scratch sc{false, s};
       bool ready = false;
       hipq::F6Make make;
       if (members <= 64 && wants_f6(std::min(nf, 4), fw, M) && (rc = f6_ready(nf, fw, M, s, sc, &ready, &make))) return rc;

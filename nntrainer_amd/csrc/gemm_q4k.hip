@@ -564,20 +564,20 @@ int launch_split_sum(const float *partials, int parts, int M, int64_t N, float *
   return HIPQ_OK;
 }
 
-static TilePlan plan(const hipq_weight *w, int64_t M) {
-  return tile_plan(COST, M, w->N, w->K, w->gt_base, w->dtype == HIPQ_Q4_K && w->gt_base);
+static TilePlan plan(const hipq_weight *w, int64_t M, int64_t parts_as) {
+  return tile_plan(COST, M, w->N, w->K, w->gt_base, w->dtype == HIPQ_Q4_K && w->gt_base, parts_as);
 }
 /* bytes of the partial products of a product in parts of K (0: whole) */
-size_t gemm_q4k_split_bytes(const hipq_weight *w, int64_t M) {
-  const TilePlan t = plan(w, M);
+size_t gemm_q4k_split_bytes(const hipq_weight *w, int64_t M, int64_t parts_as) {
+  const TilePlan t = plan(w, M, parts_as);
   return t.parts > 1 ? (size_t)t.parts * (size_t)split_stride(M, w->N) * 4 : 0;
 }
 
 int launch_gemm_q4k(const hipq_weight *w, const QActTiled *qa, int M, float *C, int64_t ldc, hipStream_t s,
-                    void *partials) {
+                    void *partials, int64_t parts_as) {
   if ((M + 127) / 128 != qa->mtiles || qa->K != w->K)
     return fail(HIPQ_ERR_INVALID_ARGUMENT, "tiled activations do not match the matmul shape");
-  const TilePlan tp = plan(w, M);
+  const TilePlan tp = plan(w, M, parts_as);
   const int parts = tp.parts;
   if (partials && parts > 1) {
     const int tm = tp.rows / 32;

@@ -333,21 +333,21 @@ static int launch_tiles6(const hipq_weight *w, const QActTiled *qa, int M, float
 }
 
 static constexpr TileCost COST = {{0.f, 1.32f, 2.01f, 2.72f, 3.2f}, {0.f, 1.68f, 2.43f, 3.2f}, {0.f, 2.56f, 3.62f}};
-static TilePlan plan(const hipq_weight *w, int64_t M) {
-  return tile_plan(COST, M, w->N, w->K, w->gt_base, w->dtype == HIPQ_Q6_K && w->gt_base);
+static TilePlan plan(const hipq_weight *w, int64_t M, int64_t parts_as) {
+  return tile_plan(COST, M, w->N, w->K, w->gt_base, w->dtype == HIPQ_Q6_K && w->gt_base, parts_as);
 }
 /* bytes of the partial products of a product in parts of K (0: whole) */
-size_t gemm_q6k_split_bytes(const hipq_weight *w, int64_t M) {
-  const TilePlan t = plan(w, M);
+size_t gemm_q6k_split_bytes(const hipq_weight *w, int64_t M, int64_t parts_as) {
+  const TilePlan t = plan(w, M, parts_as);
   return t.parts > 1 ? (size_t)t.parts * (size_t)split_stride(M, w->N) * 4 : 0;
 }
 
 int launch_gemm_q6k(const hipq_weight *w, const QActTiled *qa, int M, float *C, int64_t ldc, hipStream_t s,
-                    void *partials) {
+                    void *partials, int64_t parts_as) {
   if ((M + 127) / 128 != qa->mtiles || qa->K != w->K)
     return fail(HIPQ_ERR_INVALID_ARGUMENT, "tiled activations do not match the matmul shape");
   if (!w->gt_base) return fail(HIPQ_ERR_INVALID_ARGUMENT, "the Q6_K prefill product needs the weight's tile copy");
-  const TilePlan tp = plan(w, M);
+  const TilePlan tp = plan(w, M, parts_as);
   const int parts = tp.parts;
   if (partials && parts > 1) {
     const int tm = tp.rows / 32;

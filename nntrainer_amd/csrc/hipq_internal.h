@@ -304,14 +304,16 @@ int launch_gemm_q4k_gated(const hipq_weight *wa, const hipq_weight *wm, const QA
  * where those of 64 take 1.35 / 1.68, and are the faster ones up to about 200 rows wherever the chip is not full otherwise:
  * over 89 + 63 sizes of 17 to 320 rows (700 x 1536 to 40000 x 2048) 10 % less a call, 30 % at the smallest (us, Q6_K, 64 rows
  * -> 32: 32 rows of 1000 x 4096 16.9 -> 14.9, of 16822 x 3328 26.6 -> 22.5, 96 of 6000 x 1024 14.7 -> 12.3; Q4_K 160 of 12288 x
- * 4096 39.2 -> 32.7). `copy`: the weight has its tile copy, which they read; `split`: parts are possible. */
+ * 4096 39.2 -> 32.7). `copy`: the weight has its tile copy, which they read; `split`: parts are possible; `parts_as`: the
+ * product takes as many parts as one of that many rows, whose sums it then has (0: its own number). */
 struct TileCost {
   float c32[5], c64[4], c128[3];
 };
 struct TilePlan {
   int rows, parts;
 };
-inline TilePlan tile_plan(const TileCost &c, int64_t M, int64_t N, int64_t K, bool copy, bool split) {
+inline TilePlan tile_plan(const TileCost &c, int64_t M, int64_t N, int64_t K, bool copy, bool split, int64_t parts_as = 0) {
+  const int given = parts_as && split ? tile_plan(c, parts_as, N, K, copy, split).parts : 0;
   const int64_t nsb = K / 256, nt = (N + 127) / 128;
   TilePlan best{64, 1};
   double least = 1e30;
@@ -319,7 +321,7 @@ inline TilePlan tile_plan(const TileCost &c, int64_t M, int64_t N, int64_t K, bo
     const int64_t mt = (M + h - 1) / h;
     const int fit = h == 32 ? 4 : h == 64 ? 3 : 2;
     const float *t = h == 32 ? c.c32 : h == 64 ? c.c64 : c.c128;
-    for (int p = 1; p <= (split ? 8 : 1); ++p) {
+    for (int p = given ? given : 1; p <= (given ? given : split ? 8 : 1); ++p) {
       if (p > 1 && (nsb < 3 * p || p * M * N * 4 > ((int64_t)64 << 20))) break;
       const int64_t per = (nsb + p - 1) / p, parts = (nsb + per - 1) / per, a_cu = (mt * nt * parts + 255) / 256;
       double us = (double)per * ((double)(a_cu / fit) * t[fit] + t[a_cu % fit]);
@@ -338,13 +340,13 @@ int launch_split_sum(const float *partials, int parts, int M, int64_t N, float *
 int launch_gemm_q4k_multi(int count, const hipq_weight *const *w, const QActTiled *qa, int M, float *const *C,
                           const int64_t *ldc, hipStream_t s);
 int launch_gemm_q6k(const hipq_weight *w, const QActTiled *qa, int M, float *C, int64_t ldc, hipStream_t s,
-                    void *partials = nullptr);
-size_t gemm_q6k_split_bytes(const hipq_weight *w, int64_t M);
-/* partials: gemm_q4k_split_bytes(w, M) bytes of device memory (or null): with few tiles the product
+                    void *partials = nullptr, int64_t parts_as = 0);
+size_t gemm_q6k_split_bytes(const hipq_weight *w, int64_t M, int64_t parts_as = 0);
+/* partials: gemm_q4k_split_bytes(w, M, parts_as) bytes of device memory (or null): with few tiles the product
  * is formed in parts of K that run side by side and are then added */
 int launch_gemm_q4k(const hipq_weight *w, const QActTiled *qa, int M, float *C,
-                    int64_t ldc, hipStream_t s, void *partials = nullptr);
-size_t gemm_q4k_split_bytes(const hipq_weight *w, int64_t M);
+                    int64_t ldc, hipStream_t s, void *partials = nullptr, int64_t parts_as = 0);
+size_t gemm_q4k_split_bytes(const hipq_weight *w, int64_t M, int64_t parts_as = 0);
 /* gemm_rows_q4k.hip: Q4_K for a few rows on the matrix cores with the reference's bits; fits: the row
  * counts and shapes that should take it (up to 16 rows, in passes of up to 8 for the launcher); qa in
  * the form of launch_quantize_q8_K_rowmma, the first pair_rows rows under the 4-row quantizer's rule;

@@ -198,9 +198,9 @@ def test_grouped_calls_on_a_few_page_locked_rows(hipq, cr, kind, m):
     ("q4_0", 1400, 1024, 3072, 0),      # five steps of 256 rows, the last of 376
     ("q4_0", 2100, 1024, 2048, 8),      # eight steps; strided rows on both sides
     ("q4_K", 700, 2048, 12288, 0),      # every step takes the prefill GEMM on whole K: two steps
-    ("q4_K", 1100, 2048, 4096, 0),      # a step would run in parts of K (other bits): one piece
+    ("q4_K", 1100, 2048, 4096, 0),      # a step alone would be formed in parts of K, the whole call is not
     ("q6_K", 1100, 1024, 4096, 4),
-    ("q6_K", 520, 3072, 8448, 0),       # the whole call walks K whole, a step alone would not: two steps on whole K
+    ("q6_K", 520, 3072, 8448, 0),       # likewise
     ("q4_0", 512, 1024, 3072, 0),       # outputs of 6 MB: one piece
 ])
 def test_prefill_rows_in_steps_give_the_device_bits(hipq, cr, kind, m, k, n, pad):
@@ -253,3 +253,48 @@ def test_prefill_rows_in_steps_give_the_device_bits(hipq, cr, kind, m, k, n, pad
             p.free()
         for x in (w, w2, wd):
             x.destroy()
+
+
+@pytest.mark.parametrize("entry,m,k,n,nd", [("multi", 520, 3072, 8448, 0), ("swiglu", 520, 3072, 8448, 0), ("down", 520, 1024, 6400, 8192),
+                                               ("down", 520, 2048, 8448, 8448), ("multi", 1100, 1536, 3072, 0)])
+def test_grouped_q6_K_prefill_rows_cross_in_steps(hipq, cr, entry, m, k, n, nd):
+    """The calls of several weights: 512 rows and more cross in steps of 256, the last of up to 511, whatever a step's 256 rows
+    alone would be formed in. At the first three sizes that would be parts of K where the whole call walks K whole, at the
+    fourth the down projection of the whole call is formed in parts of K. A step's products take the whole call's parts, so
+    that the outputs have the bits of the device-memory call."""
+    import gpu_util as gu
+    import torch
+
+    def weight(j, rows, cols):
+        few = cr.quantize_weights(cr.oracle(), "q6_K", synth.normal(9800 + j, (61, cols), 0.05)).reshape(61, -1)
+        return capi.Weight("q6_K", rows, cols, np.ascontiguousarray(few[np.random.RandomState(j).randint(0, 61, rows)]))
+
+    ws = [weight(0, n, k), weight(1, n, k)] + ([weight(2, nd, n)] if nd else [])
+    a = synth.normal(9810 + m, (m, k))
+    pa = _Pinned((m, k), a)
+    shapes = [(m, n), (m, n)] if entry == "multi" else [(m, nd or n)]
+    out = [_Pinned(x, np.nan) for x in shapes]
+    dev = [torch.full(x, float("nan"), device="cuda") for x in shapes]
+
+    def call(rows, res, **kw):
+        if entry == "multi":
+            capi.matmul_multi(ws, rows, m, res, **kw)
+        else:
+            (capi.mlp_swiglu if entry == "swiglu" else capi.mlp_swiglu_down)(*ws, rows, m, res[0], **kw)
+
+    try:
+        with capi.LaunchTiming(64) as t:
+            call(gu.dev(a), dev, stream=gu.stream())
+            torch.cuda.synchronize()
+        in_parts = ["split" in name for name, _ in t.launches if name.startswith("gemm_q6k")]
+        with capi.LaunchTiming(64) as t:
+            call(pa.addr, [o.addr for o in out], mem=capi.MEM_HOST)
+        steps = ["split" in name for name, _ in t.launches if name.startswith("gemm_q6k")]
+        for o, d in zip(out, dev):
+            assert np.array_equal(o.arr.view(np.uint32), d.cpu().numpy().view(np.uint32))
+        assert len(in_parts) == len(ws) and steps == (m // 256) * in_parts, (in_parts, steps)
+    finally:
+        for x in [pa] + out:
+            x.free()
+        for w in ws:
+            w.destroy()
