@@ -168,13 +168,7 @@ __device__ __forceinline__ void store_chunk(const Chunk &c, SmemQ40 &sm) {
 
 /* da * dw with da taken from lane R of the DPP row (16 lanes) inside the multiply itself */
 #define HIPQ_MUL_BCAST(DA, DW, R)                                                                   \
-  ({                                                                                                \
-    float t_;                                                                                       \
-    asm("v_mul_f32_dpp %0, %1, %2 row_newbcast:" #R " row_mask:0xf bank_mask:0xf"                   \
-        : "=v"(t_)                                                                                  \
-        : "v"(DA), "v"(DW));                                                                        \
-    t_;                                                                                             \
-  })
+  (__builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, DA), 0x150 + (R), 0xf, 0xf, true)) * (DW))
 
 /* What one wavefront's 16 x 16 tile needs of four blocks (half a chunk): its lane's 8 bytes of
  * each block on both sides (av[p]: blocks 2 p and 2 p + 1) and the four weight scales of its column. */

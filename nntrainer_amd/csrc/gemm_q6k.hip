@@ -13,7 +13,7 @@
  * (|v| <= 4064) does not fit int8 and neither factor splits into digits whose products do
  * (one of them has eight bits), so the PRODUCT is split into a signed low byte and a signed
  * high byte:  4 v = 256 * h + l  (the factor 4 puts the split on a byte boundary of the
- * 16-bit lanes the product is formed in, see scale_split), and
+ * 16-bit lanes the product is formed in, see q6k_device.h), and
  *       4 I = sum_k l[k] * q8[k]  +  256 * sum_k h[k] * q8[k]
  * is two chains of v_mfma_i32_32x32x32_i8, exact int32 (|4 I| < 2^30). There is no min term
  * (the format is symmetric). Per super-block and output the ALU does
@@ -30,7 +30,7 @@
  * of a Q6_K weight): lane (n, g) of a wavefront owns half g (128 weights) of column n's
  * super-block, eight steps of sixteen weights with one scale each.
  */
-#include "gemv_device.h"
+#include "q6k_device.h"
 
 namespace {
 
@@ -107,26 +107,6 @@ template <int TM> struct InFlight6 {
   static constexpr int SECOND = TM + 4; /* the same and the next super-block's scales */
 };
 
-/* a * b + c in both 16-bit lanes (the compiler's own choice for the expression is a subtract
- * and a multiply) */
-__device__ __forceinline__ uint32_t pk_mad(uint32_t a, uint32_t b, uint32_t c) {
-  uint32_t r;
-  asm("v_pk_mad_i16 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return r;
-}
-/* Four 6-bit weights u, one per byte of x, times the step's scale s. In 16-bit lanes
- *     t = u * 4s + (128 - 128 s) = 4 (u - 32) s + 128,     |4 (u - 32) s| <= 16256,
- * so that 4 (u - 32) s = 256 * hi(t) + (lo(t) - 128) with hi the signed high byte of t and
- * lo(t) - 128 = lo(t) ^ 0x80 a signed byte: both operand bytes come out of t by byte
- * selection, no shifts or masks. The two planes then hold four times the product; the
- * factor leaves with the column scale. */
-__device__ __forceinline__ void scale_split(uint32_t x, uint32_t s2, uint32_t c2, int &l, int &h) {
-  const uint32_t ta = pk_mad(__builtin_amdgcn_perm(x, x, 0x0c020c00u), s2, c2); /* bytes 0 and 2 */
-  const uint32_t tb = pk_mad(__builtin_amdgcn_perm(x, x, 0x0c030c01u), s2, c2); /* bytes 1 and 3 */
-  l = (int)(__builtin_amdgcn_perm(tb, ta, 0x06020400u) ^ 0x80808080u); /* low bytes: a0 b0 a1 b1 */
-  h = (int)__builtin_amdgcn_perm(tb, ta, 0x07030501u);                 /* high bytes */
-}
-
 /* four 32-deep steps of one 128-deep stage: H = which half of the lane's eight steps */
 template <int H, int TM>
 __device__ __forceinline__ void stage_mma(const Smem6<TM> &sm, int slot, const WHalf6 &W, uint2 sc8, int lane,
@@ -145,21 +125,8 @@ __device__ __forceinline__ void stage_mma(const Smem6<TM> &sm, int slot, const W
     }
     const uint32_t x0 = ks & 1 ? W.q[ks >> 1].z : W.q[ks >> 1].x, x1 = ks & 1 ? W.q[ks >> 1].w : W.q[ks >> 1].y;
     const uint32_t hb = ks == 0 ? W.h.x : ks == 1 ? W.h.y : ks == 2 ? W.h.z : W.h.w;
-    /* four times the scale, sign-extended, in both 16-bit lanes; c2 = 128 - 128 * scale */
-    const int s = __builtin_amdgcn_sbfe((int)scw, 8 * ks, 8) << 2;
-    const uint32_t s2 = __builtin_amdgcn_perm((uint32_t)s, (uint32_t)s, 0x05040100u);
-    const uint32_t c2 = pk_mad(s2, 0xffe0ffe0u, 0x00800080u);
-    /* 6-bit weights, one per byte: the even ones (0, 2 .. 14), then the odd ones */
-    const uint32_t e0 = (x0 & HIPQ_M4) | ((hb << 4) & 0x30303030u);
-    const uint32_t e1 = (x1 & HIPQ_M4) | ((hb << 2) & 0x30303030u);
-    const uint32_t o0 = ((x0 >> 4) & HIPQ_M4) | (hb & 0x30303030u);
-    const uint32_t o1 = ((x1 >> 4) & HIPQ_M4) | ((hb >> 2) & 0x30303030u);
-    int l0, l1, l2, l3, h0, h1, h2, h3;
-    scale_split(e0, s2, c2, l0, h0);
-    scale_split(e1, s2, c2, l1, h1);
-    scale_split(o0, s2, c2, l2, h2);
-    scale_split(o1, s2, c2, l3, h3);
-    const v4i bl = {l0, l1, l2, l3}, bh = {h0, h1, h2, h3};
+    const hipq_q6k_planes p = hipq_q6k_expand(x0, x1, hb, __builtin_amdgcn_sbfe((int)scw, 8 * ks, 8));
+    const v4i bl = {(int)p.l[0], (int)p.l[1], (int)p.l[2], (int)p.l[3]}, bh = {(int)p.h[0], (int)p.h[1], (int)p.h[2], (int)p.h[3]};
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm) {
       Dl[tm] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[ks & 1][tm], bl, (H == 0 && ks == 0) ? zero16 : Dl[tm], 0, 0, 0);

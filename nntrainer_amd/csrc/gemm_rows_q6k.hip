@@ -18,7 +18,7 @@
  * instructions (430 a super-block and wavefront) and a round's latency; what it takes against the GEMV engine stands at gemm_rows_q6k_fits.
  */
 #include "hipq_internal.h"
-#include "gemv_device.h"
+#include "q6k_device.h"
 #include <algorithm>
 
 namespace {
@@ -39,20 +39,6 @@ constexpr int LDS_REC = (LDS_DA + 4 * SBR * TC * 4 + 255) / 256 * 256; /* [wavef
 constexpr int LDS_DW = LDS_REC + SBR * NREG * 2 * 256 * 4;
 constexpr int LDS_BYTES = LDS_DW + SBR * 32 * 4;
 static_assert(ACT_BYTES % 16 == 0 && 3 * LDS_BYTES <= 160 * 1024, "three workgroups a CU");
-
-__device__ __forceinline__ uint32_t pk_mad(uint32_t a, uint32_t b, uint32_t c) {
-  uint32_t r;
-  asm("v_pk_mad_i16 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return r;
-}
-/* four 6-bit weights times their scale as a low and a high int8 plane of four times the product (scale_split of
- * gemm_q6k.hip, which derives it) */
-__device__ __forceinline__ void scale_split(uint32_t x, uint32_t s2, uint32_t c2, uint32_t &l, uint32_t &h) {
-  const uint32_t ta = pk_mad(__builtin_amdgcn_perm(x, x, 0x0c020c00u), s2, c2);
-  const uint32_t tb = pk_mad(__builtin_amdgcn_perm(x, x, 0x0c030c01u), s2, c2);
-  l = __builtin_amdgcn_perm(tb, ta, 0x06020400u) ^ 0x80808080u;
-  h = __builtin_amdgcn_perm(tb, ta, 0x07030501u);
-}
 
 struct Regs { /* a lane's half of a super-block: steps s = 0 .. 7 of sixteen weights, blocks s / 2 of its half */
   v4i q[4], h[2], hd;
@@ -144,33 +130,27 @@ __global__ __launch_bounds__(NT, 2) void gemm_rows_q6k_kernel(WView w, QView a, 
           const int s = 2 * b + hh;
           const uint32_t x0 = (uint32_t)W.q[s >> 1][2 * (s & 1)], x1 = (uint32_t)W.q[s >> 1][2 * (s & 1) + 1];
           const uint32_t hb = (uint32_t)W.h[s >> 2][s & 3];
-          const int sc = __builtin_amdgcn_sbfe(W.hd[s >> 2], 8 * (s & 3), 8) << 2;
-          const uint32_t s2 = __builtin_amdgcn_perm((uint32_t)sc, (uint32_t)sc, 0x05040100u);
-          const uint32_t c2 = pk_mad(s2, 0xffe0ffe0u, 0x00800080u);
-          /* 6-bit weights, one a byte: the even ones, then the odd ones */
-          const uint32_t e0 = (x0 & HIPQ_M4) | ((hb << 4) & 0x30303030u), e1 = (x1 & HIPQ_M4) | ((hb << 2) & 0x30303030u);
-          const uint32_t o0 = ((x0 >> 4) & HIPQ_M4) | (hb & 0x30303030u), o1 = ((x1 >> 4) & HIPQ_M4) | ((hb >> 2) & 0x30303030u);
-          uint32_t l0, l1, l2, l3, h0, h1, h2, h3;
-          scale_split(e0, s2, c2, l0, h0);
-          scale_split(e1, s2, c2, l1, h1);
-          scale_split(o0, s2, c2, l2, h2);
-          scale_split(o1, s2, c2, l3, h3);
+          const hipq_q6k_planes p = hipq_q6k_expand(x0, x1, hb, __builtin_amdgcn_sbfe(W.hd[s >> 2], 8 * (s & 3), 8));
           /* weights 4 k .. 4 k + 3 in order: the block's dword of sum 4 hh + k */
-          bl[0][b] = (int)__builtin_amdgcn_perm(l2, l0, 0x05010400u), bl[1][b] = (int)__builtin_amdgcn_perm(l2, l0, 0x07030602u);
-          bl[2][b] = (int)__builtin_amdgcn_perm(l3, l1, 0x05010400u), bl[3][b] = (int)__builtin_amdgcn_perm(l3, l1, 0x07030602u);
-          bh[0][b] = (int)__builtin_amdgcn_perm(h2, h0, 0x05010400u), bh[1][b] = (int)__builtin_amdgcn_perm(h2, h0, 0x07030602u);
-          bh[2][b] = (int)__builtin_amdgcn_perm(h3, h1, 0x05010400u), bh[3][b] = (int)__builtin_amdgcn_perm(h3, h1, 0x07030602u);
+          bl[0][b] = (int)__builtin_amdgcn_perm(p.l[2], p.l[0], 0x05010400u), bl[1][b] = (int)__builtin_amdgcn_perm(p.l[2], p.l[0], 0x07030602u);
+          bl[2][b] = (int)__builtin_amdgcn_perm(p.l[3], p.l[1], 0x05010400u), bl[3][b] = (int)__builtin_amdgcn_perm(p.l[3], p.l[1], 0x07030602u);
+          bh[0][b] = (int)__builtin_amdgcn_perm(p.h[2], p.h[0], 0x05010400u), bh[1][b] = (int)__builtin_amdgcn_perm(p.h[2], p.h[0], 0x07030602u);
+          bh[2][b] = (int)__builtin_amdgcn_perm(p.h[3], p.h[1], 0x05010400u), bh[3][b] = (int)__builtin_amdgcn_perm(p.h[3], p.h[1], 0x07030602u);
         }
         int S[4][NREG];
+        v16i Dl[2], Dh[2];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const v16i Dl = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[k], bl[k], zero16, 0, 0, 0);
-          const v16i Dh = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[k], bh[k], zero16, 0, 0, 0);
+        for (int k = 0; k <= 4; ++k) { /* a sum's results are read behind the next one's steps, not waited for */
+          if (k < 4) {
+            Dl[k & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[k], bl[k], zero16, 0, 0, 0);
+            Dh[k & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[k], bh[k], zero16, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          if (k > 0) {
 #pragma unroll
-          for (int r = 0; r < NREG; ++r) S[k][r] = ((Dh[r] << 8) + Dl[r]) >> 2; /* the planes hold four times the product */
-          /* The registers of the twelve results that nobody reads stay taken until the step is over: written by the assembly of
-           * pk_mad, whose hazards the compiler does not see, they would be overwritten by the step's late results. */
-          asm volatile("" ::"v"(Dl), "v"(Dh));
+            for (int r = 0; r < NREG; ++r) /* the planes hold four times the product */
+              S[k - 1][r] = ((Dh[(k - 1) & 1][r] << 8) + Dl[(k - 1) & 1][r]) >> 2;
+          }
         }
 #pragma unroll
         for (int r = 0; r < NREG; ++r) *(v4i *)(rec + (r * 2 + hh) * 256) = v4i{S[0][r], S[1][r], S[2][r], S[3][r]};

@@ -1,0 +1,24 @@
+"""Rules that the device sources keep, read off their text."""
+import glob
+import os
+import re
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "nntrainer_amd", "csrc")
+SOURCES = sorted(glob.glob(os.path.join(CSRC, "*.hip")) + glob.glob(os.path.join(CSRC, "*.h")))
+
+
+@pytest.mark.parametrize("path", [p for p in SOURCES if "__builtin_amdgcn_mfma" in open(p).read()], ids=os.path.basename)
+def test_no_assembly_computes_beside_matrix_instructions(path):
+    """A matrix instruction writes its results many cycles after it was issued, and the compiler keeps other vector
+    instructions away from them; inline assembly it does not look into. Where a file issues matrix instructions, and in what
+    it includes from here for them, assembly may wait and order, but names no vector instruction."""
+    files = [path]
+    text = open(path).read()
+    files += [os.path.join(CSRC, x) for x in re.findall(r'#include "(q6k_device\.h|moe_tile_device\.h)"', text)]
+    found = []
+    for f in files:
+        for template in re.findall(r'\basm\s*(?:volatile\s*)?\(\s*((?:"[^"]*"\s*)*)', open(f).read()):
+            found += [(os.path.basename(f), x) for x in re.findall(r"\b(?:v|buffer|global|flat|ds)_\w+", template)]
+    assert not found
