@@ -148,28 +148,36 @@ HIPQ_API int hipq_quantize_q8_K(const float *A, int64_t M, int64_t K, int64_t ld
  *  form of gemm_q4_0 / gemm_q4_K / gemm_q6_K (x86_compute_backend.cpp:301-341)
  *  as reached from FloatTensor::dotQnK (float_tensor.cpp:923-969). M == 1 runs
  *  the decode GEMV kernels, M > 1 the prefill GEMM kernels. lda >= K and
- *  ldc >= N are row strides in elements. With M == 1, K <= 4096, N < 32768 and
- *  device memory the call is a single kernel launch (the GEMV quantizes the row
- *  itself) and uses no workspace.
+ *  ldc >= N are row strides in elements. With M == 1, A on 16 bytes, device memory and
+ *  N < 32768 (K <= 4096), N <= 8192 (K <= 12288) or N <= 4096 (K <= 16384) the call is a
+ *  single kernel launch (the GEMV quantizes the row itself) and uses no workspace.
  *  Outputs carry the bits of the reference's AVX2 kernels for every Q4_0 product and for
- *  Q4_K with up to 8 rows (up to 16 against 1024 columns or more, up to 64 where
- *  columns / 32 x rows / 8 x K / 256 <= 8192, once the weight's copy described below exists
- *  or may be made) and Q6_K with up to 16 rows (up to 8 for matrices
+ *  Q4_K with up to 8 rows (against 1024 columns or more, once the weight's copy described
+ *  below exists or may be made, up to 16, and up to 64 where, the first two quotients rounded up,
+ *  columns / 32 x rows / 8 x K / 256 <= 8192) and Q6_K with up to 16 rows (up to 8 for matrices
  *  of 2^24 weights or more, up to 4 from 2^25, up to 2 from 2^28: there the matrix cores are
  *  faster, up to several times); with more rows the K-formats run on the
  *  int8 matrix cores and agree with the reference to 1e-4 of the output's maximum (same
- *  quantized activations, another order of the fp32 sums). The first product of many rows of
- *  a weight adds a copy of it in the kernels' load order, kept until hipq_weight_destroy,
- *  beside the weight as it is stored: Q4_K 0.56 bytes per weight beside 0.56, Q6_K 0.875
- *  beside 0.82, Q4_0 0.8125 beside 0.5625 (rows padded to 32, K to 256; from nine to 65 rows
- *  on, by size). The copies of Q4_0 weights lie in blocks of 64 MiB (larger ones in blocks of
- *  their own) that are given back with the last copy in them, one empty block excepted, which
- *  hipq_shutdown frees. Q4_K with 5..16 rows and 1024
- *  columns or more (4 rows from 4096, 3 from 8192 columns) reads the same copy: those row
+ *  quantized activations, another order of the fp32 sums; the sums of few columns are formed in
+ *  parts of K). The first product of a weight on a matrix-core kernel that reads it adds a copy of
+ *  the weight in the kernels' load order, kept until hipq_weight_destroy,
+ *  beside the weight as it is stored: Q4_K 0.56 bytes per weight beside 0.56 (from two to nine rows
+ *  on, by size), Q6_K 0.875 beside 0.82 (from two to 17 rows on, by size, the rows of
+ *  hipq_matmul_each_row too: 545 MB for an lm_head of 151936 x 4096 that only ever sees a batch's
+ *  decode rows), Q4_0 0.8125 beside 0.5625 (rows padded to 32, K to 256; from nine to 65 rows
+ *  on, by size). That first product of a Q4_K or Q6_K weight allocates the copy (hipMalloc) and
+ *  waits on the null stream until it is made. The copies of Q4_0 weights lie in blocks of 64 MiB
+ *  (larger ones in blocks of their own) that are given back with the last copy in them, one empty
+ *  block excepted, which hipq_shutdown frees. Q4_K with 5..16 rows and 1024 columns or more (4 rows
+ *  from 4096 columns, from 6144 where K >= 4096, 3 from 8192 or 12288, 2 from 16384 where K <= 1024)
+ *  reads the same copy: those row
  *  counts run on the matrix cores as well, with the reference's bits (a batch of decode
  *  rows against a 12288 x 4096 matrix: 11 us for eight, 14 us for sixteen, 8 us for one).
  *  Q4_0 has the same kind of kernel for a few rows (gemm_rows_q40.hip, off the weight as it is
- *  stored: eight rows against 12288 x 4096 in 11 us, against 151936 x 1024 in 26 us); every Q4_0
+ *  stored: eight rows against 12288 x 4096 in 11 us, against 151936 x 1024 in 26 us), and Q6_K with
+ *  two to sixteen rows where that is the faster (gemm_rows_q6k.hip, off the copy; a call that is being
+ *  captured or meets a full device before the weight has its copy reads the weight as it is stored, with
+ *  the same bits); every Q4_0
  *  kernel carries the reference's bits, so there the row count only selects the fastest, and a
  *  product of many rows that cannot have the weight's copy takes a slower kernel that reads the
  *  weight as it is stored: on a full device, in a call that is being captured into a graph before
@@ -204,15 +212,15 @@ HIPQ_API int hipq_matmul_each_row(hipq_weight_t w, const float *A, int64_t rows,
  *  and Q4_K) returns HIPQ_ERR_NOT_SUPPORTED. The call performs no device
  *  allocation and no free and enqueues the same kernels as hipq_matmul, so
  *  results are the same bits wherever the same kernel runs. Where the two may take
- *  different kernels: a weight that has no tile copy yet (only an allocating call builds
+ *  different kernels: a Q6_K weight that has no tile copy yet (only an allocating call builds
  *  one) goes through the GEMV engine here, which carries the reference's bits where
- *  hipq_matmul's matrix-core product agrees to 1e-4; and a Q4_K or Q6_K product of up to
- *  128 rows that hipq_matmul forms in parts of K takes whole rows here when the parts'
- *  partial sums do not fit the slot beside the activations, or when C is not 16-byte
- *  aligned with ldc a multiple of four (both entry points then): the fp32 sums then have
- *  another order, within the 1e-4 of every matrix-core product. Results of the K-formats'
- *  matrix-core products are therefore stable to the tolerance, not to the bit, across ldc,
- *  alignment and entry point. */
+ *  hipq_matmul's matrix-core product agrees to 1e-4; a Q4_K weight without one is read as it is
+ *  stored, by the GEMV engine up to 8 rows (the reference's bits) and by the prefill GEMM beyond
+ *  (1e-4, also where hipq_matmul has the bits); and a Q4_K or Q6_K product that hipq_matmul forms
+ *  in parts of K walks K whole here when the parts' partial sums do not fit the slot beside the
+ *  activations: the fp32 sums then have another order, within the 1e-4 of every matrix-core
+ *  product. Results of the K-formats' matrix-core products are therefore stable to the tolerance,
+ *  not to the bit, across entry points; across ldc and the alignment of C they are the same bits. */
 HIPQ_API int hipq_matmul_noalloc(hipq_weight_t w, const float *A, int64_t M, int64_t lda,
                                  float *C, int64_t ldc, void *stream);
 
@@ -225,8 +233,8 @@ HIPQ_API int hipq_matmul_noalloc(hipq_weight_t w, const float *A, int64_t M, int
  *  Q4_K weights with 2 to 16 rows (a decode step of a batch; to 64 rows on narrow weights),
  *  through the few-rows kernels, with the reference's bits. Every output equals what
  *  hipq_matmul gives for that weight alone bit for bit, except where the single call of a
- *  Q4_K weight takes the prefill GEMM for those rows (then to 1e-4, as every product of that
- *  kernel). */
+ *  Q4_K weight has not the reference's bits but those of the prefill GEMM (then to 1e-4, as every
+ *  product of that kernel: several weights together walk K whole, or take the few-rows kernel). */
 HIPQ_API int hipq_matmul_multi(int count, const hipq_weight_t *w, const float *A,
                                int64_t M, int64_t lda, float *const *C,
                                const int64_t *ldc, int mem, void *stream);
@@ -237,8 +245,8 @@ HIPQ_API int hipq_matmul_multi(int count, const hipq_weight_t *w, const float *A
  *  "ffn_up" (Y) and "ffn_gate" (Z) and the SwiGLULayer on their outputs
  *  (Applications/CausalLM/layers/swiglu.cpp:40-62, causal_lm.cpp:672-695); here one call that
  *  quantizes A once, and for one row (K <= 4096, 2 N < 32768, device memory) one kernel launch
- *  in which the two products never leave the registers. The products are those of hipq_matmul
- *  bit for bit; the exponential is the device's expf. */
+ *  in which the two products never leave the registers. The products are those of
+ *  hipq_matmul_multi, and so of hipq_matmul to the same extent; the exponential is the device's expf. */
 HIPQ_API int hipq_mlp_swiglu(hipq_weight_t w_act, hipq_weight_t w_mul, const float *A, int64_t M,
                              int64_t lda, float *out, int64_t ldo, int mem, void *stream);
 
@@ -343,7 +351,7 @@ HIPQ_API int hipq_device_download(void *dst_host, const void *src_device, size_t
  *  context, cl_context.cpp:83). Tensors that live in it cross to the GPU by DMA as they are
  *  (a prefill of 512 rows and more with 16 MiB of outputs in steps of 256 rows, a step's output
  *  leaving on a second stream of the library's while the next step's rows arrive and are
- *  multiplied; up to 128 rows of at most 2 MiB a side without a copy engine at all);
+ *  multiplied, with the bits of the call in one piece; up to 128 rows of at most 2 MiB a side without a copy engine at all);
  *  any other host memory passed with HIPQ_MEM_HOST goes through a pinned staging ring inside
  *  the library (8 MiB), at the speed of a host memcpy. */
 HIPQ_API int hipq_host_alloc(void **ptr, size_t bytes);

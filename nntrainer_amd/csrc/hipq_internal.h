@@ -297,10 +297,13 @@ int launch_gemm_q4k_gated(const hipq_weight *wa, const hipq_weight *wm, const QA
  * whole), by what each choice should take. Per super-block a CU's tiles of 64 rows x 128 columns take c64[n] us with n of
  * them on it (three fit), those of 32 rows c32[n] (four fit), those of 128 c128[n] (two fit); a CU has the launch's tiles in rounds of as many as fit;
  * parts write and read their sums (0.26 us a megabyte, and a launch of 1 us). The figures are fitted (rms 5 %) to 99 sizes
- * a format, 65 to 1000 rows of 1024 x 4096 to 4096 x 12288, each with both heights and 1 to 8 parts: by them the products
- * take 1.7 % (Q4_K) and 2.9 % (Q6_K) less than by the rule before (parts up to 192 tiles of 64 rows), 1 % (Q4_K) and 2 % more
- * than the fastest choice; where that rule had left the chip unevenly filled, 400 rows of 4096 x 12288, 84 -> 69 and 100 ->
- * 72 us. Parts change the order of a sum, so they have to gain 1.5 us. Tiles of 32 rows walk a super-block in 0.92 / 1.32 us
+ * a format, 65 to 1000 rows of 1024 x 4096 to 4096 x 12288, each with both heights and 1 to 8 parts. What they are used for is
+ * the order of the choices: over 730 sizes a format, 17 to 2048 rows of 512 to 152000 columns and K of 512 to 12288, each
+ * timed with every height and number of parts, the choice takes 0.8 % (Q4_K) and 1.1 % (Q6_K) more than the fastest one on
+ * average, 14 and 15 % less than by the rule before (parts up to 192 tiles of 64 rows; more than 2 % faster at 447 and 417
+ * sizes, slower at 8 and 33, at worst 123 -> 134 us, 400 rows of 17536 x 6400 Q4_K, and 125 -> 156, 696 of 8781 x 7168 Q6_K, where
+ * 128-row tiles are the faster ones). The time itself they give within 4 % up to 25 us; a full chip runs at a lower clock
+ * (1.6 to 1.9 of 2.4 GHz), so that 60 us take a quarter more than the estimate and 150 a third. Parts change the order of a sum, so they have to gain 1.5 us. Tiles of 32 rows walk a super-block in 0.92 / 1.32 us
  * where those of 64 take 1.35 / 1.68, and are the faster ones up to about 200 rows wherever the chip is not full otherwise:
  * over 89 + 63 sizes of 17 to 320 rows (700 x 1536 to 40000 x 2048) 10 % less a call, 30 % at the smallest (us, Q6_K, 64 rows
  * -> 32: 32 rows of 1000 x 4096 16.9 -> 14.9, of 16822 x 3328 26.6 -> 22.5, 96 of 6000 x 1024 14.7 -> 12.3; Q4_K 160 of 12288 x
