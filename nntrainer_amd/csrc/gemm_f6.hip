@@ -28,7 +28,7 @@
  * Per 32 x 32 x 32 that is two matrix instructions and 16 multiply-adds, 90 clk of a SIMD by themselves
  * (210 with the int8 step).
  * Measured, kernel us, int8 kernel -> this one: 512 rows of 12288 x 4096 151 -> 62, of 3072 x 1024 14.7 -> 9.6,
- * 1024 x 1024 7.6 -> 6.7, 1024 x 3072 14.1 -> 12.0; 333 of 5000 x 2048 29 -> 14; 300 of 1000 x 896 (a K that the int8
+ * 1024 x 1024 7.6 -> 6.7, 1024 x 3072 14.1 -> 12.0 (10.4 with two wavefronts a tile, HALF_TILES); 333 of 5000 x 2048 29 -> 14; 300 of 1000 x 896 (a K that the int8
  * kernel does not take: eight-row GEMV passes) 135 us a call -> 11. At the first shape the clock falls to about
  * 1.85 GHz under this mix, and 115 clk a step at that clock are 48 us of the 62.
  *
@@ -64,6 +64,13 @@ typedef __attribute__((address_space(3))) void *lds_ptr;
 constexpr int BM = 32, BN = 128, NT = 256;
 constexpr int PARTS = 32 * 384;     /* the activations' parts of 32 rows and one chunk: [block 8]{[64 lanes][16], [64 lanes][8]} */
 constexpr int BUF = PARTS + 32 * 16; /* a row buffer in LDS: the parts, then the block scales [32 rows][8] fp16 */
+constexpr int MAX_Y = 65535; /* of a grid */
+/* Up to so many workgroups of 32 x 128 two wavefronts share a tile (NS = 8): half of the chip's SIMDs would have no wavefront,
+ * and a wavefront alone on its SIMD takes a step's vector instructions one after the other, 150 clk with sixteen sums and 115
+ * with eight. us a call, a wavefront a tile / two: 512 rows of 1024 x 1024 9.8 / 9.4, x 3072 17.6 / 16.1, 100 of 4096 x 4096 17.1 / 15.2,
+ * 200 of 673 x 7200 29.6 / 26.2; with more tiles the halves fill the chip twice: 192 (512 of 1536 x 2048) 13.7 / 15.0, 256 (256 of
+ * 4096 x 4096) 19.3 / 23.9. */
+constexpr int HALF_TILES = 128;
 constexpr int CHUNK = hipq::F6_CHUNK, WTILE = hipq::F6_WTILE; /* bytes of 64 rows / 32 columns and one chunk */
 
 __device__ __forceinline__ rsrc_t make_rsrc(const void *p, uint32_t bytes) {
@@ -85,7 +92,7 @@ struct MultiF6 { /* up to four weights of one K, their column tiles side by side
 
 /* The copies made in front of this launch are complete, by stream order: said to the host (no fence is needed for it) */
 __device__ __forceinline__ void set_word(uint32_t *word) {
-  if (word && blockIdx.x == 0 && threadIdx.x == 0) __hip_atomic_store(word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (word && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) __hip_atomic_store(word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 /* What a launch reads its rows from (QActF6). */
@@ -99,11 +106,12 @@ struct ActF6 {
  * instruction may have nothing but the one block's scales on either side: infinity times the zeros that stand for the
  * other blocks would be NaN in all of them. Masking the rows' side as well in the loop below cost 8 % of every product;
  * this plain one runs for such tiles only. */
+template <int NS>
 __device__ __forceinline__ void f6_sums_plain(const uint8_t *wbase, int N, int chunks, const ActF6 &act, int mt, int tile,
-                                              float (&acc)[16]) {
+                                              int swap, float (&acc)[NS]) {
   const int lane = threadIdx.x & 63, i32 = lane & 31, g = lane >> 5;
 #pragma unroll
-  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  for (int r = 0; r < NS; ++r) acc[r] = 0.f;
   const uint8_t *w = wbase + (size_t)min(tile, ((N + 31) >> 5) - 1) * chunks * WTILE;
   const uint8_t *rows = act.p + (size_t)(mt >> 1) * chunks * CHUNK;
 #pragma unroll 1
@@ -111,8 +119,8 @@ __device__ __forceinline__ void f6_sums_plain(const uint8_t *wbase, int N, int c
 #pragma unroll 1
     for (int j = 0; j < 8; ++j) {
       const uint8_t *p = rows + (mt & 1) * PARTS + j * 1536;
-      const v4i a0 = *(const v4i *)(p + lane * 16);
-      const v2i a1 = *(const v2i *)(p + 1024 + lane * 8);
+      const v4i a0 = *(const v4i *)(p + (lane ^ swap) * 16);
+      const v2i a1 = *(const v2i *)(p + 1024 + (lane ^ swap) * 8);
       v8i b;
 #pragma unroll
       for (int e = 0; e < 3; ++e) {
@@ -120,26 +128,28 @@ __device__ __forceinline__ void f6_sums_plain(const uint8_t *wbase, int N, int c
         b[e] = b[3 + e] = *(const int *)(w + (q >> 2) * 1024 + lane * 16 + (q & 3) * 4);
       }
       b[6] = b[7] = 0;
-      const v2i da{g ? 0 : (int)*(const uint16_t *)(rows + 2 * PARTS + (mt & 1) * 512 + i32 * 16 + j * 2), 0},
+      const v2i da{g ? 0 : (int)*(const uint16_t *)(rows + 2 * PARTS + (mt & 1) * 512 + (i32 ^ swap) * 16 + j * 2), 0},
         dw{g ? 0 : (int)*(const uint16_t *)(w + 6144 + i32 * 16 + j * 2), 0};
       const v16f D = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(v8i{a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], 0, 0}, b, zero16(),
                                                                      3, 2, 0, 127 + 4, 0, 127 + 3);
       const v16f P = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(v4h, da), __builtin_bit_cast(v4h, dw), zero16(), 0, 0, 0);
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[r] = fmaf(D[r], P[r], acc[r]);
+      for (int r = 0; r < NS; ++r) acc[r] = fmaf(D[r], P[r], acc[r]);
     }
 }
 
 /* The sums of row tile mt and the wavefront's column tile `tile` (lane (column, g), sum r: row 8 (r / 4) + 4 g + r % 4).
- * LOOK: steps an operand is read ahead of its matrix instruction, 1 or 3 */
-template <int LOOK>
+ * LOOK: steps an operand is read ahead of its matrix instruction, 1 or 3. NS = 8: the sums of half of the rows only; swap:
+ * 16 for a wavefront whose half is the upper one, which takes the rows with the halves exchanged. */
+template <int LOOK, int NS = 16>
 __device__ __forceinline__ void f6_sums(const uint8_t *wbase, int N, int chunks, const ActF6 &act, int mt, int tile,
-                                        float (&acc)[16]) {
+                                        float (&acc)[NS], int swap = 0) {
   const uint32_t flag = act.flags[mt]; /* the same for the whole workgroup */
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int lane = threadIdx.x & 63, i32 = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int half = mt & 1; /* of the quantizer's 64 rows */
+  const int al = NS == 16 ? lane : lane ^ swap;
   const rsrc_t ra = make_rsrc(act.p + (size_t)(mt >> 1) * chunks * CHUNK, (uint32_t)chunks * CHUNK);
   /* a tile past the last repeats it; it is not stored */
   const rsrc_t rw = make_rsrc(wbase + (size_t)min(tile, ((N + 31) >> 5) - 1) * chunks * WTILE, (uint32_t)chunks * WTILE);
@@ -171,36 +181,53 @@ __device__ __forceinline__ void f6_sums(const uint8_t *wbase, int N, int chunks,
     load_w(min(k, last), k, 0, 6);
     load_dw(min(k, last), k);
   }
-  asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+  /* chunk 0 is there; the second chunk's loads, three or four of rows and seven of weights, may be under way */
+  asm volatile("s_waitcnt vmcnt(10)\n\ts_barrier" ::: "memory");
   if (flag == act.token) { /* looked at only here, behind the other loads */
-    f6_sums_plain(wbase, N, chunks, act, mt, tile, acc);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); /* the copies under way: the caller uses the LDS */
+    f6_sums_plain(wbase, N, chunks, act, mt, tile, swap, acc);
     return;
   }
 
 #pragma unroll
-  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  for (int r = 0; r < NS; ++r) acc[r] = 0.f;
   v8i a[LOOK + 1], b;
   v16f D[2], P[2];
   v4h da[2]; /* the row's block scales of an even and an odd chunk */
   auto read_a = [&](int st, int at) {
     const unsigned char *p = smem + at + st * 1536;
-    const v4i a0 = *(const v4i *)(p + lane * 16);
-    const v2i a1 = *(const v2i *)(p + 1024 + lane * 8);
+    const v4i a0 = *(const v4i *)(p + al * 16);
+    const v2i a1 = *(const v2i *)(p + 1024 + al * 8);
     a[st & LOOK] = v8i{a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], 0, 0};
   };
-  auto read_da = [&](int k, int at) { da[k] = *(const v4h *)(smem + at + PARTS + i32 * 16 + g * 8); };
-  auto start = [&](int j, int k) { /* block j of the chunk whose weights are in set k */
+  auto read_da = [&](int k, int at) { da[k] = *(const v4h *)(smem + at + PARTS + (al & 31) * 16 + g * 8); };
+  /* Block j of the chunk whose weights are in set k. A wavefront with a SIMD of its own (LOOK = 3) has half of a step's sums
+   * between the two matrix instructions: the second waits for the first to leave the matrix core. */
+  auto start_d = [&](int j, int k) {
 #pragma unroll
     for (int e = 0; e < 3; ++e) b[e] = b[3 + e] = W[k][(3 * j + e) >> 2][(3 * j + e) & 3];
     b[6] = b[7] = 0;
     /* 2^4 and 2^3 make whole numbers of the units 1/16 and 1/8 */
     D[j & 1] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a[j & LOOK], b, zero16(), 3, 2, 0, 127 + 4, 0, 127 + 3);
+    if (LOOK == 3) asm volatile("" ::"v"(D[j & 1])); /* a use here: the instruction is not moved down to its sums */
+  };
+  auto start_p = [&](int j, int k) {
     /* lane (row, g) supplies the row's scales of blocks 4 g .. 4 g + 3, lane (column, g) the column's scale of block j
      * at the place of block j and zeros elsewhere */
     const uint32_t h = (uint32_t)dw[k][j >> 1] & (g == (j >> 2) ? ((j & 1) ? 0xffff0000u : 0xffffu) : 0u);
     const v2i dw2 = (j & 2) ? v2i{0, (int)h} : v2i{(int)h, 0};
     P[j & 1] = __builtin_amdgcn_mfma_f32_32x32x8f16(da[k], __builtin_bit_cast(v4h, dw2), zero16(), 0, 0, 0);
-    asm volatile("" ::"v"(D[j & 1]), "v"(P[j & 1])); /* a use here: the instructions are not moved down to their sums */
+    asm volatile("" ::"v"(D[j & 1]), "v"(P[j & 1]));
+  };
+  auto sums = [&](int j, int r0, int r1) {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int r = r0; r < r1; ++r) acc[r] = fmaf(D[j & 1][r], P[j & 1][r], acc[r]);
+#pragma unroll
+    for (int r = r0; r < r1; ++r) asm volatile("" : "+v"(acc[r])); /* the sums stay at this step */
+    /* half of the sums: the other half's registers are not free either while the instructions write them */
+    if (NS == 8) asm volatile("" ::"v"(D[j & 1]), "v"(P[j & 1]));
+    __builtin_amdgcn_sched_barrier(0);
   };
   /* Chunk c: its rows at `at`, the next chunk's at at_next, its weights in set k. The middle of the chunk waits for the
    * next chunk's rows (copied since the middle of the previous one), publishes them and gives the previous chunk's buffer
@@ -211,13 +238,10 @@ __device__ __forceinline__ void f6_sums(const uint8_t *wbase, int N, int chunks,
     for (int j = 0; j < 8; ++j) {
       read_a((j + LOOK) & 7, j + LOOK < 8 ? at : at_next);
       if (j == 8 - LOOK - 1) read_da(k ^ 1, at_next);
-      start((j + 1) & 7, j + 1 < 8 ? k : k ^ 1);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[r] = fmaf(D[j & 1][r], P[j & 1][r], acc[r]);
-#pragma unroll
-      for (int r = 0; r < 16; ++r) asm volatile("" : "+v"(acc[r])); /* the sums stay at this step */
-      __builtin_amdgcn_sched_barrier(0);
+      start_d((j + 1) & 7, j + 1 < 8 ? k : k ^ 1);
+      if (LOOK == 3) sums(j, 0, NS / 2);
+      start_p((j + 1) & 7, j + 1 < 8 ? k : k ^ 1);
+      sums(j, LOOK == 3 ? NS / 2 : 0, NS);
       if (j == 3) {
         /* the seven weight loads behind the next chunk's rows may be under way */
         asm volatile("s_waitcnt vmcnt(7)\n\ts_barrier" ::: "memory");
@@ -234,7 +258,8 @@ __device__ __forceinline__ void f6_sums(const uint8_t *wbase, int N, int chunks,
 #pragma unroll
   for (int i = 0; i < LOOK; ++i) read_a(i, 0);
   read_da(0, 0);
-  start(0, 0);
+  start_d(0, 0);
+  start_p(0, 0);
   int c = 0, at = 0, at_next = BUF, at_free = 2 * BUF;
   auto turn = [&]() {
     const int t = at;
@@ -252,42 +277,51 @@ __device__ __forceinline__ void f6_sums(const uint8_t *wbase, int N, int chunks,
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
-template <int LOOK>
+template <int LOOK, int NS>
 __device__ __forceinline__ void f6_tile(const uint8_t *wbase, int N, int chunks, const ActF6 &act, int M, int mt, int nt,
                                         float *__restrict__ C, int64_t ldc) {
   const int lane = threadIdx.x & 63, i32 = lane & 31, g = lane >> 5;
-  const int tile = nt * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  float acc[16];
-  f6_sums<LOOK>(wbase, N, chunks, act, mt, tile, acc);
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int tile = NS == 16 ? nt * 4 + wave : nt * 2 + (wave & 1), swap = NS == 16 ? 0 : (wave >> 1) * 16;
+  float acc[NS];
+  f6_sums<LOOK, NS>(wbase, N, chunks, act, mt, tile, acc, swap);
 
-  const int m0 = mt * BM, n = tile * 32 + i32;
+  const int m0 = mt * BM + swap, n = tile * 32 + i32;
   const uint32_t off = (uint32_t)(4 * g) * (uint32_t)ldc + (uint32_t)n; /* the rest of an address is uniform */
+  if (m0 + 2 * NS <= M && tile * 32 + 32 <= N) { /* uniform: the whole tile */
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
+    for (int r = 0; r < NS; ++r) (C + (int64_t)(m0 + 8 * (r >> 2) + (r & 3)) * ldc)[off] = acc[r];
+    return;
+  }
+#pragma unroll
+  for (int r = 0; r < NS; ++r) {
     const int m = m0 + 8 * (r >> 2) + (r & 3);
     if (m + 4 * g < M && n < N) (C + (int64_t)m * ldc)[off] = acc[r];
   }
 }
 
-/* LOOK = 3 takes 182 registers (two workgroups a CU), LOOK = 1 fits three */
-template <int LOOK>
-__global__ __launch_bounds__(NT, LOOK == 1 ? 3 : 2) void gemm_f6_kernel(MultiF6 mw, int chunks, ActF6 act, int M,
-                                                                        int mtiles) {
-  const int id = blockIdx.x;
-  const int xcd = id & 7, qd = id >> 3;
-  const int mt = qd % mtiles;
-  int nt = (qd / mtiles) * 8 + xcd;
+/* Grid: (8 XCDs x row tiles, eighths of the workgroup columns), so that the row tiles sharing weights run on one XCD. All
+ * arguments are asked for at once: each that is loaded where it is first used adds a round trip in front of the first
+ * load of the tile, and so does a division by the number of row tiles (together with the stores of a whole tile without a
+ * condition each, us a call: 512 rows of 2048 x 1024 10.6 -> 9.8, of 1024 x 3072 18.5 -> 17.6).
+ * LOOK = 3 takes 182 registers (two workgroups a CU), LOOK = 1 fits three. NS = 8: two wavefronts a tile, half of its sums
+ * each, the matrix instructions twice. */
+template <int LOOK, int NS>
+__global__ __launch_bounds__(NT, LOOK == 1 ? 3 : 2) void gemm_f6_kernel(MultiF6 mw, int chunks, ActF6 act, int M, int y0) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) asm volatile("" ::"s"(mw.w[i]), "s"(mw.C[i]), "s"(mw.ldc[i]), "s"(mw.N[i]), "s"(mw.tile_end[i]));
+  asm volatile("" ::"s"(mw.word), "s"(chunks), "s"(act.p), "s"(act.flags), "s"(act.token), "s"(M), "s"(y0));
+  const int mt = (int)(blockIdx.x >> 3);
+  int nt = (int)((y0 + blockIdx.y) * 8 + (blockIdx.x & 7));
   if (nt >= mw.tile_end[3]) return; /* uniform per workgroup */
-  int wi = 0;
-  if (nt >= mw.tile_end[0]) wi = 1;
-  if (nt >= mw.tile_end[1]) wi = 2;
-  if (nt >= mw.tile_end[2]) wi = 3;
-  if (wi) nt -= mw.tile_end[wi - 1];
-  const uint8_t *w = wi == 0 ? mw.w[0] : wi == 1 ? mw.w[1] : wi == 2 ? mw.w[2] : mw.w[3];
-  float *C = wi == 0 ? mw.C[0] : wi == 1 ? mw.C[1] : wi == 2 ? mw.C[2] : mw.C[3];
-  const int64_t ldc = wi == 0 ? mw.ldc[0] : wi == 1 ? mw.ldc[1] : wi == 2 ? mw.ldc[2] : mw.ldc[3];
-  const int N = wi == 0 ? mw.N[0] : wi == 1 ? mw.N[1] : wi == 2 ? mw.N[2] : mw.N[3];
-  f6_tile<LOOK>(w, N, chunks, act, M, mt, nt, C, ldc);
+  const uint8_t *w = mw.w[0];
+  float *C = mw.C[0];
+  int64_t ldc = mw.ldc[0];
+  int N = mw.N[0], begin = 0;
+#pragma unroll
+  for (int i = 1; i < 4; ++i)
+    if (nt >= mw.tile_end[i - 1]) w = mw.w[i], C = mw.C[i], ldc = mw.ldc[i], N = mw.N[i], begin = mw.tile_end[i - 1];
+  f6_tile<LOOK, NS>(w, N, chunks, act, M, mt, nt - begin, C, ldc);
   set_word(mw.word);
 }
 
@@ -402,11 +436,10 @@ __device__ __forceinline__ void f6_gated_tile(const GatedF6 &p, int chunks, cons
   }
 }
 template <int LOOK, bool QUANT>
-__global__ __launch_bounds__(NT, LOOK == 1 ? 3 : 2) void gemm_f6_gated_kernel(GatedF6 p, int chunks, ActF6 act, int M,
-                                                                              int mtiles) {
-  const int id = blockIdx.x;
-  const int xcd = id & 7, qd = id >> 3;
-  const int mt = qd % mtiles, nt = (qd / mtiles) * 8 + xcd;
+__global__ __launch_bounds__(NT, LOOK == 1 ? 3 : 2) void gemm_f6_gated_kernel(GatedF6 p, int chunks, ActF6 act, int M, int y0) {
+  asm volatile("" ::"s"(p.act), "s"(p.mul), "s"(p.out), "s"(p.ldo), "s"(p.N), "s"(p.ntiles), "s"(p.word), "s"(p.q), "s"(p.flags),
+               "s"(p.token), "s"(chunks), "s"(act.p), "s"(act.flags), "s"(act.token), "s"(M), "s"(y0));
+  const int mt = (int)(blockIdx.x >> 3), nt = (int)((y0 + blockIdx.y) * 8 + (blockIdx.x & 7));
   if (nt < p.ntiles) f6_gated_tile<LOOK, QUANT>(p, chunks, act, M, mt, nt); /* uniform per workgroup */
   set_word(p.word);
 }
@@ -863,15 +896,24 @@ int launch_gemm_f6(int count, const hipq_weight *const *w, const QActF6 *qa, int
   }
   mw.word = qa->word;
   const int mtiles = (M + BM - 1) / BM;
-  const dim3 grid((unsigned)(mtiles * ((tiles + 7) / 8) * 8));
+  auto go = [&](const char *name, auto kernel) {
+    for (int y0 = 0, end = (tiles + 7) / 8; y0 < end; y0 += MAX_Y)
+      launch_kernel(name, kernel, dim3((unsigned)(8 * mtiles), (unsigned)std::min(end - y0, MAX_Y)), dim3(NT), 3 * BUF, s, mw, qa->chunks,
+                    ActF6{qa->p, qa->flags, qa->token}, M, y0);
+  };
   /* up to two workgroups a CU: the deeper read-ahead (512 rows of 1024 x 3072 13.1 -> 12.0 us, 1024 x 1024 7.5 -> 6.7);
    * beyond, three workgroups a CU cover the reads (512 of 12288 x 4096 67 -> 62 us) */
-  if ((int64_t)mtiles * tiles <= 512)
-    launch_kernel("gemm_f6_kernel<3>", gemm_f6_kernel<3>, grid, dim3(NT), 3 * BUF, s, mw, qa->chunks, ActF6{qa->p, qa->flags, qa->token}, M,
-                  mtiles);
+  if (mtiles * (int64_t)tiles <= HALF_TILES) {
+    tiles = 0;
+    for (int i = 0; i < 4; ++i) {
+      if (i < count) tiles += (int)((w[i]->N + BN / 2 - 1) / (BN / 2));
+      mw.tile_end[i] = tiles;
+    }
+    go("gemm_f6_kernel<3, 8>", gemm_f6_kernel<3, 8>);
+  } else if (mtiles * (int64_t)tiles <= 512)
+    go("gemm_f6_kernel<3, 16>", gemm_f6_kernel<3, 16>);
   else
-    launch_kernel("gemm_f6_kernel<1>", gemm_f6_kernel<1>, grid, dim3(NT), 3 * BUF, s, mw, qa->chunks, ActF6{qa->p, qa->flags, qa->token}, M,
-                  mtiles);
+    go("gemm_f6_kernel<1, 16>", gemm_f6_kernel<1, 16>);
   HIPQ_HIP(hipGetLastError());
   return HIPQ_OK;
 }
@@ -889,11 +931,12 @@ int launch_gemm_f6_gated(const hipq_weight *wa, const hipq_weight *wm, const QAc
     p.q = qh->p, p.flags = qh->flags, p.token = qh->token;
   }
   const int mtiles = (M + BM - 1) / BM;
-  const dim3 grid((unsigned)(mtiles * ((p.ntiles + 7) / 8) * 8));
   /* the bound of launch_gemm_f6 */
   const bool few = (int64_t)mtiles * p.ntiles <= 512;
   auto go = [&](const char *name, auto kernel) {
-    launch_kernel(name, kernel, grid, dim3(NT), 3 * BUF, s, p, qa->chunks, ActF6{qa->p, qa->flags, qa->token}, M, mtiles);
+    for (int y0 = 0, end = (p.ntiles + 7) / 8; y0 < end; y0 += MAX_Y)
+      launch_kernel(name, kernel, dim3((unsigned)(8 * mtiles), (unsigned)std::min(end - y0, MAX_Y)), dim3(NT), 3 * BUF, s, p, qa->chunks,
+                    ActF6{qa->p, qa->flags, qa->token}, M, y0);
   };
   if (qh) {
     if (few)

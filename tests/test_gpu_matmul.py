@@ -224,6 +224,29 @@ def test_q4_0_on_six_bit_operands_matches_oracle(hipq, cr, m, n, k):
     w.destroy()
 
 
+@pytest.mark.parametrize("m,ns,k", [(128, (4096,), 288), (97, (4097,), 544), (129, (4000,), 256), (70, (33, 130, 64, 31), 800),
+                                    (160, (1000, 2072), 288), (65, (64, 1, 65), 32), (512, (4096,), 256)])
+def test_q4_0_on_six_bit_operands_with_few_tiles(hipq, cr, m, ns, k):
+    """gemm_f6.hip up to 128 workgroups of 32 x 128, where two wavefronts share a tile, each with the sums of half of its
+    rows, and right above, alone and several weights a launch: columns that end inside the 64 of a workgroup and in front of
+    its second tile, rows that end inside the upper and the lower half. Same bits as the reference."""
+    import gpu_util as gu
+    import torch
+    blocks = [_weights(cr, "q4_0", n, k, seed=1500 + n) for n in ns]
+    a = synth.normal(1501 + k + m, (m, k))
+    w = [capi.Weight("q4_0", n, k, b) for n, b in zip(ns, blocks)]
+    da = gu.dev(a)
+    out = [torch.full((m, n + 3), float("nan"), device="cuda") for n in ns]
+    capi.matmul_multi(w, da, m, out, ldc=[n + 3 for n in ns], stream=gu.stream())
+    torch.cuda.synchronize()
+    for x, n, b, o in zip(w, ns, blocks, out):
+        ref, got = cr.gemm(cr.oracle(), "q4_0", a, b, n), o.cpu().numpy()
+        assert np.array_equal(np.ascontiguousarray(got[:, :n]).view(np.uint32), ref.view(np.uint32))
+        assert np.isnan(got[:, n:]).all()
+        assert np.array_equal(gu.gpu_matmul(x, a).view(np.uint32), ref.view(np.uint32))
+        x.destroy()
+
+
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("n,k", [(32800, 1024), (33000, 512), (40010, 256), (32768, 768), (50000, 1280)])
 def test_single_row_against_wide_matrices_of_short_rows(hipq, cr, kind, n, k):
