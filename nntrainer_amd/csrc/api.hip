@@ -55,7 +55,8 @@ struct Workspace {
   void *pin = nullptr;
   size_t pin_bytes = 0;
   /* a page-locked word the last launch of such a call writes and the host polls */
-  uint32_t *done = nullptr;
+  uint32_t *done = nullptr, *done_dev = nullptr; /* host and device address */
+  uint32_t *done_count = nullptr;                /* HostDone::count */
   uint32_t done_seq = 0;
   /* a second stream and an event: a prefill's finished rows go back to page-locked host memory on it
    * while the kernels work on the following rows (RowSteps) */
@@ -296,37 +297,51 @@ int pinned_staging(hipStream_t s, size_t bytes, void **out) {
   return HIPQ_OK;
 }
 
-/* The end of a short synchronous call: a one-thread kernel behind the call's launches writes the
+/* The end of a short synchronous call: the last workgroup of the call's last launch (HostDone), or a one-thread kernel
+ * behind launches that do not take it, writes the
  * call's number into a page-locked word and the host polls that word. Waking a thread out of
  * hipStreamSynchronize costs several microseconds more than the poll sees the store; a call that
  * takes longer than the poll is patient falls back to the stream's wait. */
 __global__ void signal_done_kernel(uint32_t *word, uint32_t value) {
   __hip_atomic_store(word, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
-int wait_done(hipStream_t s) {
-  uint32_t *word = nullptr, seq = 0;
-  {
-    std::lock_guard<std::mutex> lk(g.mu);
-    Workspace &w = g.ws[s];
-    if (!w.done) {
-      hipError_t e = hipHostMalloc((void **)&w.done, 64, hipHostMallocDefault);
-      if (e != hipSuccess) {
-        w.done = nullptr;
-        (void)hipGetLastError();
-      } else
-        *w.done = 0;
+/* the word and the counters of the stream; without them (a full device) the call ends in the stream's wait */
+void begin_end(hipStream_t s, hipq::HostEnd *end) {
+  std::lock_guard<std::mutex> lk(g.mu);
+  Workspace &w = g.ws[s];
+  if (!w.done) {
+    static const char zeros[hipq::HOST_DONE_BYTES] = {};
+    void *word = nullptr, *dev = nullptr, *count = nullptr;
+    if (hipHostMalloc(&word, 64, hipHostMallocDefault) != hipSuccess || hipHostGetDevicePointer(&dev, word, 0) != hipSuccess ||
+        hipMalloc(&count, sizeof zeros) != hipSuccess || hipMemcpy(count, zeros, sizeof zeros, hipMemcpyHostToDevice) != hipSuccess) {
+      (void)hipGetLastError();
+      if (count) (void)hipFree(count);
+      if (word) (void)hipHostFree(word);
+      return;
     }
-    word = w.done;
-    seq = ++w.done_seq;
+    w.done = (uint32_t *)word, w.done_dev = (uint32_t *)dev, w.done_count = (uint32_t *)count;
+    *w.done = 0;
   }
-  if (!word) {
+  end->d.count = w.done_count;
+  end->d.word = w.done_dev;
+  end->d.value = ++w.done_seq;
+}
+int wait_done(hipStream_t s, const hipq::HostEnd &end) {
+  if (!end.d.word) {
     HIPQ_HIP(hipStreamSynchronize(s));
     return HIPQ_OK;
   }
-  hipq::launch_kernel("signal_done_kernel", signal_done_kernel, dim3(1), dim3(1), 0, s, (uint32_t *)pinned_device_ptr(word), seq);
-  HIPQ_HIP(hipGetLastError());
+  uint32_t *word;
+  {
+    std::lock_guard<std::mutex> lk(g.mu);
+    word = g.ws[s].done;
+  }
+  if (!end.taken) {
+    hipq::launch_kernel("signal_done_kernel", signal_done_kernel, dim3(1), dim3(1), 0, s, end.d.word, end.d.value);
+    HIPQ_HIP(hipGetLastError());
+  }
   for (int spin = 0; spin < 200000; ++spin) { /* about a tenth of a millisecond */
-    if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == seq) return HIPQ_OK;
+    if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == end.d.value) return HIPQ_OK;
     __builtin_ia32_pause();
   }
   HIPQ_HIP(hipStreamSynchronize(s));
@@ -355,6 +370,7 @@ struct DirectIO {
   const float *a_dev = nullptr; /* device-side address of the rows to fetch */
   int64_t a_ld = 0;
   std::vector<Out> outs;
+  hipq::HostEnd end; /* for the call's last launch */
 
   /* false: the call does not qualify (too many rows or bytes, odd K) and takes the copy engines */
   bool begin(hipStream_t stream, const float *A, int64_t M, int64_t lda, int64_t K, int count, float *const *C,
@@ -366,7 +382,8 @@ struct DirectIO {
     if (out_bytes > DIRECT_BYTES) return false;
     s = stream;
     rows = M;
-    const bool a_direct = !(lda & 3) && !((uintptr_t)A & 15) && pinned_device_ptr(A);
+    a_dev = !(lda & 3) && !((uintptr_t)A & 15) ? (const float *)pinned_device_ptr(A) : nullptr;
+    const bool a_direct = a_dev != nullptr;
     if (!a_direct) stage_bytes += ((size_t)M * K * 4 + 255) & ~(size_t)255;
     outs.resize(count);
     for (int i = 0; i < count; ++i) {
@@ -380,7 +397,6 @@ struct DirectIO {
       stage = (char *)p;
     }
     if (a_direct) {
-      a_dev = (const float *)pinned_device_ptr(A);
       a_ld = lda;
     } else {
       for (int64_t r = 0; r < M; ++r) memcpy(stage + (size_t)r * K * 4, A + r * lda, (size_t)K * 4);
@@ -395,6 +411,7 @@ struct DirectIO {
         o.dld = o.N;
         stage += ((size_t)M * o.N * 4 + 255) & ~(size_t)255;
       }
+    begin_end(s, &end);
     return true;
   }
   /* the rows into dense device memory dst [rows x K] */
@@ -407,7 +424,7 @@ struct DirectIO {
   }
   /* waits for the kernels; staged outputs go to where the caller wants them */
   int finish() const {
-    if (int rc = wait_done(s)) return rc;
+    if (int rc = wait_done(s, end)) return rc;
     for (const Out &o : outs)
       if (o.bounce)
         for (int64_t r = 0; r < rows; ++r) memcpy(o.host + r * o.hld, o.bounce + r * o.N, (size_t)o.N * 4);
@@ -692,7 +709,7 @@ int rows_q6k_copy(const hipq_weight *w, int64_t M, hipStream_t s) {
 
 /* Block-dot stage on already quantized activations. */
 int multiply(const hipq_weight *w, const QAct &qa, int64_t M, float *C, int64_t ldc,
-             hipStream_t s, bool each_row = false) {
+             hipStream_t s, bool each_row = false, hipq::HostEnd *end = nullptr) {
   const int is_k = w->dtype != HIPQ_Q4_0;
   /* rows the reference sends through its 4-row GEMM kernel (Q4_K, M > 1) */
   const int pair_rows = (w->dtype == HIPQ_Q4_K && M > 1 && !each_row) ? (int)((M / 4) * 4) : 0;
@@ -701,8 +718,8 @@ int multiply(const hipq_weight *w, const QAct &qa, int64_t M, float *C, int64_t 
    * that one does not apply (narrow matrices), the prefill GEMM also takes five to eight rows from
    * 2^25 weights up, where the GEMV engine's eight-row pass is the slower of the two */
   const bool q40_gemm = w->dtype == HIPQ_Q4_0 && w->K % 256 == 0;
-  if (hipq::gemm_rows_q40_fits(w, M)) return hipq::launch_gemm_rows_q40(w, &qa, (int)M, C, ldc, s);
-  if (w->gt_base && hipq::gemm_rows_q6k_fits(w, M)) return hipq::launch_gemm_rows_q6k(w, &qa, (int)M, C, ldc, s);
+  if (hipq::gemm_rows_q40_fits(w, M)) return hipq::launch_gemm_rows_q40(w, &qa, (int)M, C, ldc, s, end);
+  if (w->gt_base && hipq::gemm_rows_q6k_fits(w, M)) return hipq::launch_gemm_rows_q6k(w, &qa, (int)M, C, ldc, s, end);
   if (M <= 8 && !(q40_gemm && M >= 5 && w->N * w->K >= (int64_t(1) << 25)))
     return hipq::launch_gemv(w, &qa, (int)M, pair_rows, C, ldc, s);
   if (q40_gemm) return hipq::launch_gemm(w, &qa, (int)M, C, ldc, s);
@@ -766,7 +783,7 @@ bool wants_rows(const hipq_weight *w, int64_t M, bool may_allocate) {
 }
 
 int matmul_rows(const hipq_weight *w, const float *A, int64_t M, int64_t lda, float *C, int64_t ldc,
-                hipStream_t s, int phase, const Scratch &sc, bool each_row = false) {
+                hipStream_t s, int phase, const Scratch &sc, bool each_row = false, hipq::HostEnd *end = nullptr) {
   void *mem = nullptr;
   int rc = sc.get(qact_bytes(1, M, w->K), &mem);
   if (rc) return rc;
@@ -775,7 +792,7 @@ int matmul_rows(const hipq_weight *w, const float *A, int64_t M, int64_t lda, fl
   if (phase != 1) rc = hipq::launch_quantize_q8_K_rowmma(A, M, w->K, lda, &qa, s, mat_rows);
   if (rc || phase == 2) return rc;
   if (!w->gt_base && (rc = hipq::ensure_gemm_tiles(const_cast<hipq_weight *>(w)))) return rc;
-  return hipq::launch_gemm_rows_q4k(w, &qa, (int)M, (int)mat_rows, C, ldc, s); /* up to two passes of eight rows */
+  return hipq::launch_gemm_rows_q4k(w, &qa, (int)M, (int)mat_rows, C, ldc, s, end); /* up to two passes of eight rows */
 }
 
 /* Whether a launch of Q4_0 weights of one K takes the six-bit GEMM (gemm_f6.hip; the reference's bits like every
@@ -882,7 +899,7 @@ int mlp_f6(const hipq_weight *wa, const hipq_weight *wm, const hipq_weight *wd, 
  * and Q6_K that is what up to 16 rows give anyway; Q4_K drops the 4-row quantizer and the pairwise
  * sums the reference applies to rows it multiplies together. The caller passes at most 16 rows. */
 int matmul_device(hipq_weight_t w, const float *A, int64_t M, int64_t lda, float *C, int64_t ldc,
-                  hipStream_t s, const Scratch &sc, bool each_row = false) {
+                  hipStream_t s, const Scratch &sc, bool each_row = false, hipq::HostEnd *end = nullptr) {
   if (M == 0) return HIPQ_OK;
   const hipq_weight *one = w;
   if (wants_f6(1, &one, M)) {
@@ -891,10 +908,10 @@ int matmul_device(hipq_weight_t w, const float *A, int64_t M, int64_t lda, float
     if (int rc = f6_ready(1, &one, M, s, sc, &ready, &make)) return rc;
     if (ready) return matmul_f6(1, &one, A, M, lda, &C, &ldc, s, sc, &make);
   }
-  if (wants_rows(w, M, !sc.fixed)) return matmul_rows(w, A, M, lda, C, ldc, s, 0, sc, each_row);
+  if (wants_rows(w, M, !sc.fixed)) return matmul_rows(w, A, M, lda, C, ldc, s, 0, sc, each_row, end);
   if (!each_row && wants_tiled(w, M, !sc.fixed)) return matmul_tiled(w, A, M, lda, C, ldc, s, 0, sc);
   if (M == 1 && hipq::gemv_fuses_quantizer(w, A)) return hipq::launch_gemv_fused(w, A, C, s);
-  if (hipq::gemm_rows_q40_fuses(1, &one, M, A, lda)) return hipq::launch_gemm_rows_q40_fused(1, &one, A, lda, (int)M, &C, &ldc, s);
+  if (hipq::gemm_rows_q40_fuses(1, &one, M, A, lda)) return hipq::launch_gemm_rows_q40_fused(1, &one, A, lda, (int)M, &C, &ldc, s, end);
   const int is_k = w->dtype != HIPQ_Q4_0;
   void *mem = nullptr;
   int rc;
@@ -913,7 +930,7 @@ int matmul_device(hipq_weight_t w, const float *A, int64_t M, int64_t lda, float
     }
     return rc;
   }
-  return multiply(w, qa, M, C, ldc, s, each_row);
+  return multiply(w, qa, M, C, ldc, s, each_row, end);
 }
 
 /* Whether a product of M rows has a launch of its own that quantizes them: it reads each value once, so the rows can stay in
@@ -1007,6 +1024,7 @@ int hipq_shutdown(void) {
     if (kv.second.io) (void)hipFree(kv.second.io);
     if (kv.second.pin) (void)hipHostFree(kv.second.pin);
     if (kv.second.done) (void)hipHostFree(kv.second.done);
+    if (kv.second.done_count) (void)hipFree(kv.second.done_count);
     if (kv.second.step_done) (void)hipEventDestroy(kv.second.step_done);
     if (kv.second.copy) (void)hipStreamDestroy(kv.second.copy);
     for (void *p : kv.second.retired) (void)hipFree(p);
@@ -1051,6 +1069,7 @@ int hipq_stream_release(void *stream) {
   if (it->second.io) (void)hipFree(it->second.io);
   if (it->second.pin) (void)hipHostFree(it->second.pin);
   if (it->second.done) (void)hipHostFree(it->second.done);
+  if (it->second.done_count) (void)hipFree(it->second.done_count);
   if (it->second.step_done) (void)hipEventDestroy(it->second.step_done);
   if (it->second.copy) (void)hipStreamDestroy(it->second.copy);
   for (void *p : it->second.retired) (void)hipFree(p);
@@ -1356,7 +1375,7 @@ int hipq_matmul(hipq_weight_t w, const float *A, int64_t M, int64_t lda, float *
       if (reads_rows_once(w, M, dio.a_dev, dio.a_ld))
         dA = const_cast<float *>(dio.a_dev), a_ld = dio.a_ld;
       else if ((rc = dio.fetch(dA, w->K))) return rc;
-      if ((rc = matmul_device(w, dA, M, a_ld, dio.outs[0].dev, dio.outs[0].dld, s, sc))) return rc;
+      if ((rc = matmul_device(w, dA, M, a_ld, dio.outs[0].dev, dio.outs[0].dld, s, sc, false, &dio.end))) return rc;
       return dio.finish();
     }
     if (rc) return rc;
@@ -1416,7 +1435,7 @@ int hipq_matmul_each_row(hipq_weight_t w, const float *A, int64_t rows, int64_t 
           break;
         }
       }
-    rc = matmul_device(w, dA + r0 * a_ld, n, a_ld, dC + r0 * c_ld, c_ld, s, sc, true);
+    rc = matmul_device(w, dA + r0 * a_ld, n, a_ld, dC + r0 * c_ld, c_ld, s, sc, true, r0 + n == rows ? &dio.end : nullptr);
     r0 += n;
   }
   if (rc || mem == HIPQ_MEM_DEVICE) return rc;
@@ -1439,7 +1458,7 @@ int hipq_matmul_noalloc(hipq_weight_t w, const float *A, int64_t M, int64_t lda,
 }
 
 static int multi_device(int count, const hipq_weight_t *w, const float *A, int64_t M, int64_t lda, float *const *C,
-                        const int64_t *ldc, hipStream_t s, const Scratch &sc);
+                        const int64_t *ldc, hipStream_t s, const Scratch &sc, hipq::HostEnd *end = nullptr);
 
 int hipq_mlp_swiglu(hipq_weight_t w_act, hipq_weight_t w_mul, const float *A, int64_t M, int64_t lda,
                     float *out, int64_t ldo, int mem, void *stream) {
@@ -1584,7 +1603,7 @@ int hipq_mlp_swiglu_down(hipq_weight_t w_act, hipq_weight_t w_mul, hipq_weight_t
       if ((rr = multi_device(2, ws, a, n, a_ld, cr, lds, s, sc))) return rr;
       if ((rr = hipq::launch_swiglu_rows(cr[0], cr[1], n, N, dH + r0 * N, N, s))) return rr;
     }
-    return matmul_device(w_down, dH + r0 * N, n, N, o_dev + r0 * o_ld, o_ld, s, sc);
+    return matmul_device(w_down, dH + r0 * N, n, N, o_dev + r0 * o_ld, o_ld, s, sc, false, &dio.end);
   };
   if (mem == HIPQ_MEM_DEVICE || direct) {
     if ((rc = rows(0, M, Scratch{false, s}))) return rc;
@@ -1641,7 +1660,7 @@ int hipq_matmul_multi(int count, const hipq_weight_t *w, const float *A, int64_t
     if (dio.begin(s, A, M, lda, Kh, count, C, ldc, ns.data(), &rc)) {
       for (int i = 0; i < count; ++i) dC[i] = dio.outs[i].dev, dld[i] = dio.outs[i].dld;
       if ((rc = dio.fetch((float *)io, Kh))) return rc;
-      if ((rc = multi_device(count, w, (const float *)io, M, Kh, dC.data(), dld.data(), s, Scratch{false, s}))) return rc;
+      if ((rc = multi_device(count, w, (const float *)io, M, Kh, dC.data(), dld.data(), s, Scratch{false, s}, &dio.end))) return rc;
       return dio.finish();
     }
     if (rc) return rc;
@@ -1673,7 +1692,7 @@ int hipq_matmul_multi(int count, const hipq_weight_t *w, const float *A, int64_t
 
 /* Several weights of one K against rows in device memory; M > 0 */
 static int multi_device(int count, const hipq_weight_t *w, const float *A, int64_t M, int64_t lda, float *const *C,
-                        const int64_t *ldc, hipStream_t s, const Scratch &sc) {
+                        const int64_t *ldc, hipStream_t s, const Scratch &sc, hipq::HostEnd *end) {
   int rc;
   if (M == 1 && hipq::gemv_fuses_quantizer_multi(count, w, A))
     return hipq::launch_gemv_fused_multi(count, w, A, C, s);
@@ -1742,7 +1761,7 @@ static int multi_device(int count, const hipq_weight_t *w, const float *A, int64
       }
       if (ng == 4 || (i == count && ng)) {
         if ((rc = workspace_unmoved(s, gen))) return rc;
-        if ((rc = hipq::launch_gemm_rows_q4k_multi(ng, gw, &qa, (int)M, (int)((M / 4) * 4), gc, gl, s))) return rc;
+        if ((rc = hipq::launch_gemm_rows_q4k_multi(ng, gw, &qa, (int)M, (int)((M / 4) * 4), gc, gl, s, ng == count ? end : nullptr))) return rc;
         ng = 0;
       }
     }
@@ -1819,7 +1838,7 @@ static int multi_device(int count, const hipq_weight_t *w, const float *A, int64
           ++members;
         }
       if (members <= 4 && hipq::gemm_rows_q40_fuses(nf, fw, M, A, lda)) {
-        if ((rc = hipq::launch_gemm_rows_q40_fused(nf, fw, A, lda, (int)M, fc, fl, s))) return rc;
+        if ((rc = hipq::launch_gemm_rows_q40_fused(nf, fw, A, lda, (int)M, fc, fl, s, nf == count ? end : nullptr))) return rc;
         continue;
       }
     }
@@ -1838,7 +1857,7 @@ static int multi_device(int count, const hipq_weight_t *w, const float *A, int64
       int frc = workspace_unmoved(s, gen);
       if (frc) return frc;
       if (k == 0 && ng > 1 && hipq::gemm_rows_q40_fits_multi(ng, gw, M))
-        frc = hipq::launch_gemm_rows_q40_multi(ng, gw, &qa, (int)M, gc, gl, s);
+        frc = hipq::launch_gemm_rows_q40_multi(ng, gw, &qa, (int)M, gc, gl, s, ng == count ? end : nullptr);
       else if (k == 0 && M > 8 && gw[0]->K % 256 == 0)
         frc = hipq::launch_gemm_multi(ng, gw, &qa, (int)M, gc, gl, s);
       else

@@ -44,8 +44,10 @@ struct Regs { /* a lane's half of a super-block: steps s = 0 .. 7 of sixteen wei
   v4i q[4], h[2], hd;
 };
 
-__global__ __launch_bounds__(NT, 2) void gemm_rows_q6k_kernel(WView w, QView a, int M_all, float *__restrict__ C, int64_t ldc) {
+__global__ __launch_bounds__(NT, 2) void gemm_rows_q6k_kernel(WView w, QView a, int M_all, float *__restrict__ C, int64_t ldc,
+                                                              hipq::HostDone hd) {
   extern __shared__ __attribute__((aligned(16))) unsigned char rows_lds[];
+  asm volatile("" ::"s"(w.qs), "s"(w.qh), "s"(w.hdr), "s"(w.N), "s"(w.K), "s"(a.q), "s"(a.d), "s"(M_all), "s"(C), "s"(ldc), "s"(hd.word));
   const int tile = blockIdx.x, K = w.K, nsb = K >> 8;
   const int r0 = blockIdx.y * TC, M = min(TC, M_all - r0);
   a.q += (size_t)r0 * K;
@@ -189,7 +191,8 @@ __global__ __launch_bounds__(NT, 2) void gemm_rows_q6k_kernel(WView w, QView a, 
   }
   const int col = tile * 32 + cn;
   if (cm < M && col < w.N)
-    C[(int64_t)cm * ldc + col] = ((acc[0] + acc[4]) + (acc[2] + acc[6])) + ((acc[1] + acc[5]) + (acc[3] + acc[7]));
+    hipq::store_out(C + (int64_t)cm * ldc + col, ((acc[0] + acc[4]) + (acc[2] + acc[6])) + ((acc[1] + acc[5]) + (acc[3] + acc[7])), hd);
+  hipq::host_done(hd);
 }
 
 } // namespace
@@ -217,15 +220,15 @@ bool gemm_rows_q6k_fits(const hipq_weight *w, int64_t M) {
   return 6.8 + (double)((w->K + 1023) / 1024) * std::max(2.05, 0.6 + 1.95 * a_cu) < engine;
 }
 
-int launch_gemm_rows_q6k(const hipq_weight *w, const QAct *qa, int M, float *C, int64_t ldc, hipStream_t s) {
+int launch_gemm_rows_q6k(const hipq_weight *w, const QAct *qa, int M, float *C, int64_t ldc, hipStream_t s, HostEnd *end) {
   if (!w->gt_base || w->dtype != HIPQ_Q6_K || qa->K != w->K || M < 1 || M > 16)
     return fail(HIPQ_ERR_INVALID_ARGUMENT, "the few-rows Q6_K product takes 1 to 16 rows and a weight with its tile copy");
   WView v = wview(w);
   v.qs = w->gt_qs;
   v.qh = w->gt_qh;
   v.hdr = w->gt_hdr;
-  launch_kernel("gemm_rows_q6k_kernel", gemm_rows_q6k_kernel, dim3((unsigned)((w->N + 31) / 32), (unsigned)((M + TC - 1) / TC)), dim3(NT),
-                LDS_BYTES, s, v, qview(*qa), M, C, ldc);
+  const dim3 grid((unsigned)((w->N + 31) / 32), (unsigned)((M + TC - 1) / TC));
+  launch_kernel("gemm_rows_q6k_kernel", gemm_rows_q6k_kernel, grid, dim3(NT), LDS_BYTES, s, v, qview(*qa), M, C, ldc, take_end(end, grid));
   HIPQ_HIP(hipGetLastError());
   return HIPQ_OK;
 }

@@ -220,6 +220,55 @@ inline void launch_kernel(const char *name, void (*kernel)(KArgs...), dim3 grid,
                           hipGetErrorString(e_), __FILE__, __LINE__);         \
   } while (0)
 
+/* The end of a synchronous call on a few rows of host memory, for a product whose launch is the call's last (the kernels of
+ * gemm_rows_*.hip): its outputs are stored past the caches as the workgroups end (store_out), where the end of the kernel had
+ * written all of them back at once, and the last workgroup writes `value` to the page-locked word that the host polls
+ * (host_done), where a launch behind it did. word: null where the outputs are in device memory. us a call of page-locked rows,
+ * before -> with the stores -> with both: eight rows of 12288 x 4096 Q4_K 29.6 -> 27.9 -> 27.1; before -> both: sixteen rows 44.5 ->
+ * 41.0, eight of Q4_0 31.6 -> 28.6, of Q6_K 37.2 -> 32.3, two of 2000 x 1024 Q4_0 16.3 -> 15.8. The one-row kernels, whose
+ * wavefronts store a few columns each, lose by it (20000 x 2048 Q4_0 18.3 -> 28.0: small writes over the bus). */
+struct HostDone {
+  uint32_t *count = nullptr; /* device memory, zero between calls: [16 lines of 64 bytes][a line for their ends] */
+  uint32_t *word = nullptr;
+  uint32_t value = 0;
+  uint32_t width = 0, groups = 0; /* the launch's workgroups along x, and all of them (gridDim would bring its own arguments) */
+};
+/* The device side: every workgroup of the launch calls host_done with all its lanes behind its stores. */
+__device__ __forceinline__ void store_out(float *p, float v, const HostDone &hd) {
+  if (hd.word)
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  else
+    *p = v;
+}
+__device__ __forceinline__ void host_done(const HostDone &hd) {
+  if (!hd.word) return; /* uniform */
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); /* the stores have arrived in host memory */
+  __syncthreads();
+  if (threadIdx.x) return;
+  /* sixteen counters and one of them, so that few atomics meet on a line */
+  const uint32_t line = (blockIdx.x + blockIdx.y * hd.width) & 15, mine = (hd.groups + 15 - line) >> 4, lines = hd.groups < 16 ? hd.groups : 16;
+  uint32_t *c = hd.count + line * 16, *all = hd.count + 256;
+  if (__hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 != mine) return;
+  __hip_atomic_store(c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (__hip_atomic_fetch_add(all, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 != lines) return;
+  __hip_atomic_store(all, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(hd.word, hd.value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+constexpr size_t HOST_DONE_BYTES = 17 * 64;
+/* The host side: a call's HostDone on its way to the launch that is its last; taken: that launch ends the call */
+struct HostEnd {
+  HostDone d;
+  bool taken = false;
+};
+inline HostDone take_end(HostEnd *e, dim3 grid) {
+  if (!e || !e->d.word) return HostDone{};
+  e->taken = true;
+  HostDone d = e->d;
+  d.width = grid.x;
+  d.groups = grid.x * grid.y;
+  return d;
+}
+
 /* quantize.hip ------------------------------------------------------------ */
 /* Rows [0, M) of A (row stride lda). `canonical_out` != nullptr writes ggml
  * blocks there, otherwise the internal planes of `qa` are written.
@@ -356,32 +405,34 @@ size_t gemm_q4k_split_bytes(const hipq_weight *w, int64_t M, int64_t parts_as = 
  * the weight with its tile copy (ensure_gemm_tiles) */
 bool gemm_rows_q4k_fits(const hipq_weight *w, int64_t M);
 int launch_gemm_rows_q4k(const hipq_weight *w, const QAct *qa, int M, int pair_rows, float *C, int64_t ldc,
-                         hipStream_t s);
+                         hipStream_t s, HostEnd *end = nullptr);
 /* up to four weights of one K against the same rows in one launch (the column tiles side by side in the grid) */
 bool gemm_rows_q4k_fits_multi(int count, const hipq_weight *const *w, int64_t M);
 int launch_gemm_rows_q4k_multi(int count, const hipq_weight *const *w, const QAct *qa, int M, int pair_rows,
-                               float *const *C, const int64_t *ldc, hipStream_t s);
+                               float *const *C, const int64_t *ldc, hipStream_t s, HostEnd *end = nullptr);
 
 /* gemm_rows_q6k.hip: Q6_K for a few rows on the matrix cores with the reference's bits (rows are independent in this
  * format); fits: the row counts and shapes that should take it; qa in the form of launch_quantize_q8_K; the weight with its
  * tile copy (ensure_gemm_tiles) */
 bool gemm_rows_q6k_fits(const hipq_weight *w, int64_t M);
-int launch_gemm_rows_q6k(const hipq_weight *w, const QAct *qa, int M, float *C, int64_t ldc, hipStream_t s);
+int launch_gemm_rows_q6k(const hipq_weight *w, const QAct *qa, int M, float *C, int64_t ldc, hipStream_t s,
+                         HostEnd *end = nullptr);
 
 /* gemm_rows_q40.hip: Q4_0 for a few rows on the matrix cores with the reference's bits (rows are
  * independent in this format); fits: the row counts and shapes that should take it; qa in the form
  * of launch_quantize_q8_0; the weight's planes as they are */
 bool gemm_rows_q40_fits(const hipq_weight *w, int64_t M);
-int launch_gemm_rows_q40(const hipq_weight *w, const QAct *qa, int M, float *C, int64_t ldc, hipStream_t s);
+int launch_gemm_rows_q40(const hipq_weight *w, const QAct *qa, int M, float *C, int64_t ldc, hipStream_t s,
+                         HostEnd *end = nullptr);
 /* up to four weights of one K against the same rows in one launch (the column tiles side by side in the grid) */
 bool gemm_rows_q40_fits_multi(int count, const hipq_weight *const *w, int64_t M);
 int launch_gemm_rows_q40_multi(int count, const hipq_weight *const *w, const QAct *qa, int M, float *const *C,
-                               const int64_t *ldc, hipStream_t s);
+                               const int64_t *ldc, hipStream_t s, HostEnd *end = nullptr);
 /* the same on the fp32 rows themselves (the workgroups quantize them: no quantizer launch, no workspace),
  * for small launches; fuses: whether a product should take it */
 bool gemm_rows_q40_fuses(int count, const hipq_weight *const *w, int64_t M, const float *A, int64_t lda);
 int launch_gemm_rows_q40_fused(int count, const hipq_weight *const *w, const float *A, int64_t lda, int M,
-                               float *const *C, const int64_t *ldc, hipStream_t s);
+                               float *const *C, const int64_t *ldc, hipStream_t s, HostEnd *end = nullptr);
 
 /* moe.hip ----------------------------------------------------------------- */
 /* Variant of the expert MLP. kind 0: h = silu(g) * u, y = down(h) (qwen_moe_layer.cpp:332-392).

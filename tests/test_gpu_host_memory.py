@@ -298,3 +298,49 @@ def test_grouped_q6_K_prefill_rows_cross_in_steps(hipq, cr, entry, m, k, n, nd):
             x.free()
         for w in ws:
             w.destroy()
+
+
+@pytest.mark.parametrize("kind,m,k,ns", [
+    ("q4_K", 8, 512, (1024,)), ("q4_K", 6, 256, (4099,)),       # 32 workgroups; 129, the last with three columns
+    ("q4_K", 64, 256, (1030,)), ("q4_K", 4, 512, (384, 640, 31)),  # eight passes; three weights of a launch
+    ("q4_0", 2, 1024, (512,)), ("q4_0", 16, 2048, (520,)),      # rows quantized by the kernel; 17 workgroups a pass
+    ("q4_0", 3, 512, (600, 200, 300, 32)), ("q6_K", 16, 256, (33,)), ("q6_K", 5, 1024, (6001,)),
+])
+def test_calls_that_their_last_workgroup_ends(hipq, cr, kind, m, k, ns):
+    """A few rows of host memory through the kernels of gemm_rows_*.hip: the last workgroup of the launch tells the host that
+    the outputs are there. Launches of fewer workgroups than arrival counters, of no whole multiple of them, of several
+    passes and weights; many calls one after the other, each with outputs of its own (a flag that came early would show the
+    values of the call before). The device call's bits, page-locked and pageable."""
+    ws = [capi.Weight(kind, n, k, cr.quantize_weights(cr.oracle(), kind, synth.normal(9700 + n, (n, k), 0.02))) for n in ns]
+    a = synth.normal(9701 + m, (m, k))
+    want = [_device_result(w, a) for w in ws] if len(ws) == 1 else None
+    if want is None:
+        import gpu_util as gu
+        import torch
+        out = [torch.empty((m, n), device="cuda") for n in ns]
+        capi.matmul_multi(ws, gu.dev(a), m, out, stream=gu.stream())
+        torch.cuda.synchronize()
+        want = [o.cpu().numpy() for o in out]
+    pa, pc = capi.host_alloc(m * k * 4), [capi.host_alloc(m * n * 4) for n in ns]
+    try:
+        a_pin = np.ctypeslib.as_array(ctypes.cast(pa, ctypes.POINTER(ctypes.c_float)), (m, k))
+        c_pin = [np.ctypeslib.as_array(ctypes.cast(p, ctypes.POINTER(ctypes.c_float)), (m, n)) for p, n in zip(pc, ns)]
+        c_page = [np.empty((m, n), np.float32) for n in ns]
+        for rep in range(40):
+            scale = np.float32(2.0 ** (rep % 5))  # powers of two: the outputs scale exactly
+            a_pin[:] = a * scale
+            pinned = rep % 4 != 3
+            for c in c_pin + c_page:
+                c[:] = np.nan
+            outs = c_pin if pinned else c_page
+            if len(ws) == 1:
+                capi.matmul(ws[0], pa, m, pc[0] if pinned else c_page[0], mem=capi.MEM_HOST)
+            else:
+                capi.matmul_multi(ws, pa, m, pc if pinned else c_page, mem=capi.MEM_HOST)
+            for got, ref in zip(outs, want):
+                assert np.array_equal(got, ref * scale)
+    finally:
+        for p in [pa] + pc:
+            capi.host_free(p)
+        for w in ws:
+            w.destroy()
