@@ -55,7 +55,6 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef unsigned short v2us __attribute__((ext_vector_type(2)));
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 
 constexpr int BN = 128;
@@ -73,10 +72,6 @@ template <int TM> struct Smem {
 static_assert(sizeof(Smem<1>) * 4 <= 160 * 1024 && sizeof(Smem<2>) * 3 <= 160 * 1024 && sizeof(Smem<4>) * 2 <= 160 * 1024,
               "four workgroups of 32 rows, three of 64 or two of 128 per CU must fit the 160 KB LDS");
 
-__device__ __forceinline__ uint32_t pk_scale(uint32_t x, uint32_t digit2) {
-  const v2us r = __builtin_bit_cast(v2us, x) * __builtin_bit_cast(v2us, digit2);
-  return __builtin_bit_cast(uint32_t, r);
-}
 __device__ __forceinline__ rsrc_t make_rsrc(const void *p, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, (int)bytes, 0x00020000);
 }
@@ -147,7 +142,7 @@ template <int TM> struct InFlight {
 
 /* four 32-deep steps of one 128-deep stage: H = which half of the super-block */
 template <int H, int TM>
-__device__ __forceinline__ void stage_mma(const Smem<TM> &sm, int slot, const WHalf &W, uint32_t slo, uint32_t shi,
+__device__ __forceinline__ void stage_mma(const Smem<TM> &sm, int slot, const WHalf &W, const HipqDigits &dg, uint32_t m4,
                                           int lane, v16i (&Dlo)[TM], v16i (&Dhi)[TM]) {
   const v16i zero16 = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
   const int8_t *pa = sm.a[0] + slot * Smem<TM>::ASTAGE + lane * 16;
@@ -161,12 +156,10 @@ __device__ __forceinline__ void stage_mma(const Smem<TM> &sm, int slot, const WH
 #pragma unroll
       for (int tm = 0; tm < TM; ++tm) a[(ks + 1) & 1][tm] = *(const v4i *)(pa + (tm * 4 + ks + 1) * 1024);
     }
-    const uint32_t dl = __builtin_amdgcn_perm(slo, slo, 0x0c000c00u | (uint32_t)j | ((uint32_t)j << 16));
-    const uint32_t dh = __builtin_amdgcn_perm(shi, shi, 0x0c000c00u | (uint32_t)j | ((uint32_t)j << 16));
     const uint32_t x0 = half ? W.q[j & 1].z : W.q[j & 1].x, x1 = half ? W.q[j & 1].w : W.q[j & 1].y;
-    const uint32_t e0 = x0 & HIPQ_M4, e1 = x1 & HIPQ_M4, o0 = (x0 >> 4) & HIPQ_M4, o1 = (x1 >> 4) & HIPQ_M4;
-    const v4i bl = {(int)pk_scale(e0, dl), (int)pk_scale(e1, dl), (int)pk_scale(o0, dl), (int)pk_scale(o1, dl)};
-    const v4i bh = {(int)pk_scale(e0, dh), (int)pk_scale(e1, dh), (int)pk_scale(o0, dh), (int)pk_scale(o1, dh)};
+    const uint32_t e0 = x0 & m4, e1 = x1 & m4, o0 = (x0 >> 4) & m4, o1 = (x1 >> 4) & m4;
+    const v4i bl = {hipq_scale4(e0, dg.lo, j), hipq_scale4(e1, dg.lo, j), hipq_scale4(o0, dg.lo, j), hipq_scale4(o1, dg.lo, j)};
+    const v4i bh = {hipq_scale4(e0, dg.hi, j), hipq_scale4(e1, dg.hi, j), hipq_scale4(o0, dg.hi, j), hipq_scale4(o1, dg.hi, j)};
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm) {
       Dlo[tm] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[ks & 1][tm], bl, (H == 0 && ks == 0) ? zero16 : Dlo[tm], 0, 0, 0);
@@ -182,15 +175,9 @@ __device__ __forceinline__ void epilogue(const Smem<TM> &sm, int buf, const uint
   const v16f zero16f = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
   const int i32 = lane & 31, g = lane >> 5;
   const float dcol = hipq_h2f((uint16_t)(hd.x & 0xffff));
-  const float ndmin = -hipq_h2f((uint16_t)(hd.x >> 16));
-  const uint32_t mlo = (hd.w & 0x0f0f0f0fu) | ((hd.y >> 2) & 0x30303030u);
-  const uint32_t mhi = ((hd.w >> 4) & 0x0f0f0f0fu) | ((hd.z >> 2) & 0x30303030u);
-  v8h bmin;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    bmin[j] = (_Float16)(float)((mlo >> (8 * j)) & 0xff);
-    bmin[4 + j] = (_Float16)(float)((mhi >> (8 * j)) & 0xff);
-  }
+  float ndmin = -hipq_h2f((uint16_t)(hd.x >> 16));
+  asm("" : "+v"(ndmin)); /* as fp32: with an fp16 operand the multiply-adds below are of half the rate */
+  const v8h bmin = hipq_mins8(hd.y, hd.z, hd.w);
 #pragma unroll
   for (int tm = 0; tm < TM; ++tm) {
     const int rbase = tm * 32;
@@ -256,6 +243,12 @@ __device__ __forceinline__ void gemm_q4k_sums(const WView &w, const int8_t *__re
   sr.lane = lane;
 
   v16i Dlo[TM], Dhi[TM];
+  uint32_t m4 = HIPQ_M4;
+  /* An operand in a scalar register halves a vector instruction's rate on this chip (1.9 instead of 1.03 ns an instruction and
+   * SIMD), and so do perm, fma_mix and conversions: the mask stands in a vector register, the digits are spread by the packed
+   * multiply itself and the mins' factor is fp32. 1777 rows of 12288 x 4096 209.5 -> 206.8 us, of 4096 x 12288 213.1 -> 210.2,
+   * 512 of 12288 x 4096 63.3 -> 62.5. */
+  asm("" : "+v"(m4));
 #pragma unroll
   for (int a = 0; a < TM; ++a)
 #pragma unroll
@@ -279,15 +272,14 @@ __device__ __forceinline__ void gemm_q4k_sums(const WView &w, const int8_t *__re
    * flight. hd / hdn and Wa / Wb alternate between consecutive super-blocks. */
   auto super_block = [&](int sb, const uint4 &hd, uint4 &hdn, int eb) {
     /* 6-bit scales of sub-blocks 4g .. 4g+3, one per byte, as two 3-bit digits */
-    const uint32_t sc = (g ? hd.z : hd.y) & 0x3f3f3f3fu;
-    const uint32_t slo = sc & 0x07070707u, shi = (sc >> 3) & 0x07070707u;
+    const HipqDigits dg = hipq_digits(g ? hd.z : hd.y);
     const int sbn = min(sb + 1, nsb - 1);
     {
       const int s2 = slot >= 1 ? slot - 1 : 2; /* the slot read last stage */
       dma_a(sr, sm, min(2 * sb + 2, nstage - 1), s2);
       dma_rows(sr, sm, sbn, eb ^ 1);
       load_wh<TILES>(Wb, sr, sb, 1);
-      stage_mma<0>(sm, slot, Wa, slo, shi, lane, Dlo, Dhi);
+      stage_mma<0>(sm, slot, Wa, dg, m4, lane, Dlo, Dhi);
       slot = slot == 2 ? 0 : slot + 1;
       sync_lds<InFlight<TM>::FIRST>();
     }
@@ -296,7 +288,7 @@ __device__ __forceinline__ void gemm_q4k_sums(const WView &w, const int8_t *__re
       dma_a(sr, sm, min(2 * sb + 3, nstage - 1), s2);
       load_wh<TILES>(Wa, sr, sbn, 0);
       hdn = TILES ? ld16(sr.rh, i32 * 16, (uint32_t)sbn * 512) : hipq_ld_global(sr.whd + sbn * HSTRIDE);
-      stage_mma<1>(sm, slot, Wb, slo, shi, lane, Dlo, Dhi);
+      stage_mma<1>(sm, slot, Wb, dg, m4, lane, Dlo, Dhi);
       slot = slot == 2 ? 0 : slot + 1;
     }
     epilogue(sm, eb, hd, lane, Dlo, Dhi, acc);

@@ -85,6 +85,37 @@ __device__ __forceinline__ int hipq_dot32_u4(const uint4 &w, const uint4 &lo, co
   return (int)((h << 4) + l) - (int)(s << 7);
 }
 
+/* Q4_K's two 3-bit digits of four 6-bit scales, one a byte of sc, as the even and the odd ones' 16-bit halves: a packed multiply
+ * takes either half for both of its lanes, so no instruction spreads a digit. */
+struct HipqDigits {
+  uint32_t lo[2], hi[2];
+};
+__device__ __forceinline__ HipqDigits hipq_digits(uint32_t sc) {
+  const uint32_t odd = sc >> 8;
+  return HipqDigits{{sc & 0x00070007u, odd & 0x00070007u}, {(sc >> 3) & 0x00070007u, (odd >> 3) & 0x00070007u}};
+}
+typedef unsigned short hipq_v2us __attribute__((ext_vector_type(2)));
+/* the four bytes of x, each at most 15, times digit j of d = {even, odd} */
+__device__ __forceinline__ int hipq_scale4(uint32_t x, const uint32_t (&d)[2], int j) {
+  const hipq_v2us v = __builtin_bit_cast(hipq_v2us, d[j & 1]);
+  const unsigned short s = v[j >> 1];
+  return __builtin_bit_cast(int, __builtin_bit_cast(hipq_v2us, x) * hipq_v2us{s, s});
+}
+typedef _Float16 hipq_v2h __attribute__((ext_vector_type(2)));
+typedef _Float16 hipq_v8h __attribute__((ext_vector_type(8)));
+/* the eight 6-bit mins of a Q4_K header as fp16: 1024 + m is the bit pattern 0x6400 | m */
+__device__ __forceinline__ hipq_v8h hipq_mins8(uint32_t hy, uint32_t hz, uint32_t hw) {
+  const uint32_t m[2] = {(hw & 0x0f0f0f0fu) | ((hy >> 2) & 0x30303030u), ((hw >> 4) & 0x0f0f0f0fu) | ((hz >> 2) & 0x30303030u)};
+  hipq_v8h r;
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {
+    const uint32_t t = __builtin_amdgcn_perm(0x64646464u, m[p >> 1], p & 1 ? 0x04030402u : 0x04010400u);
+    const hipq_v2h v = __builtin_bit_cast(hipq_v2h, t) - hipq_v2h{(_Float16)1024, (_Float16)1024};
+    r[2 * p] = v[0], r[2 * p + 1] = v[1];
+  }
+  return r;
+}
+
 __device__ __forceinline__ int hipq_dot16(const uint32_t (&w)[4], const int4 &a) {
   int s = hipq_dot4((int)w[0], a.x, 0);
   s = hipq_dot4((int)w[1], a.y, s);
