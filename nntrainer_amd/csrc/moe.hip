@@ -2071,24 +2071,27 @@ __global__ __launch_bounds__(256, 4) void down_self_kernel(const WView *__restri
   }
 }
 
-/* y[t][c] = sum of the token's contributions, ascending expert id */
+/* y[t][c .. c + V - 1] = sum of the token's contributions, ascending expert id. V = 4 where the rows of y are 16-byte aligned
+ * (8000 contributions of 2048 columns 12.8 -> 11.8 us: 73 MB at 6.2 TB/s, and the launch) */
+template <int V>
 __global__ __launch_bounds__(256) void combine_kernel(const int *__restrict__ tok_slots, int topk,
                                                       int H, const float *__restrict__ contrib,
                                                       float *__restrict__ y) {
+  typedef float vf __attribute__((ext_vector_type(V)));
   const int t = blockIdx.y;
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+  const int c = (blockIdx.x * blockDim.x + threadIdx.x) * V;
   if (c >= H) return;
-  float acc = 0.f;
+  vf acc = {};
   for (int k0 = 0; k0 < topk; k0 += 8) { /* eight loads in flight, added in order */
-    float v[8];
+    vf v[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k)
-      v[k] = k0 + k < topk ? contrib[(size_t)tok_slots[t * topk + k0 + k] * H + c] : 0.f;
+      v[k] = k0 + k < topk ? *(const vf *)(contrib + (size_t)tok_slots[t * topk + k0 + k] * H + c) : vf{};
 #pragma unroll
     for (int k = 0; k < 8; ++k)
       if (k0 + k < topk) acc = acc + v[k];
   }
-  y[(size_t)t * H + c] = acc;
+  *(vf *)(y + (size_t)t * H + c) = acc;
 }
 
 /* Lanes per weight row, chunk size and weight rows per wavefront for rows of K
@@ -2504,8 +2507,12 @@ int launch_moe(const MoeArgs *a, void *workspace, size_t workspace_bytes, const 
   else
     rc = launch_grouped<HIPQ_Q6_K>(a, b, views, xq, hq, s);
   if (rc) return rc;
-  hipq::launch_kernel("combine_kernel", combine_kernel, dim3((d.hidden + 255) / 256, T), dim3(256), 0, s, b.tok_slots,
-                     d.topk, d.hidden, b.contrib, a->y);
+  if (!((uintptr_t)a->y & 15)) /* hidden is whole blocks of a weight */
+    hipq::launch_kernel("combine_kernel<4>", combine_kernel<4>, dim3((d.hidden + 1023) / 1024, T), dim3(256), 0, s, b.tok_slots, d.topk,
+                        d.hidden, (const float *)b.contrib, a->y);
+  else
+    hipq::launch_kernel("combine_kernel<1>", combine_kernel<1>, dim3((d.hidden + 255) / 256, T), dim3(256), 0, s, b.tok_slots, d.topk,
+                        d.hidden, (const float *)b.contrib, a->y);
   HIPQ_HIP(hipGetLastError());
   return HIPQ_OK;
 }

@@ -101,6 +101,31 @@ def test_moe_seeded_blocks(hipq, cr):
             w.destroy()
 
 
+@pytest.mark.parametrize("h", [256, 1280])
+def test_moe_outputs_of_any_alignment(hipq, cr, h):
+    """Outputs are summed four a lane where y is 16-byte aligned, one a lane elsewhere: the same bits, nothing written outside;
+    1280 columns end inside a workgroup of either width."""
+    import gpu_util as gu
+    import torch
+    t, i, e, k = 72, 256, 8, 3
+    gate, up, down = _experts(cr, e, i, h, seed=1100)
+    wg = [capi.Weight("q4_K", i, h, b) for b in gate]
+    wu = [capi.Weight("q4_K", i, h, b) for b in up]
+    wd = [capi.Weight("q4_K", h, i, b) for b in down]
+    dx, dl = gu.dev(synth.normal(2100, (t, h))), gu.dev(synth.normal(2101, (t, e)))
+    out = []
+    for shift in (0, 1, 2):
+        flat = torch.full((t * h + 8,), 7.0, device="cuda")
+        y = flat[shift:shift + t * h].view(t, h)
+        capi.moe_forward(t, h, i, e, k, wg, wu, wd, dx, y, router_logits=dl, stream=gu.stream())
+        torch.cuda.synchronize()
+        assert (flat[:shift] == 7).all() and (flat[shift + t * h:] == 7).all()
+        out.append(y.clone())
+    assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
+    for w in wg + wu + wd:
+        w.destroy()
+
+
 @pytest.mark.parametrize("t,h,i,e,k", [(64, 512, 256, 32, 2), (64, 256, 256, 16, 2), (96, 256, 256, 8, 2)])
 def test_moe_skewed_routing(hipq, cr, t, h, i, e, k):
     """Every token chooses expert 0: it holds far more slots than a work item (8, 16 or
