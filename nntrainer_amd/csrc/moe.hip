@@ -1715,13 +1715,17 @@ __device__ __forceinline__ bool tile_item(int cols, int rows, const int *__restr
 template <int TM>
 __device__ __forceinline__ void gate_up_tile_pass(moe_tile::Lds &l, const QView &xq, int T, int col, int e, int s0, int n,
                                                   const WView &wg, const WView &wu, int I, float *__restrict__ h,
-                                                  const hipq::MoeEpi &ep) {
+                                                  const hipq::MoeEpi &ep, int pair, int topk) {
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   const int tile = 2 * col + (wave & 1); /* I % 256 == 0 */
   const bool up = wave >= 2;
   float v[TM * 16];
   moe_tile::run<TM>(
     l, xq, (uint32_t)T, (up ? wu : wg).qs + (size_t)tile * (size_t)((xq.K >> 8) * hipq::EXPERT_TILE_BYTES),
+    [&] {
+      if (threadIdx.x < moe_tile::ROWS) l.rows[threadIdx.x] = pair / topk;
+    },
+    [] {},
     [&](const float(&acc)[TM][16], const float(&accm)[TM][16]) {
 #pragma unroll
       for (int i = 0; i < TM * 16; ++i) v[i] = acc[i >> 4][i & 15] - accm[i >> 4][i & 15];
@@ -1732,12 +1736,30 @@ __device__ __forceinline__ void gate_up_tile_pass(moe_tile::Lds &l, const QView 
 #pragma unroll
   for (int i = 0; i < HALF; ++i) mine[i * 64] = up ? v[i] : v[HALF + i];
   __syncthreads();
+  const int c = tile * 32 + (lane & 31);
 #pragma unroll
-  for (int i = 0; i < HALF; ++i) {
-    const float other = theirs[i * 64];
-    const int k = (up ? HALF : 0) + i, row = moe_tile::out_row(k >> 4, k & 15, lane), c = tile * 32 + (lane & 31);
-    const float own = up ? v[HALF + i] : v[i];
-    if (row < n) h[(size_t)(s0 + row) * I + c] = moe_act(ep, e, I, c, up ? other : own, up ? own : other);
+  for (int i0 = 0; i0 < HALF; i0 += 4) {
+    /* four values at a time, those of rows past the item's too (copies of its last row): a value's double exponential is
+     * a chain of thirty dependent instructions */
+    float o[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float other = theirs[(i0 + i) * 64], own = up ? v[HALF + i0 + i] : v[i0 + i];
+      o[i] = up ? other : own;
+      v[i0 + i] = up ? own : other;
+    }
+    if (ep.kind == 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = silu_ref(o[i]) * v[i0 + i];
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = moe_act(ep, e, I, c, o[i], v[i0 + i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int k = (up ? HALF : 0) + i0 + i, row = moe_tile::out_row(k >> 4, k & 15, lane);
+      if (row < n) h[(size_t)(s0 + row) * I + c] = o[i];
+    }
   }
 }
 __global__ __launch_bounds__(256, 3) void gate_up_tile_kernel(const WView *__restrict__ views, int E_, QView xq, int T,
@@ -1750,12 +1772,11 @@ __global__ __launch_bounds__(256, 3) void gate_up_tile_kernel(const WView *__res
   int col, e, s0, n;
   if (!tile_item(I >> 6, rows, items, offsets, col, e, s0, n)) return;
   const WView wg = views[e], wu = views[E_ + e];
-  if (threadIdx.x < moe_tile::ROWS) l.rows[threadIdx.x] = slot_pair[s0 + min((int)threadIdx.x, n - 1)] / topk;
-  __syncthreads();
+  const int pair = slot_pair[s0 + min((int)threadIdx.x, n - 1)]; /* of row threadIdx.x */
   if (n > 32)
-    gate_up_tile_pass<2>(l, xq, T, col, e, s0, n, wg, wu, I, h, ep);
+    gate_up_tile_pass<2>(l, xq, T, col, e, s0, n, wg, wu, I, h, ep, pair, topk);
   else
-    gate_up_tile_pass<1>(l, xq, T, col, e, s0, n, wg, wu, I, h, ep);
+    gate_up_tile_pass<1>(l, xq, T, col, e, s0, n, wg, wu, I, h, ep, pair, topk);
 }
 
 /* contrib of 128 columns, a tile a wavefront; the rows of h are quantized (a row of the activation planes is a slot). With
@@ -1764,12 +1785,18 @@ __global__ __launch_bounds__(256, 3) void gate_up_tile_kernel(const WView *__res
  * top 4, 93.2 -> 85.0, 1000 of 128 of 2048 x 768, top 8, 199.9 -> 195.7 (without the router). */
 template <int TM>
 __device__ __forceinline__ void down_tile_pass(moe_tile::Lds &l, const QView &hq, int P, int col, int e, int s0, int n,
-                                               const WView &wd, const float *wrow, int H, float *__restrict__ contrib,
-                                               const hipq::MoeEpi &ep) {
+                                               const WView &wd, float *wrow, int pair, const float *__restrict__ wgt, int H,
+                                               float *__restrict__ contrib, const hipq::MoeEpi &ep) {
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   const int tile = col * 4 + wave; /* H % 256 == 0 */
   moe_tile::run<TM>(
     l, hq, (uint32_t)P, wd.qs + (size_t)tile * (size_t)((hq.K >> 8) * hipq::EXPERT_TILE_BYTES),
+    [&] {
+      if (threadIdx.x < moe_tile::ROWS) l.rows[threadIdx.x] = s0 + min((int)threadIdx.x, n - 1);
+    },
+    [&] {
+      if (threadIdx.x < moe_tile::ROWS) wrow[threadIdx.x] = wgt[pair];
+    },
     [&](const float(&acc)[TM][16], const float(&accm)[TM][16]) {
       const int c = tile * 32 + (lane & 31), g4 = 4 * (lane >> 5);
       const uint32_t off = (uint32_t)(g4 * H + c); /* the rest of an address is uniform */
@@ -1795,16 +1822,11 @@ __global__ __launch_bounds__(256, 3) void down_tile_kernel(const WView *__restri
   int col, e, s0, n;
   if (!tile_item(H >> 7, rows, items, offsets, col, e, s0, n)) return;
   const WView wd = views[2 * E_ + e];
-  if (threadIdx.x < moe_tile::ROWS) {
-    const int slot = s0 + min((int)threadIdx.x, n - 1);
-    l.rows[threadIdx.x] = slot;
-    wrow[threadIdx.x] = wgt[slot_pair[slot]];
-  }
-  __syncthreads();
+  const int pair = slot_pair[s0 + min((int)threadIdx.x, n - 1)]; /* of row threadIdx.x */
   if (n > 32)
-    down_tile_pass<2>(l, hq, P, col, e, s0, n, wd, wrow, H, contrib, ep);
+    down_tile_pass<2>(l, hq, P, col, e, s0, n, wd, wrow, pair, wgt, H, contrib, ep);
   else
-    down_tile_pass<1>(l, hq, P, col, e, s0, n, wd, wrow, H, contrib, ep);
+    down_tile_pass<1>(l, hq, P, col, e, s0, n, wd, wrow, pair, wgt, H, contrib, ep);
 }
 
 /* ---- The block without a pair sort ------------------------------------------------------

@@ -13,12 +13,15 @@
  * I = Dlo + 8 Dhi is the exact integer the few-token kernels form. The fp32 chains behind it
  * are theirs (and the single-row product's), acc = fma(float(I), d * dA, acc) and
  * accm = fma(float(Im), dmin * dA, accm), so the outputs keep those bits. The expansion of the
- * weights is shared by the two row tiles of 32: 175 vector instructions per 32 x 32 x 256.
+ * weights is shared by the two row tiles of 32: 135 vector instructions per 32 x 32 x 256.
  *
  * Rows go from the quantized planes straight to one of two LDS buffers, a super-block ahead, with
  * buffer_load ... lds: sixteen lanes fetch the 256 consecutive bytes of a row (four rows an
  * instruction, whole cache lines), wherever the row lies, so nothing is gathered or copied
- * beforehand. A row's sixteen 16-byte pieces are stored rotated by an exclusive-or with its number
+ * beforehand. The row sums of the mins' pass arrive during the products, in LDS of their own (the first eight super-blocks
+ * of them), and its headers eight at a time: with one header under way ahead of its use, and the sums copied when they were due, the
+ * pass was a chain of L2 latencies. 1000 tokens of 128 experts of 2048 x 768, top 8: gate/up 107 -> 97 us, with the activation
+ * evaluated four values at a time, down 65.5 -> 56.6; the block 222 -> 212 us by the wall. A row's sixteen 16-byte pieces are stored rotated by an exclusive-or with its number
  * (the lane asks for piece slot ^ row), which spreads the 128-bit reads of eight neighbouring rows
  * over all banks. Weights stream through registers from the expert tiles (hipq_internal.h), a
  * super-block ahead.
@@ -34,38 +37,54 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef unsigned short v2us __attribute__((ext_vector_type(2)));
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 
 constexpr int ROWS = 64; /* rows of a work item, at most */
 
-constexpr int MINS_SB = 12; /* super-blocks whose row sums are in LDS at once in the mins' pass */
+constexpr int MINS_SB = 8; /* super-blocks whose row sums are in LDS at once in the mins' pass */
+struct MinsLds {
+  uint8_t amin[MINS_SB][ROWS * 32]; /* [row][8 low parts, 8 high parts of the sub-block sums, fp16] */
+  float dA[MINS_SB][ROWS];
+};
 struct Lds {
   int8_t q[2][ROWS * 256]; /* per buffer [row][16 pieces of 16 bytes, piece p of row r at place p ^ (r & 15)] */
   float dA[2][ROWS];
   int rows[ROWS]; /* where the item's rows lie in the activation planes */
+  MinsLds m;
 };
-struct MinsLds { /* in the place of the row buffers */
-  uint8_t amin[MINS_SB][ROWS * 32]; /* [row][8 low parts, 8 high parts of the sub-block sums, fp16] */
-  float dA[MINS_SB][ROWS];
-};
-static_assert(sizeof(MinsLds) <= sizeof(Lds::q), "the mins' pass reuses the row buffers");
+static_assert(sizeof(Lds) * 3 + 3 * 256 <= 160 * 1024, "three workgroups per CU must fit the 160 KB LDS");
 
-__device__ __forceinline__ uint32_t scale2(uint32_t x, uint32_t digit2) {
-  return __builtin_bit_cast(uint32_t, __builtin_bit_cast(v2us, x) * __builtin_bit_cast(v2us, digit2));
-}
 __device__ __forceinline__ int out_row(int tm, int r, int lane) { return 32 * tm + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
 
 /* The wavefront's column tile (its first byte is tile[0]) over the whole of K for the item's 32 * TM rows (l.rows, all of
  * them valid plane rows). done(acc, accm) receives the sums: acc[tm][r] - accm[tm][r] is row out_row(tm, r, lane), column
  * lane & 31. */
-template <int TM, typename Done>
-__device__ __forceinline__ void run(Lds &l, const QView &a, uint32_t a_rows, const uint8_t *tile, Done done) {
+template <int TM, typename Rows, typename Late, typename Done>
+__device__ __forceinline__ void run(Lds &l, const QView &a, uint32_t a_rows, const uint8_t *tile, Rows rows, Late late,
+                                    Done done) {
   const int K = a.K, nsb = K >> 8;
   const int lane = threadIdx.x & 63, i32 = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const v16i zero16 = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
   const v16f zero16f = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+
+  const uint32_t tile_bytes = (uint32_t)nsb * hipq::EXPERT_TILE_BYTES;
+  const rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)tile, 0, (int)tile_bytes, 0x00020000);
+  auto load_q = [&](int sb, int i) {
+    return __builtin_bit_cast(
+      v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, lane * 16, sb * hipq::EXPERT_TILE_BYTES + i * 1024, 0));
+  };
+  auto load_hd = [&](int sb) {
+    return __builtin_bit_cast(
+      v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, 4096 + i32 * 16, sb * hipq::EXPERT_TILE_BYTES, 0));
+  };
+  /* the weights are asked for before the rows are known */
+  v4i W[4], hd0, hd1;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) W[i] = load_q(0, i);
+  hd0 = load_hd(0);
+  rows();
+  __syncthreads();
 
   const rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc((void *)a.q, 0, (int)(a_rows * (uint32_t)K), 0x00020000);
   const rsrc_t rm = __builtin_amdgcn_make_buffer_rsrc((void *)a.bsum, 0, (int)(a_rows * (uint32_t)nsb * 32), 0x00020000);
@@ -87,25 +106,16 @@ __device__ __forceinline__ void run(Lds &l, const QView &a, uint32_t a_rows, con
     if (wave == 0) __builtin_amdgcn_raw_ptr_buffer_load_lds(rd, lds_ptr(l.dA[buf]), 4, (int)vd, sb * 4, 0, 0);
   };
 
-  const uint32_t tile_bytes = (uint32_t)nsb * hipq::EXPERT_TILE_BYTES;
   /* LDS byte of this lane's operand of step j: row i32, piece 2 j + g */
   const uint32_t abase = (uint32_t)(i32 * 256 + ((g ^ (i32 & 15)) << 4));
 
-  const rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)tile, 0, (int)tile_bytes, 0x00020000);
-  auto load_q = [&](int sb, int i) {
-    return __builtin_bit_cast(
-      v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, lane * 16, sb * hipq::EXPERT_TILE_BYTES + i * 1024, 0));
-  };
-  auto load_hd = [&](int sb) {
-    return __builtin_bit_cast(
-      v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, 4096 + i32 * 16, sb * hipq::EXPERT_TILE_BYTES, 0));
-  };
   float acc[TM][16];
 #pragma unroll
   for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[tm][r] = 0.f;
-  v4i W[4], hd0, hd1;
+  uint32_t m4 = HIPQ_M4;
+  asm("" : "+v"(m4)); /* an operand in a scalar register halves an instruction's rate */
 
   /* One super-block: the rows of the next are asked for first; a quarter of the nibbles is asked for
    * again (for the next super-block) as soon as its two steps have taken it, so one set of registers holds
@@ -114,7 +124,8 @@ __device__ __forceinline__ void run(Lds &l, const QView &a, uint32_t a_rows, con
     const int sbn = min(sb + 1, nsb - 1); /* past the end the last one again: a fixed number of loads in flight */
     copy_rows(sbn, buf ^ 1);
     const int8_t *pq = l.q[buf];
-    const uint32_t hx = (uint32_t)hd[0], hy = (uint32_t)hd[1], hz = (uint32_t)hd[2];
+    const uint32_t hx = (uint32_t)hd[0];
+    const HipqDigits dgy = hipq_digits((uint32_t)hd[1]), dgz = hipq_digits((uint32_t)hd[2]);
     v16i Dlo[TM], Dhi[TM];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -123,14 +134,13 @@ __device__ __forceinline__ void run(Lds &l, const QView &a, uint32_t a_rows, con
       asm("" : "+v"(at)); /* one instruction a step instead of eight registers */
 #pragma unroll
       for (int tm = 0; tm < TM; ++tm) av[tm] = *(const v4i *)(pq + (at ^ (j * 32)) + tm * 8192);
-      const uint32_t sel = 0x0c000c00u | (uint32_t)(j & 3) | ((uint32_t)(j & 3) << 16);
-      const uint32_t sc = j < 4 ? hy : hz;
-      const uint32_t slo = sc & 0x07070707u, shi = (sc >> 3) & 0x07070707u;
-      const uint32_t dl = __builtin_amdgcn_perm(slo, slo, sel), dh = __builtin_amdgcn_perm(shi, shi, sel);
+      const HipqDigits &dg = j < 4 ? dgy : dgz;
       const uint32_t x0 = (uint32_t)W[j >> 1][2 * (j & 1)], x1 = (uint32_t)W[j >> 1][2 * (j & 1) + 1];
-      const uint32_t e0 = x0 & HIPQ_M4, e1 = x1 & HIPQ_M4, o0 = (x0 >> 4) & HIPQ_M4, o1 = (x1 >> 4) & HIPQ_M4;
-      const v4i bl = {(int)scale2(e0, dl), (int)scale2(e1, dl), (int)scale2(o0, dl), (int)scale2(o1, dl)};
-      const v4i bh = {(int)scale2(e0, dh), (int)scale2(e1, dh), (int)scale2(o0, dh), (int)scale2(o1, dh)};
+      const uint32_t e0 = x0 & m4, e1 = x1 & m4, o0 = (x0 >> 4) & m4, o1 = (x1 >> 4) & m4;
+      const v4i bl = {hipq_scale4(e0, dg.lo, j & 3), hipq_scale4(e1, dg.lo, j & 3), hipq_scale4(o0, dg.lo, j & 3),
+                      hipq_scale4(o1, dg.lo, j & 3)};
+      const v4i bh = {hipq_scale4(e0, dg.hi, j & 3), hipq_scale4(e1, dg.hi, j & 3), hipq_scale4(o0, dg.hi, j & 3),
+                      hipq_scale4(o1, dg.hi, j & 3)};
 #pragma unroll
       for (int tm = 0; tm < TM; ++tm) {
         Dlo[tm] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[tm], bl, j == 0 ? zero16 : Dlo[tm], 0, 0, 0);
@@ -161,11 +171,20 @@ __device__ __forceinline__ void run(Lds &l, const QView &a, uint32_t a_rows, con
     asm volatile("s_waitcnt vmcnt(5) lgkmcnt(0)\n\ts_barrier" ::: "memory");
   };
 
+  /* row sums and scales of the super-blocks m0 .. of the mins' pass */
+  const uint32_t vm = (uint32_t)l.rows[(32 * (wave & 1) + (lane >> 1)) & (32 * TM - 1)] * (uint32_t)(nsb * 32) + (lane & 1) * 16;
+  auto copy_mins = [&](int m0, int mn) {
+    for (int k = wave; k < TM * mn; k += 4) { /* 32 rows of a super-block; k % TM is wave % TM, as in vm */
+      const int b = k / TM, part = k % TM;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rm, lds_ptr(l.m.amin[b] + part * 1024), 16, (int)vm, (m0 + b) * 32, 0, 0);
+    }
+    for (int b = wave; b < mn; b += 4)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rd, lds_ptr(l.m.dA[b]), 4, (int)vd, (m0 + b) * 4, 0, 0);
+  };
+
   copy_rows(0, 0);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) W[i] = load_q(0, i);
-  hd0 = load_hd(0);
   asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+  copy_mins(0, min(MINS_SB, nsb)); /* the first of them arrive during the products */
   int sb = 0;
   for (; sb + 1 < nsb; sb += 2) {
     super_block(sb, 0, hd0, hd1);
@@ -174,54 +193,46 @@ __device__ __forceinline__ void run(Lds &l, const QView &a, uint32_t a_rows, con
   if (sb < nsb) super_block(sb, 0, hd0, hd1);
 
   /* the mins: accm = fma(Im, dmin * dA, accm) over the super-blocks, in a pass of its own so that its
-   * chains do not occupy registers during the products */
+   * chains do not occupy registers during the products. The headers come again, eight at once into the registers that
+   * the products no longer need. */
   float accm[TM][16];
 #pragma unroll
   for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
     for (int r = 0; r < 16; ++r) accm[tm][r] = 0.f;
-  MinsLds &ml = *reinterpret_cast<MinsLds *>(&l.q[0][0]);
-  const uint32_t vm = (uint32_t)l.rows[(32 * (wave & 1) + (lane >> 1)) & (32 * TM - 1)] * (uint32_t)(nsb * 32) + (lane & 1) * 16;
+  late();
   for (int m0 = 0; m0 < nsb; m0 += MINS_SB) {
     const int mn = min(MINS_SB, nsb - m0);
-    /* copies of the last super-block of the products may still be under way into the row buffers */
-    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-    for (int k = wave; k < TM * mn; k += 4) { /* 32 rows of a super-block; k % TM is wave % TM, as in vm */
-      const int b = k / TM, part = k % TM;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rm, lds_ptr(ml.amin[b] + part * 1024), 16, (int)vm, (m0 + b) * 32, 0, 0);
+    if (m0) {
+      __syncthreads(); /* the sums in LDS have been read */
+      copy_mins(m0, mn);
     }
-    for (int b = wave; b < mn; b += 4)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rd, lds_ptr(ml.dA[b]), 4, (int)vd, (m0 + b) * 4, 0, 0);
-    v4i hd = load_hd(m0);
+    v4i hd[MINS_SB];
+#pragma unroll
+    for (int b = 0; b < MINS_SB; ++b)
+      if (b < mn) hd[b] = load_hd(m0 + b);
+    /* also the last copies of rows, which nothing reads: the row buffers are free behind this */
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-    for (int b = 0; b < mn; ++b) {
-      const uint32_t hx = (uint32_t)hd[0], hy = (uint32_t)hd[1], hz = (uint32_t)hd[2], hw = (uint32_t)hd[3];
-      hd = load_hd(m0 + min(b + 1, mn - 1));
-      const float dmin = hipq_h2f((uint16_t)(hx >> 16));
-      const uint32_t mlo = (hw & 0x0f0f0f0fu) | ((hy >> 2) & 0x30303030u);
-      const uint32_t mhi = ((hw >> 4) & 0x0f0f0f0fu) | ((hz >> 2) & 0x30303030u);
-      v8h bmin;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        bmin[j] = (_Float16)(float)((mlo >> (8 * j)) & 0xff);
-        bmin[4 + j] = (_Float16)(float)((mhi >> (8 * j)) & 0xff);
-      }
+    for (int b = 0; b < MINS_SB; ++b)
+      if (b < mn) { /* uniform */
+        const float dmin = hipq_h2f((uint16_t)((uint32_t)hd[b][0] >> 16));
+        const v8h bmin = hipq_mins8((uint32_t)hd[b][1], (uint32_t)hd[b][2], (uint32_t)hd[b][3]);
 #pragma unroll
-      for (int tm = 0; tm < TM; ++tm) {
-        const v8h amin = __builtin_bit_cast(v8h, *(const v4i *)(ml.amin[b] + (32 * tm + i32) * 32 + g * 16));
-        const v16f Sm = __builtin_amdgcn_mfma_f32_32x32x16_f16(amin, bmin, zero16f, 0, 0, 0);
+        for (int tm = 0; tm < TM; ++tm) {
+          const v8h amin = __builtin_bit_cast(v8h, *(const v4i *)(l.m.amin[b] + (32 * tm + i32) * 32 + g * 16));
+          const v16f Sm = __builtin_amdgcn_mfma_f32_32x32x16_f16(amin, bmin, zero16f, 0, 0, 0);
 #pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4) {
-          const v4i dv = *(const v4i *)((const int8_t *)ml.dA[b] + (32 * tm + 8 * q4 + 4 * g) * 4);
+          for (int q4 = 0; q4 < 4; ++q4) {
+            const v4i dv = *(const v4i *)((const int8_t *)l.m.dA[b] + (32 * tm + 8 * q4 + 4 * g) * 4);
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            accm[tm][4 * q4 + e] = fmaf(Sm[4 * q4 + e], dmin * __int_as_float(dv[e]), accm[tm][4 * q4 + e]);
+            for (int e = 0; e < 4; ++e)
+              accm[tm][4 * q4 + e] = fmaf(Sm[4 * q4 + e], dmin * __int_as_float(dv[e]), accm[tm][4 * q4 + e]);
+          }
         }
       }
-    }
   }
   done(acc, accm);
-  __syncthreads(); /* the row buffers are free again */
 }
 
 } // namespace moe_tile
