@@ -1710,58 +1710,65 @@ __device__ __forceinline__ bool tile_item(int cols, int rows, const int *__restr
   return true;
 }
 
+/* Rows of an output, n of them from base on: stores to rows past them are dropped, so that all are issued without conditions. */
+struct OutRows {
+  moe_tile::rsrc_t r;
+  __device__ __forceinline__ OutRows(float *base, int n, int cols) {
+    r = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, n * cols * (int)sizeof(float), 0x00020000);
+  }
+  __device__ __forceinline__ void put(int lane_at, int uniform_at, float v) const {
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(v), r, lane_at * 4, uniform_at * 4, 0);
+  }
+};
+
 /* h of 64 columns: wavefronts 0 and 1 form the two gate tiles, 2 and 3 the up tiles; each pair then
  * exchanges half its sums through LDS, so that all four evaluate the activation. */
-template <int TM>
+template <int TM, bool BIASED>
 __device__ __forceinline__ void gate_up_tile_pass(moe_tile::Lds &l, const QView &xq, int T, int col, int e, int s0, int n,
                                                   const WView &wg, const WView &wu, int I, float *__restrict__ h,
                                                   const hipq::MoeEpi &ep, int pair, int topk) {
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   const int tile = 2 * col + (wave & 1); /* I % 256 == 0 */
   const bool up = wave >= 2;
-  float v[TM * 16];
   moe_tile::run<TM>(
     l, xq, (uint32_t)T, (up ? wu : wg).qs + (size_t)tile * (size_t)((xq.K >> 8) * hipq::EXPERT_TILE_BYTES),
     [&] {
       if (threadIdx.x < moe_tile::ROWS) l.rows[threadIdx.x] = pair / topk;
     },
     [] {},
-    [&](const float(&acc)[TM][16], const float(&accm)[TM][16]) {
+    [&](const float(&acc)[TM][16], const float(&accm)[TM][16], int8_t *free) {
+      constexpr int HALF = TM * 8;
+      float v[TM * 16];
 #pragma unroll
       for (int i = 0; i < TM * 16; ++i) v[i] = acc[i >> 4][i & 15] - accm[i >> 4][i & 15];
+      float *mine = (float *)free + wave * 1024 + lane, *theirs = (float *)free + (wave ^ 2) * 1024 + lane; /* [HALF][64 lanes] */
+#pragma unroll
+      for (int i = 0; i < HALF; ++i) mine[i * 64] = up ? v[i] : v[HALF + i];
+      __syncthreads();
+      const int c = tile * 32 + (lane & 31);
+      const OutRows out(h + (size_t)s0 * I, n, I);
+#pragma unroll
+      for (int i0 = 0; i0 < HALF; i0 += 4) {
+        /* four values at a time, those of rows past the item's too (copies of its last row): a value's double exponential
+         * is a chain of thirty dependent instructions */
+        float o[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float other = theirs[(i0 + i) * 64], own = up ? v[HALF + i0 + i] : v[i0 + i];
+          o[i] = up ? other : own;
+          v[i0 + i] = up ? own : other;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = BIASED ? moe_act(ep, e, I, c, o[i], v[i0 + i]) : silu_ref(o[i]) * v[i0 + i];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int k = (up ? HALF : 0) + i0 + i;
+          out.put(4 * (lane >> 5) * I + c, moe_tile::out_row(k >> 4, k & 15, 0) * I, o[i]);
+        }
+      }
     });
-  constexpr int HALF = TM * 8;
-  float *xch = (float *)l.q[0]; /* [wavefront][HALF][64 lanes] */
-  float *mine = xch + (size_t)wave * HALF * 64 + lane, *theirs = xch + (size_t)(wave ^ 2) * HALF * 64 + lane;
-#pragma unroll
-  for (int i = 0; i < HALF; ++i) mine[i * 64] = up ? v[i] : v[HALF + i];
-  __syncthreads();
-  const int c = tile * 32 + (lane & 31);
-#pragma unroll
-  for (int i0 = 0; i0 < HALF; i0 += 4) {
-    /* four values at a time, those of rows past the item's too (copies of its last row): a value's double exponential is
-     * a chain of thirty dependent instructions */
-    float o[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float other = theirs[(i0 + i) * 64], own = up ? v[HALF + i0 + i] : v[i0 + i];
-      o[i] = up ? other : own;
-      v[i0 + i] = up ? own : other;
-    }
-    if (ep.kind == 0) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) o[i] = silu_ref(o[i]) * v[i0 + i];
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) o[i] = moe_act(ep, e, I, c, o[i], v[i0 + i]);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int k = (up ? HALF : 0) + i0 + i, row = moe_tile::out_row(k >> 4, k & 15, lane);
-      if (row < n) h[(size_t)(s0 + row) * I + c] = o[i];
-    }
-  }
 }
+template <bool BIASED>
 __global__ __launch_bounds__(256, 3) void gate_up_tile_kernel(const WView *__restrict__ views, int E_, QView xq, int T,
                                                               const int *__restrict__ offsets,
                                                               const int *__restrict__ items,
@@ -1774,42 +1781,47 @@ __global__ __launch_bounds__(256, 3) void gate_up_tile_kernel(const WView *__res
   const WView wg = views[e], wu = views[E_ + e];
   const int pair = slot_pair[s0 + min((int)threadIdx.x, n - 1)]; /* of row threadIdx.x */
   if (n > 32)
-    gate_up_tile_pass<2>(l, xq, T, col, e, s0, n, wg, wu, I, h, ep, pair, topk);
+    gate_up_tile_pass<2, BIASED>(l, xq, T, col, e, s0, n, wg, wu, I, h, ep, pair, topk);
   else
-    gate_up_tile_pass<1>(l, xq, T, col, e, s0, n, wg, wu, I, h, ep, pair, topk);
+    gate_up_tile_pass<1, BIASED>(l, xq, T, col, e, s0, n, wg, wu, I, h, ep, pair, topk);
 }
 
 /* contrib of 128 columns, a tile a wavefront; the rows of h are quantized (a row of the activation planes is a slot). With
  * two tiles a wavefront, one after the other, a block of few experts left most of the chip idle and one of many ended
  * less evenly: us a block, 100 tokens of eight experts of 1536 x 1024, top 2, 43.9 -> 36.3, 250 52 / 44, of 32 of 2560 x 1280,
- * top 4, 93.2 -> 85.0, 1000 of 128 of 2048 x 768, top 8, 199.9 -> 195.7 (without the router). */
-template <int TM>
+ * top 4, 93.2 -> 85.0, 1000 of 128 of 2048 x 768, top 8, 199.9 -> 195.7 (without the router). Nor do workgroups that go on to
+ * a next tile, its first loads under way before they end one: 400 tokens of 128 experts 124 -> 134, 900 of 64 of 1280 x 1536, top 2,
+ * 94.2 -> 98. */
+template <int TM, bool BIASED>
 __device__ __forceinline__ void down_tile_pass(moe_tile::Lds &l, const QView &hq, int P, int col, int e, int s0, int n,
                                                const WView &wd, float *wrow, int pair, const float *__restrict__ wgt, int H,
                                                float *__restrict__ contrib, const hipq::MoeEpi &ep) {
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   const int tile = col * 4 + wave; /* H % 256 == 0 */
+  float own;
   moe_tile::run<TM>(
     l, hq, (uint32_t)P, wd.qs + (size_t)tile * (size_t)((hq.K >> 8) * hipq::EXPERT_TILE_BYTES),
     [&] {
       if (threadIdx.x < moe_tile::ROWS) l.rows[threadIdx.x] = s0 + min((int)threadIdx.x, n - 1);
+      own = wgt[pair];
     },
     [&] {
-      if (threadIdx.x < moe_tile::ROWS) wrow[threadIdx.x] = wgt[pair];
+      if (threadIdx.x < moe_tile::ROWS) wrow[threadIdx.x] = own;
     },
-    [&](const float(&acc)[TM][16], const float(&accm)[TM][16]) {
+    [&](const float(&acc)[TM][16], const float(&accm)[TM][16], int8_t *) {
       const int c = tile * 32 + (lane & 31), g4 = 4 * (lane >> 5);
-      const uint32_t off = (uint32_t)(g4 * H + c); /* the rest of an address is uniform */
+      const OutRows out(contrib + (size_t)s0 * H, n, H);
 #pragma unroll
       for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const int urow = 32 * tm + 8 * (r >> 2) + (r & 3); /* out_row = urow + g4 */
-          float *base = contrib + (size_t)(s0 + urow) * H;
-          if (urow + g4 < n) base[off] = moe_out(ep, e, H, c, acc[tm][r] - accm[tm][r], wrow[urow + g4]);
+          const int urow = moe_tile::out_row(tm, r, 0); /* out_row = urow + g4 */
+          const float o = acc[tm][r] - accm[tm][r], wt = wrow[urow + g4];
+          out.put(g4 * H + c, urow * H, BIASED ? moe_out(ep, e, H, c, o, wt) : o * wt);
         }
     });
 }
+template <bool BIASED>
 __global__ __launch_bounds__(256, 3) void down_tile_kernel(const WView *__restrict__ views, int E_, QView hq, int P,
                                                            const int *__restrict__ offsets,
                                                            const int *__restrict__ items,
@@ -1824,9 +1836,9 @@ __global__ __launch_bounds__(256, 3) void down_tile_kernel(const WView *__restri
   const WView wd = views[2 * E_ + e];
   const int pair = slot_pair[s0 + min((int)threadIdx.x, n - 1)]; /* of row threadIdx.x */
   if (n > 32)
-    down_tile_pass<2>(l, hq, P, col, e, s0, n, wd, wrow, pair, wgt, H, contrib, ep);
+    down_tile_pass<2, BIASED>(l, hq, P, col, e, s0, n, wd, wrow, pair, wgt, H, contrib, ep);
   else
-    down_tile_pass<1>(l, hq, P, col, e, s0, n, wd, wrow, pair, wgt, H, contrib, ep);
+    down_tile_pass<1, BIASED>(l, hq, P, col, e, s0, n, wd, wrow, pair, wgt, H, contrib, ep);
 }
 
 /* ---- The block without a pair sort ------------------------------------------------------
@@ -2294,12 +2306,13 @@ int launch_tile_mma(const hipq::MoeArgs *a, const MoeBufs &b, const WView *views
   const int64_t P = (int64_t)d.tokens * d.topk;
   const int max_items = (int)((P < d.experts ? P : d.experts) + P / rows);
   const unsigned groups = (unsigned)((max_items + 7) / 8 * 8);
-  hipq::launch_kernel("gate_up_tile_kernel", gate_up_tile_kernel, dim3(groups * (unsigned)(d.intermediate / 64)), dim3(256),
+  const bool biased = a->epi.kind != 0;
+  hipq::launch_kernel("gate_up_tile_kernel", biased ? gate_up_tile_kernel<true> : gate_up_tile_kernel<false>, dim3(groups * (unsigned)(d.intermediate / 64)), dim3(256),
                       sizeof(moe_tile::Lds), s, views, d.experts, qview(xq), d.tokens, b.offsets, b.items, b.slot_pair, rows,
                       d.topk, d.intermediate, b.h, a->epi);
   HIPQ_HIP(hipGetLastError());
   if (int rc = hipq::launch_quantize_q8_K_rowmma(b.h, P, d.intermediate, d.intermediate, &hq, s)) return rc;
-  hipq::launch_kernel("down_tile_kernel", down_tile_kernel, dim3(groups * (unsigned)(d.hidden / 128)), dim3(256),
+  hipq::launch_kernel("down_tile_kernel", biased ? down_tile_kernel<true> : down_tile_kernel<false>, dim3(groups * (unsigned)(d.hidden / 128)), dim3(256),
                       sizeof(moe_tile::Lds) + moe_tile::ROWS * sizeof(float), s, views, d.experts, qview(hq), (int)P,
                       b.offsets, b.items, b.slot_pair, (const float *)b.wgt, rows, d.hidden, b.contrib, a->epi);
   HIPQ_HIP(hipGetLastError());

@@ -18,21 +18,26 @@
  * Rows go from the quantized planes straight to one of two LDS buffers, a super-block ahead, with
  * buffer_load ... lds: sixteen lanes fetch the 256 consecutive bytes of a row (four rows an
  * instruction, whole cache lines), wherever the row lies, so nothing is gathered or copied
- * beforehand. The row sums of the mins' pass arrive during the products, in LDS of their own (the first eight super-blocks
- * of them), and its headers eight at a time: with one header under way ahead of its use, and the sums copied when they were due, the
- * pass was a chain of L2 latencies. 1000 tokens of 128 experts of 2048 x 768, top 8: gate/up 107 -> 97 us, with the activation
- * evaluated four values at a time, down 65.5 -> 56.6; the block 222 -> 212 us by the wall. A row's sixteen 16-byte pieces are stored rotated by an exclusive-or with its number
+ * beforehand. What the mins' pass reads arrives during the products too: the row sums in LDS of their own (of the first eight
+ * super-blocks), the headers in the row buffer that the last super-block leaves free. With the sums copied when they were due and one
+ * header under way, the pass was a chain of L2 latencies, and a workgroup has three to twelve super-blocks in all. 1000 tokens
+ * of 128 experts of 2048 x 768, top 8: gate/up 103 -> 92 us, with the activation evaluated four values at a time and the outputs
+ * stored without conditions, down 61 -> 52. A row's sixteen
+ * 16-byte pieces are stored rotated by an exclusive-or with its number
  * (the lane asks for piece slot ^ row), which spreads the 128-bit reads of eight neighbouring rows
  * over all banks. Weights stream through registers from the expert tiles (hipq_internal.h), a
  * super-block ahead.
  */
 #ifndef HIPQ_MOE_TILE_DEVICE_H
 #define HIPQ_MOE_TILE_DEVICE_H
+#include <type_traits>
+
 #include "gemv_device.h"
 
 namespace moe_tile {
 
 typedef int v2i __attribute__((ext_vector_type(2)));
+typedef int v3i __attribute__((ext_vector_type(3)));
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v16f __attribute__((ext_vector_type(16)));
@@ -52,16 +57,15 @@ struct Lds {
   int rows[ROWS]; /* where the item's rows lie in the activation planes */
   MinsLds m;
 };
-static_assert(sizeof(Lds) * 3 + 3 * 256 <= 160 * 1024, "three workgroups per CU must fit the 160 KB LDS");
+static_assert((sizeof(Lds) + 512) * 3 <= 158 * 1024, "three workgroups per CU must fit the 160 KB LDS");
 
 __device__ __forceinline__ int out_row(int tm, int r, int lane) { return 32 * tm + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
 
-/* The wavefront's column tile (its first byte is tile[0]) over the whole of K for the item's 32 * TM rows (l.rows, all of
- * them valid plane rows). done(acc, accm) receives the sums: acc[tm][r] - accm[tm][r] is row out_row(tm, r, lane), column
- * lane & 31. */
-template <int TM, typename Rows, typename Late, typename Done>
-__device__ __forceinline__ void run(Lds &l, const QView &a, uint32_t a_rows, const uint8_t *tile, Rows rows, Late late,
-                                    Done done) {
+/* The wavefront's column tile (its first byte is tile[0]) over the whole of K for the item's 32 * TM rows. rows() fills l.rows (valid
+ * plane rows, all of them), kept() may put into LDS what was asked for there, and done(acc, accm, free) receives the sums:
+ * acc[tm][r] - accm[tm][r] is row out_row(tm, r, lane), column lane & 31. It may use 4 KB of LDS a wavefront from free on. */
+template <int TM, typename Rows, typename Kept, typename Done>
+__device__ __forceinline__ void run(Lds &l, const QView &a, uint32_t a_rows, const uint8_t *tile, Rows rows, Kept kept, Done done) {
   const int K = a.K, nsb = K >> 8;
   const int lane = threadIdx.x & 63, i32 = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -76,19 +80,21 @@ __device__ __forceinline__ void run(Lds &l, const QView &a, uint32_t a_rows, con
   };
   auto load_hd = [&](int sb) {
     return __builtin_bit_cast(
-      v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, 4096 + i32 * 16, sb * hipq::EXPERT_TILE_BYTES, 0));
+      v3i, __builtin_amdgcn_raw_buffer_load_b96(rw, 4096 + i32 * 16, sb * hipq::EXPERT_TILE_BYTES, 0));
   };
+  v4i W[4];
+  v3i hd; /* the scales; the mins' pass reads the whole header */
   /* the weights are asked for before the rows are known */
-  v4i W[4], hd0, hd1;
 #pragma unroll
   for (int i = 0; i < 4; ++i) W[i] = load_q(0, i);
-  hd0 = load_hd(0);
+  hd = load_hd(0);
   rows();
   __syncthreads();
 
   const rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc((void *)a.q, 0, (int)(a_rows * (uint32_t)K), 0x00020000);
   const rsrc_t rm = __builtin_amdgcn_make_buffer_rsrc((void *)a.bsum, 0, (int)(a_rows * (uint32_t)nsb * 32), 0x00020000);
   const rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc((void *)a.d, 0, (int)(a_rows * (uint32_t)nsb * 4), 0x00020000);
+  auto lds_ptr = [](void *p) { return (__attribute__((address_space(3))) void *)p; };
   /* this lane's places: copy i of the wavefront moves rows 4 (2 TM wave + i) .. + 3 */
   uint32_t vq[2 * TM];
 #pragma unroll
@@ -97,7 +103,6 @@ __device__ __forceinline__ void run(Lds &l, const QView &a, uint32_t a_rows, con
     vq[i] = (uint32_t)l.rows[r] * (uint32_t)K + (uint32_t)(((lane & 15) ^ (r & 15)) * 16);
   }
   const uint32_t vd = (uint32_t)l.rows[lane & (32 * TM - 1)] * (uint32_t)(nsb * 4); /* row lane's scale */
-  auto lds_ptr = [](void *p) { return (__attribute__((address_space(3))) void *)p; };
   auto copy_rows = [&](int sb, int buf) {
 #pragma unroll
     for (int i = 0; i < 2 * TM; ++i)
@@ -105,27 +110,44 @@ __device__ __forceinline__ void run(Lds &l, const QView &a, uint32_t a_rows, con
                                                0, 0);
     if (wave == 0) __builtin_amdgcn_raw_ptr_buffer_load_lds(rd, lds_ptr(l.dA[buf]), 4, (int)vd, sb * 4, 0, 0);
   };
+  /* row sums and scales of the super-blocks m0 .. of the mins' pass */
+  const uint32_t vm = (uint32_t)l.rows[(32 * (wave & 1) + (lane >> 1)) & (32 * TM - 1)] * (uint32_t)(nsb * 32) + (lane & 1) * 16;
+  auto copy_mins = [&](int m0, int mn) {
+    for (int k = wave; k < TM * mn; k += 4) { /* 32 rows of a super-block; k % TM is wave % TM, as in vm */
+      const int b = k / TM, part = k % TM;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rm, lds_ptr(l.m.amin[b] + part * 1024), 16, (int)vm, (m0 + b) * 32, 0, 0);
+    }
+    for (int b = wave; b < mn; b += 4)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rd, lds_ptr(l.m.dA[b]), 4, (int)vd, (m0 + b) * 4, 0, 0);
+  };
+  /* headers of the super-blocks m0 .. of the mins' pass, [super-block][column] in the wavefront's 4 KB of a row buffer */
+  auto copy_headers = [&](int buf, int m0) {
+#pragma unroll
+    for (int b = 0; b < MINS_SB; b += 2) /* two of 32 columns an instruction; past the end the last one again: a fixed number of loads in flight */
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, lds_ptr(l.q[buf] + wave * 4096 + b * 512), 16,
+                                               4096 + (lane & 31) * 16 + min(m0 + b + (lane >> 5), nsb - 1) * (int)hipq::EXPERT_TILE_BYTES,
+                                               0, 0, 0);
+  };
 
   /* LDS byte of this lane's operand of step j: row i32, piece 2 j + g */
   const uint32_t abase = (uint32_t)(i32 * 256 + ((g ^ (i32 & 15)) << 4));
-
-  float acc[TM][16];
-#pragma unroll
-  for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[tm][r] = 0.f;
   uint32_t m4 = HIPQ_M4;
   asm("" : "+v"(m4)); /* an operand in a scalar register halves an instruction's rate */
+  float acc[TM][16];
 
   /* One super-block: the rows of the next are asked for first; a quarter of the nibbles is asked for
    * again (for the next super-block) as soon as its two steps have taken it, so one set of registers holds
    * the stream and most of a super-block's time covers every load. */
-  auto super_block = [&](int sb, int buf, const v4i &hd, v4i &hdn) {
-    const int sbn = min(sb + 1, nsb - 1); /* past the end the last one again: a fixed number of loads in flight */
-    copy_rows(sbn, buf ^ 1);
-    const int8_t *pq = l.q[buf];
-    const uint32_t hx = (uint32_t)hd[0];
-    const HipqDigits dgy = hipq_digits((uint32_t)hd[1]), dgz = hipq_digits((uint32_t)hd[2]);
+  auto super_block = [&](int sb, auto last) {
+    constexpr bool LAST = decltype(last)::value;
+    const int buf = sb & 1;
+    if (LAST)
+      copy_headers(buf ^ 1, 0);
+    else
+      copy_rows(sb + 1, buf ^ 1);
+    const int8_t *pq = l.q[0] + buf * (ROWS * 256);
+    HipqDigits dg;
+    const float dw = hipq_h2f((uint16_t)((uint32_t)hd[0] & 0xffff));
     v16i Dlo[TM], Dhi[TM];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -134,7 +156,7 @@ __device__ __forceinline__ void run(Lds &l, const QView &a, uint32_t a_rows, con
       asm("" : "+v"(at)); /* one instruction a step instead of eight registers */
 #pragma unroll
       for (int tm = 0; tm < TM; ++tm) av[tm] = *(const v4i *)(pq + (at ^ (j * 32)) + tm * 8192);
-      const HipqDigits &dg = j < 4 ? dgy : dgz;
+      if (j % 4 == 0) dg = hipq_digits((uint32_t)hd[1 + j / 4]);
       const uint32_t x0 = (uint32_t)W[j >> 1][2 * (j & 1)], x1 = (uint32_t)W[j >> 1][2 * (j & 1) + 1];
       const uint32_t e0 = x0 & m4, e1 = x1 & m4, o0 = (x0 >> 4) & m4, o1 = (x1 >> 4) & m4;
       const v4i bl = {hipq_scale4(e0, dg.lo, j & 3), hipq_scale4(e1, dg.lo, j & 3), hipq_scale4(o0, dg.lo, j & 3),
@@ -146,16 +168,15 @@ __device__ __forceinline__ void run(Lds &l, const QView &a, uint32_t a_rows, con
         Dlo[tm] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[tm], bl, j == 0 ? zero16 : Dlo[tm], 0, 0, 0);
         Dhi[tm] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[tm], bh, j == 0 ? zero16 : Dhi[tm], 0, 0, 0);
       }
-      if (j & 1) W[j >> 1] = load_q(sbn, j >> 1);
+      if (!LAST && (j & 1)) W[j >> 1] = load_q(sb + 1, j >> 1);
       __builtin_amdgcn_sched_barrier(0);
     }
-    hdn = load_hd(sbn);
-    const float dw = hipq_h2f((uint16_t)(hx & 0xffff));
+    if (!LAST) hd = load_hd(sb + 1);
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm) {
 #pragma unroll
       for (int q4 = 0; q4 < 4; ++q4) {
-        const v4i dv = *(const v4i *)((const int8_t *)l.dA[buf] + (32 * tm + 8 * q4 + 4 * g) * 4);
+        const v4i dv = *(const v4i *)((const int8_t *)l.dA[0] + buf * (ROWS * 4) + (32 * tm + 8 * q4 + 4 * g) * 4);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int r = 4 * q4 + e;
@@ -168,71 +189,55 @@ __device__ __forceinline__ void run(Lds &l, const QView &a, uint32_t a_rows, con
       __builtin_amdgcn_sched_barrier(0);
     }
     /* the rows copied above have arrived (they were issued before the five weight loads, which stay in flight) */
-    asm volatile("s_waitcnt vmcnt(5) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  };
-
-  /* row sums and scales of the super-blocks m0 .. of the mins' pass */
-  const uint32_t vm = (uint32_t)l.rows[(32 * (wave & 1) + (lane >> 1)) & (32 * TM - 1)] * (uint32_t)(nsb * 32) + (lane & 1) * 16;
-  auto copy_mins = [&](int m0, int mn) {
-    for (int k = wave; k < TM * mn; k += 4) { /* 32 rows of a super-block; k % TM is wave % TM, as in vm */
-      const int b = k / TM, part = k % TM;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rm, lds_ptr(l.m.amin[b] + part * 1024), 16, (int)vm, (m0 + b) * 32, 0, 0);
-    }
-    for (int b = wave; b < mn; b += 4)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rd, lds_ptr(l.m.dA[b]), 4, (int)vd, (m0 + b) * 4, 0, 0);
+    if (!LAST) asm volatile("s_waitcnt vmcnt(5) lgkmcnt(0)\n\ts_barrier" ::: "memory");
   };
 
   copy_rows(0, 0);
-  asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-  copy_mins(0, min(MINS_SB, nsb)); /* the first of them arrive during the products */
-  int sb = 0;
-  for (; sb + 1 < nsb; sb += 2) {
-    super_block(sb, 0, hd0, hd1);
-    super_block(sb + 1, 1, hd1, hd0);
-  }
-  if (sb < nsb) super_block(sb, 0, hd0, hd1);
+  kept();
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  copy_mins(0, min(MINS_SB, nsb)); /* they arrive during the products */
+#pragma unroll
+  for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[tm][r] = 0.f;
+  for (int sb = 0; sb + 1 < nsb; ++sb) super_block(sb, std::false_type{});
+  super_block(nsb - 1, std::true_type{});
 
   /* the mins: accm = fma(Im, dmin * dA, accm) over the super-blocks, in a pass of its own so that its
-   * chains do not occupy registers during the products. The headers come again, eight at once into the registers that
-   * the products no longer need. */
+   * chains do not occupy registers during the products */
+  const int hbuf = nsb & 1; /* the row buffer that the last super-block left free */
   float accm[TM][16];
 #pragma unroll
   for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
     for (int r = 0; r < 16; ++r) accm[tm][r] = 0.f;
-  late();
   for (int m0 = 0; m0 < nsb; m0 += MINS_SB) {
     const int mn = min(MINS_SB, nsb - m0);
     if (m0) {
       __syncthreads(); /* the sums in LDS have been read */
       copy_mins(m0, mn);
+      copy_headers(hbuf, m0);
     }
-    v4i hd[MINS_SB];
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    for (int b = 0; b < mn; ++b) {
+      const v4i hm = *(const v4i *)(l.q[hbuf] + wave * 4096 + b * 512 + i32 * 16);
+      const float dmin = hipq_h2f((uint16_t)((uint32_t)hm[0] >> 16));
+      const v8h bmin = hipq_mins8((uint32_t)hm[1], (uint32_t)hm[2], (uint32_t)hm[3]);
 #pragma unroll
-    for (int b = 0; b < MINS_SB; ++b)
-      if (b < mn) hd[b] = load_hd(m0 + b);
-    /* also the last copies of rows, which nothing reads: the row buffers are free behind this */
-    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+      for (int tm = 0; tm < TM; ++tm) {
+        const v8h amin = __builtin_bit_cast(v8h, *(const v4i *)(l.m.amin[b] + (32 * tm + i32) * 32 + g * 16));
+        const v16f Sm = __builtin_amdgcn_mfma_f32_32x32x16_f16(amin, bmin, zero16f, 0, 0, 0);
 #pragma unroll
-    for (int b = 0; b < MINS_SB; ++b)
-      if (b < mn) { /* uniform */
-        const float dmin = hipq_h2f((uint16_t)((uint32_t)hd[b][0] >> 16));
-        const v8h bmin = hipq_mins8((uint32_t)hd[b][1], (uint32_t)hd[b][2], (uint32_t)hd[b][3]);
+        for (int q4 = 0; q4 < 4; ++q4) {
+          const v4i dv = *(const v4i *)((const int8_t *)l.m.dA[b] + (32 * tm + 8 * q4 + 4 * g) * 4);
 #pragma unroll
-        for (int tm = 0; tm < TM; ++tm) {
-          const v8h amin = __builtin_bit_cast(v8h, *(const v4i *)(l.m.amin[b] + (32 * tm + i32) * 32 + g * 16));
-          const v16f Sm = __builtin_amdgcn_mfma_f32_32x32x16_f16(amin, bmin, zero16f, 0, 0, 0);
-#pragma unroll
-          for (int q4 = 0; q4 < 4; ++q4) {
-            const v4i dv = *(const v4i *)((const int8_t *)l.m.dA[b] + (32 * tm + 8 * q4 + 4 * g) * 4);
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              accm[tm][4 * q4 + e] = fmaf(Sm[4 * q4 + e], dmin * __int_as_float(dv[e]), accm[tm][4 * q4 + e]);
-          }
+          for (int e = 0; e < 4; ++e)
+            accm[tm][4 * q4 + e] = fmaf(Sm[4 * q4 + e], dmin * __int_as_float(dv[e]), accm[tm][4 * q4 + e]);
         }
       }
+    }
   }
-  done(acc, accm);
+  done(acc, accm, l.q[hbuf]);
 }
 
 } // namespace moe_tile

@@ -280,6 +280,34 @@ def test_moe_tiles_of_64_rows_of_many_experts(hipq, cr, h, i):
         w.destroy()
 
 
+@pytest.mark.parametrize("h,i", [(2048, 256), (2304, 512)])
+def test_moe_tiles_around_a_part_of_the_mins_pass(hipq, cr, h, i):
+    """The mins' pass takes eight super-blocks at a time: rows of exactly eight, and of one more; with and without biases, whose
+    tile kernels are forms of their own. Thirty pairs an expert: items of more than 32 rows and of fewer."""
+    import gpu_util as gu
+    import torch
+    t, e, k = 600, 40, 2
+    gate, up, down = ([m[j % 3] for j in range(e)] for m in _experts(cr, 3, i, h, seed=5200))
+    x, logits = synth.normal(5201, (t, h)), synth.normal(5202, (t, e))
+    gb, ub, db = (synth.normal(5203 + j, (e, n), 0.1) for j, n in enumerate((i, i, h)))
+    wg = [capi.Weight("q4_K", i, h, b) for b in gate]
+    wu = [capi.Weight("q4_K", i, h, b) for b in up]
+    wd = [capi.Weight("q4_K", h, i, b) for b in down]
+    ref = cr.moe_forward(x, logits, gate, up, down, k)[0]
+    y = torch.full((t, h), float("nan"), device="cuda")
+    capi.moe_forward(t, h, i, e, k, wg, wu, wd, gu.dev(x), y, router_logits=gu.dev(logits), stream=gu.stream())
+    torch.cuda.synchronize()
+    assert gu.rel_err(y.cpu().numpy(), ref) <= 2e-6  # the last bits of the softmax's sum, as above
+    ref = cr.moe_forward_gpt_oss(x, logits, gate, up, down, gb, ub, db, k)[0]
+    y.fill_(float("nan"))
+    capi.moe_forward_gpt_oss(t, h, i, e, k, wg, wu, wd, gu.dev(x), y, gu.dev(gb), gu.dev(ub), gu.dev(db),
+                             router_logits=gu.dev(logits), stream=gu.stream())
+    torch.cuda.synchronize()
+    assert gu.rel_err(y.cpu().numpy(), ref) <= gu.TOL  # the device's expf against the host's
+    for w in wg + wu + wd:
+        w.destroy()
+
+
 def test_expert_weights_serve_the_moe_block_only(hipq, cr):
     """Q4_K experts are re-stored for the expert kernels at the first block; a plain
     matmul on such a handle is refused, the block keeps giving the same bits."""
