@@ -149,13 +149,17 @@ __device__ __forceinline__ void run(Lds &l, const QView &a, uint32_t a_rows, con
     HipqDigits dg;
     const float dw = hipq_h2f((uint16_t)((uint32_t)hd[0] & 0xffff));
     v16i Dlo[TM], Dhi[TM];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      v4i av[TM];
+    v4i av[2][TM]; /* the rows of a step are read a step ahead: a block of 1000 tokens 198.4 -> 197.7 us */
+    auto read_a = [&](int j) {
       uint32_t at = abase;
       asm("" : "+v"(at)); /* one instruction a step instead of eight registers */
 #pragma unroll
-      for (int tm = 0; tm < TM; ++tm) av[tm] = *(const v4i *)(pq + (at ^ (j * 32)) + tm * 8192);
+      for (int tm = 0; tm < TM; ++tm) av[j & 1][tm] = *(const v4i *)(pq + (at ^ (j * 32)) + tm * 8192);
+    };
+    read_a(0);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (j + 1 < 8) read_a(j + 1);
       if (j % 4 == 0) dg = hipq_digits((uint32_t)hd[1 + j / 4]);
       const uint32_t x0 = (uint32_t)W[j >> 1][2 * (j & 1)], x1 = (uint32_t)W[j >> 1][2 * (j & 1) + 1];
       const uint32_t e0 = x0 & m4, e1 = x1 & m4, o0 = (x0 >> 4) & m4, o1 = (x1 >> 4) & m4;
@@ -165,8 +169,8 @@ __device__ __forceinline__ void run(Lds &l, const QView &a, uint32_t a_rows, con
                       hipq_scale4(o1, dg.hi, j & 3)};
 #pragma unroll
       for (int tm = 0; tm < TM; ++tm) {
-        Dlo[tm] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[tm], bl, j == 0 ? zero16 : Dlo[tm], 0, 0, 0);
-        Dhi[tm] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[tm], bh, j == 0 ? zero16 : Dhi[tm], 0, 0, 0);
+        Dlo[tm] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[j & 1][tm], bl, j == 0 ? zero16 : Dlo[tm], 0, 0, 0);
+        Dhi[tm] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[j & 1][tm], bh, j == 0 ? zero16 : Dhi[tm], 0, 0, 0);
       }
       if (!LAST && (j & 1)) W[j >> 1] = load_q(sb + 1, j >> 1);
       __builtin_amdgcn_sched_barrier(0);
