@@ -245,13 +245,12 @@ __device__ __forceinline__ void host_done(const HostDone &hd) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); /* the stores have arrived in host memory */
   __syncthreads();
   if (threadIdx.x) return;
-  /* sixteen counters and one of them, so that few atomics meet on a line */
+  /* Sixteen counters and one of them, so that few atomics meet on a line. The arrival that completes a counter wraps it to
+   * zero in the same atomic, so that all are zero before the word is written: the next call may come on another queue of
+   * the same handle (threads that share hipStreamPerThread), ordered behind this one by nothing but the word. */
   const uint32_t line = (blockIdx.x + blockIdx.y * hd.width) & 15, mine = (hd.groups + 15 - line) >> 4, lines = hd.groups < 16 ? hd.groups : 16;
-  uint32_t *c = hd.count + line * 16, *all = hd.count + 256;
-  if (__hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 != mine) return;
-  __hip_atomic_store(c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if (__hip_atomic_fetch_add(all, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 != lines) return;
-  __hip_atomic_store(all, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (atomicInc(hd.count + line * 16, mine - 1) != mine - 1) return;
+  if (atomicInc(hd.count + 256, lines - 1) != lines - 1) return;
   __hip_atomic_store(hd.word, hd.value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 constexpr size_t HOST_DONE_BYTES = 17 * 64;

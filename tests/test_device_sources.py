@@ -22,3 +22,13 @@ def test_no_assembly_computes_beside_matrix_instructions(path):
         for template in re.findall(r'\basm\s*(?:volatile\s*)?\(\s*((?:"[^"]*"\s*)*)', open(f).read()):
             found += [(os.path.basename(f), x) for x in re.findall(r"\b(?:v|buffer|global|flat|ds)_\w+", template)]
     assert not found
+
+
+def test_shared_arrival_counters_are_zero_before_the_word_that_ends_a_call():
+    """host_done's counters belong to a stream's handle. A call on the same handle may come from another thread's queue, behind
+    nothing but the word this call's last workgroup writes (hipStreamPerThread, hipq_stream_release in hipq.h): the counters
+    go back to zero in the arrivals themselves, not by stores of which one may be late."""
+    text = open(os.path.join(CSRC, "hipq_internal.h")).read()
+    body = text[text.index("void host_done("):text.index("constexpr size_t HOST_DONE_BYTES")]
+    assert re.findall(r"__hip_atomic_store\(([^,]+),", body) == ["hd.word"]
+    assert len(re.findall(r"atomicInc\(hd\.count", body)) == 2 and "fetch_add" not in body

@@ -344,3 +344,41 @@ def test_calls_that_their_last_workgroup_ends(hipq, cr, kind, m, k, ns):
             capi.host_free(p)
         for w in ws:
             w.destroy()
+
+
+def test_threads_in_turn_on_the_per_thread_stream(hipq, cr):
+    """Two threads that share the handle hipStreamPerThread, call after call in turn: queues of their own, one set of arrival
+    counters and one word, ordered by each call's return alone. The device call's bits, 129 and 32 workgroups."""
+    import threading
+    per_thread = 2  # hipStreamPerThread
+    work = []
+    for m, n, k in ((8, 4100, 256), (3, 1024, 512)):
+        w = capi.Weight("q4_K", n, k, cr.quantize_weights(cr.oracle(), "q4_K", synth.normal(9800 + n, (n, k), 0.02)))
+        a = synth.normal(9801 + n, (m, k))
+        work.append((w, m, n, k, a, _device_result(w, a), capi.host_alloc(m * k * 4), capi.host_alloc(m * n * 4)))
+    turn, failed = threading.Semaphore(1), []
+
+    def calls(index):
+        w, m, n, k, a, want, pa, pc = work[index]
+        a_pin = np.ctypeslib.as_array(ctypes.cast(pa, ctypes.POINTER(ctypes.c_float)), (m, k))
+        c_pin = np.ctypeslib.as_array(ctypes.cast(pc, ctypes.POINTER(ctypes.c_float)), (m, n))
+        for rep in range(100):
+            scale = np.float32(2.0 ** (rep % 5))
+            with turn:
+                a_pin[:] = a * scale
+                c_pin[:] = np.nan
+                capi.matmul(w, pa, m, pc, mem=capi.MEM_HOST, stream=per_thread)
+                if not np.array_equal(c_pin, want * scale):
+                    failed.append((index, rep))
+
+    threads = [threading.Thread(target=calls, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    capi.stream_release(per_thread)
+    for w, _, _, _, _, _, pa, pc in work:
+        capi.host_free(pa)
+        capi.host_free(pc)
+        w.destroy()
+    assert not failed
