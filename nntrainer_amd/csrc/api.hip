@@ -305,26 +305,42 @@ int pinned_staging(hipStream_t s, size_t bytes, void **out) {
 __global__ void signal_done_kernel(uint32_t *word, uint32_t value) {
   __hip_atomic_store(word, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
-/* the word and the counters of the stream; without them (a full device) the call ends in the stream's wait */
+__global__ void clear_counts_kernel(uint32_t *count) {
+  for (uint32_t i = threadIdx.x; i < hipq::HOST_DONE_BYTES / 4; i += blockDim.x) count[i] = 0;
+}
+/* The word and the counters of the stream; without them (a full device) the call ends in the stream's wait. The caller holds
+ * the stream's enqueue lock. A stream's first call makes them, outside the library's lock and with the zeros written in order
+ * on the stream: no other thread and no other stream's work is waited for. Not while the stream is being captured: the
+ * zeros would be a node of the graph. */
 void begin_end(hipStream_t s, hipq::HostEnd *end) {
-  std::lock_guard<std::mutex> lk(g.mu);
-  Workspace &w = g.ws[s];
-  if (!w.done) {
-    static const char zeros[hipq::HOST_DONE_BYTES] = {};
+  Workspace *w;
+  {
+    std::lock_guard<std::mutex> lk(g.mu);
+    w = &g.ws[s]; /* nodes of the map do not move */
+  }
+  if (!w->done) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cs) != hipSuccess) (void)hipGetLastError();
+    if (cs != hipStreamCaptureStatusNone) return;
     void *word = nullptr, *dev = nullptr, *count = nullptr;
-    if (hipHostMalloc(&word, 64, hipHostMallocDefault) != hipSuccess || hipHostGetDevicePointer(&dev, word, 0) != hipSuccess ||
-        hipMalloc(&count, sizeof zeros) != hipSuccess || hipMemcpy(count, zeros, sizeof zeros, hipMemcpyHostToDevice) != hipSuccess) {
+    bool made = hipHostMalloc(&word, 64, hipHostMallocDefault) == hipSuccess && hipHostGetDevicePointer(&dev, word, 0) == hipSuccess &&
+                hipMalloc(&count, hipq::HOST_DONE_BYTES) == hipSuccess;
+    if (made) {
+      hipq::launch_kernel("clear_counts_kernel", clear_counts_kernel, dim3(1), dim3(64), 0, s, (uint32_t *)count);
+      made = hipGetLastError() == hipSuccess;
+    }
+    if (!made) {
       (void)hipGetLastError();
       if (count) (void)hipFree(count);
       if (word) (void)hipHostFree(word);
       return;
     }
-    w.done = (uint32_t *)word, w.done_dev = (uint32_t *)dev, w.done_count = (uint32_t *)count;
-    *w.done = 0;
+    *(uint32_t *)word = 0;
+    w->done_dev = (uint32_t *)dev, w->done_count = (uint32_t *)count, w->done = (uint32_t *)word;
   }
-  end->d.count = w.done_count;
-  end->d.word = w.done_dev;
-  end->d.value = ++w.done_seq;
+  end->d.count = w->done_count;
+  end->d.word = w->done_dev;
+  end->d.value = ++w->done_seq;
 }
 int wait_done(hipStream_t s, const hipq::HostEnd &end) {
   if (!end.d.word) {

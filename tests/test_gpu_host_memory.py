@@ -382,3 +382,38 @@ def test_threads_in_turn_on_the_per_thread_stream(hipq, cr):
         capi.host_free(pc)
         w.destroy()
     assert not failed
+
+
+def test_a_streams_first_host_call_waits_for_no_other_stream(hipq, cr):
+    """What a stream's first call on host memory sets up is made in order on that stream: work under way on the default stream,
+    hundreds of milliseconds of it, is still under way when the call returns."""
+    import torch
+    m, n, k = 8, 2048, 512
+    w = capi.Weight("q4_K", n, k, cr.quantize_weights(cr.oracle(), "q4_K", synth.normal(9900, (n, k), 0.02)))
+    a = synth.normal(9901, (m, k))
+    want = _device_result(w, a)
+    pa, pc = capi.host_alloc(m * k * 4), capi.host_alloc(m * n * 4)
+    try:
+        np.ctypeslib.as_array(ctypes.cast(pa, ctypes.POINTER(ctypes.c_float)), (m, k))[:] = a
+        c_pin = np.ctypeslib.as_array(ctypes.cast(pc, ctypes.POINTER(ctypes.c_float)), (m, n))
+        x, y = (torch.ones((8192, 8192), device="cuda", dtype=torch.bfloat16) for _ in range(2))
+        other, end = torch.cuda.Stream(), torch.cuda.Event()
+        capi.matmul(w, pa, m, pc, mem=capi.MEM_HOST, stream=other.cuda_stream)
+        capi.stream_release(other.cuda_stream)
+        torch.mm(x, x, out=y)
+        torch.cuda.synchronize()
+        for _ in range(300):
+            torch.mm(x, x, out=y)
+        end.record()
+        for _ in range(2):
+            c_pin[:] = np.nan
+            capi.matmul(w, pa, m, pc, mem=capi.MEM_HOST, stream=other.cuda_stream)
+            assert np.array_equal(c_pin.view(np.uint32), want.view(np.uint32))
+        assert not end.query()
+        torch.cuda.synchronize()
+        capi.stream_release(other.cuda_stream)
+    finally:
+        torch.cuda.synchronize()
+        capi.host_free(pa)
+        capi.host_free(pc)
+        w.destroy()
