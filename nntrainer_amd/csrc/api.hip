@@ -1451,7 +1451,8 @@ int hipq_matmul_each_row(hipq_weight_t w, const float *A, int64_t rows, int64_t 
           break;
         }
       }
-    rc = matmul_device(w, dA + r0 * a_ld, n, a_ld, dC + r0 * c_ld, c_ld, s, sc, true, r0 + n == rows ? &dio.end : nullptr);
+    /* several launches write the outputs, the earlier ones through the caches: a launch behind them ends the call (HostDone) */
+    rc = matmul_device(w, dA + r0 * a_ld, n, a_ld, dC + r0 * c_ld, c_ld, s, sc, true, n == rows ? &dio.end : nullptr);
     r0 += n;
   }
   if (rc || mem == HIPQ_MEM_DEVICE) return rc;

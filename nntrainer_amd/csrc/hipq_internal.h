@@ -220,8 +220,9 @@ inline void launch_kernel(const char *name, void (*kernel)(KArgs...), dim3 grid,
                           hipGetErrorString(e_), __FILE__, __LINE__);         \
   } while (0)
 
-/* The end of a synchronous call on a few rows of host memory, for a product whose launch is the call's last (the kernels of
- * gemm_rows_*.hip): its outputs are stored past the caches as the workgroups end (store_out), where the end of the kernel had
+/* The end of a synchronous call on a few rows of host memory, for a product whose launch alone writes the call's outputs (the
+ * kernels of gemm_rows_*.hip; the word vouches for this launch's stores only, which are past the caches and waited for, and
+ * signal_done_kernel's release for those of several launches): its outputs are stored past the caches as the workgroups end (store_out), where the end of the kernel had
  * written all of them back at once, and the last workgroup writes `value` to the page-locked word that the host polls
  * (host_done), where a launch behind it did. word: null where the outputs are in device memory. us a call of page-locked rows,
  * before -> with the stores -> with both: eight rows of 12288 x 4096 Q4_K 29.6 -> 27.9 -> 27.1; before -> both: sixteen rows 44.5 ->

@@ -417,3 +417,33 @@ def test_a_streams_first_host_call_waits_for_no_other_stream(hipq, cr):
         capi.host_free(pa)
         capi.host_free(pc)
         w.destroy()
+
+
+@pytest.mark.parametrize("kind,rows,one_launch", [("q6_K", 16, True), ("q6_K", 24, False), ("q6_K", 40, False), ("q4_K", 64, True),
+                                                  ("q4_K", 72, False), ("q4_0", 24, True)])
+def test_only_a_launch_that_writes_all_outputs_ends_its_call(hipq, cr, kind, rows, one_launch):
+    """Rows as products of their own in host memory: one launch up to 16 (Q6_K) and 64 rows (Q4_K), which tells the host itself;
+    more rows take several, and a launch behind all of them ends the call. The device call's bits."""
+    n, k = 4100, 512
+    w = capi.Weight(kind, n, k, cr.quantize_weights(cr.oracle(), kind, synth.normal(9950 + rows, (n, k), 0.02)))
+    a = synth.normal(9951, (rows, k))
+    import gpu_util as gu
+    import torch
+    want = torch.empty((rows, n), device="cuda")
+    capi.matmul_each_row(w, gu.dev(a), rows, want, stream=gu.stream())
+    torch.cuda.synchronize()
+    pa, pc = capi.host_alloc(rows * k * 4), capi.host_alloc(rows * n * 4)
+    try:
+        np.ctypeslib.as_array(ctypes.cast(pa, ctypes.POINTER(ctypes.c_float)), (rows, k))[:] = a
+        c_pin = np.ctypeslib.as_array(ctypes.cast(pc, ctypes.POINTER(ctypes.c_float)), (rows, n))
+        c_pin[:] = np.nan
+        with capi.LaunchTiming(64) as t:
+            capi.matmul_each_row(w, pa, rows, pc, mem=capi.MEM_HOST, stream=gu.stream())
+        assert np.array_equal(c_pin.view(np.uint32), want.cpu().numpy().view(np.uint32))
+        names = [name for name, _ in t.launches]
+        products = [x for x in names if x.startswith("gemm_rows_")]
+        assert (len(products) == 1) == one_launch and (names[-1] != "signal_done_kernel") == one_launch, names
+    finally:
+        capi.host_free(pa)
+        capi.host_free(pc)
+        w.destroy()
