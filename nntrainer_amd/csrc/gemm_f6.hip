@@ -178,8 +178,10 @@ __device__ __forceinline__ void f6_sums(const uint8_t *wbase, int N, int chunks,
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
     copy(min(k, last), k * BUF);
+    __builtin_amdgcn_sched_barrier(0); /* the counted waits here and in the first chunk rest on this order */
     load_w(min(k, last), k, 0, 6);
     load_dw(min(k, last), k);
+    __builtin_amdgcn_sched_barrier(0);
   }
   /* chunk 0 is there; the second chunk's loads, three or four of rows and seven of weights, may be under way */
   asm volatile("s_waitcnt vmcnt(10)\n\ts_barrier" ::: "memory");

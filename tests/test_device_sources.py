@@ -32,3 +32,17 @@ def test_shared_arrival_counters_are_zero_before_the_word_that_ends_a_call():
     body = text[text.index("void host_done("):text.index("constexpr size_t HOST_DONE_BYTES")]
     assert re.findall(r"__hip_atomic_store\(([^,]+),", body) == ["hd.word"]
     assert len(re.findall(r"atomicInc\(hd\.count", body)) == 2 and "fetch_add" not in body
+
+
+def test_loads_before_a_counted_wait_keep_their_order():
+    """f6_sums waits for copies into LDS by the number of loads issued behind them (s_waitcnt vmcnt with a count): each chunk's
+    copies are fenced off from the weight loads behind them, and those from the next chunk's copies, in the prologue as in
+    the loop."""
+    text = open(os.path.join(CSRC, "gemm_f6.hip")).read()
+    body = text[text.index("f6_sums(const uint8_t *wbase"):text.index("f6_tile(const uint8_t *wbase")]
+    assert re.findall(r"vmcnt\((\d+)\)", body) == ["10", "0", "7", "0"]
+    fence = r"__builtin_amdgcn_sched_barrier\(0\);"
+    calls = [m.end() for m in re.finditer(r"^ +(?:copy|load_dw)\([^;]*\);", body, re.M)]
+    assert len(calls) == 4  # one of each in the prologue and in the loop
+    for end in calls:
+        assert re.match(r"\s*" + fence, body[end:]), body[end - 40:end + 80]
