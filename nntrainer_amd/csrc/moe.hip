@@ -1710,14 +1710,16 @@ __device__ __forceinline__ bool tile_item(int cols, int rows, const int *__restr
   return true;
 }
 
-/* Rows of an output, n of them from base on: stores to rows past them are dropped, so that all are issued without conditions. */
+/* Rows of an output, n of them from base on: stores to rows past them are dropped, so that all are issued without conditions.
+ * The whole of a place stands in the lane's operand: that is what the hardware's check against the descriptor's size is
+ * defined on, a scalar offset beside it is not. */
 struct OutRows {
   moe_tile::rsrc_t r;
   __device__ __forceinline__ OutRows(float *base, int n, int cols) {
     r = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, n * cols * (int)sizeof(float), 0x00020000);
   }
-  __device__ __forceinline__ void put(int lane_at, int uniform_at, float v) const {
-    __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(v), r, lane_at * 4, uniform_at * 4, 0);
+  __device__ __forceinline__ void put(int at, float v) const {
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(v), r, at * (int)sizeof(float), 0, 0);
   }
 };
 
@@ -1763,7 +1765,7 @@ __device__ __forceinline__ void gate_up_tile_pass(moe_tile::Lds &l, const QView 
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int k = (up ? HALF : 0) + i0 + i;
-          out.put(4 * (lane >> 5) * I + c, moe_tile::out_row(k >> 4, k & 15, 0) * I, o[i]);
+          out.put(4 * (lane >> 5) * I + c + moe_tile::out_row(k >> 4, k & 15, 0) * I, o[i]);
         }
       }
     });
@@ -1817,7 +1819,7 @@ __device__ __forceinline__ void down_tile_pass(moe_tile::Lds &l, const QView &hq
         for (int r = 0; r < 16; ++r) {
           const int urow = moe_tile::out_row(tm, r, 0); /* out_row = urow + g4 */
           const float o = acc[tm][r] - accm[tm][r], wt = wrow[urow + g4];
-          out.put(g4 * H + c, urow * H, BIASED ? moe_out(ep, e, H, c, o, wt) : o * wt);
+          out.put(g4 * H + c + urow * H, BIASED ? moe_out(ep, e, H, c, o, wt) : o * wt);
         }
     });
 }

@@ -308,6 +308,33 @@ def test_moe_tiles_around_a_part_of_the_mins_pass(hipq, cr, h, i):
         w.destroy()
 
 
+def test_moe_items_that_end_in_front_of_another_experts(hipq, cr):
+    """Items of one row and of one row more than a row tile, each in front of another expert's rows and one as the block's last:
+    the tiles store their rows without conditions, those past an item dropped by the buffer's size. Every row has the bits
+    of its token alone, whose kernels are others."""
+    import gpu_util as gu
+    import torch
+    counts = [65, 64, 33, 96, 1, 70, 129]
+    t, e, k, h, i = sum(counts), len(counts), 1, 512, 256
+    gate, up, down = _experts(cr, e, i, h, seed=9700)
+    x = synth.normal(9701, (t, h))
+    logits = synth.normal(9702, (t, e))
+    logits[np.arange(t), np.repeat(np.arange(e), counts)] += 20.0
+    ws = [[capi.Weight("q4_K", n, c, b) for b in m] for m, n, c in ((gate, i, h), (up, i, h), (down, h, i))]
+    ex = capi.Experts(*ws)
+    dx, dl = gu.dev(x), gu.dev(logits)
+    y, one = (torch.full((t, h), float("nan"), device="cuda") for _ in range(2))
+    with capi.LaunchTiming(64) as timing:
+        capi.moe_forward(t, h, i, e, k, ex, None, None, dx, y, router_logits=dl, stream=gu.stream())
+    assert "down_tile_kernel" in [name for name, _ in timing.launches]
+    for r in range(t):
+        capi.moe_forward(1, h, i, e, k, ex, None, None, dx[r:], one[r:], router_logits=dl[r:], stream=gu.stream())
+    torch.cuda.synchronize()
+    assert torch.equal(y, one)
+    for w in sum(ws, []):
+        w.destroy()
+
+
 def test_expert_weights_serve_the_moe_block_only(hipq, cr):
     """Q4_K experts are re-stored for the expert kernels at the first block; a plain
     matmul on such a handle is refused, the block keeps giving the same bits."""
