@@ -83,11 +83,9 @@ struct SRegs {
 /* Up to four weights of one K against the same quantized rows as ONE launch: the grid's columns are
  * the concatenation of the weights' column tiles (Q, K, V or gate, up of a layer). */
 struct MultiRowsQ40 {
-  const uint8_t *qs[4];
-  const uint16_t *d[4];
+  WView w[4];
   float *C[4];
   int64_t ldc[4];
-  int N[4];
   int tile_end[4]; /* running sum of the weights' column tiles */
 };
 
@@ -95,23 +93,21 @@ struct MultiRowsQ40 {
  * itself, a round ahead, with the arithmetic of the Q8_0 quantizer kernel (the same bits): no
  * quantizer launch and no workspace. For launches of few workgroups, where that launch costs more
  * than the repeated quantization. */
-template <bool FUSED>
+template <bool FUSED, bool HOST>
 __global__ __launch_bounds__(NT, 2) void gemm_rows_q40_kernel(MultiRowsQ40 mw, QView a, const float *__restrict__ Af,
                                                               int64_t lda, int M_all, hipq::HostDone hd) {
   extern __shared__ __attribute__((aligned(16))) unsigned char rows_lds[];
-  asm volatile("" ::"s"(hd.word)); /* asked for here, not at the end */
+  if (HOST) asm volatile("" ::"s"(hd.word)); /* asked for here, not at the end */
   /* which weight this workgroup's column tile belongs to (uniform) */
   int tile = blockIdx.x, wi = 0;
   if (tile >= mw.tile_end[0]) wi = 1;
   if (tile >= mw.tile_end[1]) wi = 2;
   if (tile >= mw.tile_end[2]) wi = 3;
-  tile -= wi == 0 ? 0 : wi == 1 ? mw.tile_end[0] : wi == 2 ? mw.tile_end[1] : mw.tile_end[2];
-  const uint8_t *qs = wi == 0 ? mw.qs[0] : wi == 1 ? mw.qs[1] : wi == 2 ? mw.qs[2] : mw.qs[3];
-  const uint16_t *wd = wi == 0 ? mw.d[0] : wi == 1 ? mw.d[1] : wi == 2 ? mw.d[2] : mw.d[3];
-  const int N = wi == 0 ? mw.N[0] : wi == 1 ? mw.N[1] : wi == 2 ? mw.N[2] : mw.N[3];
+  if (wi) tile -= mw.tile_end[wi - 1];
+  const WView w = wi == 0 ? mw.w[0] : wi == 1 ? mw.w[1] : wi == 2 ? mw.w[2] : mw.w[3];
   float *__restrict__ C = wi == 0 ? mw.C[0] : wi == 1 ? mw.C[1] : wi == 2 ? mw.C[2] : mw.C[3];
   const int64_t ldc = wi == 0 ? mw.ldc[0] : wi == 1 ? mw.ldc[1] : wi == 2 ? mw.ldc[2] : mw.ldc[3];
-  const int K = a.K, nb = K >> 5;
+  const int K = w.K, nb = K >> 5;
   const int r0 = blockIdx.y * TC;
   const int M = min(TC, M_all - r0);
   if (FUSED) {
@@ -122,14 +118,14 @@ __global__ __launch_bounds__(NT, 2) void gemm_rows_q40_kernel(MultiRowsQ40 mw, Q
   }
   C += (int64_t)r0 * ldc;
   const int n0 = tile * 32;
-  const int ncols = min(32, N - n0);
+  const int ncols = min(32, w.N - n0);
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int lane = threadIdx.x & 63, i32 = lane & 31, g = lane >> 5;
   const int t = threadIdx.x;
   uint32_t *const lrec = (uint32_t *)(rows_lds + LDS_REC);
 
   /* the tile's nibbles as a buffer descriptor in scalar registers; columns past N repeat the last */
-  const qrsrc_t rq = __builtin_amdgcn_make_buffer_rsrc((void *)(qs + (size_t)n0 * (size_t)(K >> 1)), 0,
+  const qrsrc_t rq = __builtin_amdgcn_make_buffer_rsrc((void *)(w.qs + (size_t)n0 * (size_t)(K >> 1)), 0,
                                                        ncols * (K >> 1), 0x00020000);
   /* load i of a lane: 16 bytes of column 8 i + lane / 8, so that eight lanes cover the 128-byte line a
    * column's eight blocks are and a load instruction eight whole lines (a lane loading its own
@@ -160,7 +156,7 @@ __global__ __launch_bounds__(NT, 2) void gemm_rows_q40_kernel(MultiRowsQ40 mw, Q
       *(qv4i *)(rows_lds + LDS_Q + (c >> 6) * QROW + (c & 63) * 16) = r[u];
     }
   };
-  const uint16_t *const dcol = wd + (size_t)(n0 + min(t >> 3, ncols - 1)) * nb;
+  const uint16_t *const dcol = w.d + (size_t)(n0 + min(t >> 3, ncols - 1)) * nb;
   auto s_load = [&](SRegs &r, int rho) {
     if (!FUSED) r.meta = a.meta[(size_t)min(t >> 5, M - 1) * nb + min(rho * BR + (t & 31), nb - 1)];
     r.dw = *(const uint2 *)(dcol + min(rho * BR + (t & 7) * 4, nb - 4));
@@ -310,8 +306,11 @@ __global__ __launch_bounds__(NT, 2) void gemm_rows_q40_kernel(MultiRowsQ40 mw, Q
     }
   }
   const int col = n0 + cn;
-  if (cm < M && col < N) hipq::store_out(C + (int64_t)cm * ldc + col, acc, hd);
-  hipq::host_done(hd);
+  if (HOST) {
+    if (cm < M && col < w.N) hipq::store_out(C + (int64_t)cm * ldc + col, acc);
+    hipq::host_done(hd);
+  } else if (cm < M && col < w.N)
+    C[(int64_t)cm * ldc + col] = acc;
 }
 
 } // namespace
@@ -387,23 +386,23 @@ static int launch_rows_q40(int count, const hipq_weight *const *w, const QAct *q
         return fail(HIPQ_ERR_INVALID_ARGUMENT, "the few-rows Q4_0 product takes Q4_0 weights of the rows' K, in whole 256s");
       tiles += (int)((w[i]->N + 31) / 32);
     }
-    mw.qs[i] = w[j]->qs;
-    mw.d[i] = w[j]->d;
-    mw.N[i] = (int)w[j]->N;
+    mw.w[i] = wview(w[j]);
     mw.C[i] = C[j];
     mw.ldc[i] = ldc[j];
     mw.tile_end[i] = tiles; /* unused entries repeat the total: no workgroup lands in them */
   }
   const dim3 grid((unsigned)tiles, (unsigned)((M + TC - 1) / TC));
-  if (qa) {
-    hipq::launch_kernel("gemm_rows_q40_kernel<false>", gemm_rows_q40_kernel<false>, grid, dim3(NT), LDS_BYTES, s, mw, qview(*qa), (const float *)nullptr,
-                       (int64_t)0, M, take_end(end, grid));
-  } else {
-    QView none{};
-    none.K = (int)w[0]->K;
-    hipq::launch_kernel("gemm_rows_q40_kernel<true>", gemm_rows_q40_kernel<true>, grid, dim3(NT), LDS_BYTES, s, mw, none, A, lda, M,
-                        take_end(end, grid));
-  }
+  QView rows{};
+  rows.K = (int)w[0]->K;
+  if (qa) rows = qview(*qa);
+  const HostDone hd = take_end(end, grid);
+  auto go = [&](const char *name, auto kernel) { launch_kernel(name, kernel, grid, dim3(NT), LDS_BYTES, s, mw, rows, A, lda, M, hd); };
+  if (qa)
+    hd.word ? go("gemm_rows_q40_kernel<false, true>", gemm_rows_q40_kernel<false, true>)
+            : go("gemm_rows_q40_kernel<false, false>", gemm_rows_q40_kernel<false, false>);
+  else
+    hd.word ? go("gemm_rows_q40_kernel<true, true>", gemm_rows_q40_kernel<true, true>)
+            : go("gemm_rows_q40_kernel<true, false>", gemm_rows_q40_kernel<true, false>);
   HIPQ_HIP(hipGetLastError());
   return HIPQ_OK;
 }

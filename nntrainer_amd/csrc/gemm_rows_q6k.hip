@@ -44,10 +44,11 @@ struct Regs { /* a lane's half of a super-block: steps s = 0 .. 7 of sixteen wei
   v4i q[4], h[2], hd;
 };
 
+template <bool HOST>
 __global__ __launch_bounds__(NT, 2) void gemm_rows_q6k_kernel(WView w, QView a, int M_all, float *__restrict__ C, int64_t ldc,
                                                               hipq::HostDone hd) {
   extern __shared__ __attribute__((aligned(16))) unsigned char rows_lds[];
-  asm volatile("" ::"s"(w.qs), "s"(w.qh), "s"(w.hdr), "s"(w.N), "s"(w.K), "s"(a.q), "s"(a.d), "s"(M_all), "s"(C), "s"(ldc), "s"(hd.word));
+  if (HOST) asm volatile("" ::"s"(w.qs), "s"(w.qh), "s"(w.hdr), "s"(w.N), "s"(w.K), "s"(a.q), "s"(a.d), "s"(M_all), "s"(C), "s"(ldc), "s"(hd.word));
   const int tile = blockIdx.x, K = w.K, nsb = K >> 8;
   const int r0 = blockIdx.y * TC, M = min(TC, M_all - r0);
   a.q += (size_t)r0 * K;
@@ -190,9 +191,12 @@ __global__ __launch_bounds__(NT, 2) void gemm_rows_q6k_kernel(WView w, QView a, 
     }
   }
   const int col = tile * 32 + cn;
-  if (cm < M && col < w.N)
-    hipq::store_out(C + (int64_t)cm * ldc + col, ((acc[0] + acc[4]) + (acc[2] + acc[6])) + ((acc[1] + acc[5]) + (acc[3] + acc[7])), hd);
-  hipq::host_done(hd);
+  const float sum = ((acc[0] + acc[4]) + (acc[2] + acc[6])) + ((acc[1] + acc[5]) + (acc[3] + acc[7]));
+  if (HOST) {
+    if (cm < M && col < w.N) hipq::store_out(C + (int64_t)cm * ldc + col, sum);
+    hipq::host_done(hd);
+  } else if (cm < M && col < w.N)
+    C[(int64_t)cm * ldc + col] = sum;
 }
 
 } // namespace
@@ -228,7 +232,9 @@ int launch_gemm_rows_q6k(const hipq_weight *w, const QAct *qa, int M, float *C, 
   v.qh = w->gt_qh;
   v.hdr = w->gt_hdr;
   const dim3 grid((unsigned)((w->N + 31) / 32), (unsigned)((M + TC - 1) / TC));
-  launch_kernel("gemm_rows_q6k_kernel", gemm_rows_q6k_kernel, grid, dim3(NT), LDS_BYTES, s, v, qview(*qa), M, C, ldc, take_end(end, grid));
+  const HostDone hd = take_end(end, grid);
+  auto go = [&](const char *name, auto kernel) { launch_kernel(name, kernel, grid, dim3(NT), LDS_BYTES, s, v, qview(*qa), M, C, ldc, hd); };
+  hd.word ? go("gemm_rows_q6k_kernel<true>", gemm_rows_q6k_kernel<true>) : go("gemm_rows_q6k_kernel<false>", gemm_rows_q6k_kernel<false>);
   HIPQ_HIP(hipGetLastError());
   return HIPQ_OK;
 }

@@ -222,12 +222,16 @@ inline void launch_kernel(const char *name, void (*kernel)(KArgs...), dim3 grid,
 
 /* The end of a synchronous call on a few rows of host memory, for a product whose launch alone writes the call's outputs (the
  * kernels of gemm_rows_*.hip; the word vouches for this launch's stores only, which are past the caches and waited for, and
- * signal_done_kernel's release for those of several launches): its outputs are stored past the caches as the workgroups end (store_out), where the end of the kernel had
- * written all of them back at once, and the last workgroup writes `value` to the page-locked word that the host polls
- * (host_done), where a launch behind it did. word: null where the outputs are in device memory. us a call of page-locked rows,
- * before -> with the stores -> with both: eight rows of 12288 x 4096 Q4_K 29.6 -> 27.9 -> 27.1; before -> both: sixteen rows 44.5 ->
- * 41.0, eight of Q4_0 31.6 -> 28.6, of Q6_K 37.2 -> 32.3, two of 2000 x 1024 Q4_0 16.3 -> 15.8. The one-row kernels, whose
- * wavefronts store a few columns each, lose by it (20000 x 2048 Q4_0 18.3 -> 28.0: small writes over the bus). */
+ * signal_done_kernel's release for those of several launches): its outputs are stored past the caches as the workgroups end
+ * (store_out), where the end of the kernel had written all of them back at once, and the last workgroup writes `value` to the
+ * page-locked word that the host polls (host_done), where a launch behind it did. us a call of page-locked rows, before -> with
+ * the stores -> with both: eight rows of 12288 x 4096 Q4_K 29.6 -> 27.9 -> 27.1; before -> both: sixteen rows 44.5 -> 41.0, eight
+ * of Q4_0 31.6 -> 28.6, of Q6_K 37.2 -> 32.3, two of 2000 x 1024 Q4_0 16.3 -> 15.8. Rows that are no whole cache lines gain the
+ * same: eight of 12289 x 4096 Q4_K 29.4 -> 27.3, of 4096 x 4096 with a row stride of 4097 24.4 -> 23.4. At 257 to 264 workgroups,
+ * where one to eight CUs have a second one, both take about the same (Q4_K 2 to 4 % less, Q4_0 0 to 2 % less, Q6_K 0 to 3 % more).
+ * The one-row kernels, whose wavefronts store a few columns each, lose by it (20000 x 2048 Q4_0 18.3 -> 28.0: small writes over
+ * the bus). It is a form of the kernels of its own (HOST): the same code with a test of the word was scheduled otherwise in the
+ * device calls too, eight rows of 4096 x 12288 Q4_0 23.0 -> 24.0, sixteen of 2500 x 6144 14.2 -> 14.8. */
 struct HostDone {
   uint32_t *count = nullptr; /* device memory, zero between calls: [16 lines of 64 bytes][a line for their ends] */
   uint32_t *word = nullptr;
@@ -235,14 +239,8 @@ struct HostDone {
   uint32_t width = 0, groups = 0; /* the launch's workgroups along x, and all of them (gridDim would bring its own arguments) */
 };
 /* The device side: every workgroup of the launch calls host_done with all its lanes behind its stores. */
-__device__ __forceinline__ void store_out(float *p, float v, const HostDone &hd) {
-  if (hd.word)
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-  else
-    *p = v;
-}
+__device__ __forceinline__ void store_out(float *p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
 __device__ __forceinline__ void host_done(const HostDone &hd) {
-  if (!hd.word) return; /* uniform */
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); /* the stores have arrived in host memory */
   __syncthreads();
   if (threadIdx.x) return;
