@@ -28,7 +28,7 @@
  * Per 32 x 32 x 32 that is two matrix instructions and 16 multiply-adds, 90 clk of a SIMD by themselves
  * (210 with the int8 step).
  * Measured, kernel us, int8 kernel -> this one: 512 rows of 12288 x 4096 151 -> 62, of 3072 x 1024 14.7 -> 9.6,
- * 1024 x 1024 7.6 -> 6.7, 1024 x 3072 14.1 -> 12.0 (10.4 with two wavefronts a tile, HALF_TILES); 333 of 5000 x 2048 29 -> 14; 300 of 1000 x 896 (a K that the int8
+ * 1024 x 1024 7.6 -> 6.7, 1024 x 3072 14.1 -> 12.0 (10.4 with two wavefronts a tile); 333 of 5000 x 2048 29 -> 14; 300 of 1000 x 896 (a K that the int8
  * kernel does not take: eight-row GEMV passes) 135 us a call -> 11. At the first shape the clock falls to about
  * 1.85 GHz under this mix, and 115 clk a step at that clock are 48 us of the 62.
  *
@@ -65,12 +65,9 @@ constexpr int BM = 32, BN = 128, NT = 256;
 constexpr int PARTS = 32 * 384;     /* the activations' parts of 32 rows and one chunk: [block 8]{[64 lanes][16], [64 lanes][8]} */
 constexpr int BUF = PARTS + 32 * 16; /* a row buffer in LDS: the parts, then the block scales [32 rows][8] fp16 */
 constexpr int MAX_Y = 65535; /* of a grid */
-/* Up to so many workgroups of 32 x 128 two wavefronts share a tile (NS = 8): half of the chip's SIMDs would have no wavefront,
- * and a wavefront alone on its SIMD takes a step's vector instructions one after the other, 150 clk with sixteen sums and 115
- * with eight. us a call, a wavefront a tile / two: 512 rows of 1024 x 1024 9.8 / 9.4, x 3072 17.6 / 16.1, 100 of 4096 x 4096 17.1 / 15.2,
- * 200 of 673 x 7200 29.6 / 26.2; with more tiles the halves fill the chip twice: 192 (512 of 1536 x 2048) 13.7 / 15.0, 256 (256 of
- * 4096 x 4096) 19.3 / 23.9. */
-constexpr int HALF_TILES = 128;
+/* Whether `groups` workgroup columns of `mtiles` row tiles leave every workgroup a CU of its own: an XCD takes every eighth
+ * column with all its row tiles and has 32 CUs. */
+inline bool f6_alone(int mtiles, int64_t groups) { return mtiles * ((groups + 7) / 8) <= 32; }
 constexpr int CHUNK = hipq::F6_CHUNK, WTILE = hipq::F6_WTILE; /* bytes of 64 rows / 32 columns and one chunk */
 
 __device__ __forceinline__ rsrc_t make_rsrc(const void *p, uint32_t bytes) {
@@ -885,6 +882,7 @@ int launch_gemm_f6(int count, const hipq_weight *const *w, const QActF6 *qa, int
   if (count < 1 || count > 4) return fail(HIPQ_ERR_INVALID_ARGUMENT, "1 to 4 weights per launch, got %d", count);
   MultiF6 mw;
   int tiles = 0;
+  int64_t halves = 0; /* workgroup columns of 64, of two tiles */
   for (int i = 0; i < 4; ++i) {
     const int k = i < count ? i : count - 1;
     if (!w[k]->gf_base || w[k]->K != w[0]->K || w[k]->K != qa->K || M != qa->M)
@@ -893,7 +891,7 @@ int launch_gemm_f6(int count, const hipq_weight *const *w, const QActF6 *qa, int
     mw.N[i] = (int)w[k]->N;
     mw.C[i] = C[k];
     mw.ldc[i] = ldc[k];
-    if (i < count) tiles += (int)((w[k]->N + BN - 1) / BN);
+    if (i < count) tiles += (int)((w[k]->N + BN - 1) / BN), halves += (w[k]->N + BN / 2 - 1) / (BN / 2);
     mw.tile_end[i] = tiles; /* unused entries repeat the total: no workgroup lands in them */
   }
   mw.word = qa->word;
@@ -905,7 +903,13 @@ int launch_gemm_f6(int count, const hipq_weight *const *w, const QActF6 *qa, int
   };
   /* up to two workgroups a CU: the deeper read-ahead (512 rows of 1024 x 3072 13.1 -> 12.0 us, 1024 x 1024 7.5 -> 6.7);
    * beyond, three workgroups a CU cover the reads (512 of 12288 x 4096 67 -> 62 us) */
-  if (mtiles * (int64_t)tiles <= HALF_TILES) {
+  if (f6_alone(mtiles, halves) || (halves <= 8 && mtiles * (int64_t)tiles <= 128)) {
+    /* Two wavefronts a tile (NS = 8), where their workgroups, twice as many, still have a CU each: a wavefront alone on its SIMD
+     * takes a step's vector instructions one after the other, 150 clk with sixteen sums and 115 with eight. us a call, a
+     * wavefront a tile / two: 512 rows of 1024 x 1024 9.8 / 9.2, x 3072 17.9 / 16.8, x 12288 47.2 / 43.7, 128 of 4096 x 4096 17.3 / 15.8.
+     * With more of them the halves take a CU twice: 525 rows of 865 x 1024 10.2 / 11.0, x 7168 32.5 / 37.3, x 12288 48.3 / 56.5 (238
+     * workgroups, 34 of them on an XCD), 512 of 1536 x 2048 13.7 / 15.0. Not with up to eight workgroup columns, where an XCD has one
+     * of either kind and the halves run on twice the XCDs: 2000 of 256 x 1024 17.6 / 15.9, 4096 of 128 x 4096 66.0 / 59.4. */
     tiles = 0;
     for (int i = 0; i < 4; ++i) {
       if (i < count) tiles += (int)((w[i]->N + BN / 2 - 1) / (BN / 2));

@@ -227,8 +227,8 @@ def test_q4_0_on_six_bit_operands_matches_oracle(hipq, cr, m, n, k):
 @pytest.mark.parametrize("m,ns,k", [(128, (4096,), 288), (97, (4097,), 544), (129, (4000,), 256), (70, (33, 130, 64, 31), 800),
                                     (160, (1000, 2072), 288), (65, (64, 1, 65), 32), (512, (4096,), 256)])
 def test_q4_0_on_six_bit_operands_with_few_tiles(hipq, cr, m, ns, k):
-    """gemm_f6.hip up to 128 workgroups of 32 x 128, where two wavefronts share a tile, each with the sums of half of its
-    rows, and right above, alone and several weights a launch: columns that end inside the 64 of a workgroup and in front of
+    """gemm_f6.hip with few tiles, where two wavefronts share one, each with the sums of half of its rows, and right above
+    (f6_alone), alone and several weights a launch: columns that end inside the 64 of a workgroup and in front of
     its second tile, rows that end inside the upper and the lower half. Same bits as the reference."""
     import gpu_util as gu
     import torch
@@ -245,6 +245,27 @@ def test_q4_0_on_six_bit_operands_with_few_tiles(hipq, cr, m, ns, k):
         assert np.isnan(got[:, n:]).all()
         assert np.array_equal(gu.gpu_matmul(x, a).view(np.uint32), ref.view(np.uint32))
         x.destroy()
+
+
+@pytest.mark.parametrize("m,n,half", [(512, 1024, True), (513, 1024, False), (525, 865, False), (128, 4096, True), (128, 4097, False),
+                                      (33, 8192, True), (33, 8193, False), (1024, 512, True), (1025, 512, False), (1024, 513, False), (1300, 300, True),
+                                      (4096, 128, True), (4097, 128, False)])
+def test_q4_0_tiles_are_shared_where_their_workgroups_have_a_cu_each(hipq, cr, m, n, half):
+    """Two wavefronts a tile make twice the workgroups, of which an XCD's 32 CUs hold one each: its eighth of the
+    workgroup columns, with all row tiles, decides and not their total; up to eight columns either way are one an XCD. Both
+    sides of the lines, the reference's bits."""
+    import gpu_util as gu
+    k = 64
+    blocks = _weights(cr, "q4_0", n, k, seed=1600 + n)
+    a = synth.normal(1601 + m, (m, k))
+    w = capi.Weight("q4_0", n, k, blocks)
+    gu.gpu_matmul(w, a)  # makes the six-bit copy
+    with capi.LaunchTiming(16) as t:
+        got = gu.gpu_matmul(w, a)
+    names = [name for name, _ in t.launches if name.startswith("gemm_f6_kernel")]
+    assert len(names) == 1 and (names[0] == "gemm_f6_kernel<3, 8>") == half, names
+    assert np.array_equal(got.view(np.uint32), cr.gemm(cr.oracle(), "q4_0", a, blocks, n).view(np.uint32))
+    w.destroy()
 
 
 @pytest.mark.parametrize("kind", KINDS)
