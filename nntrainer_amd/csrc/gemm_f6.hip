@@ -136,9 +136,10 @@ __device__ __forceinline__ void f6_sums_plain(const uint8_t *wbase, int N, int c
 }
 
 /* The sums of row tile mt and the wavefront's column tile `tile` (lane (column, g), sum r: row 8 (r / 4) + 4 g + r % 4).
- * LOOK: steps an operand is read ahead of its matrix instruction, 1 or 3. NS = 8: the sums of half of the rows only; swap:
- * 16 for a wavefront whose half is the upper one, which takes the rows with the halves exchanged. */
-template <int LOOK, int NS = 16>
+ * LOOK: steps an operand is read ahead of its matrix instruction, 1 or 3. ALONE: the wavefront has a SIMD to itself. NS = 8: the
+ * sums of half of the rows only; swap: 16 for a wavefront whose half is the upper one, which takes the rows with the halves
+ * exchanged. */
+template <int LOOK, bool ALONE, int NS = 16>
 __device__ __forceinline__ void f6_sums(const uint8_t *wbase, int N, int chunks, const ActF6 &act, int mt, int tile,
                                         float (&acc)[NS], int swap = 0) {
   const uint32_t flag = act.flags[mt]; /* the same for the whole workgroup */
@@ -200,15 +201,17 @@ __device__ __forceinline__ void f6_sums(const uint8_t *wbase, int N, int chunks,
     a[st & LOOK] = v8i{a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], 0, 0};
   };
   auto read_da = [&](int k, int at) { da[k] = *(const v4h *)(smem + at + PARTS + (al & 31) * 16 + g * 8); };
-  /* Block j of the chunk whose weights are in set k. A wavefront with a SIMD of its own (LOOK = 3) has half of a step's sums
-   * between the two matrix instructions: the second waits for the first to leave the matrix core. */
+  /* Block j of the chunk whose weights are in set k. ALONE: half of a step's sums stand between the two matrix instructions,
+   * since the second waits for the first to leave the matrix core (us a call, both instructions first / so: 512 rows of 2048 x 4096
+   * 23.1 / 22.8, 525 of 865 x 7168 32.9 / 32.0). With a second wavefront on the SIMD that one has the gap, and the fences of the
+   * split cost: 512 of 4096 x 12288 73.0 / 76.9, 77 of 12288 x 7168 36.2 / 38.0. */
   auto start_d = [&](int j, int k) {
 #pragma unroll
     for (int e = 0; e < 3; ++e) b[e] = b[3 + e] = W[k][(3 * j + e) >> 2][(3 * j + e) & 3];
     b[6] = b[7] = 0;
     /* 2^4 and 2^3 make whole numbers of the units 1/16 and 1/8 */
     D[j & 1] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a[j & LOOK], b, zero16(), 3, 2, 0, 127 + 4, 0, 127 + 3);
-    if (LOOK == 3) asm volatile("" ::"v"(D[j & 1])); /* a use here: the instruction is not moved down to its sums */
+    if (ALONE) asm volatile("" ::"v"(D[j & 1])); /* a use here: the instruction is not moved down to its sums */
   };
   auto start_p = [&](int j, int k) {
     /* lane (row, g) supplies the row's scales of blocks 4 g .. 4 g + 3, lane (column, g) the column's scale of block j
@@ -238,9 +241,9 @@ __device__ __forceinline__ void f6_sums(const uint8_t *wbase, int N, int chunks,
       read_a((j + LOOK) & 7, j + LOOK < 8 ? at : at_next);
       if (j == 8 - LOOK - 1) read_da(k ^ 1, at_next);
       start_d((j + 1) & 7, j + 1 < 8 ? k : k ^ 1);
-      if (LOOK == 3) sums(j, 0, NS / 2);
+      if (ALONE) sums(j, 0, NS / 2);
       start_p((j + 1) & 7, j + 1 < 8 ? k : k ^ 1);
-      sums(j, LOOK == 3 ? NS / 2 : 0, NS);
+      sums(j, ALONE ? NS / 2 : 0, NS);
       if (j == 3) {
         /* the seven weight loads behind the next chunk's rows may be under way */
         asm volatile("s_waitcnt vmcnt(7)\n\ts_barrier" ::: "memory");
@@ -276,14 +279,14 @@ __device__ __forceinline__ void f6_sums(const uint8_t *wbase, int N, int chunks,
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
-template <int LOOK, int NS>
+template <int LOOK, bool ALONE, int NS>
 __device__ __forceinline__ void f6_tile(const uint8_t *wbase, int N, int chunks, const ActF6 &act, int M, int mt, int nt,
                                         float *__restrict__ C, int64_t ldc) {
   const int lane = threadIdx.x & 63, i32 = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int tile = NS == 16 ? nt * 4 + wave : nt * 2 + (wave & 1), swap = NS == 16 ? 0 : (wave >> 1) * 16;
   float acc[NS];
-  f6_sums<LOOK, NS>(wbase, N, chunks, act, mt, tile, acc, swap);
+  f6_sums<LOOK, ALONE, NS>(wbase, N, chunks, act, mt, tile, acc, swap);
 
   const int m0 = mt * BM + swap, n = tile * 32 + i32;
   const uint32_t off = (uint32_t)(4 * g) * (uint32_t)ldc + (uint32_t)n; /* the rest of an address is uniform */
@@ -303,9 +306,9 @@ __device__ __forceinline__ void f6_tile(const uint8_t *wbase, int N, int chunks,
  * arguments are asked for at once: each that is loaded where it is first used adds a round trip in front of the first
  * load of the tile, and so does a division by the number of row tiles (together with the stores of a whole tile without a
  * condition each, us a call: 512 rows of 2048 x 1024 10.6 -> 9.8, of 1024 x 3072 18.5 -> 17.6).
- * LOOK = 3 takes 182 registers (two workgroups a CU), LOOK = 1 fits three. NS = 8: two wavefronts a tile, half of its sums
+ * LOOK = 3 takes 184 registers, 188 ALONE and 196 with NS = 8 (two workgroups a CU), LOOK = 1 takes 163 and fits three. NS = 8: two wavefronts a tile, half of its sums
  * each, the matrix instructions twice. */
-template <int LOOK, int NS>
+template <int LOOK, bool ALONE, int NS>
 __global__ __launch_bounds__(NT, LOOK == 1 ? 3 : 2) void gemm_f6_kernel(MultiF6 mw, int chunks, ActF6 act, int M, int y0) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) asm volatile("" ::"s"(mw.w[i]), "s"(mw.C[i]), "s"(mw.ldc[i]), "s"(mw.N[i]), "s"(mw.tile_end[i]));
@@ -320,7 +323,7 @@ __global__ __launch_bounds__(NT, LOOK == 1 ? 3 : 2) void gemm_f6_kernel(MultiF6 
 #pragma unroll
   for (int i = 1; i < 4; ++i)
     if (nt >= mw.tile_end[i - 1]) w = mw.w[i], C = mw.C[i], ldc = mw.ldc[i], N = mw.N[i], begin = mw.tile_end[i - 1];
-  f6_tile<LOOK, NS>(w, N, chunks, act, M, mt, nt - begin, C, ldc);
+  f6_tile<LOOK, ALONE, NS>(w, N, chunks, act, M, mt, nt - begin, C, ldc);
   set_word(mw.word);
 }
 
@@ -390,7 +393,7 @@ struct GatedF6 {
   uint8_t *q;     /* QUANT: where the quantized rows go (QActF6) */
   uint32_t *flags, token;
 };
-template <int LOOK, bool QUANT>
+template <int LOOK, bool ALONE, bool QUANT>
 __device__ __forceinline__ void f6_gated_tile(const GatedF6 &p, int chunks, const ActF6 &act, int M, int mt, int nt) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int lane = threadIdx.x & 63, i32 = lane & 31, g = lane >> 5;
@@ -398,7 +401,7 @@ __device__ __forceinline__ void f6_gated_tile(const GatedF6 &p, int chunks, cons
   const bool second = wave >= 2;
   const int tile = nt * 2 + (wave & 1);
   float acc[16];
-  f6_sums<LOOK>(second ? p.mul : p.act, p.N, chunks, act, mt, tile, acc);
+  f6_sums<LOOK, ALONE>(second ? p.mul : p.act, p.N, chunks, act, mt, tile, acc);
 
   __syncthreads(); /* no wavefront reads or fills its row buffers any more */
   float *mine = (float *)smem + wave * 512, *other = (float *)smem + (wave ^ 2) * 512;
@@ -434,12 +437,12 @@ __device__ __forceinline__ void f6_gated_tile(const GatedF6 &p, int chunks, cons
     if (m + 4 * g < M && n < p.N) (p.out + (int64_t)m * p.ldo)[off] = h;
   }
 }
-template <int LOOK, bool QUANT>
+template <int LOOK, bool ALONE, bool QUANT>
 __global__ __launch_bounds__(NT, LOOK == 1 ? 3 : 2) void gemm_f6_gated_kernel(GatedF6 p, int chunks, ActF6 act, int M, int y0) {
   asm volatile("" ::"s"(p.act), "s"(p.mul), "s"(p.out), "s"(p.ldo), "s"(p.N), "s"(p.ntiles), "s"(p.word), "s"(p.q), "s"(p.flags),
                "s"(p.token), "s"(chunks), "s"(act.p), "s"(act.flags), "s"(act.token), "s"(M), "s"(y0));
   const int mt = (int)(blockIdx.x >> 3), nt = (int)((y0 + blockIdx.y) * 8 + (blockIdx.x & 7));
-  if (nt < p.ntiles) f6_gated_tile<LOOK, QUANT>(p, chunks, act, M, mt, nt); /* uniform per workgroup */
+  if (nt < p.ntiles) f6_gated_tile<LOOK, ALONE, QUANT>(p, chunks, act, M, mt, nt); /* uniform per workgroup */
   set_word(p.word);
 }
 
@@ -915,11 +918,13 @@ int launch_gemm_f6(int count, const hipq_weight *const *w, const QActF6 *qa, int
       if (i < count) tiles += (int)((w[i]->N + BN / 2 - 1) / (BN / 2));
       mw.tile_end[i] = tiles;
     }
-    go("gemm_f6_kernel<3, 8>", gemm_f6_kernel<3, 8>);
-  } else if (mtiles * (int64_t)tiles <= 512)
-    go("gemm_f6_kernel<3, 16>", gemm_f6_kernel<3, 16>);
+    go("gemm_f6_kernel<3, true, 8>", gemm_f6_kernel<3, true, 8>);
+  } else if (f6_alone(mtiles, tiles))
+    go("gemm_f6_kernel<3, true, 16>", gemm_f6_kernel<3, true, 16>);
+  else if (mtiles * (int64_t)tiles <= 512)
+    go("gemm_f6_kernel<3, false, 16>", gemm_f6_kernel<3, false, 16>);
   else
-    go("gemm_f6_kernel<1, 16>", gemm_f6_kernel<1, 16>);
+    go("gemm_f6_kernel<1, false, 16>", gemm_f6_kernel<1, false, 16>);
   HIPQ_HIP(hipGetLastError());
   return HIPQ_OK;
 }
@@ -937,23 +942,27 @@ int launch_gemm_f6_gated(const hipq_weight *wa, const hipq_weight *wm, const QAc
     p.q = qh->p, p.flags = qh->flags, p.token = qh->token;
   }
   const int mtiles = (M + BM - 1) / BM;
-  /* the bound of launch_gemm_f6 */
-  const bool few = (int64_t)mtiles * p.ntiles <= 512;
+  /* the bounds of launch_gemm_f6 */
+  const bool alone = f6_alone(mtiles, p.ntiles), few = (int64_t)mtiles * p.ntiles <= 512;
   auto go = [&](const char *name, auto kernel) {
     for (int y0 = 0, end = (p.ntiles + 7) / 8; y0 < end; y0 += MAX_Y)
       launch_kernel(name, kernel, dim3((unsigned)(8 * mtiles), (unsigned)std::min(end - y0, MAX_Y)), dim3(NT), 3 * BUF, s, p, qa->chunks,
                     ActF6{qa->p, qa->flags, qa->token}, M, y0);
   };
   if (qh) {
-    if (few)
-      go("gemm_f6_gated_kernel<3, true>", gemm_f6_gated_kernel<3, true>);
+    if (alone)
+      go("gemm_f6_gated_kernel<3, true, true>", gemm_f6_gated_kernel<3, true, true>);
+    else if (few)
+      go("gemm_f6_gated_kernel<3, false, true>", gemm_f6_gated_kernel<3, false, true>);
     else
-      go("gemm_f6_gated_kernel<1, true>", gemm_f6_gated_kernel<1, true>);
+      go("gemm_f6_gated_kernel<1, false, true>", gemm_f6_gated_kernel<1, false, true>);
   } else {
-    if (few)
-      go("gemm_f6_gated_kernel<3, false>", gemm_f6_gated_kernel<3, false>);
+    if (alone)
+      go("gemm_f6_gated_kernel<3, true, false>", gemm_f6_gated_kernel<3, true, false>);
+    else if (few)
+      go("gemm_f6_gated_kernel<3, false, false>", gemm_f6_gated_kernel<3, false, false>);
     else
-      go("gemm_f6_gated_kernel<1, false>", gemm_f6_gated_kernel<1, false>);
+      go("gemm_f6_gated_kernel<1, false, false>", gemm_f6_gated_kernel<1, false, false>);
   }
   HIPQ_HIP(hipGetLastError());
   return HIPQ_OK;

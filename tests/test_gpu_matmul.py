@@ -247,13 +247,16 @@ def test_q4_0_on_six_bit_operands_with_few_tiles(hipq, cr, m, ns, k):
         x.destroy()
 
 
-@pytest.mark.parametrize("m,n,half", [(512, 1024, True), (513, 1024, False), (525, 865, False), (128, 4096, True), (128, 4097, False),
-                                      (33, 8192, True), (33, 8193, False), (1024, 512, True), (1025, 512, False), (1024, 513, False), (1300, 300, True),
-                                      (4096, 128, True), (4097, 128, False)])
-def test_q4_0_tiles_are_shared_where_their_workgroups_have_a_cu_each(hipq, cr, m, n, half):
-    """Two wavefronts a tile make twice the workgroups, of which an XCD's 32 CUs hold one each: its eighth of the
-    workgroup columns, with all row tiles, decides and not their total; up to eight columns either way are one an XCD. Both
-    sides of the lines, the reference's bits."""
+@pytest.mark.parametrize("m,n,form", [
+    (512, 1024, "<3, true, 8>"), (513, 1024, "<3, true, 16>"), (525, 865, "<3, true, 16>"), (128, 4096, "<3, true, 8>"),
+    (128, 4097, "<3, true, 16>"), (33, 8192, "<3, true, 8>"), (33, 8193, "<3, true, 16>"), (1024, 512, "<3, true, 8>"),
+    (1025, 512, "<3, false, 16>"), (1024, 513, "<3, true, 16>"), (1300, 300, "<3, true, 8>"), (4096, 128, "<3, true, 8>"),
+    (4097, 128, "<3, false, 16>"), (512, 2048, "<3, true, 16>"), (513, 2048, "<3, false, 16>"), (512, 2049, "<3, false, 16>"),
+    (512, 4096, "<3, false, 16>"), (512, 4097, "<1, false, 16>")])
+def test_q4_0_tile_forms_by_an_xcds_workgroups(hipq, cr, m, n, form):
+    """gemm_f6.hip: two wavefronts a tile, and the sums between the matrix instructions, where every workgroup has a CU of its own: an
+    XCD's eighth of the workgroup columns, with all row tiles, against its 32 CUs, not their total (up to eight columns of two
+    tiles are one an XCD however many rows there are). Both sides of the lines, the reference's bits."""
     import gpu_util as gu
     k = 64
     blocks = _weights(cr, "q4_0", n, k, seed=1600 + n)
@@ -262,10 +265,35 @@ def test_q4_0_tiles_are_shared_where_their_workgroups_have_a_cu_each(hipq, cr, m
     gu.gpu_matmul(w, a)  # makes the six-bit copy
     with capi.LaunchTiming(16) as t:
         got = gu.gpu_matmul(w, a)
-    names = [name for name, _ in t.launches if name.startswith("gemm_f6_kernel")]
-    assert len(names) == 1 and (names[0] == "gemm_f6_kernel<3, 8>") == half, names
+    assert [name for name, _ in t.launches if name.startswith("gemm_f6_kernel")] == ["gemm_f6_kernel" + form]
     assert np.array_equal(got.view(np.uint32), cr.gemm(cr.oracle(), "q4_0", a, blocks, n).view(np.uint32))
     w.destroy()
+
+
+@pytest.mark.parametrize("m,n,form", [(512, 1024, "<3, true, "), (513, 1024, "<3, false, "), (512, 1056, "<3, false, "),
+                                      (1024, 1024, "<3, false, "), (1025, 1024, "<1, false, ")])
+def test_q4_0_gated_tile_forms_by_an_xcds_workgroups(hipq, cr, m, n, form):
+    """The gated pair keeps to the same lines; its result as rows and as the down projection's operand."""
+    import gpu_util as gu
+    import torch
+    k, nd = 64, 64
+    ws = [capi.Weight("q4_0", r, c, _weights(cr, "q4_0", r, c, seed=1700 + i)) for i, (r, c) in enumerate([(n, k), (n, k), (nd, n)])]
+    a = synth.normal(1701 + m, (m, k))
+    da, h, out, two = gu.dev(a), torch.empty((m, n), device="cuda"), *(torch.empty((m, nd), device="cuda") for _ in range(2))
+    for _ in range(2):  # the first calls make the six-bit copies
+        with capi.LaunchTiming(32) as t:
+            capi.mlp_swiglu(ws[0], ws[1], da, m, h, stream=gu.stream())
+            capi.mlp_swiglu_down(*ws, da, m, out, stream=gu.stream())
+        torch.cuda.synchronize()
+    assert [name for name, _ in t.launches if "gated" in name] == ["gemm_f6_gated_kernel%s%s>" % (form, q) for q in ("false", "true")]
+    y, z = gu.gpu_matmul(ws[0], a), gu.gpu_matmul(ws[1], a)
+    ref = cr.swiglu(y, z)
+    assert np.abs(h.cpu().numpy() - ref).max() <= 1e-6 * np.abs(ref).max()  # the device's expf against the host's
+    capi.matmul(ws[2], h, m, two, stream=gu.stream())
+    torch.cuda.synchronize()
+    assert torch.equal(out, two)
+    for w in ws:
+        w.destroy()
 
 
 @pytest.mark.parametrize("kind", KINDS)
