@@ -86,7 +86,7 @@ struct MultiRowsQ4K {
 
 /* blockIdx.y: the pass, rows 8 y .. 8 y + 7 of the call's M_all (the first pair_all of them under
  * the 4-row rule); the passes of one launch run side by side */
-template <bool PAIRS, bool HOST>
+template <bool PAIRS>
 __global__ __launch_bounds__(NT, PAIRS ? 2 : 3) void gemm_rows_q4k_kernel(MultiRowsQ4K mw, QView a, int M_all, int pair_all,
                                                                           hipq::HostDone hd) {
   typedef Rows<PAIRS> R;
@@ -98,8 +98,7 @@ __global__ __launch_bounds__(NT, PAIRS ? 2 : 3) void gemm_rows_q4k_kernel(MultiR
 #pragma unroll
   for (int i = 0; i < 4; ++i)
     asm volatile("" ::"s"(mw.qs[i]), "s"(mw.hdr[i]), "s"(mw.C[i]), "s"(mw.ldc[i]), "s"(mw.N[i]), "s"(mw.tile_end[i]));
-  asm volatile("" ::"s"(a.q), "s"(a.d), "s"(a.bsum), "s"(a.K), "s"(M_all), "s"(pair_all));
-  if (HOST) asm volatile("" ::"s"(hd.word));
+  asm volatile("" ::"s"(a.q), "s"(a.d), "s"(a.bsum), "s"(a.K), "s"(M_all), "s"(pair_all), "s"(hd.word));
   /* which weight this workgroup's column tile belongs to (uniform) */
   int tile = blockIdx.x, wi = 0;
   if (tile >= mw.tile_end[0]) wi = 1;
@@ -345,11 +344,14 @@ __global__ __launch_bounds__(NT, PAIRS ? 2 : 3) void gemm_rows_q4k_kernel(MultiR
     }
   }
   const int col = tile * 32 + cn;
-  if (HOST) {
-    if (cm < M && col < N) hipq::store_out(C + (int64_t)cm * ldc + col, acc - accm);
-    hipq::host_done(hd);
-  } else if (cm < M && col < N)
-    C[(int64_t)cm * ldc + col] = acc - accm;
+  if (cm < M && col < N) {
+    float *const o = C + (int64_t)cm * ldc + col;
+    if (hd.word)
+      hipq::store_out(o, acc - accm);
+    else
+      *o = acc - accm;
+  }
+  if (hd.word) hipq::host_done(hd); /* uniform */
 }
 
 } // namespace
@@ -428,16 +430,12 @@ int launch_gemm_rows_q4k_multi(int count, const hipq_weight *const *w, const QAc
     mw.tile_end[i] = tiles; /* unused entries repeat the total: no workgroup lands in them */
   }
   const dim3 grid((unsigned)tiles, (unsigned)((M + TC - 1) / TC));
-  const HostDone hd = take_end(end, grid);
-  auto go = [&](const char *name, auto kernel, size_t lds, int pairs) {
-    launch_kernel(name, kernel, grid, dim3(NT), lds, s, mw, qview(*qa), M, pairs, hd);
-  };
   if (pair_rows)
-    hd.word ? go("gemm_rows_q4k_kernel<true, true>", gemm_rows_q4k_kernel<true, true>, Rows<true>::LDS_BYTES, pair_rows)
-            : go("gemm_rows_q4k_kernel<true, false>", gemm_rows_q4k_kernel<true, false>, Rows<true>::LDS_BYTES, pair_rows);
+    hipq::launch_kernel("gemm_rows_q4k_kernel<true>", gemm_rows_q4k_kernel<true>, grid, dim3(NT), Rows<true>::LDS_BYTES, s, mw,
+                        qview(*qa), M, pair_rows, take_end(end, grid));
   else
-    hd.word ? go("gemm_rows_q4k_kernel<false, true>", gemm_rows_q4k_kernel<false, true>, Rows<false>::LDS_BYTES, 0)
-            : go("gemm_rows_q4k_kernel<false, false>", gemm_rows_q4k_kernel<false, false>, Rows<false>::LDS_BYTES, 0);
+    hipq::launch_kernel("gemm_rows_q4k_kernel<false>", gemm_rows_q4k_kernel<false>, grid, dim3(NT), Rows<false>::LDS_BYTES, s,
+                        mw, qview(*qa), M, 0, take_end(end, grid));
   HIPQ_HIP(hipGetLastError());
   return HIPQ_OK;
 }

@@ -230,8 +230,9 @@ inline void launch_kernel(const char *name, void (*kernel)(KArgs...), dim3 grid,
  * same: eight of 12289 x 4096 Q4_K 29.4 -> 27.3, of 4096 x 4096 with a row stride of 4097 24.4 -> 23.4. At 257 to 264 workgroups,
  * where one to eight CUs have a second one, both take about the same (Q4_K 2 to 4 % less, Q4_0 0 to 2 % less, Q6_K 0 to 3 % more).
  * The one-row kernels, whose wavefronts store a few columns each, lose by it (20000 x 2048 Q4_0 18.3 -> 28.0: small writes over
- * the bus). It is a form of the kernels of its own (HOST): the same code with a test of the word was scheduled otherwise in the
- * device calls too, eight rows of 4096 x 12288 Q4_0 23.0 -> 24.0, sixteen of 2500 x 6144 14.2 -> 14.8. */
+ * the bus). A form of their own (HOST) of the kernels of Q4_0 and Q6_K: one form with a test of the word was scheduled otherwise
+ * in the device calls too, eight rows of 4096 x 12288 Q4_0 23.0 -> 24.0, sixteen of 2500 x 6144 14.2 -> 14.8. The kernel of Q4_K
+ * takes the device calls 0.5 % less time with the test in it than without. */
 struct HostDone {
   uint32_t *count = nullptr; /* device memory, zero between calls: [16 lines of 64 bytes][a line for their ends] */
   uint32_t *word = nullptr;
