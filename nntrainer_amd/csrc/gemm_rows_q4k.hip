@@ -93,8 +93,8 @@ __global__ __launch_bounds__(NT, PAIRS ? 2 : 3) void gemm_rows_q4k_kernel(MultiR
   constexpr int QROW = R::QROW, ACT_Q = R::ACT_Q, ACT_AMIN = R::ACT_AMIN, ACT_BYTES = R::ACT_BYTES, LDS_REC = R::LDS_REC,
                 LDS_DW = R::LDS_DW;
   extern __shared__ __attribute__((aligned(16))) unsigned char rows_lds[];
-  /* all arguments at once: each that is loaded where it is first used adds a round trip (eight rows of 12288 x 4096 14.4 -> 13.9
-   * us, 24 of 4096 x 4096 13.2 -> 12.7) */
+  /* all arguments at once: each that is loaded where it is first used adds a round trip (calls from a graph, eight rows of
+   * 12288 x 4096 11.9 -> 11.8 us, 24 of 4096 x 4096 11.3 -> 11.1, of 12288 x 4096 26.0 -> 25.9, 48 42.7 -> 41.9) */
 #pragma unroll
   for (int i = 0; i < 4; ++i)
     asm volatile("" ::"s"(mw.qs[i]), "s"(mw.hdr[i]), "s"(mw.C[i]), "s"(mw.ldc[i]), "s"(mw.N[i]), "s"(mw.tile_end[i]));

@@ -21,8 +21,9 @@
  * beforehand. What the mins' pass reads arrives during the products too: the row sums in LDS of their own (of the first eight
  * super-blocks), the headers in the row buffer that the last super-block leaves free. With the sums copied when they were due and one
  * header under way, the pass was a chain of L2 latencies, and a workgroup has three to twelve super-blocks in all. 1000 tokens
- * of 128 experts of 2048 x 768, top 8: gate/up 103 -> 92 us, with the activation evaluated four values at a time and the outputs
- * stored without conditions, down 61 -> 52. A row's sixteen
+ * of 128 experts of 2048 x 768, top 8, traced, medians of 400 launches: gate/up 110 -> 98 us, with the activation evaluated four values
+ * at a time and the outputs stored without conditions, down 67 -> 57. What is beyond eight super-blocks of a row is
+ * copied when it is due, as all of it was: blocks of 2304 to 3072 hidden or intermediate columns take 2 to 14 % less all the same. A row's sixteen
  * 16-byte pieces are stored rotated by an exclusive-or with its number
  * (the lane asks for piece slot ^ row), which spreads the 128-bit reads of eight neighbouring rows
  * over all banks. Weights stream through registers from the expert tiles (hipq_internal.h), a
@@ -149,7 +150,7 @@ __device__ __forceinline__ void run(Lds &l, const QView &a, uint32_t a_rows, con
     HipqDigits dg;
     const float dw = hipq_h2f((uint16_t)((uint32_t)hd[0] & 0xffff));
     v16i Dlo[TM], Dhi[TM];
-    v4i av[2][TM]; /* the rows of a step are read a step ahead: a block of 1000 tokens 198.4 -> 197.7 us */
+    v4i av[2][TM]; /* the rows of a step are read a step ahead: a block of 1000 tokens 0.4 % less */
     auto read_a = [&](int j) {
       uint32_t at = abase;
       asm("" : "+v"(at)); /* one instruction a step instead of eight registers */
